@@ -125,3 +125,19 @@ def test_cpp_remove_peaks_demo(cuda, tmp_path, layers):
     else:
         exp, _ = oracle.match(pair.left, pair.right, 0, 128, peaks_ratio=0.003)
     _eq(got, exp, "demo")
+
+
+# the edges of the 64 x 16 labelling tiles: maps one pixel short of, at and
+# past them, single rows and columns, and strips that cut tiles
+@pytest.mark.parametrize("H,W,nstrips,ratio", [
+    (1, 1, 1, 1.0), (1, 200, 1, 0.05), (200, 1, 1, 0.05), (15, 63, 1, 0.01), (16, 64, 1, 0.01),
+    (17, 65, 1, 0.01), (33, 129, 1, 0.005), (33, 129, 3, 0.02), (48, 192, 5, 0.01),
+])
+@pytest.mark.parametrize("levels", [1, 3, 40])
+def test_remove_peaks_tile_edges(cuda, H, W, nstrips, ratio, levels):
+    print(f"[peaks tiles] {W}x{H} strips={nstrips} levels={levels}", flush=True)
+    rng = np.random.default_rng(1000 * H + W + levels)
+    d = _map(rng, H, W, levels, 0.3)
+    exp, _ = oracle.remove_peaks(d, nstrips, ratio)
+    got = stages.remove_peaks(torch.from_numpy(d).to(cuda), nstrips, ratio).cpu().numpy()
+    _eq(got, exp, "remove_peaks")
