@@ -72,6 +72,14 @@ int wide_min_groups() {
     return v;
 }
 
+unsigned spread_lds(int n, int used) {
+    constexpr int kLds = 160 * 1024, kUnit = 1280;   // per CU; allocation granule
+    const int cus = wide_min_groups() / 8;
+    const int want = std::max(4, (n + cus - 1) / cus);   // one per SIMD at least
+    const int bytes = kLds / want / kUnit * kUnit;
+    return bytes > used ? (unsigned)(bytes - used) : 0u;
+}
+
 // Stored-cost plans: the four directions and then the WTA, or bottom->top
 // fused with the WTA after the other three.  The fused bottom->top walk is
 // latency-bound on a small plan (about 250 ns per step), so when the
@@ -136,10 +144,11 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     const int nj = (int)jobs.size(), np = (int)posts.size();
     std::vector<int> oc(nj + 1, 0), ok(nj + 1, 0), oa(nj + 1, 0), ow(nj + 1, 0), op(np + 1, 0);
     std::vector<int> o3(nj + 1, 0), od(nj + 1, 0), w3(nj + 1, 0), wd(nj + 1, 0), wf(nj + 1, 0);
-    int dmax = 64;
-    bool wide = true;
+    int dmax = 64, dmin = kMaxD;
+    bool wide = true, big = false;
     for (int i = 0; i < nj; ++i) {
         wide = wide && wide_ok(jobs[i]);
+        big = big || wide_big(jobs[i]);
         const bool w = jobs[i].D <= 256;
         w3[i + 1] = w3[i] + (w ? wide_h_items(jobs[i]) : 0);
         wd[i + 1] = wd[i] + (w ? wide_v_items(jobs[i], kWideV) : 0);
@@ -151,6 +160,7 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
         o3[i + 1] = o3[i] + agg3_items(jobs[i]);
         od[i + 1] = od[i] + dw_items(jobs[i]);
         dmax = std::max(dmax, jobs[i].D);
+        dmin = std::min(dmin, jobs[i].D);
     }
     for (int i = 0; i < np; ++i) op[i + 1] = op[i] + post_items(posts[i]);
     const size_t s_jobs = align256(sizeof(SgmJob) * std::max(nj, 1));
@@ -209,9 +219,11 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     plan->n_wv = wd[nj];
     plan->n_wf = wf[nj];
     plan->wide = choose_wide(wide, w3[nj]);
+    plan->wide_big = big;
     plan->squarish = squarish_jobs(jobs, nj);
     plan->n_post = op[np];
     plan->dmax = dmax;
+    plan->dmin = dmin;
     return SGM_OK;
 }
 
@@ -1327,21 +1339,37 @@ int sgm_stage_aggregate_wta_otf(const uint64_t* d_census_base, const uint64_t* d
     if (!wide_ok(j))
         return fail(nullptr, SGM_E_UNSUPPORTED,
                     "the on-the-fly cost takes D <= 256 and not the 5x5 right view");
-    for (int r : {(int)kUD, (int)kLR, (int)kRL}) {
+    for (int r : {(int)kUD, (int)kLR, (int)kRL})
         if (!d_paths[r]) return fail(nullptr, SGM_E_INVALID_ARG, "NULL path pointer");
-        j.path[r] = d_paths[r];
-    }
     j.disp = d_disp;
     j.p1 = p1; j.p2 = p2;
     j.uniqueness = uniqueness;
+    // the launches keep their volumes in an order of their own: they fill
+    // temporary ones, which are then written out plainly
+    TmpPlan t;
+    const size_t vol = align256((size_t)width * height * disp_range);
+    struct TmpMem {
+        void* p = nullptr;
+        ~TmpMem() { if (p) (void)hipFree(p); }
+    } tmp;
+    HIP_TRY(nullptr, hipMalloc(&tmp.p, 3 * vol));
+    uint8_t* next = static_cast<uint8_t*>(tmp.p);
+    for (int r : {(int)kUD, (int)kLR, (int)kRL}) {
+        j.path[r] = next;
+        next += vol;
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
     // the fused WTA writes the columns from roi_x on; the ones left of them
     // are INVALID, as the WTA stage writes them
-    HIP_TRY(nullptr, launch_invalid_columns(d_disp, width, height, j.roi_x,
-                                            static_cast<hipStream_t>(stream)));
-    return run_stage(j, nullptr, [](const StagePlan& p, hipStream_t s) {
-        const hipError_t e = launch_wide3(p, s);
-        return e != hipSuccess ? e : launch_wide_wta(p, s);
-    }, stream);
+    HIP_TRY(nullptr, launch_invalid_columns(d_disp, width, height, j.roi_x, s));
+    if (int rc = upload_plan({j}, {}, &t.plan, &t.block, nullptr)) return rc;
+    HIP_TRY(nullptr, launch_wide3(t.plan, s));
+    HIP_TRY(nullptr, launch_wide_wta(t.plan, s));
+    const uint8_t* const src[4] = {j.path[0], j.path[1], nullptr, j.path[3]};
+    uint8_t* const dst[4] = {d_paths[0], d_paths[1], nullptr, d_paths[3]};
+    HIP_TRY(nullptr, launch_wide_export(j, src, dst, s));
+    HIP_TRY(nullptr, hipStreamSynchronize(s));
+    return SGM_OK;
 }
 
 int sgm_stage_wta(uint8_t* const d_paths[4], int32_t width, int32_t height,

@@ -97,6 +97,9 @@ inline int wide_v_items(const SgmJob& j, int kind) {
 }
 // Whether a job's cost can come from the census on the fly: D <= 256, and not
 // the 5x5 right view, whose skipped-pixel rule needs the stored cost.
+// Penalties whose sums leave the positive finite f16 patterns (below 0x7C00):
+// the on-the-fly kernels then take integer minima.
+inline bool wide_big(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
 inline bool wide_ok(const SgmJob& j) { return j.D <= 256 && !(j.is_right && j.cs_type == 0); }
 
 // Caller buffers bound for one launch sequence in place of the plan's own:
@@ -129,8 +132,9 @@ struct StagePlan {
     int njobs_ctw = 0;            // if > 0: jobs [0, njobs_ctw) run cost..wta
     int n_census = 0, n_cost = 0, n_agg = 0, n_wta = 0, n_post = 0, n_agg3 = 0, n_dw = 0;
     int n_wh = 0, n_wv = 0, n_wf = 0;
-    int dmax = 64;
+    int dmax = 64, dmin = 64;     // over all jobs; dmin over the matched ones
     bool wide = false;            // matching uses the on-the-fly cost kernels
+    bool wide_big = false;        // some job's penalties need their integer minima
     bool squarish = false;        // every matched job has W - roi_x <= 2.5 H
     IoBind io{};                  // host-side: bound caller buffers, if any
 };
@@ -158,11 +162,21 @@ hipError_t launch_aggregate_wta_sched(const StagePlan& p, const AggSchedule& sc,
 // Resident 64-lane workgroups per compute unit of the persistent kernels.
 hipError_t persistent_occupancy(const StagePlan& p, int* per_cu);
 hipError_t launch_reset_counters(uint32_t* counters, int n, hipStream_t s);
+// Dynamic LDS (bytes) for a launch of n single-wave workgroups that spreads
+// them evenly: the dispatcher fills a compute unit up to its occupancy before
+// the waves are even (3072 waves that fit 16 to a CU ran on 192 CUs, a third
+// slower than 12 to each of 256), so a grid that fits at once is held to
+// ceil(n / CUs) workgroups per CU by the LDS each one claims.  `used` is the
+// kernel's static LDS.
+unsigned spread_lds(int n, int used);
 // sgm_wide.hip: aggregation with the cost computed from the census words
 hipError_t launch_wide3(const StagePlan& p, hipStream_t s);
 hipError_t launch_wide_wta(const StagePlan& p, hipStream_t s);
 hipError_t launch_wide3_sched(const StagePlan& p, const AggSchedule& sc, hipStream_t s);
 hipError_t launch_wide_wta_sched(const StagePlan& p, const AggSchedule& sc, hipStream_t s);
+// direction volumes as the launches above leave them (kUD, kLR, kRL) to plain ones
+hipError_t launch_wide_export(const SgmJob& j, const uint8_t* const (&src)[4],
+                              uint8_t* const (&dst)[4], hipStream_t s);
 hipError_t wide_occupancy(const StagePlan& p, int* per_cu);
 // Process-wide SGM_COST_* mode, read when a plan is built; choose_wide
 // applies it to a plan whose views all allow the on-the-fly cost

@@ -17,13 +17,26 @@
 //     lane loads the entering word.  The window slots rotate at compile time
 //     over a 16-step unrolled block.  A direction whose window would slide the
 //     other way runs with the disparity order reversed inside the lanes (the
-//     recurrence is symmetric in d); only the byte order of its stores changes.
+//     recurrence is symmetric in d).
 //   * vertical directions load the census words of the next PF steps into
 //     registers (PF = FSGM_PF_V or FSGM_PF_F) and stage, per step, the wave's
 //     own words and the D + lines - 1 partner words into one of two LDS
 //     slots private to the (single-wave) workgroup; each lane reads its DPL
 //     partners from there.
-//   * cost(x, t) = popcount(own(x) ^ partner(x, t)): 2 v_xor + 2 v_bcnt.
+//   * cost(x, t) = popcount(own(x) ^ partner(x, t)): 2 v_xor + 2 v_bcnt, the
+//     v_bcnt accumulating onto the step's packed -m'.
+//
+// The volumes these kernels hand each other are in an order of their own
+// (wide_export_kernel undoes it for the stage entry point):
+//   * top->bottom: [H][W][D]; left->right and right->left: row tiles, the
+//     rows of one horizontal wave side by side per column
+//     ([H / lines][W][lines][D], the last tile lower), so that a step of that
+//     wave stores 1 KB in one piece instead of `lines` pieces of D bytes.  At
+//     D = 64 the pieces are half a cache line, and 32 pairs of 1242x375 took
+//     1.63 ms for the two directions against 1.27 ms (the bottom->top kernel,
+//     which reads them column by column, went from 1.34 to 1.40 ms).
+//   * a reversed direction stays reversed, and a word's bytes are in the order
+//     d, d + 2, d + 1, d + 3 (pack_lane).
 #include <algorithm>
 
 #include "sgm_device.h"
@@ -107,25 +120,62 @@ __device__ __forceinline__ uint32_t pk_min_halves(uint32_t v) {
     return as_u(__builtin_elementwise_min(as_v(v), as_v(v).yx));
 }
 
-template <int LPL, int NP>
-__device__ __forceinline__ void line_init(Line<NP>& s, const uint32_t (&c)[NP]) {
-    uint32_t t = c[0];
-#pragma unroll
-    for (int k = 0; k < NP; ++k) {
-        s.L[k] = c[k];
-        t = pk_min(t, c[k]);
+// min of three packed pairs.  Costs and penalties below 2^15 - 2^10 are
+// positive finite f16 bit patterns, which order as the integers they are, so
+// one v_pk_minimum3_f16 stands for two v_pk_min_u16 (one 4-cycle issue
+// instead of two); BIG plans (see wide_big) keep the integer form.
+template <bool BIG>
+__device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
+    if constexpr (BIG) {
+        return pk_min(pk_min(a, b), c);
+    } else {
+        uint32_t r;
+        asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return r;
     }
-    s.m = line_min<LPL>(pk_min_halves(t));
+}
+// packed minimum over N registers
+template <bool BIG, int N>
+__device__ __forceinline__ uint32_t pk_min_all(const uint32_t (&v)[N]) {
+    uint32_t t[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) t[k] = v[k];
+    int n = N;
+#pragma unroll
+    for (int round = 0; round < 4; ++round) {   // 3^4 > N
+        int o = 0;
+#pragma unroll
+        for (int k = 0; k < N; k += 3) {
+            if (k >= n) continue;
+            t[o++] = k + 2 < n ? pk_min3<BIG>(t[k], t[k + 1], t[k + 2])
+                     : k + 1 < n ? pk_min(t[k], t[k + 1]) : t[k];
+        }
+        n = o;
+    }
+    return t[0];
 }
 
-template <int LPL, int NP>
+template <bool BIG, int LPL, int NP>
+__device__ __forceinline__ void line_init(Line<NP>& s, const uint32_t (&c)[NP]) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) s.L[k] = c[k];
+    s.m = line_min<LPL>(pk_min_halves(pk_min_all<BIG>(s.L)));
+}
+
+// The sums of a step never carry or borrow between the u16 halves: costs are
+// at most 64, the line minimum is at most the cost at the previous minimum's
+// disparity (so below every term, 127 included) and P1 + P2 <= 65000.  So
+// they are 32-bit adds and subtracts, which issue in 2 cycles where the packed
+// forms take 4.
+
+template <bool BIG, int LPL, int NP>
 __device__ __forceinline__ void line_step(Line<NP>& s, const uint32_t (&c)[NP], uint32_t P1v,
                                           uint32_t P2v, bool first, bool last) {
     const uint32_t mv = s.m;
-    const uint32_t mp2 = pk_add(mv, P2v);
+    const uint32_t mp2 = mv + P2v;
     uint32_t R[NP];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) R[k] = pk_add(s.L[k], P1v);
+    for (int k = 0; k < NP; ++k) R[k] = s.L[k] + P1v;
     const uint32_t prev_last = from_prev<LPL>(R[NP - 1], 127u << 16, first);
     const uint32_t next_first = from_next<LPL>(R[0], 127u, last);
     uint32_t E[NP + 1];
@@ -133,71 +183,98 @@ __device__ __forceinline__ void line_step(Line<NP>& s, const uint32_t (&c)[NP], 
 #pragma unroll
     for (int k = 1; k < NP; ++k) E[k] = __builtin_amdgcn_alignbit(R[k], R[k - 1], 16);
     E[NP] = __builtin_amdgcn_alignbit(next_first, R[NP - 1], 16);
-    uint32_t T[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        const uint32_t b = pk_min(E[k], E[k + 1]);
-        const uint32_t v = pk_min(pk_min(s.L[k], b), mp2);
-        s.L[k] = pk_sub(pk_add(c[k], v), mv);
-        T[k] = s.L[k];
+        const uint32_t v = pk_min(pk_min3<BIG>(s.L[k], E[k], E[k + 1]), mp2);
+        s.L[k] = c[k] + v;
     }
-    // tree minimum over the pairs
-#pragma unroll
-    for (int w = 1; w < NP; w *= 2)
-#pragma unroll
-        for (int k = 0; k + w < NP; k += 2 * w) T[k] = pk_min(T[k], T[k + w]);
-    s.m = line_min<LPL>(pk_min_halves(T[0]));
+    s.m = line_min<LPL>(pk_min_halves(pk_min_all<BIG>(s.L)));
 }
 
-// the lane's 2 NP bytes (uint8 truncation) in memory order; `sel` reverses
-// the bytes of each word, `revmask` (all ones or zero, wave-uniform) the
-// order of the words.  The mask select keeps the word order a bit operation:
-// a conditional on `rev` is turned by the compiler into a per-step indexed
-// select chain.
+// The lane's 2 NP bytes (uint8 truncation).  The volumes these kernels hand
+// each other keep a word's bytes in the order d, d + 2, d + 1, d + 3, so the
+// reader gets two packed u16 pairs from a word with a 2-cycle mask and one
+// packed shift instead of two v_perm.
 template <int NP>
-__device__ __forceinline__ void pack_lane(const Line<NP>& s, uint32_t sel, uint32_t revmask,
-                                          uint32_t (&o)[NP / 2]) {
-    uint32_t w[NP / 2];
+__device__ __forceinline__ void pack_lane(const Line<NP>& s, uint32_t sel, uint32_t (&o)[NP / 2]) {
 #pragma unroll
-    for (int k = 0; k < NP / 2; ++k) w[k] = __builtin_amdgcn_perm(s.L[2 * k + 1], s.L[2 * k], sel);
-#pragma unroll
-    for (int k = 0; k < NP / 2; ++k) o[k] = (w[NP / 2 - 1 - k] & revmask) | (w[k] & ~revmask);
+    for (int k = 0; k < NP / 2; ++k) o[k] = __builtin_amdgcn_perm(s.L[2 * k + 1], s.L[2 * k], sel);
+}
+// pairs 2k and 2k + 1 of a word
+__device__ __forceinline__ uint32_t word_pair(uint32_t w, int odd) {
+    return odd ? as_u(as_v(w) >> (u16x2)8) : (w & 0x00FF00FFu);
 }
 
-constexpr uint32_t kSelFwd = 0x06040200u;   // bytes d, d+1, d+2, d+3
-constexpr uint32_t kSelRev = 0x00020406u;   // the same bytes, reversed
+constexpr uint32_t kSelFwd = 0x06020400u;   // bytes d, d+2, d+1, d+3
+// lanes that hold the disparities in reversed order swap a pair's halves, so
+// that the reader (which takes their words in reversed order) finds d before d + 1
+constexpr uint32_t kSelRev = 0x04000602u;
 
 __device__ __forceinline__ uint64_t g64(const uint64_t* p) { return gld(p); }
 
 __device__ __forceinline__ int clampcol(int p, int W) { return (p >= 0 && p < W) ? p : 0; }
 
-// value of lane lane0 + SRC (SRC < LPL) of the line, on every lane of the line
-template <int LPL>
-__device__ __forceinline__ uint32_t line_bcast(uint32_t v, int src, int lane0) {
+// value of lane `src` (a compile-time constant after unrolling) of the line,
+// on every lane of the line: quad_perm, or row_newbcast (the broadcast of one
+// lane of a 16-lane DPP row; two of them, by halves, where a line is 8 lanes)
+template <int LPL, int SRC>
+__device__ __forceinline__ uint32_t line_bcast_c(uint32_t v) {
     if constexpr (LPL == 4) {
-        switch (src) {   // quad_perm [src, src, src, src]
-            case 0: return dpp0<0x00>(v);
-            case 1: return dpp0<0x55>(v);
-            case 2: return dpp0<0xAA>(v);
-            default: return dpp0<0xFF>(v);
-        }
+        return dpp0<SRC * 0x55>(v);
+    } else if constexpr (LPL == 16) {
+        return dpp0<0x150 + SRC>(v);
     } else {
-        return (uint32_t)__builtin_amdgcn_ds_bpermute((lane0 + src) << 2, (int)v);
+        const int lo = (int)dpp0<0x150 + SRC>(v);
+        return (uint32_t)__builtin_amdgcn_update_dpp(lo, (int)v, 0x150 + SRC + 8, 0xF, 0xC, false);
     }
 }
 template <int LPL>
-__device__ __forceinline__ uint64_t line_bcast64(uint64_t v, int src, int lane0) {
-    const uint32_t lo = line_bcast<LPL>((uint32_t)v, src, lane0);
-    const uint32_t hi = line_bcast<LPL>((uint32_t)(v >> 32), src, lane0);
+__device__ __forceinline__ uint32_t line_bcast(uint32_t v, int src) {
+    switch (src) {
+        case 0: return line_bcast_c<LPL, 0>(v);
+        case 1: return line_bcast_c<LPL, 1>(v);
+        case 2: return line_bcast_c<LPL, 2>(v);
+        case 3: return line_bcast_c<LPL, 3>(v);
+        default: break;
+    }
+    if constexpr (LPL >= 8)
+        switch (src) {
+            case 4: return line_bcast_c<LPL, 4>(v);
+            case 5: return line_bcast_c<LPL, 5>(v);
+            case 6: return line_bcast_c<LPL, 6>(v);
+            case 7: return line_bcast_c<LPL, 7>(v);
+            default: break;
+        }
+    if constexpr (LPL >= 16)
+        switch (src) {
+            case 8: return line_bcast_c<LPL, 8>(v);
+            case 9: return line_bcast_c<LPL, 9>(v);
+            case 10: return line_bcast_c<LPL, 10>(v);
+            case 11: return line_bcast_c<LPL, 11>(v);
+            case 12: return line_bcast_c<LPL, 12>(v);
+            case 13: return line_bcast_c<LPL, 13>(v);
+            case 14: return line_bcast_c<LPL, 14>(v);
+            case 15: return line_bcast_c<LPL, 15>(v);
+            default: break;
+        }
+    return v;
+}
+template <int LPL>
+__device__ __forceinline__ uint64_t line_bcast64(uint64_t v, int src) {
+    const uint32_t lo = line_bcast<LPL>((uint32_t)v, src);
+    const uint32_t hi = line_bcast<LPL>((uint32_t)(v >> 32), src);
     return ((uint64_t)hi << 32) | lo;
 }
 
 // packed costs of one lane: pair k = (partner 2k, partner 2k + 1)
 template <int NP, class F>
-__device__ __forceinline__ void lane_costs(uint64_t own, F&& partner, uint32_t (&c)[NP]) {
+__device__ __forceinline__ void lane_costs(uint64_t own, uint32_t base, F&& partner, uint32_t (&c)[NP]) {
 #pragma unroll
-    for (int k = 0; k < NP; ++k)
-        c[k] = popc_acc(own ^ partner(2 * k), popc64(own ^ partner(2 * k + 1)) << 16);
+    for (int k = 0; k < NP; ++k) {
+        uint32_t t;
+        asm("v_lshl_add_u32 %0, %1, 16, %2" : "=v"(t) : "v"(popc_acc(own ^ partner(2 * k + 1), 0u)), "v"(base));
+        c[k] = popc_acc(own ^ partner(2 * k), t);
+    }
 }
 
 // ------------------------------------------------------------ horizontal ---
@@ -206,7 +283,7 @@ __device__ __forceinline__ void lane_costs(uint64_t own, F&& partner, uint32_t (
 //   p(x, t') = a + x + st * t',   and   p(x + dx, t') = p(x, t' - 1),
 // so every step the window moves up by one: lane q takes lane q-1's element
 // t' = DPL q - 1 and the line's lane 0 loads p(x, 0) = a + x.
-template <int D>
+template <int D, bool BIG>
 __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int group, int lane) {
     constexpr int DPL = wide_dpl(kWideH, D), NP = DPL / 2, LPL = D / DPL, LPW = 64 / LPL;
     const int q = lane % LPL, sub = lane / LPL;
@@ -226,11 +303,12 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
     const uint64_t* cm = J.census_other + (int64_t)y * W;
     const uint32_t P1v = (uint32_t)J.p1 * 0x10001u, P2v = (uint32_t)J.p2 * 0x10001u;
     const uint32_t sel = rev ? kSelRev : kSelFwd;
-    const uint32_t revmask = rev ? ~0u : 0u;
-    const int chunk = rev ? LPL - 1 - q : q;
     uint8_t* const out_base = (path == kLR) ? J.path[kLR] : J.path[kRL];
-    uint8_t* const dst0 = out_base + ((int64_t)y * W + x0) * D + chunk * DPL;
-    const int64_t dstep = (int64_t)dx * D;
+    // row tile: the wave's rows side by side per column
+    const int ty = group * LPW, trows = min(LPW, H - ty);
+    uint8_t* const dst0 =
+        out_base + ((int64_t)ty * W + (int64_t)x0 * trows + (y - ty)) * D + q * DPL;
+    const int64_t dstep = (int64_t)dx * trows * D;
 
     // window: slot j holds element t' = DPL q + j at the start of a block
     uint64_t win[DPL];
@@ -239,10 +317,10 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
     Line<NP> s;
     {
         uint32_t c[NP];
-        lane_costs<NP>(g64(cb + x0), [&](int j) { return win[j]; }, c);
-        line_init<LPL>(s, c);
+        lane_costs<NP>(g64(cb + x0), 0u, [&](int j) { return win[j]; }, c);
+        line_init<BIG, LPL>(s, c);
         uint32_t o[NP / 2];
-        pack_lane(s, sel, revmask, o);
+        pack_lane(s, sel, o);
         if (active) store_words<NP / 2>(dst0, o);
     }
 
@@ -251,6 +329,9 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
     // q + LPL k (k < E), and each step takes them from the line's lane
     // (step mod LPL) by a lane broadcast.  Few, early loads keep the census
     // traffic (many scattered 8-byte reads) off the step's critical path.
+    // (Refilling each slot right after its last step instead saves 16
+    // registers at D = 64 but waits for stores every LPL steps: 1.62 against
+    // 1.27 ms for 32 pairs of 1242x375.)
     constexpr int E = DPL / LPL;
     static_assert(E * LPL == DPL, "a block's steps spread evenly over the line's lanes");
     uint64_t c_own[E], c_in[E], n_own[E], n_in[E];   // this block, next block
@@ -263,7 +344,6 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
             in[k] = g64(cm + clampcol(a + x, W));
         }
     };
-    const int lane0 = lane - q;   // first lane of the line
     load_block(1, c_own, c_in);
     // blocks of DPL steps: the window slots rotate once per block
     for (int i0 = 1; i0 < n; i0 += DPL) {
@@ -271,8 +351,8 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
 #pragma unroll
         for (int sb = 0; sb < DPL; ++sb) {
             const int i = i0 + sb;
-            const uint64_t own = line_bcast64<LPL>(c_own[sb / LPL], sb % LPL, lane0);
-            const uint64_t in = line_bcast64<LPL>(c_in[sb / LPL], sb % LPL, lane0);
+            const uint64_t own = line_bcast64<LPL>(c_own[sb / LPL], sb % LPL);
+            const uint64_t in = line_bcast64<LPL>(c_in[sb / LPL], sb % LPL);
             // the slot of the leaving element t' = DPL q + DPL - 1 takes the
             // entering one; element j then sits in slot (e + j) mod DPL
             const int e = (DPL - 1 - sb) & (DPL - 1);
@@ -281,10 +361,10 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
             const uint32_t nhi = from_prev<LPL>((uint32_t)(lv >> 32), (uint32_t)(in >> 32), first);
             win[e] = ((uint64_t)nhi << 32) | nlo;
             uint32_t c[NP];
-            lane_costs<NP>(own, [&](int j) { return win[(e + j) & (DPL - 1)]; }, c);
-            line_step<LPL>(s, c, P1v, P2v, first, last);
+            lane_costs<NP>(own, 0u - s.m, [&](int j) { return win[(e + j) & (DPL - 1)]; }, c);
+            line_step<BIG, LPL>(s, c, P1v, P2v, first, last);
             uint32_t o[NP / 2];
-            pack_lane(s, sel, revmask, o);
+            pack_lane(s, sel, o);
             if (active && i < n) store_words<NP / 2>(dst0 + (int64_t)i * dstep, o);
         }
 #pragma unroll
@@ -313,7 +393,7 @@ struct VertLds {
                                             : VertGeom<64, wide_dpl(KIND, 64)>::NV;
 };
 
-template <int D, bool FUSE>
+template <int D, bool FUSE, bool BIG>
 __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int lane, uint64_t* lds,
                                               uint16_t* sums /* FUSE: [lines][D] */) {
     constexpr int KIND = FUSE ? kWideF : kWideV;
@@ -345,6 +425,23 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
     uint8_t* const out_base = FUSE ? J.path[kDU] : J.path[kUD];
 
     // census words staged for step i: lane loads v = lane + 64 r
+    // the other three directions' bytes of step i (FUSE): top->bottom by rows,
+    // the horizontal pair in the row tiles of the horizontal kernel, one of
+    // them (left->right of the right view, right->left of the left view) with
+    // the disparity order reversed
+    constexpr int TR = wide_lines(kWideH, D);
+    const uint8_t* const src_fwd = right ? J.path[kRL] : J.path[kLR];
+    const uint8_t* const src_rev = right ? J.path[kLR] : J.path[kRL];
+    auto load_others = [&](int i, uint32_t (&w)[3][NW]) __attribute__((always_inline)) {
+        const int y = y0 + dy * min(i, H - 1);
+        const int ty = y & -TR, trows = min(TR, H - ty);
+        load_words<NW>(J.path[kUD] + ((int64_t)y * W + c0) * D + loff, w[0]);
+        const int64_t to = ((int64_t)ty * W + (int64_t)c0 * trows + (y - ty)) * D;
+        const uint32_t tv = (uint32_t)((x - c0) * trows * D + q * DPL);
+        const uint32_t tr = (uint32_t)((x - c0) * trows * D + (LPL - 1 - q) * DPL);
+        load_words<NW>(src_fwd + to + tv, w[1]);
+        load_words<NW>(src_rev + to + tr, w[2]);
+    };
     auto load_step = [&](int i, uint64_t (&g)[NR]) __attribute__((always_inline)) {
         const int y = y0 + dy * min(i, H - 1);
         const uint64_t* cb = J.census + (int64_t)y * W;
@@ -362,9 +459,26 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
             if (v < NV) lds[slot * NV + v] = g[r];
         }
     };
-    auto costs = [&](int slot, uint32_t (&c)[NP]) __attribute__((always_inline)) {
+    // The fused kernel up to D = 128 reads a step's words back from LDS beside
+    // the arithmetic of the step before: 34 registers more, two waves per SIMD
+    // instead of three, and still 1.42 -> 1.39 ms for 32 pairs of 1242x375 and
+    // 3.86 -> 3.71 ms for a mixed batch.  At D = 256 (7.1 against 6.7 ms for
+    // 4800x3409) and in the top->bottom kernel (10.0 -> 10.7 ms there with the
+    // horizontal one, no change at D = 64) it does not pay.
+    constexpr bool AHEAD = FUSE && D <= 128;
+    uint64_t wo = 0, wp[AHEAD ? DPL : 1];
+    auto fetch = [&](int slot) __attribute__((always_inline)) {
+        if constexpr (AHEAD) {
+            const uint64_t* b = lds + slot * NV;
+            wo = b[kown];
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) wp[j] = right ? b[kp + j] : b[kp - j];
+        }
+    };
+    auto costs = [&](int slot, uint32_t base, uint32_t (&c)[NP]) __attribute__((always_inline)) {
         const uint64_t* b = lds + slot * NV;
-        lane_costs<NP>(b[kown], [&](int j) { return right ? b[kp + j] : b[kp - j]; }, c);
+        if constexpr (AHEAD) lane_costs<NP>(wo, base, [&](int j) { return wp[j]; }, c);
+        else lane_costs<NP>(b[kown], base, [&](int j) { return right ? b[kp + j] : b[kp - j]; }, c);
     };
 
     // WTA (FUSE): lane q < 4 of a line keeps the integer result of step
@@ -373,7 +487,6 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
     const float uthr = 1.0f - J.uniqueness;
     uint32_t kb = 0u, kboth = 0u;
     uint16_t* const sline = sums + sub * D;   // this line's sums (FUSE)
-    const uint8_t* srcs[3] = {J.path[kUD], J.path[kLR], J.path[kRL]};
     auto wta_flush = [&](int i0) __attribute__((always_inline)) {
         const int i = i0 + q;
         const int y = y0 - i;
@@ -403,24 +516,23 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             const int w = k >> 1;
-            const uint32_t a0 = (k & 1) ? bytes23(o3[0][w]) : bytes01(o3[0][w]);
-            const uint32_t a1 = (k & 1) ? bytes23(o3[1][w]) : bytes01(o3[1][w]);
-            const uint32_t a2 = (k & 1) ? bytes23(o3[2][w]) : bytes01(o3[2][w]);
+            const uint32_t a0 = word_pair(o3[0][w], k & 1), a1 = word_pair(o3[1][w], k & 1);
+            const uint32_t a2 = word_pair(o3[2][NW - 1 - w], (k & 1) ^ 1);
             S[k] = a0 + a1 + a2 + (s.L[k] & 0x00FF00FFu);   // each half <= 1020
         }
         // argmin with the smallest d: inside the lane on u16 keys S * DPL + j
-        // (S <= 4 * 255 < 2^10 and j < DPL <= 64: the keys fit in 16 bits, so
+        // (S <= 4 * 255 < 2^10 and j < DPL <= 16: the keys are below 2^14, so
         // one 32-bit v_lshl_or_b32 per pair shifts both halves without a carry
         // between them), then across the line's lanes on (S << 16) | d
-        static_assert(DPL <= 64 && (DPL & (DPL - 1)) == 0, "u16 argmin keys S * DPL + j");
+        static_assert(DPL <= 16 && (DPL & (DPL - 1)) == 0, "u16 argmin keys S * DPL + j");
         constexpr int kLog = __builtin_ctz(DPL);
-        uint32_t key = 0xFFFFFFFFu;
+        uint32_t keys[NP];
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             const uint32_t jk = (uint32_t)(2 * k) | ((uint32_t)(2 * k + 1) << 16);
-            key = pk_min(key, (S[k] << kLog) | jk);
+            keys[k] = (S[k] << kLog) | jk;
         }
-        key = pk_min_halves(key) & 0xFFFFu;
+        const uint32_t key = pk_min_halves(pk_min_all<false>(keys)) & 0xFFFFu;
         uint32_t best = ((key / DPL) << 16) | (uint32_t)(DPL * q + key % DPL);
         best = line_min<LPL>(best);
         const int ds = (int)(best & 0xFFFFu);
@@ -440,8 +552,10 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
 
     // rings (PF steps ahead) of census words and, with FUSE, of the other
     // three directions' bytes; the loop body covers BLK steps (with FUSE one
-    // 4-step WTA block)
-    constexpr int PF = FUSE ? FSGM_PF_F : FSGM_PF_V;
+    // 4-step WTA block).  The fused kernel at D = 256 looks 2 steps ahead: its
+    // 5 census words per step and lane made 179 registers, two waves per SIMD
+    // (4800x3409: 7.8 -> 6.7 ms at 139).
+    constexpr int PF = FUSE ? (D == 256 ? 2 : FSGM_PF_F) : FSGM_PF_V;
     constexpr int BLK = (PF > 4) ? PF : 4;
     static_assert(BLK % PF == 0, "the loop body must hold whole ring turns");
     static_assert(!FUSE || BLK == 4, "the WTA finishes its pixels in 4-step blocks");
@@ -458,22 +572,25 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
         load_step(1 + p, gr[p]);
-        if constexpr (FUSE) {
-#pragma unroll
-            for (int u = 0; u < 3; ++u)
-                load_words<NW>(srcs[u] + off0 + (int64_t)min(1 + p, H - 1) * ostep, pr[p][u]);
-        }
+        if constexpr (FUSE) load_others(1 + p, pr[p]);
         __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_wave_barrier();
     Line<NP> s;
     {
         uint32_t c[NP];
-        costs(0, c);
-        line_init<LPL>(s, c);
+        fetch(0);
+        costs(0, 0u, c);
+        if constexpr (AHEAD) {
+            stage(1, gr[0]);
+            load_step(1 + PF, gr[0]);
+            __builtin_amdgcn_wave_barrier();
+            fetch(1);
+        }
+        line_init<BIG, LPL>(s, c);
         if constexpr (!FUSE) {
             uint32_t o[NW];
-            pack_lane(s, kSelFwd, 0u, o);
+            pack_lane(s, kSelFwd, o);
             if (active) store_words<NW>(out_base + off0, o);
         } else {
             // row H - 1 is a border row of the WTA
@@ -488,26 +605,27 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
 #pragma unroll
         for (int b = 0; b < BLK; ++b) {
             const int i = i0 + b, p = b % PF;
-            // stage step i (slot i & 1); the other slot still holds step i - 1
-            stage(i & 1, gr[p]);
-            load_step(i + PF, gr[p]);
+            // stage step i (slot i & 1), or with AHEAD step i + 1, whose words
+            // replace those of step i once its costs are taken; the other slot
+            // still holds the step before
+            const int a = AHEAD ? 1 : 0, pa = (p + a) % PF;
+            stage((i + a) & 1, gr[pa]);
+            load_step(i + a + PF, gr[pa]);
             __builtin_amdgcn_wave_barrier();
             uint32_t c[NP];
-            costs(i & 1, c);
-            line_step<LPL>(s, c, P1v, P2v, first, last);
+            costs(i & 1, 0u - s.m, c);
+            fetch((i + 1) & 1);
+            line_step<BIG, LPL>(s, c, P1v, P2v, first, last);
             if constexpr (!FUSE) {
                 uint32_t o[NW];
-                pack_lane(s, kSelFwd, 0u, o);
+                pack_lane(s, kSelFwd, o);
                 int64_t r = row_i;
                 asm volatile("" : "+s"(r));   // keep it a scalar of its own
                 if (active && i < H) store_words<NW>(out_base + r + loff, o);
             } else {
                 // consume the slot, then refill it for step i + PF
                 wta_step(s, pr[p], i);
-                int64_t r = (i + PF <= H - 1) ? row_f : row_last;
-                asm volatile("" : "+s"(r));
-#pragma unroll
-                for (int u = 0; u < 3; ++u) load_words<NW>(srcs[u] + r + loff, pr[p][u]);
+                load_others(i + PF, pr[p]);
             }
             row_i += ostep;
             row_f += ostep;
@@ -521,7 +639,7 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
 // separate kernels: each fits 4+ waves per SIMD on its own, together they
 // would not.  Grid form: item `local` of a job is its scanline group
 // (horizontal: left->right groups, then right->left groups).
-template <int DMAX>
+template <int DMAX, bool BIG, bool ONLY>
 __global__ __launch_bounds__(64) void wide_h_kernel(const SgmJob* __restrict__ jobs,
                                                     const int* __restrict__ offs, int njobs) {
     const int item = blockIdx.x;
@@ -532,9 +650,9 @@ __global__ __launch_bounds__(64) void wide_h_kernel(const SgmJob* __restrict__ j
     const int nh = (J.H + lw - 1) / lw;
     const int path = local < nh ? kLR : kRL, group = local < nh ? local : local - nh;
     switch (J.D) {
-        case 64: wide_horizontal<64>(J, path, group, threadIdx.x); break;
-        case 128: if constexpr (DMAX >= 128) wide_horizontal<128>(J, path, group, threadIdx.x); break;
-        case 256: if constexpr (DMAX >= 256) wide_horizontal<256>(J, path, group, threadIdx.x); break;
+        case 64: if constexpr (!ONLY || DMAX == 64) wide_horizontal<64, BIG>(J, path, group, threadIdx.x); break;
+        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_horizontal<128, BIG>(J, path, group, threadIdx.x); break;
+        case 256: if constexpr (DMAX >= 256) wide_horizontal<256, BIG>(J, path, group, threadIdx.x); break;
         default: break;
     }
 }
@@ -543,7 +661,7 @@ __global__ __launch_bounds__(64) void wide_h_kernel(const SgmJob* __restrict__ j
 template <int DMAX>
 constexpr int kSumsLen = 64 * wide_dpl(kWideF, DMAX);
 
-template <int DMAX, bool FUSE>
+template <int DMAX, bool FUSE, bool BIG, bool ONLY>
 __global__ __launch_bounds__(64) void wide_v_kernel(const SgmJob* __restrict__ jobs,
                                                     const int* __restrict__ offs, int njobs) {
     __shared__ uint64_t lds[2 * VertLds<DMAX, FUSE ? kWideF : kWideV>::NV];
@@ -553,9 +671,9 @@ __global__ __launch_bounds__(64) void wide_v_kernel(const SgmJob* __restrict__ j
     const SgmJob& J = jobs[j];
     const int group = item - offs[j];
     switch (J.D) {
-        case 64: wide_vertical<64, FUSE>(J, group, threadIdx.x, lds, sums); break;
-        case 128: if constexpr (DMAX >= 128) wide_vertical<128, FUSE>(J, group, threadIdx.x, lds, sums); break;
-        case 256: if constexpr (DMAX >= 256) wide_vertical<256, FUSE>(J, group, threadIdx.x, lds, sums); break;
+        case 64: if constexpr (!ONLY || DMAX == 64) wide_vertical<64, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_vertical<128, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+        case 256: if constexpr (DMAX >= 256) wide_vertical<256, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
         default: break;
     }
 }
@@ -572,27 +690,29 @@ __device__ __forceinline__ bool next_item(const uint32_t* items, int n, uint32_t
     return true;
 }
 
-template <int DMAX>
+template <int DMAX, bool BIG>
 __global__ __launch_bounds__(64) void wide_h_persistent(const SgmJob* __restrict__ jobs,
                                                         const uint32_t* __restrict__ items, int n,
                                                         uint32_t* __restrict__ counter) {
+    constexpr bool ONLY = false;
     uint32_t it;
     while (next_item(items, n, counter, &it)) {
         const SgmJob& J = jobs[it >> 16];
         const int path = (int)((it >> 14) & 3u), group = (int)(it & 0x3FFFu);
         switch (J.D) {
-            case 64: wide_horizontal<64>(J, path, group, threadIdx.x); break;
-            case 128: if constexpr (DMAX >= 128) wide_horizontal<128>(J, path, group, threadIdx.x); break;
-            case 256: if constexpr (DMAX >= 256) wide_horizontal<256>(J, path, group, threadIdx.x); break;
+            case 64: if constexpr (!ONLY || DMAX == 64) wide_horizontal<64, BIG>(J, path, group, threadIdx.x); break;
+            case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_horizontal<128, BIG>(J, path, group, threadIdx.x); break;
+            case 256: if constexpr (DMAX >= 256) wide_horizontal<256, BIG>(J, path, group, threadIdx.x); break;
             default: break;
         }
     }
 }
 
-template <int DMAX, bool FUSE>
+template <int DMAX, bool FUSE, bool BIG>
 __global__ __launch_bounds__(64) void wide_v_persistent(const SgmJob* __restrict__ jobs,
                                                         const uint32_t* __restrict__ items, int n,
                                                         uint32_t* __restrict__ counter) {
+    constexpr bool ONLY = false;
     __shared__ uint64_t lds[2 * VertLds<DMAX, FUSE ? kWideF : kWideV>::NV];
     __shared__ __align__(16) uint16_t sums[FUSE ? kSumsLen<DMAX> : 1];
     uint32_t it;
@@ -600,20 +720,24 @@ __global__ __launch_bounds__(64) void wide_v_persistent(const SgmJob* __restrict
         const SgmJob& J = jobs[it >> 16];
         const int group = (int)(it & 0x3FFFu);
         switch (J.D) {
-            case 64: wide_vertical<64, FUSE>(J, group, threadIdx.x, lds, sums); break;
-            case 128: if constexpr (DMAX >= 128) wide_vertical<128, FUSE>(J, group, threadIdx.x, lds, sums); break;
-            case 256: if constexpr (DMAX >= 256) wide_vertical<256, FUSE>(J, group, threadIdx.x, lds, sums); break;
+            case 64: if constexpr (!ONLY || DMAX == 64) wide_vertical<64, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+            case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_vertical<128, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+            case 256: if constexpr (DMAX >= 256) wide_vertical<256, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
             default: break;
         }
     }
 }
 
+// A plan whose jobs all have one D runs the kernel of that D alone: the code
+// of several ranges in one kernel takes the registers of the largest.
 hipError_t launch_h(const StagePlan& p, hipStream_t s) {
     if (p.n_wh <= 0) return hipSuccess;
     const dim3 g(p.n_wh), b(64);
-    if (p.dmax <= 64) hipLaunchKernelGGL(wide_h_kernel<64>, g, b, 0, s, p.jobs, p.offs_wh, p.njobs);
-    else if (p.dmax <= 128) hipLaunchKernelGGL(wide_h_kernel<128>, g, b, 0, s, p.jobs, p.offs_wh, p.njobs);
-    else hipLaunchKernelGGL(wide_h_kernel<256>, g, b, 0, s, p.jobs, p.offs_wh, p.njobs);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, p.offs_wh, p.njobs); };
+    if (p.wide_big) go(wide_h_kernel<256, true, false>);
+    else if (p.dmax <= 64) go(wide_h_kernel<64, false, true>);
+    else if (p.dmin == p.dmax) p.dmax == 128 ? go(wide_h_kernel<128, false, true>) : go(wide_h_kernel<256, false, true>);
+    else p.dmax <= 128 ? go(wide_h_kernel<128, false, false>) : go(wide_h_kernel<256, false, false>);
     return hipGetLastError();
 }
 
@@ -623,12 +747,11 @@ hipError_t launch_v(const StagePlan& p, hipStream_t s) {
     const int* offs = FUSE ? p.offs_wf : p.offs_wv;
     if (n <= 0) return hipSuccess;
     const dim3 g(n), b(64);
-    if (p.dmax <= 64)
-        hipLaunchKernelGGL((wide_v_kernel<64, FUSE>), g, b, 0, s, p.jobs, offs, p.njobs);
-    else if (p.dmax <= 128)
-        hipLaunchKernelGGL((wide_v_kernel<128, FUSE>), g, b, 0, s, p.jobs, offs, p.njobs);
-    else
-        hipLaunchKernelGGL((wide_v_kernel<256, FUSE>), g, b, 0, s, p.jobs, offs, p.njobs);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs); };
+    if (p.wide_big) go(wide_v_kernel<256, FUSE, true, false>);
+    else if (p.dmax <= 64) go(wide_v_kernel<64, FUSE, false, true>);
+    else if (p.dmin == p.dmax) p.dmax == 128 ? go(wide_v_kernel<128, FUSE, false, true>) : go(wide_v_kernel<256, FUSE, false, true>);
+    else p.dmax <= 128 ? go(wide_v_kernel<128, FUSE, false, false>) : go(wide_v_kernel<256, FUSE, false, false>);
     return hipGetLastError();
 }
 
@@ -636,9 +759,10 @@ hipError_t launch_h_persistent(const StagePlan& p, const uint32_t* items, int n,
                                int grid, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const dim3 g(grid), b(64);
-    if (p.dmax <= 64) hipLaunchKernelGGL(wide_h_persistent<64>, g, b, 0, s, p.jobs, items, n, counter);
-    else if (p.dmax <= 128) hipLaunchKernelGGL(wide_h_persistent<128>, g, b, 0, s, p.jobs, items, n, counter);
-    else hipLaunchKernelGGL(wide_h_persistent<256>, g, b, 0, s, p.jobs, items, n, counter);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, items, n, counter); };
+    if (p.wide_big) go(wide_h_persistent<256, true>);
+    else if (p.dmax <= 64) go(wide_h_persistent<64, false>);
+    else p.dmax <= 128 ? go(wide_h_persistent<128, false>) : go(wide_h_persistent<256, false>);
     return hipGetLastError();
 }
 
@@ -647,13 +771,32 @@ hipError_t launch_v_persistent(const StagePlan& p, const uint32_t* items, int n,
                                int grid, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const dim3 g(grid), b(64);
-    if (p.dmax <= 64)
-        hipLaunchKernelGGL((wide_v_persistent<64, FUSE>), g, b, 0, s, p.jobs, items, n, counter);
-    else if (p.dmax <= 128)
-        hipLaunchKernelGGL((wide_v_persistent<128, FUSE>), g, b, 0, s, p.jobs, items, n, counter);
-    else
-        hipLaunchKernelGGL((wide_v_persistent<256, FUSE>), g, b, 0, s, p.jobs, items, n, counter);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, items, n, counter); };
+    if (p.wide_big) go(wide_v_persistent<256, FUSE, true>);
+    else if (p.dmax <= 64) go(wide_v_persistent<64, FUSE, false>);
+    else p.dmax <= 128 ? go(wide_v_persistent<128, FUSE, false>) : go(wide_v_persistent<256, FUSE, false>);
     return hipGetLastError();
+}
+
+// Internal direction volumes to plain [H][W][D] ones: a word's bytes back in
+// order, and for the horizontal directions (`tiled`) the row tiles and the
+// reversed disparity order of `rev` undone.
+__global__ __launch_bounds__(256) void wide_export_kernel(const uint32_t* __restrict__ src,
+                                                          uint32_t* __restrict__ dst, int W, int H,
+                                                          int D, int roi_x, int tile, int rev) {
+    const int nw = D / 4;
+    const int64_t n = (int64_t)H * W * nw;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int k = (int)(i % nw);
+        const int64_t pix = i / nw;
+        const int x = (int)(pix % W), y = (int)(pix / W);
+        if (x < roi_x) continue;   // not matched: left as it is
+        const int ty = y / tile * tile, trows = min(tile, H - ty);
+        const int64_t sp = (int64_t)ty * W + (int64_t)x * trows + (y - ty);
+        const uint32_t w = src[sp * nw + (rev ? nw - 1 - k : k)];
+        const uint32_t a = w & 0x00FF00FFu, b = (w >> 8) & 0x00FF00FFu;   // pairs (0, 1), (2, 3)
+        dst[i] = rev ? pack4(b, a) : pack4(a, b);
+    }
 }
 
 }  // namespace
@@ -679,22 +822,36 @@ hipError_t launch_wide_wta_sched(const StagePlan& p, const AggSchedule& sc, hipS
     return launch_v_persistent<true>(p, sc.items_dw, sc.ndw, sc.counters + 1, sc.grid, s);
 }
 
+hipError_t launch_wide_export(const SgmJob& j, const uint8_t* const (&src)[4],
+                              uint8_t* const (&dst)[4], hipStream_t s) {
+    const int64_t n = (int64_t)j.H * j.W * (j.D / 4);
+    const unsigned blocks = (unsigned)std::min<int64_t>((n + 255) / 256, 65535);
+    for (int r : {(int)kUD, (int)kLR, (int)kRL}) {
+        const int tile = r == kUD ? 1 : wide_lines(kWideH, j.D);
+        const int rev = r != kUD && (j.is_right != 0) != (r == kRL);
+        hipLaunchKernelGGL(wide_export_kernel, dim3(blocks), dim3(256), 0, s,
+                           reinterpret_cast<const uint32_t*>(src[r]),
+                           reinterpret_cast<uint32_t*>(dst[r]), j.W, j.H, j.D, j.roi_x, tile, rev);
+    }
+    return hipGetLastError();
+}
+
 // resident waves per CU: the smallest over the three persistent kernels
 hipError_t wide_occupancy(const StagePlan& p, int* per_cu) {
     int a = 0, b = 0, c = 0;
     hipError_t e;
     if (p.dmax <= 64) {
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<64>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<64, false>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<64, true>, 64, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<64, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<64, false, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<64, true, false>, 64, 0);
     } else if (p.dmax <= 128) {
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<128>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<128, false>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<128, true>, 64, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<128, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<128, false, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<128, true, false>, 64, 0);
     } else {
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<256>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<256, false>, 64, 0);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<256, true>, 64, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, wide_h_persistent<256, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, wide_v_persistent<256, false, false>, 64, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, wide_v_persistent<256, true, false>, 64, 0);
     }
     if (e == hipSuccess) *per_cu = std::max(1, std::min(a, std::min(b, c)));
     return e;

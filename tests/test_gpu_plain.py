@@ -126,6 +126,29 @@ def test_on_the_fly_stages_match_oracle(cuda, case):
         _eq_float(raw.cpu().numpy(), ref[f"wta_{view}"], f"raw wta {view}")
 
 
+# heights one short of, at and past the row tiles of the horizontal volumes
+# (16, 8 and 4 rows for D = 64, 128, 256), and penalties on both sides of the
+# line where the kernels change from f16 to integer minima
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("H,p1,p2", [(1, 10, 150), (3, 10, 150), (4, 20000, 10000), (7, 20000, 10001),
+                                     (9, 10, 65000 - 10), (15, 30, 30000), (17, 10, 29990)])
+def test_on_the_fly_tiles_and_penalties(cuda, D, H, p1, p2):
+    W = 41
+    print(f"[otf tiles] {W}x{H} D{D} p{p1},{p2}", flush=True)
+    rng = np.random.default_rng(D + H)
+    cl = rng.integers(0, 1 << 63, (H, W), dtype=np.uint64)
+    cr = rng.integers(0, 1 << 63, (H, W), dtype=np.uint64)
+    dev = [torch.from_numpy(c.view(np.int64)).to(cuda) for c in (cl, cr)]
+    for is_right, (b, m) in ((False, (0, 1)), (True, (1, 0))):
+        cost = oracle.cost((cl, cr)[b], (cl, cr)[m], 0, D, not is_right, 1)
+        ref = [oracle.aggregate(cost, 0, r, p1, p2) for r in range(4)]
+        paths, raw = stages.aggregate_wta_otf(dev[b], dev[m], 0, D, is_right, 1, p1, p2, UNIQ)
+        for r in (0, 1, 3):
+            np.testing.assert_array_equal(paths[r].cpu().numpy(), ref[r],
+                                          err_msg=f"path {stages.DIRS[r]}")
+        _eq_float(raw.cpu().numpy(), oracle.wta(ref, 0, 0, UNIQ), "raw wta")
+
+
 @pytest.mark.parametrize("case", CASES[:6], ids=_ids)
 @pytest.mark.parametrize("lr,median", [(True, True), (False, True), (True, False)])
 def test_stereocuda_match_matches_oracle(cuda, case, lr, median):
