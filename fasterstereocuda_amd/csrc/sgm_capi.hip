@@ -148,7 +148,7 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     bool wide = true, big = false;
     for (int i = 0; i < nj; ++i) {
         wide = wide && wide_ok(jobs[i]);
-        big = big || wide_big(jobs[i]);
+        big = big || big_penalties(jobs[i]);
         const bool w = jobs[i].D <= 256;
         w3[i + 1] = w3[i] + (w ? wide_h_items(jobs[i]) : 0);
         wd[i + 1] = wd[i] + (w ? wide_v_items(jobs[i], kWideV) : 0);
@@ -219,7 +219,8 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     plan->n_wv = wd[nj];
     plan->n_wf = wf[nj];
     plan->wide = choose_wide(wide, w3[nj]);
-    plan->wide_big = big;
+    plan->big = big;
+    plan->fast = !big;
     plan->squarish = squarish_jobs(jobs, nj);
     plan->n_post = op[np];
     plan->dmax = dmax;
@@ -1270,6 +1271,7 @@ int run_stage(const SgmJob& j, const SgmPost* post, hipError_t (*fn)(const Stage
     std::vector<SgmPost> posts;
     if (post) posts.push_back(*post);
     if (int rc = upload_plan(jobs, posts, &t.plan, &t.block, nullptr)) return rc;
+    t.plan.fast = false;   // a caller's cost volume holds any byte
     hipStream_t s = static_cast<hipStream_t>(stream);
     HIP_TRY(nullptr, fn(t.plan, s));
     HIP_TRY(nullptr, hipStreamSynchronize(s));

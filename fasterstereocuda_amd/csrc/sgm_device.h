@@ -18,6 +18,41 @@ __device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
     return as_u(__builtin_elementwise_min(as_v(a), as_v(b)));
 }
 
+// min of three packed pairs.  Costs and penalties below 2^15 - 2^10 are
+// positive finite f16 bit patterns, which order as the integers they are, so
+// one v_pk_minimum3_f16 stands for two v_pk_min_u16 (one 4-cycle issue
+// instead of two); BIG keeps the integer form (see big_penalties).
+template <bool BIG>
+__device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
+    if constexpr (BIG) {
+        return pk_min(pk_min(a, b), c);
+    } else {
+        uint32_t r;
+        asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return r;
+    }
+}
+// packed minimum over N registers
+template <bool BIG, int N>
+__device__ __forceinline__ uint32_t pk_min_all(const uint32_t (&v)[N]) {
+    uint32_t t[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) t[k] = v[k];
+    int n = N;
+#pragma unroll
+    for (int round = 0; round < 4; ++round) {   // 3^4 > N
+        int o = 0;
+#pragma unroll
+        for (int k = 0; k < N; k += 3) {
+            if (k >= n) continue;
+            t[o++] = k + 2 < n ? pk_min3<BIG>(t[k], t[k + 1], t[k + 2])
+                     : k + 1 < n ? pk_min(t[k], t[k + 1]) : t[k];
+        }
+        n = o;
+    }
+    return t[0];
+}
+
 // byte <-> packed-u16 conversions (v_perm_b32)
 __device__ __forceinline__ uint32_t bytes01(uint32_t w) { return __builtin_amdgcn_perm(0u, w, 0x0C010C00u); }
 __device__ __forceinline__ uint32_t bytes23(uint32_t w) { return __builtin_amdgcn_perm(0u, w, 0x0C030C02u); }
@@ -50,6 +85,20 @@ __device__ __forceinline__ uint32_t row_min16(uint32_t m) {
     return m;
 }
 
+constexpr int kQuadXor1 = 0xB1;        // quad_perm [1, 0, 3, 2]
+constexpr int kQuadXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
+constexpr int kRowHalfMirror = 0x141;  // lane i <-> 7 - i within 8 lanes
+constexpr int kRowMirror = 0x140;      // lane i <-> 15 - i within 16 lanes
+
+// reductions over the LPL lanes of a line (LPL = 4, 8, 16); every lane gets it
+template <int LPL>
+__device__ __forceinline__ uint32_t line_min(uint32_t v) {
+    v = min(v, dpp0<kQuadXor1>(v));
+    v = min(v, dpp0<kQuadXor2>(v));
+    if constexpr (LPL >= 8) v = min(v, dpp0<kRowHalfMirror>(v));
+    if constexpr (LPL >= 16) v = min(v, dpp0<kRowMirror>(v));
+    return v;
+}
 __device__ __forceinline__ int find_job(const int* __restrict__ offs, int n, int item) {
     int lo = 0, hi = n - 1;
     while (lo < hi) {

@@ -62,7 +62,12 @@ inline int cost_items(const SgmJob& j) { return j.H * ((j.W - j.roi_x + kCostSeg
 inline int agg_items(const SgmJob& j) { return 2 * ((j.H + 3) / 4) + 2 * ((j.W - j.roi_x + 3) / 4); }
 inline int agg3_items(const SgmJob& j) { return 2 * ((j.H + 3) / 4) + ((j.W - j.roi_x + 3) / 4); }
 inline int dw_items(const SgmJob& j) { return (j.W - j.roi_x + 3) / 4; }
-inline int wta_items(const SgmJob& j) { return j.H * ((j.W + 15) / 16); }
+// lanes per pixel of the WTA kernel (16 disparities a lane, 32 for D = 512)
+__host__ __device__ constexpr int wta_lpp(int D) { return D <= 256 ? D / 16 : 16; }
+inline int wta_items(const SgmJob& j) {
+    const int px = 256 / wta_lpp(j.D);
+    return j.H * ((j.W + px - 1) / px);
+}
 inline int post_items(const SgmPost& p) { return ((p.W + 63) / 64) * ((p.H + 15) / 16); }
 // On-the-fly cost aggregation (sgm_wide.hip).  Each kernel holds DPL
 // disparities per lane, so a scanline takes D / DPL lanes (at most one
@@ -98,8 +103,8 @@ inline int wide_v_items(const SgmJob& j, int kind) {
 // Whether a job's cost can come from the census on the fly: D <= 256, and not
 // the 5x5 right view, whose skipped-pixel rule needs the stored cost.
 // Penalties whose sums leave the positive finite f16 patterns (below 0x7C00):
-// the on-the-fly kernels then take integer minima.
-inline bool wide_big(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
+// the aggregation then takes integer minima.
+inline bool big_penalties(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
 inline bool wide_ok(const SgmJob& j) { return j.D <= 256 && !(j.is_right && j.cs_type == 0); }
 
 // Caller buffers bound for one launch sequence in place of the plan's own:
@@ -134,7 +139,8 @@ struct StagePlan {
     int n_wh = 0, n_wv = 0, n_wf = 0;
     int dmax = 64, dmin = 64;     // over all jobs; dmin over the matched ones
     bool wide = false;            // matching uses the on-the-fly cost kernels
-    bool wide_big = false;        // some job's penalties need their integer minima
+    bool big = false;             // some job's penalties need integer minima
+    bool fast = false;            // not big, and every cost is a census distance (at most 64)
     bool squarish = false;        // every matched job has W - roi_x <= 2.5 H
     IoBind io{};                  // host-side: bound caller buffers, if any
 };

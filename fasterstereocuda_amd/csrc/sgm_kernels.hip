@@ -240,7 +240,85 @@ __global__ __launch_bounds__(256) void cost_kernel(const SgmJob* __restrict__ jo
 // stored directions + this one's value mod 256, argmin with the smallest d,
 // c1 / c3 gathered with one row OR-reduction, then the reference's
 // uniqueness and subpixel rules (see wta_pixel below).
-template <int D, bool FUSE>
+//
+// A lone wave issues an instruction every 4 to 5 cycles whatever it is, and
+// the long scanlines of one pair run about one wave per SIMD, so a step costs
+// its instruction count (a D = 64 step of 48 instructions and its waits took
+// 115 ns, this one of 33 takes 82 ns: 1242x375, both views, three directions
+// 142 -> 102 us).  Hence:
+//   * loads and stores are buffer accesses, a wave-uniform base per block of
+//     PF steps plus a scalar offset per step: no vector address arithmetic;
+//   * every step stores, so the wait counts are exact and a step waits only
+//     for the load issued PF steps earlier, not for its recent stores (and the
+//     fused form, whose loads are issued after a step's arithmetic, has PF = 8
+//     at D = 64 and 128: at 4 and 2, 1920x1080 D = 128 took 0.64 ms).  The
+//     lines of a last, partial group past the region repeat its last line:
+//     the same bytes to the same place;
+//   * the pads of the lane shifts stay in the shifts' destination registers,
+//     whose out-of-row lanes no shift writes;
+//   * FAST (costs of at most 64, P1 + P2 <= 30000): no sum carries or borrows
+//     between u16 halves, so sums are 32-bit, and values are positive finite
+//     f16 patterns, so two minima are one v_pk_minimum3_f16.
+
+// Where a block of up to PF steps starts and how its steps lie from there:
+// byte offset `base` of its lowest address, the scalar offset of its first
+// step, the step's change and the offset of its far end (steps past the
+// line's last stay on it).
+struct BlockWalk {
+    int64_t base;
+    int s, inc, last;
+};
+__device__ __forceinline__ BlockWalk block_walk(int64_t first, int64_t step, int j, int count, int n) {
+    const int jc = min(j, n - 1), km = min(count - 1, n - 1 - jc);
+    const int st = (int)(step < 0 ? -step : step);
+    BlockWalk w;
+    w.last = km * st;
+    w.base = first + (int64_t)(step < 0 ? jc + km : jc) * step;
+    w.s = step < 0 ? w.last : 0;
+    w.inc = (int)step;
+    return w;
+}
+
+typedef unsigned int buf_u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int buf_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const uint8_t* p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, 0x7fffffff, 0x00020000);
+}
+template <int NW>
+__device__ __forceinline__ void buf_load(__amdgpu_buffer_rsrc_t r, uint32_t v, int s, uint32_t (&w)[NW]) {
+    if constexpr (NW == 1) {
+        w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)v, s, 0);
+    } else if constexpr (NW == 2) {
+        const buf_u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, s, 0);
+        w[0] = t.x; w[1] = t.y;
+    } else {
+#pragma unroll
+        for (int k = 0; k < NW; k += 4) {
+            const buf_u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(v + 4 * k), s, 0);
+            w[k] = t.x; w[k + 1] = t.y; w[k + 2] = t.z; w[k + 3] = t.w;
+        }
+    }
+}
+// A 128-bit store takes its step offset in the vector offset: with a scalar
+// offset register the compiler leaves the data registers free to be rewritten
+// by the next instruction, and under load such stores have written the later
+// values (D = 256 beside two larger pairs); without one it keeps the wait
+// state that stores of more than 64 bits need.
+template <int NW>
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t v, int s, const uint32_t (&w)[NW]) {
+    if constexpr (NW == 1) {
+        __builtin_amdgcn_raw_buffer_store_b32(w[0], r, (int)v, s, 0);
+    } else if constexpr (NW == 2) {
+        __builtin_amdgcn_raw_buffer_store_b64(buf_u32x2{w[0], w[1]}, r, (int)v, s, 0);
+    } else {
+#pragma unroll
+        for (int k = 0; k < NW; k += 4)
+            __builtin_amdgcn_raw_buffer_store_b128(buf_u32x4{w[k], w[k + 1], w[k + 2], w[k + 3]}, r,
+                                                   (int)(v + 4 * k + s), 0, 0);
+    }
+}
+
+template <int D, bool FUSE, bool FAST>
 __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, int lane) {
     constexpr int DPD = D / 16;   // disparities per lane
     constexpr int NW = DPD / 4;   // u32 words of cost per lane
@@ -254,40 +332,61 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
     const bool active = line < nlines;
     if (!active) line = nlines - 1;
     const int n = horiz ? (W - roi_x) : H;
-    int64_t x0, y0, step;
-    if (horiz) {
-        y0 = line; x0 = fwd ? roi_x : W - 1; step = fwd ? D : -D;
-    } else {
-        x0 = roi_x + line; y0 = fwd ? 0 : H - 1;
-        step = fwd ? (int64_t)W * D : -(int64_t)W * D;
-    }
-    // Addresses = wave-uniform base (first line of the group, scalar
-    // registers) + a small per-lane offset, so the per-step part of every
-    // address is scalar arithmetic.
+    // first column (horizontal) or row (vertical) of the lines, wave-uniform
+    const int xs = fwd ? roi_x : W - 1, ys = fwd ? 0 : H - 1;
+    const int64_t x0 = horiz ? xs : roi_x + line, y0 = horiz ? line : ys;
+    const int64_t step = (fwd ? 1 : -1) * (horiz ? (int64_t)D : (int64_t)W * D);
+    // Addresses = wave-uniform base (first line of the group) + a small
+    // per-lane offset + a scalar offset per step.
     const int line0 = group * 4;
-    const int64_t offL = horiz ? ((int64_t)line0 * W + x0) * D
-                               : (y0 * W + roi_x + line0) * D;
+    const int64_t offL = horiz ? ((int64_t)line0 * W + xs) * D
+                               : ((int64_t)ys * W + roi_x + line0) * D;
     const uint32_t voff = (uint32_t)((line - line0) * (horiz ? W * D : D) + l * DPD);
-    const uint8_t* const src0 = J.cost + offL;
     uint8_t* const out_base = (path == 0) ? J.path[0] : (path == 1) ? J.path[1]
                             : (path == 2) ? J.path[2] : J.path[3];
-    uint8_t* const dst0 = out_base + offL;
     const uint32_t P1v = (uint32_t)J.p1 * 0x10001u;
     const uint32_t P2v = (uint32_t)J.p2 * 0x10001u;
     const float uthr = 1.0f - J.uniqueness;
     const int min_d = J.min_d;
+    auto add = [](uint32_t a, uint32_t b) __attribute__((always_inline)) { return FAST ? a + b : pk_add(a, b); };
+    auto sub2 = [](uint32_t a, uint32_t b) __attribute__((always_inline)) { return FAST ? a - b : pk_sub(a, b); };
 
-    uint32_t w[NW];
-    load_words<NW>(src0 + voff, w);
+    // Register ring of prefetched words (the cost, and with FUSE the three
+    // other directions).  Slot p holds step i0 + p of the current block.
+    constexpr int NSRC = FUSE ? 4 : 1;
+    constexpr int PF = FUSE ? (NW == 1 ? 8 : 16 / NW) : (NW >= 2 ? 32 / NW : 16);
+    const uint8_t* srcs[4] = {J.cost, J.path[0], J.path[1], J.path[3]};
+    uint32_t buf[PF][NSRC][NW];
+
     uint32_t L[NP];
+    uint32_t m;   // the line minimum in both u16 halves
+    auto line_minimum = [&]() __attribute__((always_inline)) {
+        const uint32_t t = pk_min_all<!FAST>(L);
+        return row_min16(as_u(__builtin_elementwise_min(as_v(t), as_v(t).yx)));
+    };
+    {
+        const BlockWalk w0 = block_walk(offL, step, 0, 1, n);
+        uint32_t w[NW];
+        buf_load<NW>(buf_at(srcs[0] + w0.base), voff, w0.s, w);
+        // the ring's slots in the loop's own order (the scheduler may not
+        // interleave them): the wait counts at the loop head are the merge of
+        // both paths, and any other order collapses them to zero
+        __builtin_amdgcn_sched_barrier(0);
+        const BlockWalk b = block_walk(offL, step, 1, PF, n);
+        int so = b.s;
 #pragma unroll
-    for (int k = 0; k < NW; ++k) { L[2 * k] = bytes01(w[k]); L[2 * k + 1] = bytes23(w[k]); }
-    if (active && !FUSE) store_words<NW>(dst0 + (int64_t)0 + voff, w);
-    if (FUSE && active && l == 0) gst(J.disp + y0 * W + x0, kInvalidDisp);   // row H-1: border
-    uint32_t t0 = L[0];
+        for (int p = 0; p < PF; ++p) {
 #pragma unroll
-    for (int k = 1; k < NP; ++k) t0 = pk_min(t0, L[k]);
-    uint32_t m = row_min16(min(t0 & 0xFFFFu, t0 >> 16));
+            for (int q = 0; q < NSRC; ++q) buf_load<NW>(buf_at(srcs[q] + b.base), voff, so, buf[p][q]);
+            so = max(min(so + b.inc, b.last), 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int k = 0; k < NW; ++k) { L[2 * k] = bytes01(w[k]); L[2 * k + 1] = bytes23(w[k]); }
+        if constexpr (!FUSE) buf_store<NW>(buf_at(out_base + w0.base), voff, w0.s, w);
+        else if (active && l == 0) gst(J.disp + y0 * W + x0, kInvalidDisp);   // row H-1: border
+        m = line_minimum();
+    }
 
     // WTA of the pixel at step i from this direction's L and the other three
     // stored directions (FUSE only).  The integer part (sum, argmin with the
@@ -359,117 +458,100 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
         if (l == ((i - 1) & 15)) { kb = best; kboth = both; }
     };
 
-    // one recurrence step: consumes the cost words of step i, updates L, m
-    auto advance = [&](const uint32_t (&c8)[NW], int i) __attribute__((always_inline)) {
-        const uint32_t mv = m * 0x10001u;
-        const uint32_t mp2 = pk_add(mv, P2v);
+    // one recurrence step: consumes the cost words of a step, updates L, m
+    uint32_t prev_last = 127u << 16, next_first = 127u;
+    auto advance = [&](const uint32_t (&c8)[NW]) __attribute__((always_inline)) {
+        const uint32_t mp2 = add(m, P2v);
         uint32_t R[NP];
 #pragma unroll
-        for (int k = 0; k < NP; ++k) R[k] = pk_add(L[k], P1v);
-        // neighbours across lanes; lane 0 / lane 15 of a row get the 127 term
-        const uint32_t prev_last = dpp<kRowShr1>(127u << 16, R[NP - 1]);
-        const uint32_t next_first = dpp<kRowShl1>(127u, R[0]);
+        for (int k = 0; k < NP; ++k) R[k] = add(L[k], P1v);
+        // neighbours across lanes; lane 0 / lane 15 of a row keep the 127 term
+        prev_last = dpp<kRowShr1>(prev_last, R[NP - 1]);
+        next_first = dpp<kRowShl1>(next_first, R[0]);
         uint32_t E[NP + 1];
         E[0] = __builtin_amdgcn_alignbit(R[0], prev_last, 16);
 #pragma unroll
         for (int k = 1; k < NP; ++k) E[k] = __builtin_amdgcn_alignbit(R[k], R[k - 1], 16);
         E[NP] = __builtin_amdgcn_alignbit(next_first, R[NP - 1], 16);
-        uint32_t t = 0xFFFFFFFFu;
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             const uint32_t c = (k & 1) ? bytes23(c8[k >> 1]) : bytes01(c8[k >> 1]);
-            const uint32_t b = pk_min(E[k], E[k + 1]);
-            const uint32_t v = pk_min(pk_min(L[k], b), mp2);
-            L[k] = pk_sub(pk_add(c, v), mv);
-            t = pk_min(t, L[k]);
+            const uint32_t v = pk_min(pk_min3<!FAST>(L[k], E[k], E[k + 1]), mp2);
+            L[k] = add(sub2(c, m), v);
         }
-        if constexpr (!FUSE) {
-            uint32_t o[NW];
+        m = line_minimum();
+    };
+    auto pack = [&](uint32_t (&o)[NW]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < NW; ++k) o[k] = pack4(L[2 * k], L[2 * k + 1]);
-            if (active) store_words<NW>(dst0 + (int64_t)i * step + voff, o);
-        }
-        m = row_min16(min(t & 0xFFFFu, t >> 16));
+        for (int k = 0; k < NW; ++k) o[k] = pack4(L[2 * k], L[2 * k + 1]);
     };
 
-    // Register ring of prefetched words (the cost, and with FUSE the three
-    // other directions), about 64 bytes per lane in flight so a wave covers
-    // many steps of memory latency.  Slot p holds step base + p; refills are
-    // unconditional, clamped to the last step.
-    constexpr int NSRC = FUSE ? 4 : 1;
-    constexpr int PF = FUSE ? ((NW >= 4) ? 2 : 4 / NW) : ((NW >= 8) ? 2 : 16 / NW);
-    const uint8_t* srcs[4] = {src0, J.path[0] + offL, J.path[1] + offL, J.path[3] + offL};
-    uint32_t buf[PF][NSRC][NW];
-    // The prologue issues the slots in the loop's own order (the scheduler
-    // may not interleave them): the wait counts at the loop head are the
-    // merge of both paths, and any other order collapses them to zero.
+    // Blocks of PF steps, refilling each slot with the step PF later (the last
+    // one again near the end of the line), then the steps left over.
+    int i = 1;
+    if constexpr (!FUSE) {
+        for (; i + PF <= n; i += PF) {
+            const BlockWalk in = block_walk(offL, step, i + PF, PF, n);
+            const BlockWalk out = block_walk(offL, step, i, PF, n);
+            const auto rin = buf_at(srcs[0] + in.base);
+            const auto rout = buf_at(out_base + out.base);
+            int si = in.s, so = out.s;
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
+            for (int p = 0; p < PF; ++p) {
+                advance(buf[p][0]);
+                buf_load<NW>(rin, voff, si, buf[p][0]);
+                uint32_t o[NW];
+                pack(o);
+                buf_store<NW>(rout, voff, so, o);
+                si = max(min(si + in.inc, in.last), 0);
+                so += out.inc;
+            }
+        }
+        const BlockWalk out = block_walk(offL, step, i, PF, n);
+        const auto rout = buf_at(out_base + out.base);
+        int so = out.s;
 #pragma unroll
-        for (int q = 0; q < NSRC; ++q)
-            load_words<NW>(srcs[q] + (int64_t)min(1 + p, n - 1) * step + voff, buf[p][q]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    auto consume = [&](uint32_t (&cur)[NSRC][NW], int i) __attribute__((always_inline)) {
-        advance(cur[0], i);
-        if constexpr (FUSE) {
+        for (int p = 0; p < PF - 1; ++p) {
+            if (i + p < n) {
+                advance(buf[p][0]);
+                uint32_t o[NW];
+                pack(o);
+                buf_store<NW>(rout, voff, so, o);
+                so += out.inc;
+            }
+        }
+    } else {
+        auto consume = [&](const uint32_t (&cur)[NSRC][NW], int at) __attribute__((always_inline)) {
+            advance(cur[0]);
             uint32_t other[3][NW];
 #pragma unroll
             for (int q = 0; q < 3; ++q)
 #pragma unroll
                 for (int k = 0; k < NW; ++k) other[q][k] = cur[q + 1][k];
-            wta_step(other, i);
-        }
-    };
-    // Steps i .. i + PF - 1, refilling each slot with step + PF (clamped to
-    // step n - 1 near the end of the line).  Without FUSE the refill offsets
-    // come from one multiply per turn and scalar adds / selects, so each load
-    // adds a scalar offset to the lane's loop-invariant address instead of a
-    // 64-bit multiply-add per load.  The fused kernel keeps the multiply: the
-    // scalar form gives it four 64-bit lane bases and 37 more VGPRs, and its
-    // larger plans run slower at the lower occupancy.
-    const int64_t last_off = (int64_t)(n - 1) * step;
-    auto ring_turn = [&](int i) __attribute__((always_inline)) {
-        int64_t so = (int64_t)(i + PF) * step;
+            wta_step(other, at);
+        };
+        auto turn = [&](int at) __attribute__((always_inline)) {
+            const BlockWalk in = block_walk(offL, step, at + PF, PF, n);
+            int si = in.s;
 #pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            uint32_t cur[NSRC][NW];
+            for (int p = 0; p < PF; ++p) {
+                consume(buf[p], at + p);
 #pragma unroll
-            for (int q = 0; q < NSRC; ++q)
-#pragma unroll
-                for (int k = 0; k < NW; ++k) cur[q][k] = buf[p][q][k];
-            int64_t o;
-            if constexpr (FUSE) {
-                o = (int64_t)min(i + p + PF, n - 1) * step;
-            } else {
-                o = (i + p + PF <= n - 1) ? so : last_off;
-                asm volatile("" : "+s"(o));   // keep it a scalar of its own
+                for (int q = 0; q < NSRC; ++q) buf_load<NW>(buf_at(srcs[q] + in.base), voff, si, buf[p][q]);
+                si = max(min(si + in.inc, in.last), 0);
             }
-#pragma unroll
-            for (int q = 0; q < NSRC; ++q) load_words<NW>(srcs[q] + o + voff, buf[p][q]);
-            so += step;
-            consume(cur, i + p);
-        }
-    };
-    int i = 1;
-    if constexpr (FUSE) {
+        };
         // blocks of 16 steps (steps 16b + 1 .. 16b + 16), then their pixels
         constexpr int kUnroll = (D <= 128) ? 16 / PF : 1;
         for (; i + 16 <= n; i += 16) {
 #pragma unroll kUnroll
-            for (int s0 = 0; s0 < 16; s0 += PF) ring_turn(i + s0);
+            for (int s0 = 0; s0 < 16; s0 += PF) turn(i + s0);
             wta_flush(i, 16);
         }
-    } else {
-        for (; i + PF <= n; i += PF) ring_turn(i);
-    }
-    for (; i < n; ++i) {
-        uint32_t cur[NSRC][NW];
+        for (; i + PF <= n; i += PF) turn(i);
 #pragma unroll
-        for (int q = 0; q < NSRC; ++q) load_words<NW>(srcs[q] + (int64_t)i * step + voff, cur[q]);
-        consume(cur, i);
-    }
-    if constexpr (FUSE) {
+        for (int p = 0; p < PF - 1; ++p)
+            if (i + p < n) consume(buf[p], i + p);
         // pixels of the last, partial block of 16 steps
         const int last = (n - 2) & 15;   // slot of step n - 1
         if (n > 1 && last != 15) wta_flush(n - 1 - last, last + 1);
@@ -478,7 +560,8 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
 
 // MODE 0: all four directions (stage entry point); MODE 1: left->right,
 // right->left, top->bottom; MODE 2: bottom->top fused with the WTA.
-template <int DMAX, int MODE>
+// ONLY: every job has D = DMAX (other ranges' code would take its registers).
+template <int DMAX, int MODE, bool FAST, bool ONLY>
 __global__ __launch_bounds__(64) void aggregate_kernel(const SgmJob* __restrict__ jobs,
                                                        const int* __restrict__ offs, int njobs) {
     const int item = blockIdx.x;
@@ -496,10 +579,10 @@ __global__ __launch_bounds__(64) void aggregate_kernel(const SgmJob* __restrict_
     const int lane = threadIdx.x;
     constexpr bool F = (MODE == 2);
     switch (J.D) {
-        case 64: agg_lines<64, F>(J, path, group, lane); break;
-        case 128: if constexpr (DMAX >= 128) agg_lines<128, F>(J, path, group, lane); break;
-        case 256: if constexpr (DMAX >= 256) agg_lines<256, F>(J, path, group, lane); break;
-        case 512: if constexpr (DMAX >= 512) agg_lines<512, F>(J, path, group, lane); break;
+        case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST>(J, path, group, lane); break;
+        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) agg_lines<128, F, FAST>(J, path, group, lane); break;
+        case 256: if constexpr (ONLY ? DMAX == 256 : DMAX >= 256) agg_lines<256, F, FAST>(J, path, group, lane); break;
+        case 512: if constexpr (ONLY ? DMAX == 512 : DMAX >= 512) agg_lines<512, F, FAST>(J, path, group, lane); break;
         default: break;
     }
 }
@@ -508,7 +591,7 @@ __global__ __launch_bounds__(64) void aggregate_kernel(const SgmJob* __restrict_
 // packed items (job << 16 | direction << 14 | group) from a device counter
 // until the list is exhausted; every wave leaves through that one test.  The
 // list order is the scanline schedule (e.g. longest scanlines first).
-template <int DMAX, int MODE>
+template <int DMAX, int MODE, bool FAST>
 __global__ __launch_bounds__(64) void aggregate_persistent_kernel(
     const SgmJob* __restrict__ jobs, const uint32_t* __restrict__ items, int n_items,
     uint32_t* __restrict__ counter) {
@@ -523,10 +606,10 @@ __global__ __launch_bounds__(64) void aggregate_persistent_kernel(
         const SgmJob& J = jobs[it >> 16];
         const int path = (int)((it >> 14) & 3u), group = (int)(it & 0x3FFFu);
         switch (J.D) {
-            case 64: agg_lines<64, F>(J, path, group, lane); break;
-            case 128: if constexpr (DMAX >= 128) agg_lines<128, F>(J, path, group, lane); break;
-            case 256: if constexpr (DMAX >= 256) agg_lines<256, F>(J, path, group, lane); break;
-            case 512: if constexpr (DMAX >= 512) agg_lines<512, F>(J, path, group, lane); break;
+            case 64: agg_lines<64, F, FAST>(J, path, group, lane); break;
+            case 128: if constexpr (DMAX >= 128) agg_lines<128, F, FAST>(J, path, group, lane); break;
+            case 256: if constexpr (DMAX >= 256) agg_lines<256, F, FAST>(J, path, group, lane); break;
+            case 512: if constexpr (DMAX >= 512) agg_lines<512, F, FAST>(J, path, group, lane); break;
             default: break;
         }
     }
@@ -538,41 +621,41 @@ __global__ void reset_counters_kernel(uint32_t* c, int n) {
 
 // ------------------------------------------------------------------- wta ---
 // cusgm_ca.cu:3606-3699 (D=64), :3701-3809 (D=128), :3149-3232 (generic),
-// SubPixBias :150-154.  16 lanes per pixel, D/16 disparities per lane.
-// argmin ties -> smallest d (key = S << 16 | d).
+// SubPixBias :150-154.  A pixel takes wta_lpp(D) lanes of 16 disparities (32
+// for D = 512): one 16-byte load per direction and lane, and the float rules
+// on one lane in 4 (D = 64) instead of one in 16 (450x375, both views: 20.5 ->
+// 15.7 us).  argmin ties -> smallest d.
 template <int D>
-__device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int l,
-                                          uint16_t* __restrict__ s) {
-    constexpr int DPD = D / 16, NW = DPD / 4, NP = DPD / 2;
+__device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int q, uint16_t* __restrict__ s) {
+    constexpr int LPP = wta_lpp(D), DPL = D / LPP, NW = DPL / 4, NP = DPL / 2;
     const bool inimg = x < J.W;
     const int xc = inimg ? x : J.W - 1;
-    const int64_t off = ((int64_t)y * J.W + xc) * D + l * DPD;
-    uint32_t S[NP];
+    const int64_t off = ((int64_t)y * J.W + xc) * D + q * DPL;
+    uint32_t w[4][NW];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) S[k] = 0u;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        uint32_t w[NW];
-        load_words<NW>(J.path[r] + off, w);
-#pragma unroll
-        for (int k = 0; k < NW; ++k) {
-            S[2 * k] = pk_add(S[2 * k], bytes01(w[k]));
-            S[2 * k + 1] = pk_add(S[2 * k + 1], bytes23(w[k]));
-        }
-    }
-    uint32_t best = 0xFFFFFFFFu;
+    for (int r = 0; r < 4; ++r) load_words<NW>(J.path[r] + off, w[r]);
+    // pair 2k = (S(4k), S(4k + 2)), pair 2k + 1 = (S(4k + 1), S(4k + 3)): at
+    // most 4 x 255 per half, so the sums are 32-bit and the keys S * DPL + j
+    // (j the disparity inside the lane) fit the halves, below 2^15
+    constexpr int kLog = __builtin_ctz(DPL);
+    uint32_t S[NP], keys[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        const uint32_t d0 = (uint32_t)(l * DPD + 2 * k);
-        best = min(best, (S[k] << 16) | d0);
-        best = min(best, (S[k] & 0xFFFF0000u) | (d0 + 1));
+        const int i = k >> 1, o = k & 1;
+        auto half = [&](uint32_t v) { return o ? as_u(as_v(v) >> (u16x2)8) : (v & 0x00FF00FFu); };
+        S[k] = half(w[0][i]) + half(w[1][i]) + half(w[2][i]) + half(w[3][i]);
+        keys[k] = (S[k] << kLog) | (uint32_t)((4 * i + o) | ((4 * i + o + 2) << 16));
     }
-    best = row_min16(best);
+    const uint32_t t = pk_min_all<false>(keys);
+    const uint32_t key = min(t & 0xFFFFu, t >> 16);
+    uint32_t best = ((key >> kLog) << 16) | (uint32_t)(DPL * q + (int)(key & (DPL - 1)));
+    best = line_min<LPP>(best);
     uint32_t* s32 = reinterpret_cast<uint32_t*>(s);
 #pragma unroll
-    for (int k = 0; k < NP; ++k) s32[l * NP + k] = S[k];
+    for (int k = 0; k < NP; ++k) s32[q * NP + k] = S[k];
     __syncthreads();
-    if (l == 0 && inimg) {
+    auto sum_at = [&](int d) { return (float)s[(d & ~3) | ((d & 1) << 1) | ((d >> 1) & 1)]; };
+    if (q == 0 && inimg) {
         // rows are counted in the job; the border is the image's (the frame)
         const int W = J.fW ? J.fW : J.W, H = J.fW ? J.fH : J.H;
         const int xi = x + J.fx0, yi = y + J.fy0;
@@ -583,9 +666,9 @@ __device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int l,
             const uint32_t c2 = best >> 16;
             const int ds = (int)(best & 0xFFFFu);
             if (ds > 0 && (warp_rule || ds < D - 1)) {
-                const float c1 = (float)s[ds - 1];
+                const float c1 = sum_at(ds - 1);
                 const float c2f = (float)c2;
-                const float c3 = (ds == D - 1) ? (float)(D - 1) : (float)s[ds + 1];
+                const float c3 = (ds == D - 1) ? (float)(D - 1) : sum_at(ds + 1);
                 const float a = c1 - c2f, b = c3 - c2f;
                 const float uniq = (a < b) ? a : b;
                 const float ut = 1.0f - J.uniqueness;
@@ -605,20 +688,28 @@ __device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int l,
 template <int DMAX>
 __global__ __launch_bounds__(256) void wta_kernel(const SgmJob* __restrict__ jobs,
                                                   const int* __restrict__ offs, int njobs) {
-    __shared__ __align__(16) uint16_t sS[16][DMAX];
+    // the sums of 256 / LPP pixels: 16 per thread (32 for D = 512)
+    __shared__ __align__(16) uint16_t sums[256 * (DMAX <= 256 ? 16 : 32)];
     const int item = blockIdx.x;
     const int j = find_job(offs, njobs, item);
     const SgmJob& J = jobs[j];
     const int local = item - offs[j];
-    const int segs = (J.W + 15) / 16;
-    const int y = local / segs;
-    const int pix = threadIdx.x >> 4, l = threadIdx.x & 15;
-    const int x = (local - y * segs) * 16 + pix;
+    const int px = 256 / wta_lpp(J.D), segs = (J.W + px - 1) / px;
+    const int y = local / segs, x0 = (local - y * segs) * px;
+    const int tid = threadIdx.x;
     switch (J.D) {
-        case 64: wta_pixel<64>(J, x, y, l, sS[pix]); break;
-        case 128: if constexpr (DMAX >= 128) wta_pixel<128>(J, x, y, l, sS[pix]); break;
-        case 256: if constexpr (DMAX >= 256) wta_pixel<256>(J, x, y, l, sS[pix]); break;
-        case 512: if constexpr (DMAX >= 512) wta_pixel<512>(J, x, y, l, sS[pix]); break;
+#define FSGM_WTA_CASE(DD)                                                                   \
+    case DD:                                                                                \
+        if constexpr (DMAX >= DD) {                                                         \
+            constexpr int LPP = wta_lpp(DD);                                                \
+            wta_pixel<DD>(J, x0 + tid / LPP, y, tid % LPP, sums + (tid / LPP) * DD);        \
+        }                                                                                   \
+        break;
+        FSGM_WTA_CASE(64)
+        FSGM_WTA_CASE(128)
+        FSGM_WTA_CASE(256)
+        FSGM_WTA_CASE(512)
+#undef FSGM_WTA_CASE
         default: break;
     }
 }
@@ -837,14 +928,17 @@ template <int MODE>
 static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const dim3 g(n), b(64);
-    if (p.dmax <= 64)
-        hipLaunchKernelGGL((aggregate_kernel<64, MODE>), g, b, 0, s, p.jobs, offs, p.njobs);
-    else if (p.dmax <= 128)
-        hipLaunchKernelGGL((aggregate_kernel<128, MODE>), g, b, 0, s, p.jobs, offs, p.njobs);
-    else if (p.dmax <= 256)
-        hipLaunchKernelGGL((aggregate_kernel<256, MODE>), g, b, 0, s, p.jobs, offs, p.njobs);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs); };
+    if (!p.fast) go(aggregate_kernel<512, MODE, false, false>);
+    else if (p.dmax <= 64) go(aggregate_kernel<64, MODE, true, true>);
+    else if (p.dmin == p.dmax)
+        p.dmax == 128 ? go(aggregate_kernel<128, MODE, true, true>)
+                      : p.dmax == 256 ? go(aggregate_kernel<256, MODE, true, true>)
+                                      : go(aggregate_kernel<512, MODE, true, true>);
     else
-        hipLaunchKernelGGL((aggregate_kernel<512, MODE>), g, b, 0, s, p.jobs, offs, p.njobs);
+        p.dmax == 128 ? go(aggregate_kernel<128, MODE, true, false>)
+                      : p.dmax == 256 ? go(aggregate_kernel<256, MODE, true, false>)
+                                      : go(aggregate_kernel<512, MODE, true, false>);
     return hipGetLastError();
 }
 
@@ -865,14 +959,12 @@ static hipError_t launch_persistent_mode(const StagePlan& p, const uint32_t* ite
                                          uint32_t* counter, int grid, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const dim3 g(grid), b(64);
-    if (p.dmax <= 64)
-        hipLaunchKernelGGL((aggregate_persistent_kernel<64, MODE>), g, b, 0, s, p.jobs, items, n, counter);
-    else if (p.dmax <= 128)
-        hipLaunchKernelGGL((aggregate_persistent_kernel<128, MODE>), g, b, 0, s, p.jobs, items, n, counter);
-    else if (p.dmax <= 256)
-        hipLaunchKernelGGL((aggregate_persistent_kernel<256, MODE>), g, b, 0, s, p.jobs, items, n, counter);
-    else
-        hipLaunchKernelGGL((aggregate_persistent_kernel<512, MODE>), g, b, 0, s, p.jobs, items, n, counter);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, items, n, counter); };
+    if (!p.fast) go(aggregate_persistent_kernel<512, MODE, false>);
+    else if (p.dmax <= 64) go(aggregate_persistent_kernel<64, MODE, true>);
+    else if (p.dmax <= 128) go(aggregate_persistent_kernel<128, MODE, true>);
+    else if (p.dmax <= 256) go(aggregate_persistent_kernel<256, MODE, true>);
+    else go(aggregate_persistent_kernel<512, MODE, true>);
     return hipGetLastError();
 }
 
@@ -896,12 +988,12 @@ hipError_t launch_aggregate_wta_sched(const StagePlan& p, const AggSchedule& sc,
 template <int MODE>
 static hipError_t occ_mode(int dmax, int* n) {
     if (dmax <= 64)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<64, MODE>, 64, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<64, MODE, true>, 64, 0);
     if (dmax <= 128)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<128, MODE>, 64, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<128, MODE, true>, 64, 0);
     if (dmax <= 256)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<256, MODE>, 64, 0);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<512, MODE>, 64, 0);
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<256, MODE, true>, 64, 0);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, aggregate_persistent_kernel<512, MODE, true>, 64, 0);
 }
 
 hipError_t persistent_occupancy(const StagePlan& p, int* per_cu) {

@@ -57,20 +57,6 @@ namespace {
 
 using namespace dev;
 
-constexpr int kQuadXor1 = 0xB1;        // quad_perm [1, 0, 3, 2]
-constexpr int kQuadXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
-constexpr int kRowHalfMirror = 0x141;  // lane i <-> 7 - i within 8 lanes
-constexpr int kRowMirror = 0x140;      // lane i <-> 15 - i within 16 lanes
-
-// reductions over the LPL lanes of a line (LPL = 4, 8, 16); every lane gets it
-template <int LPL>
-__device__ __forceinline__ uint32_t line_min(uint32_t v) {
-    v = min(v, dpp0<kQuadXor1>(v));
-    v = min(v, dpp0<kQuadXor2>(v));
-    if constexpr (LPL >= 8) v = min(v, dpp0<kRowHalfMirror>(v));
-    if constexpr (LPL >= 16) v = min(v, dpp0<kRowMirror>(v));
-    return v;
-}
 // value of the previous / next lane of the line; the line's first / last
 // lane gets `edge`
 template <int LPL>
@@ -118,41 +104,6 @@ struct Line {
 // a u32 minimum of such values is their u16 minimum
 __device__ __forceinline__ uint32_t pk_min_halves(uint32_t v) {
     return as_u(__builtin_elementwise_min(as_v(v), as_v(v).yx));
-}
-
-// min of three packed pairs.  Costs and penalties below 2^15 - 2^10 are
-// positive finite f16 bit patterns, which order as the integers they are, so
-// one v_pk_minimum3_f16 stands for two v_pk_min_u16 (one 4-cycle issue
-// instead of two); BIG plans (see wide_big) keep the integer form.
-template <bool BIG>
-__device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
-    if constexpr (BIG) {
-        return pk_min(pk_min(a, b), c);
-    } else {
-        uint32_t r;
-        asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-        return r;
-    }
-}
-// packed minimum over N registers
-template <bool BIG, int N>
-__device__ __forceinline__ uint32_t pk_min_all(const uint32_t (&v)[N]) {
-    uint32_t t[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) t[k] = v[k];
-    int n = N;
-#pragma unroll
-    for (int round = 0; round < 4; ++round) {   // 3^4 > N
-        int o = 0;
-#pragma unroll
-        for (int k = 0; k < N; k += 3) {
-            if (k >= n) continue;
-            t[o++] = k + 2 < n ? pk_min3<BIG>(t[k], t[k + 1], t[k + 2])
-                     : k + 1 < n ? pk_min(t[k], t[k + 1]) : t[k];
-        }
-        n = o;
-    }
-    return t[0];
 }
 
 template <bool BIG, int LPL, int NP>
@@ -734,7 +685,7 @@ hipError_t launch_h(const StagePlan& p, hipStream_t s) {
     if (p.n_wh <= 0) return hipSuccess;
     const dim3 g(p.n_wh), b(64);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, p.offs_wh, p.njobs); };
-    if (p.wide_big) go(wide_h_kernel<256, true, false>);
+    if (p.big) go(wide_h_kernel<256, true, false>);
     else if (p.dmax <= 64) go(wide_h_kernel<64, false, true>);
     else if (p.dmin == p.dmax) p.dmax == 128 ? go(wide_h_kernel<128, false, true>) : go(wide_h_kernel<256, false, true>);
     else p.dmax <= 128 ? go(wide_h_kernel<128, false, false>) : go(wide_h_kernel<256, false, false>);
@@ -748,7 +699,7 @@ hipError_t launch_v(const StagePlan& p, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const dim3 g(n), b(64);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs); };
-    if (p.wide_big) go(wide_v_kernel<256, FUSE, true, false>);
+    if (p.big) go(wide_v_kernel<256, FUSE, true, false>);
     else if (p.dmax <= 64) go(wide_v_kernel<64, FUSE, false, true>);
     else if (p.dmin == p.dmax) p.dmax == 128 ? go(wide_v_kernel<128, FUSE, false, true>) : go(wide_v_kernel<256, FUSE, false, true>);
     else p.dmax <= 128 ? go(wide_v_kernel<128, FUSE, false, false>) : go(wide_v_kernel<256, FUSE, false, false>);
@@ -760,7 +711,7 @@ hipError_t launch_h_persistent(const StagePlan& p, const uint32_t* items, int n,
     if (n <= 0) return hipSuccess;
     const dim3 g(grid), b(64);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, items, n, counter); };
-    if (p.wide_big) go(wide_h_persistent<256, true>);
+    if (p.big) go(wide_h_persistent<256, true>);
     else if (p.dmax <= 64) go(wide_h_persistent<64, false>);
     else p.dmax <= 128 ? go(wide_h_persistent<128, false>) : go(wide_h_persistent<256, false>);
     return hipGetLastError();
@@ -772,7 +723,7 @@ hipError_t launch_v_persistent(const StagePlan& p, const uint32_t* items, int n,
     if (n <= 0) return hipSuccess;
     const dim3 g(grid), b(64);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, items, n, counter); };
-    if (p.wide_big) go(wide_v_persistent<256, FUSE, true>);
+    if (p.big) go(wide_v_persistent<256, FUSE, true>);
     else if (p.dmax <= 64) go(wide_v_persistent<64, FUSE, false>);
     else p.dmax <= 128 ? go(wide_v_persistent<128, FUSE, false>) : go(wide_v_persistent<256, FUSE, false>);
     return hipGetLastError();
