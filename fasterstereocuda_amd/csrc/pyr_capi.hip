@@ -166,10 +166,12 @@ sgm_pyramid* build_pyramid(int32_t width, int32_t height, int32_t num_layers, in
     p->top_min = dmin; p->top_range = range;
     // memory
     const bool lr = opt->do_lr_check != 0;
+    const int pad = mid_pad(range, dmin);   // of the coarsest level's census rows
     size_t total = 0;
     for (int i = 0; i < layers; ++i) {
         const size_t npix = (size_t)p->lw[i] * p->lh[i];
-        total += 2 * a256(npix) + 2 * a256(npix * 8) + 2 * a256(npix * 4);
+        const size_t ncensus = census_words(p->lw[i], p->lh[i], i == top ? pad : 0);
+        total += 2 * a256(npix) + 2 * a256(ncensus * 8) + 2 * a256(npix * 4);
         if (i == top) total += (lr ? 2 : 1) * 5 * a256(npix * range) + a256(npix * 4);
         else total += a256(npix * 2) + 5 * a256(npix * level_range);
     }
@@ -192,8 +194,10 @@ sgm_pyramid* build_pyramid(int32_t width, int32_t height, int32_t num_layers, in
     for (int i = 0; i < layers; ++i) {
         const size_t npix = (size_t)p->lw[i] * p->lh[i];
         p->il[i] = take(npix); p->ir[i] = take(npix);
-        p->cl[i] = reinterpret_cast<uint64_t*>(take(npix * 8));
-        p->cr[i] = reinterpret_cast<uint64_t*>(take(npix * 8));
+        const int cp = i == top ? pad : 0;
+        const size_t ncensus = census_words(p->lw[i], p->lh[i], cp);
+        p->cl[i] = reinterpret_cast<uint64_t*>(take(ncensus * 8)) + cp;
+        p->cr[i] = reinterpret_cast<uint64_t*>(take(ncensus * 8)) + cp;
         p->out[i] = reinterpret_cast<float*>(take(npix * 4));
         p->raw[i] = reinterpret_cast<float*>(take(npix * 4));
     }
@@ -207,6 +211,13 @@ sgm_pyramid* build_pyramid(int32_t width, int32_t height, int32_t num_layers, in
             SgmJob j = census_job(v ? p->ir[top] : p->il[top], v ? p->cr[top] : p->cl[top],
                                   v ? p->cl[top] : p->cr[top], w, h, opt->cs_type, v);
             j.D = range; j.min_d = dmin; j.roi_x = std::max(0, dmin);
+            j.cpitch = w + 2 * pad; j.cpad = pad;
+            if (pad > 0 && (fill_census_pads(j, p->stream) != hipSuccess ||
+                            hipStreamSynchronize(p->stream) != hipSuccess)) {
+                set_global_error(SGM_E_HIP, "pyramid: census pads");
+                free_pyramid(p);
+                return nullptr;
+            }
             j.p1 = opt->p1; j.p2 = opt->p2_init;
             j.uniqueness = (top > 0) ? 1.0f : opt->unique_threshold;
             if (v == 0 || lr) {

@@ -80,19 +80,26 @@ unsigned spread_lds(int n, int used) {
     return bytes > used ? (unsigned)(bytes - used) : 0u;
 }
 
+int waves_per_group(int n, int limit) {
+    const int simds = wide_min_groups() / 2;   // 4 per CU
+    return 2 * n > simds && 4 * n <= limit * simds ? 4 : 1;
+}
+
 // Stored-cost plans: the four directions and then the WTA, or bottom->top
 // fused with the WTA after the other three.  The fused bottom->top walk is
-// latency-bound on a small plan (about 250 ns per step), so when the
-// four-direction launch leaves the device at 2.5 waves per SIMD or fewer the
-// walk is better run beside the horizontal ones and the WTA left to its own
-// memory-bound launch -- unless the rows are much longer than the columns:
-// then the fused walk is short and the extra launch costs more than it saves
-// (measured on single pairs from 450x375 to 1920x1080).
+// latency-bound on a small plan, so it is better run beside the horizontal
+// ones (and the WTA left to its own memory-bound launch) while the four
+// directions have at most 2.5 waves per SIMD and the extra volume's traffic is
+// small: up to 200M cells, or 100M where the rows are much longer than the
+// columns and the fused walk is short (both views, separate / fused:
+// 1242x375 D = 64, 60M: 185 / 211 us; 640x480 D = 128, 79M: 240 / 268;
+// 1242x375 D = 128, 119M: 416 / 336; 1200x852, 131M: 405 / 429; 1280x720
+// D = 128, 236M: 643 / 626).
 bool separate_wta(const StagePlan& p) {
     const int f = g_wta_form.load();
     if (f == SGM_WTA_FUSED) return false;
     if (f == SGM_WTA_SEPARATE) return true;
-    return p.squarish && 4 * p.n_agg <= 5 * wide_min_groups();
+    return 4 * p.n_agg <= 5 * wide_min_groups() && p.cells <= (p.squarish ? 200000000 : 100000000);
 }
 
 bool squarish_jobs(const std::vector<SgmJob>& jobs, int n) {
@@ -105,6 +112,19 @@ bool choose_wide(bool eligible, int n_wh) {
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED) return false;
     return mode == SGM_COST_ON_THE_FLY || n_wh >= wide_min_groups();
+}
+
+// The 4-line on-the-fly form moves 6 bytes per cell where the stored cost
+// takes 11, but issues about 1.6 times the instructions per step: it wins once
+// memory, not the scanlines' serial steps, bounds the stored form (both views,
+// stored / on the fly: 1280x720 D = 128, 236M cells: 626 / 669 us; 1117x573
+// D = 256, 328M: 880 / 821; 1920x1080 D = 128, 531M: 1290 / 1100; 2400x1704
+// D = 256, 2.1G: 5.5 / 4.2 ms).
+constexpr int64_t kMidCells = 250000000;
+bool choose_mid(bool eligible, int n_wh, int64_t cells) {
+    const int mode = cost_mode();
+    if (!eligible || mode == SGM_COST_STORED || n_wh >= wide_min_groups()) return false;
+    return mode == SGM_COST_ON_THE_FLY || cells >= kMidCells;
 }
 }  // namespace fsgm
 
@@ -139,16 +159,26 @@ int check_option(const sgm_option* o, std::string* err, bool allow_peaks) {
 }  // namespace
 
 // Uploads jobs / posts and the per-stage item tables into one device block.
-int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost>& posts,
+int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmPost>& posts,
                 StagePlan* plan, void** block, std::string* err) {
+    std::vector<SgmJob> jobs(jobs_in);
+    for (SgmJob& j : jobs)
+        if (!j.cpitch) j.cpitch = j.W;
     const int nj = (int)jobs.size(), np = (int)posts.size();
     std::vector<int> oc(nj + 1, 0), ok(nj + 1, 0), oa(nj + 1, 0), ow(nj + 1, 0), op(np + 1, 0);
     std::vector<int> o3(nj + 1, 0), od(nj + 1, 0), w3(nj + 1, 0), wd(nj + 1, 0), wf(nj + 1, 0);
+    std::vector<int> m3(nj + 1, 0), mf(nj + 1, 0);
     int dmax = 64, dmin = kMaxD;
-    bool wide = true, big = false;
+    bool wide = true, big = false, mid = true, quirk = false;
+    int64_t cells = 0;
     for (int i = 0; i < nj; ++i) {
         wide = wide && wide_ok(jobs[i]);
         big = big || big_penalties(jobs[i]);
+        mid = mid && mid_ok(jobs[i]);
+        quirk = quirk || mid_specials(jobs[i]) > 0;
+        cells += (int64_t)(jobs[i].W - jobs[i].roi_x) * jobs[i].H * jobs[i].D;
+        m3[i + 1] = m3[i] + mid3_items(jobs[i]);
+        mf[i + 1] = mf[i] + mid_v_items(jobs[i]);
         const bool w = jobs[i].D <= 256;
         w3[i + 1] = w3[i] + (w ? wide_h_items(jobs[i]) : 0);
         wd[i + 1] = wd[i] + (w ? wide_v_items(jobs[i], kWideV) : 0);
@@ -167,7 +197,7 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     const size_t s_posts = align256(sizeof(SgmPost) * std::max(np, 1));
     const size_t s_oj = align256(sizeof(int) * (nj + 1));
     const size_t s_op = align256(sizeof(int) * (np + 1));
-    const size_t total = s_jobs + s_posts + 9 * s_oj + s_op;
+    const size_t total = s_jobs + s_posts + 11 * s_oj + s_op;
     std::vector<uint8_t> host(total, 0);
     size_t off = 0;
     auto put = [&](const void* src, size_t n, size_t slot) {
@@ -187,6 +217,8 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     const size_t a_w3 = put(w3.data(), sizeof(int) * (nj + 1), s_oj);
     const size_t a_wd = put(wd.data(), sizeof(int) * (nj + 1), s_oj);
     const size_t a_wf = put(wf.data(), sizeof(int) * (nj + 1), s_oj);
+    const size_t a_m3 = put(m3.data(), sizeof(int) * (nj + 1), s_oj);
+    const size_t a_mf = put(mf.data(), sizeof(int) * (nj + 1), s_oj);
     const size_t a_op = put(op.data(), sizeof(int) * (np + 1), s_op);
     if (*block) {
         (void)hipFree(*block);
@@ -206,6 +238,8 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     plan->offs_wh = reinterpret_cast<int*>(b + a_w3);
     plan->offs_wv = reinterpret_cast<int*>(b + a_wd);
     plan->offs_wf = reinterpret_cast<int*>(b + a_wf);
+    plan->offs_m3 = reinterpret_cast<int*>(b + a_m3);
+    plan->offs_mf = reinterpret_cast<int*>(b + a_mf);
     plan->offs_post = reinterpret_cast<int*>(b + a_op);
     plan->njobs = nj;
     plan->nposts = np;
@@ -218,7 +252,12 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
     plan->n_wh = w3[nj];
     plan->n_wv = wd[nj];
     plan->n_wf = wf[nj];
+    plan->n_m3 = m3[nj];
+    plan->n_mf = mf[nj];
     plan->wide = choose_wide(wide, w3[nj]);
+    plan->mid = choose_mid(mid, w3[nj], cells);
+    plan->cells = cells;
+    plan->quirk = quirk;
     plan->big = big;
     plan->fast = !big;
     plan->squarish = squarish_jobs(jobs, nj);
@@ -233,9 +272,17 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs, const std::vector<SgmPost
 void fsgm::restrict_matching(StagePlan* P, const std::vector<SgmJob>& jobs, int n) {
     P->njobs_ctw = n;
     P->n_cost = P->n_agg = P->n_wta = P->n_agg3 = P->n_dw = P->n_wh = P->n_wv = P->n_wf = 0;
-    bool wide = true;
+    P->n_m3 = P->n_mf = 0;
+    bool wide = true, mid = true;
+    int64_t cells = 0;
+    P->quirk = false;
     for (int i = 0; i < n; ++i) {
         wide = wide && wide_ok(jobs[i]);
+        mid = mid && mid_ok(jobs[i]);
+        P->quirk = P->quirk || mid_specials(jobs[i]) > 0;
+        cells += (int64_t)(jobs[i].W - jobs[i].roi_x) * jobs[i].H * jobs[i].D;
+        P->n_m3 += mid3_items(jobs[i]);
+        P->n_mf += mid_v_items(jobs[i]);
         if (jobs[i].D <= 256) {
             P->n_wh += wide_h_items(jobs[i]);
             P->n_wv += wide_v_items(jobs[i], kWideV);
@@ -248,6 +295,8 @@ void fsgm::restrict_matching(StagePlan* P, const std::vector<SgmJob>& jobs, int 
         P->n_dw += dw_items(jobs[i]);
     }
     P->wide = choose_wide(wide, P->n_wh);
+    P->mid = choose_mid(mid, P->n_wh, cells);
+    P->cells = cells;
     P->squarish = squarish_jobs(jobs, n);
 }
 
@@ -264,10 +313,13 @@ hipError_t fsgm::launch_match(const StagePlan& plan, bool right_invalidation, hi
     if ((e = launch_census(plan, s)) != hipSuccess) return e;
     if ((e = mark(1)) != hipSuccess) return e;
     // with the on-the-fly cost there is no cost volume to build
-    if (!plan.wide && (e = launch_cost(ctw, s)) != hipSuccess) return e;
+    const bool mid = plan.mid && !sched;
+    if (!plan.wide && !mid && (e = launch_cost(ctw, s)) != hipSuccess) return e;
     if ((e = mark(2)) != hipSuccess) return e;
-    const bool separate = !plan.wide && !sched && separate_wta(ctw);
-    if (plan.wide)
+    const bool separate = !plan.wide && !mid && !sched && separate_wta(ctw);
+    if (mid)
+        e = launch_mid3(ctw, s);
+    else if (plan.wide)
         e = sched ? launch_wide3_sched(ctw, *sched, s) : launch_wide3(ctw, s);
     else if (separate)
         e = launch_aggregate(ctw, s);
@@ -275,7 +327,9 @@ hipError_t fsgm::launch_match(const StagePlan& plan, bool right_invalidation, hi
         e = sched ? launch_aggregate_sched(ctw, *sched, s) : launch_aggregate3(ctw, s);
     if (e != hipSuccess) return e;
     if ((e = mark(3)) != hipSuccess) return e;
-    if (plan.wide)
+    if (mid)
+        e = launch_mid_wta(ctw, s);
+    else if (plan.wide)
         e = sched ? launch_wide_wta_sched(ctw, *sched, s) : launch_wide_wta(ctw, s);
     else if (separate)
         e = launch_wta(ctw, s);
@@ -302,6 +356,7 @@ struct sgm_handle {
     bool inited = false;
     int device = -1;
     int32_t W = 0, H = 0, min_d = 0, D = 0;
+    int32_t cpad = 0;             // census pad words per side (from Init's min_d)
     // D = LEVEL_RANGE (32): the handle matches around an initial disparity
     // map only (window cost, window aggregation, window WTA), as the
     // reference's finer pyramid levels do (FasterStereoCuda.cpp:282-289, 455-469)
@@ -322,9 +377,9 @@ struct sgm_handle {
 
 namespace {
 
-size_t arena_bytes(int W, int H, int D) {
-    const size_t npix = (size_t)W * H, ncell = npix * D;
-    return 2 * (align256(npix) + align256(npix * 8) + 5 * align256(ncell) + 2 * align256(npix * 4)) +
+size_t arena_bytes(int W, int H, int D, int cpad) {
+    const size_t npix = (size_t)W * H, ncell = npix * D, ncensus = census_words(W, H, cpad);
+    return 2 * (align256(npix) + align256(ncensus * 8) + 5 * align256(ncell) + 2 * align256(npix * 4)) +
            align256(npix * 2);
 }
 
@@ -335,7 +390,7 @@ void carve(sgm_handle* h) {
     for (int v = 0; v < 2; ++v) {
         ViewBuffers& b = h->view[v];
         b.img = take(npix);
-        b.census = reinterpret_cast<uint64_t*>(take(npix * 8));
+        b.census = reinterpret_cast<uint64_t*>(take(census_words(h->W, h->H, h->cpad) * 8)) + h->cpad;
         b.cost = take(ncell);
         for (int r = 0; r < 4; ++r) b.path[r] = take(ncell);
         b.raw = reinterpret_cast<float*>(take(npix * 4));
@@ -354,6 +409,7 @@ SgmJob make_job(const sgm_handle* h, int v) {
     for (int r = 0; r < 4; ++r) j.path[r] = b.path[r];
     j.disp = b.raw;
     j.W = h->W; j.H = h->H; j.D = h->D; j.min_d = h->min_d;
+    j.cpitch = h->W + 2 * h->cpad; j.cpad = h->cpad;
     j.roi_x = std::max(0, h->min_d);
     j.is_right = v;
     j.cs_type = h->opt.cs_type;
@@ -533,10 +589,15 @@ int sgm_init(sgm_handle* h, int32_t width, int32_t height, int32_t min_disparity
     h->opt = *opt;
     h->print_log = print_log != 0;
     HIP_TRY(&h->err, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-    HIP_TRY(&h->err, hipMalloc(&h->arena, arena_bytes(width, height, disp_range)));
+    h->cpad = h->window ? 0 : mid_pad(disp_range, min_disparity);
+    HIP_TRY(&h->err, hipMalloc(&h->arena, arena_bytes(width, height, disp_range, h->cpad)));
     if (opt->do_remove_peaks)
         HIP_TRY(&h->err, hipMalloc(&h->peaks, 2 * (size_t)width * height * sizeof(int)));
     carve(h);
+    if (h->cpad > 0) {
+        for (int v = 0; v < 2; ++v) HIP_TRY(&h->err, fill_census_pads(make_job(h, v), h->stream));
+        HIP_TRY(&h->err, hipStreamSynchronize(h->stream));
+    }
     if (int rc = build_handle_plan(h)) return rc;
     h->inited = true;
     if (h->print_log)
@@ -952,12 +1013,24 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
         return nullptr;
     }
     const bool lr = opt->do_lr_check != 0;
+    // census rows are padded where the batch may take the 4-line form
+    int groups = 0;
+    for (int i = 0; i < n; ++i) {
+        SgmJob j{};
+        j.H = pairs[i].height; j.D = pairs[i].disp_range;
+        groups += j.D <= 256 ? (lr ? 2 : 1) * wide_h_items(j) : 0;
+    }
+    const bool padded = groups < wide_min_groups();
+    auto pad_of = [&](const sgm_pair_desc& p) {
+        return padded ? mid_pad(p.disp_range, p.min_disparity) : 0;
+    };
     // arena: per pair two census maps; cost + 4 paths + raw map per matched view
     size_t total = 0;
     for (int i = 0; i < n; ++i) {
         const size_t npix = (size_t)pairs[i].width * pairs[i].height;
         const size_t ncell = npix * pairs[i].disp_range;
-        total += 2 * align256(npix * 8) + (lr ? 2 : 1) * (5 * align256(ncell) + align256(npix * 4));
+        const size_t ncensus = census_words(pairs[i].width, pairs[i].height, pad_of(pairs[i]));
+        total += 2 * align256(ncensus * 8) + (lr ? 2 : 1) * (5 * align256(ncell) + align256(npix * 4));
     }
     if (hipMalloc(&b->arena, total) != hipSuccess) {
         fail(nullptr, SGM_E_HIP, "hipMalloc of " + std::to_string(total) + " bytes failed");
@@ -972,8 +1045,10 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
     for (int i = 0; i < n; ++i) {
         const sgm_pair_desc& p = pairs[i];
         const size_t npix = (size_t)p.width * p.height, ncell = npix * p.disp_range;
-        uint64_t* cs[2] = {reinterpret_cast<uint64_t*>(take(npix * 8)),
-                           reinterpret_cast<uint64_t*>(take(npix * 8))};
+        const int pad = pad_of(p);
+        const size_t ncensus = census_words(p.width, p.height, pad);
+        uint64_t* cs[2] = {reinterpret_cast<uint64_t*>(take(ncensus * 8)) + pad,
+                           reinterpret_cast<uint64_t*>(take(ncensus * 8)) + pad};
         SgmPost post{};
         for (int v = 0; v < (lr ? 2 : 1); ++v) {
             SgmJob j{};
@@ -984,6 +1059,7 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
             for (int r = 0; r < 4; ++r) j.path[r] = take(ncell);
             j.disp = reinterpret_cast<float*>(take(npix * 4));
             j.W = p.width; j.H = p.height; j.D = p.disp_range; j.min_d = p.min_disparity;
+            j.cpitch = p.width + 2 * pad; j.cpad = pad;
             j.roi_x = std::max(0, p.min_disparity);
             j.is_right = v;
             j.cs_type = opt->cs_type;
@@ -1010,6 +1086,17 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
     }
     std::vector<SgmJob> jobs = left_jobs;
     jobs.insert(jobs.end(), right_jobs.begin(), right_jobs.end());
+    if (padded) {
+        hipError_t e = hipSuccess;
+        for (const SgmJob& j : jobs)
+            if (j.cpad > 0 && e == hipSuccess) e = fill_census_pads(j, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+        if (e != hipSuccess) {
+            fail(nullptr, SGM_E_HIP, std::string("census pads: ") + hipGetErrorString(e));
+            free_batch(b);
+            return nullptr;
+        }
+    }
     if (upload_plan(jobs, posts, &b->plan, &b->plan_block, &b->err)) {
         g_last_error = b->err;
         free_batch(b);

@@ -108,6 +108,13 @@ __device__ __forceinline__ int find_job(const int* __restrict__ offs, int n, int
     return lo;
 }
 
+// The item of this wave, where a workgroup is one wave or several (each an
+// item of its own; see waves_per_group).  Wave-uniform.
+__device__ __forceinline__ int wave_in_group() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+__device__ __forceinline__ int wave_item() {
+    return (int)blockIdx.x * (int)(blockDim.x >> 6) + wave_in_group();
+}
+
 // Workgroups of one launch go round-robin to the 8 XCDs (block b to XCD
 // b mod 8), and each XCD has its own L2.  This bijection on [0, n) gives each
 // XCD one contiguous run of items, so neighbouring items (adjacent column

@@ -42,6 +42,9 @@ struct SgmJob {
     // the whole image.  Border rules then use image coordinates and the map
     // written is the image's (row pitch fW).
     int32_t fx0, fy0, fW, fH;
+    // census rows: words per row (0: W) and the pad words on each side, which
+    // hold the word of column 0 (a partner column outside the image)
+    int32_t cpitch, cpad;
 };
 
 struct SgmPost {                   // one stereo pair: LR check + median
@@ -107,6 +110,34 @@ inline int wide_v_items(const SgmJob& j, int kind) {
 inline bool big_penalties(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
 inline bool wide_ok(const SgmJob& j) { return j.D <= 256 && !(j.is_right && j.cs_type == 0); }
 
+// Their 4-line form (sgm_mid.hip) for plans too small to fill the GPU that
+// way: D <= 256, 32-bit offsets, and census rows padded by every partner
+// column.  It takes the 5x5 right view: columns with the skipped-pixel rule
+// are lines of their own.
+inline int64_t mid_partners(int D, int64_t min_d) { return D - 1 + (min_d < 0 ? -min_d : min_d); }
+// pad words a plan gives its rows: none for D > 256 or an offset beyond D
+inline int mid_pad(int D, int64_t min_d) {
+    const int64_t p = mid_partners(D, min_d);
+    return D <= 256 && p < 2 * D ? (int)p : 0;
+}
+// words of a census map with pad words: a step of the vertical lines loads up
+// to 384 words from its first partner on, past the last row's end
+inline size_t census_words(int W, int H, int pad) {
+    return (size_t)(W + 2 * pad) * H + (pad > 0 ? 384 : 0);
+}
+inline bool mid_ok(const SgmJob& j) {
+    return j.D <= 256 && mid_partners(j.D, j.min_d) <= j.cpad &&
+           (int64_t)j.W * j.H * j.D < INT32_MAX && (int64_t)j.H * j.cpitch * 8 < INT32_MAX;
+}
+__host__ __device__ inline int mid_specials(const SgmJob& j) {   // columns of that rule
+    return (j.is_right && j.cs_type == 0) ? (j.W - j.roi_x + j.D - 1) / j.D : 0;
+}
+inline int mid_v_items(const SgmJob& j) {
+    const int sp = mid_specials(j);
+    return (j.W - j.roi_x - sp + 3) / 4 + (sp + 3) / 4;
+}
+inline int mid3_items(const SgmJob& j) { return 2 * ((j.H + 3) / 4) + mid_v_items(j); }
+
 // Caller buffers bound for one launch sequence in place of the plan's own:
 // the images of jobs 0 and 1 (the left and right view of a single-pair
 // plan) and the outputs of post 0.  With `on` = 0 the plan's buffers are
@@ -131,14 +162,19 @@ struct StagePlan {
     int* offs_wh = nullptr;       // on-the-fly cost: left->right + right->left groups
     int* offs_wv = nullptr;       // on-the-fly cost: top->bottom groups
     int* offs_wf = nullptr;       // on-the-fly cost: bottom->top + WTA groups
+    int* offs_m3 = nullptr;       // 4-line form: left->right, right->left, top->bottom
+    int* offs_mf = nullptr;       // 4-line form: bottom->top + WTA
     SgmPost* posts = nullptr;     // device
     int* offs_post = nullptr;
     int njobs = 0, nposts = 0;
     int njobs_ctw = 0;            // if > 0: jobs [0, njobs_ctw) run cost..wta
     int n_census = 0, n_cost = 0, n_agg = 0, n_wta = 0, n_post = 0, n_agg3 = 0, n_dw = 0;
-    int n_wh = 0, n_wv = 0, n_wf = 0;
+    int n_wh = 0, n_wv = 0, n_wf = 0, n_m3 = 0, n_mf = 0;
+    int64_t cells = 0;            // matched pixels x D, over the views
     int dmax = 64, dmin = 64;     // over all jobs; dmin over the matched ones
     bool wide = false;            // matching uses the on-the-fly cost kernels
+    bool mid = false;             // unless scheduled, it uses their 4-line form
+    bool quirk = false;           // some matched job is a 5x5 right view
     bool big = false;             // some job's penalties need integer minima
     bool fast = false;            // not big, and every cost is a census distance (at most 64)
     bool squarish = false;        // every matched job has W - roi_x <= 2.5 H
@@ -175,6 +211,14 @@ hipError_t launch_reset_counters(uint32_t* counters, int n, hipStream_t s);
 // ceil(n / CUs) workgroups per CU by the LDS each one claims.  `used` is the
 // kernel's static LDS.
 unsigned spread_lds(int n, int used);
+// Waves per workgroup of a launch of n scanline groups (one wave each): 4 from
+// half a wave per SIMD up to `limit` quarters of one, else 1.  A workgroup's waves go to
+// different SIMDs, while single-wave workgroups are placed unevenly: with few
+// waves some SIMDs get several and others none (1242x375 D = 64, four
+// directions and WTA: 211 us as 1620 single waves, 183 us by fours;
+// 1920x1080 D = 128, 2040 waves with on-the-fly cost: 1265 and 1097 us).  With
+// more waves, or where memory is the limit, the finer grain is the better one.
+int waves_per_group(int n, int limit);
 // sgm_wide.hip: aggregation with the cost computed from the census words
 hipError_t launch_wide3(const StagePlan& p, hipStream_t s);
 hipError_t launch_wide_wta(const StagePlan& p, hipStream_t s);
@@ -183,12 +227,20 @@ hipError_t launch_wide_wta_sched(const StagePlan& p, const AggSchedule& sc, hipS
 // direction volumes as the launches above leave them (kUD, kLR, kRL) to plain ones
 hipError_t launch_wide_export(const SgmJob& j, const uint8_t* const (&src)[4],
                               uint8_t* const (&dst)[4], hipStream_t s);
+// sgm_mid.hip: the 4-line form; fill_census_pads writes a job's pad words
+hipError_t launch_mid3(const StagePlan& p, hipStream_t s);
+hipError_t launch_mid_wta(const StagePlan& p, hipStream_t s);
+hipError_t fill_census_pads(const SgmJob& j, hipStream_t s);
 hipError_t wide_occupancy(const StagePlan& p, int* per_cu);
 // Process-wide SGM_COST_* mode, read when a plan is built; choose_wide
 // applies it to a plan whose views all allow the on-the-fly cost
 // (`eligible`) and that has n_wh horizontal scanline groups.
 int cost_mode();
+// choose_mid: whether an unscheduled run of it takes the 4-line form
+// (`eligible` by mid_ok; cells: matched pixels x D over the views).
 bool choose_wide(bool eligible, int n_wh);
+bool choose_mid(bool eligible, int n_wh, int64_t cells);
+int wide_min_groups();
 hipError_t launch_wta(const StagePlan& p, hipStream_t s);
 hipError_t launch_post(const StagePlan& p, hipStream_t s);
 hipError_t launch_right_invalidate(const StagePlan& p, hipStream_t s);

@@ -21,6 +21,7 @@
 
 #include "sgm_device.h"
 #include "sgm_internal.h"
+#include "sgm_line.h"
 
 #pragma clang fp contract(off)
 
@@ -156,7 +157,7 @@ __global__ __launch_bounds__(128) void census_kernel(const SgmJob* __restrict__ 
             const int x = x0 + 2 * lx + h;
             if (x >= J.W) continue;
             const bool border = x < rw || x >= J.W - rw || y < rh || y >= J.H - rh;
-            gst(J.census + (int64_t)y * J.W + x, border ? invalid : v[rr][h]);
+            gst(J.census + (int64_t)y * J.cpitch + x, border ? invalid : v[rr][h]);
         }
     }
 }
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(256) void cost_kernel(const SgmJob* __restrict__ jo
     const int segs = (W - roi_x + kCostSeg - 1) / kCostSeg;
     const int y = local / segs;
     const int x0 = roi_x + (local - y * segs) * kCostSeg;
-    const uint64_t* cb = J.census + (int64_t)y * W;
-    const uint64_t* cm = J.census_other + (int64_t)y * W;
+    const uint64_t* cb = J.census + (int64_t)y * J.cpitch;
+    const uint64_t* cm = J.census_other + (int64_t)y * J.cpitch;
     const bool l2r = !J.is_right;
     const bool quirk_job = J.is_right && J.cs_type == 0;
     const int tid = threadIdx.x;
@@ -277,45 +278,6 @@ __device__ __forceinline__ BlockWalk block_walk(int64_t first, int64_t step, int
     w.s = step < 0 ? w.last : 0;
     w.inc = (int)step;
     return w;
-}
-
-typedef unsigned int buf_u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int buf_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const uint8_t* p) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, 0x7fffffff, 0x00020000);
-}
-template <int NW>
-__device__ __forceinline__ void buf_load(__amdgpu_buffer_rsrc_t r, uint32_t v, int s, uint32_t (&w)[NW]) {
-    if constexpr (NW == 1) {
-        w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)v, s, 0);
-    } else if constexpr (NW == 2) {
-        const buf_u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, s, 0);
-        w[0] = t.x; w[1] = t.y;
-    } else {
-#pragma unroll
-        for (int k = 0; k < NW; k += 4) {
-            const buf_u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(v + 4 * k), s, 0);
-            w[k] = t.x; w[k + 1] = t.y; w[k + 2] = t.z; w[k + 3] = t.w;
-        }
-    }
-}
-// A 128-bit store takes its step offset in the vector offset: with a scalar
-// offset register the compiler leaves the data registers free to be rewritten
-// by the next instruction, and under load such stores have written the later
-// values (D = 256 beside two larger pairs); without one it keeps the wait
-// state that stores of more than 64 bits need.
-template <int NW>
-__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t v, int s, const uint32_t (&w)[NW]) {
-    if constexpr (NW == 1) {
-        __builtin_amdgcn_raw_buffer_store_b32(w[0], r, (int)v, s, 0);
-    } else if constexpr (NW == 2) {
-        __builtin_amdgcn_raw_buffer_store_b64(buf_u32x2{w[0], w[1]}, r, (int)v, s, 0);
-    } else {
-#pragma unroll
-        for (int k = 0; k < NW; k += 4)
-            __builtin_amdgcn_raw_buffer_store_b128(buf_u32x4{w[k], w[k + 1], w[k + 2], w[k + 3]}, r,
-                                                   (int)(v + 4 * k + s), 0, 0);
-    }
 }
 
 template <int D, bool FUSE, bool FAST>
@@ -562,9 +524,11 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
 // right->left, top->bottom; MODE 2: bottom->top fused with the WTA.
 // ONLY: every job has D = DMAX (other ranges' code would take its registers).
 template <int DMAX, int MODE, bool FAST, bool ONLY>
-__global__ __launch_bounds__(64) void aggregate_kernel(const SgmJob* __restrict__ jobs,
-                                                       const int* __restrict__ offs, int njobs) {
-    const int item = blockIdx.x;
+__global__ __launch_bounds__(256) void aggregate_kernel(const SgmJob* __restrict__ jobs,
+                                                        const int* __restrict__ offs, int njobs,
+                                                        int n) {
+    const int item = wave_item();
+    if (item >= n) return;
     const int j = find_job(offs, njobs, item);
     const SgmJob& J = jobs[j];
     const int local = item - offs[j];
@@ -576,7 +540,7 @@ __global__ __launch_bounds__(64) void aggregate_kernel(const SgmJob* __restrict_
     else if (local < 2 * nh) { path = kRL; group = local - nh; }
     else if (local < 2 * nh + nv) { path = kUD; group = local - 2 * nh; }
     else { path = kDU; group = local - 2 * nh - nv; }
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     constexpr bool F = (MODE == 2);
     switch (J.D) {
         case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST>(J, path, group, lane); break;
@@ -927,8 +891,9 @@ hipError_t launch_cost(const StagePlan& p, hipStream_t s) {
 template <int MODE>
 static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    const dim3 g(n), b(64);
-    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs); };
+    const int wg = p.cells <= 100000000 ? waves_per_group(n, 7) : 1;
+    const dim3 g((n + wg - 1) / wg), b(64 * wg);
+    auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs, n); };
     if (!p.fast) go(aggregate_kernel<512, MODE, false, false>);
     else if (p.dmax <= 64) go(aggregate_kernel<64, MODE, true, true>);
     else if (p.dmin == p.dmax)

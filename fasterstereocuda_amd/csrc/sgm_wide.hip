@@ -41,6 +41,7 @@
 
 #include "sgm_device.h"
 #include "sgm_internal.h"
+#include "sgm_line.h"
 
 #pragma clang fp contract(off)
 
@@ -57,176 +58,9 @@ namespace {
 
 using namespace dev;
 
-// value of the previous / next lane of the line; the line's first / last
-// lane gets `edge`
-template <int LPL>
-__device__ __forceinline__ uint32_t from_prev(uint32_t v, uint32_t edge, bool first) {
-    if constexpr (LPL == 16) {
-        return dpp<kRowShr1>(edge, v);
-    } else {
-        const uint32_t s = dpp0<kRowShr1>(v);   // every lane moves; the first then takes `edge`
-        return first ? edge : s;
-    }
-}
-template <int LPL>
-__device__ __forceinline__ uint32_t from_next(uint32_t v, uint32_t edge, bool last) {
-    if constexpr (LPL == 16) {
-        return dpp<kRowShl1>(edge, v);
-    } else {
-        const uint32_t s = dpp0<kRowShl1>(v);
-        return last ? edge : s;
-    }
-}
-
-__device__ __forceinline__ uint32_t popc64(uint64_t a) { return (uint32_t)__popcll(a); }
-// popcount(a) + acc as two accumulating v_bcnt_u32_b32.  Written out, the
-// compiler regroups the sum and packs with a v_lshl_or_b32; this form packs
-// the upper count with a v_lshlrev_b32, which issues at twice the rate.
-__device__ __forceinline__ uint32_t bcnt_acc(uint32_t x, uint32_t acc) {
-    uint32_t r;
-    asm("v_bcnt_u32_b32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(acc));
-    return r;
-}
-__device__ __forceinline__ uint32_t popc_acc(uint64_t a, uint32_t acc) {
-    return bcnt_acc((uint32_t)a, bcnt_acc((uint32_t)(a >> 32), acc));
-}
-
-// One recurrence step of a line, NP packed u16 pairs (2 NP disparities) per lane:
-//   L(d) = C(d) + min(L'(d), B-(d), B+(d), m' + P2) - m'
-//   B-(d) = d == 0 ? 127 : L'(d-1) + P1,  B+(d) = d == D-1 ? 127 : L'(d+1) + P1
-template <int NP>
-struct Line {
-    uint32_t L[NP];
-    uint32_t m;   // the line minimum in both u16 halves
-};
-
-// both halves = the smaller half (v_pk_min_u16 with swapped operand halves);
-// a u32 minimum of such values is their u16 minimum
-__device__ __forceinline__ uint32_t pk_min_halves(uint32_t v) {
-    return as_u(__builtin_elementwise_min(as_v(v), as_v(v).yx));
-}
-
-template <bool BIG, int LPL, int NP>
-__device__ __forceinline__ void line_init(Line<NP>& s, const uint32_t (&c)[NP]) {
-#pragma unroll
-    for (int k = 0; k < NP; ++k) s.L[k] = c[k];
-    s.m = line_min<LPL>(pk_min_halves(pk_min_all<BIG>(s.L)));
-}
-
-// The sums of a step never carry or borrow between the u16 halves: costs are
-// at most 64, the line minimum is at most the cost at the previous minimum's
-// disparity (so below every term, 127 included) and P1 + P2 <= 65000.  So
-// they are 32-bit adds and subtracts, which issue in 2 cycles where the packed
-// forms take 4.
-
-template <bool BIG, int LPL, int NP>
-__device__ __forceinline__ void line_step(Line<NP>& s, const uint32_t (&c)[NP], uint32_t P1v,
-                                          uint32_t P2v, bool first, bool last) {
-    const uint32_t mv = s.m;
-    const uint32_t mp2 = mv + P2v;
-    uint32_t R[NP];
-#pragma unroll
-    for (int k = 0; k < NP; ++k) R[k] = s.L[k] + P1v;
-    const uint32_t prev_last = from_prev<LPL>(R[NP - 1], 127u << 16, first);
-    const uint32_t next_first = from_next<LPL>(R[0], 127u, last);
-    uint32_t E[NP + 1];
-    E[0] = __builtin_amdgcn_alignbit(R[0], prev_last, 16);
-#pragma unroll
-    for (int k = 1; k < NP; ++k) E[k] = __builtin_amdgcn_alignbit(R[k], R[k - 1], 16);
-    E[NP] = __builtin_amdgcn_alignbit(next_first, R[NP - 1], 16);
-#pragma unroll
-    for (int k = 0; k < NP; ++k) {
-        const uint32_t v = pk_min(pk_min3<BIG>(s.L[k], E[k], E[k + 1]), mp2);
-        s.L[k] = c[k] + v;
-    }
-    s.m = line_min<LPL>(pk_min_halves(pk_min_all<BIG>(s.L)));
-}
-
-// The lane's 2 NP bytes (uint8 truncation).  The volumes these kernels hand
-// each other keep a word's bytes in the order d, d + 2, d + 1, d + 3, so the
-// reader gets two packed u16 pairs from a word with a 2-cycle mask and one
-// packed shift instead of two v_perm.
-template <int NP>
-__device__ __forceinline__ void pack_lane(const Line<NP>& s, uint32_t sel, uint32_t (&o)[NP / 2]) {
-#pragma unroll
-    for (int k = 0; k < NP / 2; ++k) o[k] = __builtin_amdgcn_perm(s.L[2 * k + 1], s.L[2 * k], sel);
-}
-// pairs 2k and 2k + 1 of a word
-__device__ __forceinline__ uint32_t word_pair(uint32_t w, int odd) {
-    return odd ? as_u(as_v(w) >> (u16x2)8) : (w & 0x00FF00FFu);
-}
-
-constexpr uint32_t kSelFwd = 0x06020400u;   // bytes d, d+2, d+1, d+3
-// lanes that hold the disparities in reversed order swap a pair's halves, so
-// that the reader (which takes their words in reversed order) finds d before d + 1
-constexpr uint32_t kSelRev = 0x04000602u;
-
 __device__ __forceinline__ uint64_t g64(const uint64_t* p) { return gld(p); }
 
 __device__ __forceinline__ int clampcol(int p, int W) { return (p >= 0 && p < W) ? p : 0; }
-
-// value of lane `src` (a compile-time constant after unrolling) of the line,
-// on every lane of the line: quad_perm, or row_newbcast (the broadcast of one
-// lane of a 16-lane DPP row; two of them, by halves, where a line is 8 lanes)
-template <int LPL, int SRC>
-__device__ __forceinline__ uint32_t line_bcast_c(uint32_t v) {
-    if constexpr (LPL == 4) {
-        return dpp0<SRC * 0x55>(v);
-    } else if constexpr (LPL == 16) {
-        return dpp0<0x150 + SRC>(v);
-    } else {
-        const int lo = (int)dpp0<0x150 + SRC>(v);
-        return (uint32_t)__builtin_amdgcn_update_dpp(lo, (int)v, 0x150 + SRC + 8, 0xF, 0xC, false);
-    }
-}
-template <int LPL>
-__device__ __forceinline__ uint32_t line_bcast(uint32_t v, int src) {
-    switch (src) {
-        case 0: return line_bcast_c<LPL, 0>(v);
-        case 1: return line_bcast_c<LPL, 1>(v);
-        case 2: return line_bcast_c<LPL, 2>(v);
-        case 3: return line_bcast_c<LPL, 3>(v);
-        default: break;
-    }
-    if constexpr (LPL >= 8)
-        switch (src) {
-            case 4: return line_bcast_c<LPL, 4>(v);
-            case 5: return line_bcast_c<LPL, 5>(v);
-            case 6: return line_bcast_c<LPL, 6>(v);
-            case 7: return line_bcast_c<LPL, 7>(v);
-            default: break;
-        }
-    if constexpr (LPL >= 16)
-        switch (src) {
-            case 8: return line_bcast_c<LPL, 8>(v);
-            case 9: return line_bcast_c<LPL, 9>(v);
-            case 10: return line_bcast_c<LPL, 10>(v);
-            case 11: return line_bcast_c<LPL, 11>(v);
-            case 12: return line_bcast_c<LPL, 12>(v);
-            case 13: return line_bcast_c<LPL, 13>(v);
-            case 14: return line_bcast_c<LPL, 14>(v);
-            case 15: return line_bcast_c<LPL, 15>(v);
-            default: break;
-        }
-    return v;
-}
-template <int LPL>
-__device__ __forceinline__ uint64_t line_bcast64(uint64_t v, int src) {
-    const uint32_t lo = line_bcast<LPL>((uint32_t)v, src);
-    const uint32_t hi = line_bcast<LPL>((uint32_t)(v >> 32), src);
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// packed costs of one lane: pair k = (partner 2k, partner 2k + 1)
-template <int NP, class F>
-__device__ __forceinline__ void lane_costs(uint64_t own, uint32_t base, F&& partner, uint32_t (&c)[NP]) {
-#pragma unroll
-    for (int k = 0; k < NP; ++k) {
-        uint32_t t;
-        asm("v_lshl_add_u32 %0, %1, 16, %2" : "=v"(t) : "v"(popc_acc(own ^ partner(2 * k + 1), 0u)), "v"(base));
-        c[k] = popc_acc(own ^ partner(2 * k), t);
-    }
-}
 
 // ------------------------------------------------------------ horizontal ---
 // Left->right or right->left over the wave's rows.  With t' the lane-local
@@ -250,8 +84,8 @@ __device__ __forceinline__ void wide_horizontal(const SgmJob& J, int path, int g
     const bool rev = right != (path == kRL);
     const int a = right ? (rev ? min_d + D - 1 : min_d) : (rev ? -min_d - (D - 1) : -min_d);
     const int st = (right != rev) ? 1 : -1;
-    const uint64_t* cb = J.census + (int64_t)y * W;
-    const uint64_t* cm = J.census_other + (int64_t)y * W;
+    const uint64_t* cb = J.census + (int64_t)y * J.cpitch;
+    const uint64_t* cm = J.census_other + (int64_t)y * J.cpitch;
     const uint32_t P1v = (uint32_t)J.p1 * 0x10001u, P2v = (uint32_t)J.p2 * 0x10001u;
     const uint32_t sel = rev ? kSelRev : kSelFwd;
     uint8_t* const out_base = (path == kLR) ? J.path[kLR] : J.path[kRL];
@@ -395,8 +229,8 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
     };
     auto load_step = [&](int i, uint64_t (&g)[NR]) __attribute__((always_inline)) {
         const int y = y0 + dy * min(i, H - 1);
-        const uint64_t* cb = J.census + (int64_t)y * W;
-        const uint64_t* cm = J.census_other + (int64_t)y * W;
+        const uint64_t* cb = J.census + (int64_t)y * J.cpitch;
+        const uint64_t* cm = J.census_other + (int64_t)y * J.cpitch;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const int v = min(lane + 64 * r, NV - 1);

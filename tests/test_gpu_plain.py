@@ -204,6 +204,73 @@ def test_cost_modes_match_oracle(cuda, cost_mode, mode, case, lr, median):
     st.Release()
 
 
+# The 4-line on-the-fly kernels at the columns of the 5x5 right view's
+# skipped-pixel rule (the last of every D-column block, and the last one): one
+# block exactly, one short, one past, several; and offsets on both sides.
+@pytest.mark.parametrize("W,H,D,min_d", [
+    (64, 9, 64, 0), (63, 13, 64, 0), (65, 12, 64, 0), (128, 10, 64, 0), (129, 11, 64, 0),
+    (340, 14, 64, 0), (340, 14, 64, 9), (333, 17, 64, -70), (290, 13, 128, 0), (520, 12, 256, -3),
+])
+def test_on_the_fly_5x5_columns(cuda, cost_mode, W, H, D, min_d):
+    print(f"[otf 5x5] {W}x{H} D{D} m{min_d}", flush=True)
+    cost_mode(2)
+    left, right = _pair(W, H, D, seed=11)
+    exp_l, exp_r = oracle.match(left, right, min_d, D, cs_type=0, p1=8, p2=32, uniqueness=UNIQ,
+                                lr_threshold=LR_THR, do_median=False)
+    st = StereoCuda()
+    opt = CuSGMOption.benchmark(cs_type=0, p1=8, p2_init=32, do_median_filter=False)
+    assert st.Init(W, H, min_d, D, opt), st.last_error
+    dl, dr = np.empty((H, W), np.float32), np.empty((H, W), np.float32)
+    assert st.Match(left, right, dl, dr), st.last_error
+    _eq_float(dl, exp_l, "left map")
+    _eq_float(dr, exp_r, "right map")
+    st.Release()
+
+
+# a handle's census rows are padded for the offset it was made with: moved
+# within the pads, back, and past them (where the stored cost takes over)
+@pytest.mark.parametrize("cs", [0, 1])
+def test_on_the_fly_moved_offset(cuda, cost_mode, cs):
+    W, H, D = 150, 21, 64
+    cost_mode(2)
+    left, right = _pair(W, H, D, seed=12)
+    st = StereoCuda()
+    assert st.Init(W, H, -6, D, CuSGMOption.benchmark(cs_type=cs)), st.last_error
+    dl, dr = np.empty((H, W), np.float32), np.empty((H, W), np.float32)
+    for min_d in (-6, 6, -7, 40, -6):
+        st.SetMinDisparity(min_d)
+        exp_l, exp_r = oracle.match(left, right, min_d, D, cs_type=cs, uniqueness=UNIQ,
+                                    lr_threshold=LR_THR)
+        assert st.Match(left, right, dl, dr), st.last_error
+        _eq_float(dl, exp_l, f"left map at {min_d}")
+        _eq_float(dr, exp_r, f"right map at {min_d}")
+    st.Release()
+
+
+# penalties past the f16 minima, and ranges mixed in one plan, on the 4-line form
+@pytest.mark.parametrize("cs,p1,p2", [(0, 20000, 10001), (1, 10, 64990), (1, 20000, 10000)])
+def test_on_the_fly_mixed_batch(cuda, cost_mode, cs, p1, p2):
+    from fasterstereocuda_amd.batch import SgmBatch
+    cost_mode(2)
+    opt = CuSGMOption.benchmark(cs_type=cs, p1=p1, p2_init=p2)
+    pairs, refs = [], []
+    for i, (W, H, D, m) in enumerate([(140, 30, 64, 0), (200, 19, 128, 3), (280, 14, 256, -2)]):
+        left, right = _pair(W, H, D, seed=20 + i)
+        refs.append(oracle.match(left, right, m, D, cs_type=cs, p1=p1, p2=p2, uniqueness=UNIQ,
+                                 lr_threshold=LR_THR))
+        pairs.append({"left": torch.from_numpy(left).to(cuda), "right": torch.from_numpy(right).to(cuda),
+                      "disp_left": torch.empty((H, W), device=cuda),
+                      "disp_right": torch.empty((H, W), device=cuda),
+                      "min_disparity": m, "disp_range": D})
+    b = SgmBatch(pairs, opt)
+    for _ in range(3):
+        b.run()
+    torch.cuda.synchronize()
+    for p, (exp_l, exp_r) in zip(pairs, refs):
+        _eq_float(p["disp_left"].cpu().numpy(), exp_l, "left map")
+        _eq_float(p["disp_right"].cpu().numpy(), exp_r, "right map")
+
+
 @pytest.fixture
 def wta_form():
     before = stages.get_wta_form()
