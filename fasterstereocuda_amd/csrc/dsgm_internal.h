@@ -40,6 +40,11 @@ __host__ __device__ inline int64_t dsgm_saved_kstar_offset(int B, int H, int W, 
     return (int64_t)B * H * W * (8 + D);
 }
 
+// dsgm_sweep.hip: the form that runs two directions together, and where it is used
+bool dsgm_sweep_ok(const DsgmArgs& A);
+hipError_t dsgm_sweep_forward(const DsgmArgs& A, hipStream_t s);
+hipError_t dsgm_sweep_backward(const DsgmArgs& A, hipStream_t s);
+
 hipError_t dsgm_launch_forward(const DsgmArgs& A, hipStream_t s);
 hipError_t dsgm_launch_backward(const DsgmArgs& A, hipStream_t s);
 

@@ -35,75 +35,14 @@
 //
 // Layout per wave as in the integer aggregation: four 16-lane DPP rows, one
 // scanline per row, D/16 disparities per lane.
-#include <algorithm>
-#include <cmath>
-
-#include "dsgm_internal.h"
+#include "dsgm_device.h"
 #include "sgm_device.h"
 
 #pragma clang fp contract(off)
 
 namespace fsgm {
+using namespace dsgm;
 namespace {
-
-template <int CTRL>
-__device__ __forceinline__ float dppf(float old, float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-        __builtin_bit_cast(int, old), __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-template <int CTRL>
-__device__ __forceinline__ int dppi(int old, int v) {
-    return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xF, 0xF, false);
-}
-constexpr int kShl1 = 0x101, kShr1 = 0x111;
-
-__device__ __forceinline__ float row_minf(float v) {
-    v = fminf(v, dppf<0x128>(0.f, v));
-    v = fminf(v, dppf<0x124>(0.f, v));
-    v = fminf(v, dppf<0x122>(0.f, v));
-    v = fminf(v, dppf<0x121>(0.f, v));
-    return v;
-}
-__device__ __forceinline__ float row_sumf(float v) {
-    v = v + dppf<0x128>(0.f, v);
-    v = v + dppf<0x124>(0.f, v);
-    v = v + dppf<0x122>(0.f, v);
-    v = v + dppf<0x121>(0.f, v);
-    return v;
-}
-__device__ __forceinline__ int row_mini(int v) {
-    v = min(v, dppi<0x128>(0, v));
-    v = min(v, dppi<0x124>(0, v));
-    v = min(v, dppi<0x122>(0, v));
-    v = min(v, dppi<0x121>(0, v));
-    return v;
-}
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) f32x4 g_f4;
-typedef __attribute__((address_space(1))) float g_f;
-
-template <int N>
-__device__ __forceinline__ void loadf(const float* p, float (&v)[N]) {
-#pragma unroll
-    for (int k = 0; k < N; k += 4) {
-        const f32x4 t = *(const g_f4*)(p + k);
-        v[k] = t.x; v[k + 1] = t.y; v[k + 2] = t.z; v[k + 3] = t.w;
-    }
-}
-template <int N>
-__device__ __forceinline__ void storef(float* p, const float (&v)[N]) {
-#pragma unroll
-    for (int k = 0; k < N; k += 4) *(g_f4*)(p + k) = f32x4{v[k], v[k + 1], v[k + 2], v[k + 3]};
-}
-__device__ __forceinline__ float loads(const float* p) { return *(const g_f*)p; }
-
-// A lane's winner codes of one step: DPD = D / 16 disparities, 2 bits each.
-template <int D> struct WinWordOf;
-template <> struct WinWordOf<64> { using type = uint8_t; };
-template <> struct WinWordOf<128> { using type = uint16_t; };
-template <> struct WinWordOf<256> { using type = uint32_t; };
-template <int D> using WinWord = typename WinWordOf<D>::type;
 
 // Geometry of one scanline of one direction.
 struct LineGeo {
@@ -135,84 +74,7 @@ __device__ __forceinline__ LineGeo line_geo(const DsgmArgs& A, int path, int gro
     return g;
 }
 
-// one forward step for a lane's DPD disparities; returns winners packed 2 bits each
-template <int DPD>
-__device__ __forceinline__ uint32_t fwd_step(float (&L)[DPD], const float (&c)[DPD], float m,
-                                             float p1, float p2) {
-    const float inf = __builtin_inff();
-    const float prev_last = dppf<kShr1>(inf, L[DPD - 1]);
-    const float next_first = dppf<kShl1>(inf, L[0]);
-    const float c3 = m + p2;
-    uint32_t wins = 0;
-    float nl[DPD];
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) {
-        const float lm = (k == 0) ? prev_last : L[k - 1];
-        const float lp = (k == DPD - 1) ? next_first : L[k + 1];
-        float best = L[k];
-        uint32_t w = 0;
-        const float c1 = lm + p1, c2 = lp + p1;
-        if (c1 < best) { best = c1; w = 1; }
-        if (c2 < best) { best = c2; w = 2; }
-        if (c3 < best) { best = c3; w = 3; }
-        nl[k] = (c[k] + best) - m;
-        wins |= w << (2 * k);
-    }
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) L[k] = nl[k];
-    return wins;
-}
-
-template <int DPD>
-__device__ __forceinline__ float lane_min(const float (&L)[DPD]) {
-    float v = L[0];
-#pragma unroll
-    for (int k = 1; k < DPD; ++k) v = fminf(v, L[k]);
-    return v;
-}
-
-// smallest d with L(d) == m over the row
-template <int DPD>
-__device__ __forceinline__ int row_argmin(const float (&L)[DPD], float m, int l) {
-    int idx = 0x7FFFFFFF;
-#pragma unroll
-    for (int k = DPD - 1; k >= 0; --k)
-        if (L[k] == m) idx = l * DPD + k;
-    return row_mini(idx);
-}
-
 // ------------------------------------------------------------- forward ---
-// Unnormalised softmax weight exp(-(s - mn) / T) = 2^((mn - s) * c) with
-// c = log2(e) / T: one v_exp_f32 after a subtraction and a product.  The
-// forward and the backward use this same form.  The argument is <= 0, and a
-// weight below 2^-126 (a cost more than 87 T above the minimum) contributes
-// nothing to the sums either way.
-__device__ __forceinline__ float soft_weight(float s, float mn, float c) {
-    return __builtin_amdgcn_exp2f((mn - s) * c);
-}
-__device__ __forceinline__ float soft_scale(float invT) { return invT * 1.44269504088896340736f; }
-
-// Soft-argmin of one pixel per 16-lane row: s holds S, every lane of the row
-// receives the disparity, the minimum mn and the normaliser z.
-template <int DPD>
-__device__ __forceinline__ float soft_argmin(const float (&s)[DPD], int l, float invT, float* mn_out,
-                                             float* z_out) {
-    const float mn = row_minf(lane_min(s));
-    const float c = soft_scale(invT);
-    float z = 0.f, acc = 0.f;
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) {
-        const float e = soft_weight(s[k], mn, c);
-        z += e;
-        acc += (float)(l * DPD + k) * e;
-    }
-    z = row_sumf(z);
-    acc = row_sumf(acc);
-    *mn_out = mn;
-    *z_out = z;
-    return acc / z;
-}
-
 // What a forward pass does with each step's L.
 enum FwdMode {
     kFwdStoreS = 0,   // S = L          (left->right, first of the horizontal pair)
@@ -360,17 +222,6 @@ __global__ __launch_bounds__(64) void dsgm_forward_last_kernel(DsgmArgs A) {
 }
 
 // ------------------------------------------------------------ backward ---
-// gS(p, d) = gdisp(p) * (-1/T) * prob(p, d) * (d - disp(p)) of one pixel,
-// from S and the forward's minimum mn and normaliser z of that pixel.
-template <int DPD>
-__device__ __forceinline__ void grad_s_from(const float (&s)[DPD], float mn, float z, float gd,
-                                            float dq, float invT, int l, float (&g)[DPD]) {
-    const float coef = gd * (-invT) / z;
-    const float c = soft_scale(invT);
-#pragma unroll
-    for (int k = 0; k < DPD; ++k)
-        g[k] = coef * soft_weight(s[k], mn, c) * ((float)(l * DPD + k) - dq);
-}
 template <int DPD>
 __device__ __forceinline__ void grad_s_at(const DsgmArgs& A, const float* Sb, const float* stats,
                                           const float* disp, const float* gdisp, int64_t q, int l,
@@ -581,6 +432,7 @@ static unsigned dsgm_items_first(const DsgmArgs& A) {
 static unsigned dsgm_items_last(const DsgmArgs& A) { return (unsigned)(A.B * ((A.W + 3) / 4)); }
 
 hipError_t dsgm_launch_forward(const DsgmArgs& A, hipStream_t s) {
+    if (dsgm_sweep_ok(A)) return dsgm_sweep_forward(A, s);
     const dim3 b1(64);
     FSGM_DSGM_DISPATCH(dsgm_forward_first_kernel, dim3(dsgm_items_first(A)), b1, A, s);
     hipError_t e = hipGetLastError();
@@ -590,6 +442,7 @@ hipError_t dsgm_launch_forward(const DsgmArgs& A, hipStream_t s) {
 }
 
 hipError_t dsgm_launch_backward(const DsgmArgs& A, hipStream_t s) {
+    if (dsgm_sweep_ok(A)) return dsgm_sweep_backward(A, s);
     const dim3 b1(64);
     FSGM_DSGM_DISPATCH(dsgm_backward_first_kernel, dim3(dsgm_items_first(A)), b1, A, s);
     hipError_t e = hipGetLastError();

@@ -54,6 +54,30 @@ def test_forward_backward_match_fp64(cuda, B, H, W, D):
             assert np.abs(g - ref).max() <= 1e-4 * np.abs(ref).max(), f"{name} max err"
 
 
+# many images of few rows, which take the form that walks bands of four rows
+# for two directions together: last bands of 1 to 4 rows, a single band (no
+# state handed between bands), lines shorter than the skew of a band's rows
+@pytest.mark.parametrize("B,H,W,D", [(141, 13, 70, 128), (188, 10, 33, 64), (560, 3, 9, 64),
+                                     (140, 16, 1, 128), (280, 7, 2, 64), (187, 12, 130, 128)])
+def test_many_images_match_fp64(cuda, B, H, W, D):
+    print(f"[dsgm] B{B} H{H} W{W} D{D}", flush=True)
+    cost, p1, p2, gt = _inputs(B, H, W, D, seed=B + H + W + D)
+    tc = torch.from_numpy(cost).to(cuda).requires_grad_(True)
+    t1 = torch.from_numpy(p1).to(cuda).requires_grad_(True)
+    t2 = torch.from_numpy(p2).to(cuda).requires_grad_(True)
+    disp = diff_sgm(tc, t1, t2, T)
+    (disp - torch.from_numpy(gt).to(cuda)).abs().mean(dim=(1, 2)).sum().backward()
+    for b in (0, 1, B // 2, B - 1):
+        _, d_ref, _ = oracle.dsgm_forward(cost[b], p1[b], p2[b], gt[b], T)
+        gC, g1, g2, _ = oracle.dsgm_backward(cost[b], p1[b], p2[b], gt[b], T)
+        d = disp[b].detach().cpu().numpy()
+        assert np.abs(d - d_ref).max() <= 1e-5 * max(1.0, np.abs(d_ref).max()), "disparity"
+        for name, got, ref in (("dC", tc.grad[b], gC), ("dP1", t1.grad[b], g1), ("dP2", t2.grad[b], g2)):
+            g = got.cpu().numpy().astype(np.float64)
+            assert _rel(g, ref) <= 1e-4, f"{name} rel err {_rel(g, ref):.2e}"
+            assert np.abs(g - ref).max() <= 1e-4 * np.abs(ref).max(), f"{name} max err"
+
+
 def test_deterministic_and_repeatable(cuda):
     cost, p1, p2, gt = _inputs(2, 40, 50, 64, seed=1)
     outs = []
