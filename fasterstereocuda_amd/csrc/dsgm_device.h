@@ -22,12 +22,19 @@ __device__ __forceinline__ int dppi(int old, int v) {
 }
 constexpr int kShl1 = 0x101, kShr1 = 0x111;
 
-__device__ __forceinline__ float row_minf(float v) {
-    v = fminf(v, dppf<0x128>(0.f, v));
-    v = fminf(v, dppf<0x124>(0.f, v));
-    v = fminf(v, dppf<0x122>(0.f, v));
-    v = fminf(v, dppf<0x121>(0.f, v));
-    return v;
+// (written out: fminf of a moved value costs a separate move and a
+// canonicalising v_max per stage)
+__device__ __forceinline__ float row_min(float a) {
+    asm("s_nop 1\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf"
+        : "+v"(a));
+    return a;
 }
 __device__ __forceinline__ float row_sumf(float v) {
     v = v + dppf<0x128>(0.f, v);
@@ -106,16 +113,6 @@ __device__ __forceinline__ float lane_min(const float (&L)[DPD]) {
     return v;
 }
 
-// smallest d with L(d) == m over the row
-template <int DPD>
-__device__ __forceinline__ int row_argmin(const float (&L)[DPD], float m, int l) {
-    int idx = 0x7FFFFFFF;
-#pragma unroll
-    for (int k = DPD - 1; k >= 0; --k)
-        if (L[k] == m) idx = l * DPD + k;
-    return row_mini(idx);
-}
-
 // Unnormalised softmax weight exp(-(s - mn) / T) = 2^((mn - s) * c) with
 // c = log2(e) / T: one v_exp_f32 after a subtraction and a product.  The
 // forward and the backward use this same form.  The argument is <= 0, and a
@@ -131,7 +128,7 @@ __device__ __forceinline__ float soft_scale(float invT) { return invT * 1.442695
 template <int DPD>
 __device__ __forceinline__ float soft_argmin(const float (&s)[DPD], int l, float invT, float* mn_out,
                                              float* z_out) {
-    const float mn = row_minf(lane_min(s));
+    const float mn = row_min(lane_min(s));
     const float c = soft_scale(invT);
     float z = 0.f, acc = 0.f;
 #pragma unroll
@@ -157,6 +154,100 @@ __device__ __forceinline__ void grad_s_from(const float (&s)[DPD], float mn, flo
 #pragma unroll
     for (int k = 0; k < DPD; ++k)
         g[k] = coef * soft_weight(s[k], mn, c) * ((float)(l * DPD + k) - dq);
+}
+
+// Row reductions of several values stage by stage: a DPP read has to wait two
+// states after the write of its register, which the other values' moves fill.
+__device__ __forceinline__ void row_min_both(float& a, float& b) {
+    asm("s_nop 1\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_min_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_min_f32_dpp %1, %1, %1 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_min_f32_dpp %1, %1, %1 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_min_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_min_f32_dpp %1, %1, %1 row_ror:1 row_mask:0xf bank_mask:0xf"
+        : "+v"(a), "+v"(b));
+}
+template <int CTRL, int N>
+__device__ __forceinline__ void add_stage(float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dppf<CTRL>(0.f, v[i]);
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int N>
+__device__ __forceinline__ void row_sums(float (&v)[N]) {
+    add_stage<0x128>(v);
+    add_stage<0x124>(v);
+    add_stage<0x122>(v);
+    add_stage<0x121>(v);
+}
+// smallest d with L(d) == m in a lane (none: a large value)
+template <int DPD>
+__device__ __forceinline__ int lane_argmin(const float (&L)[DPD], float m, int l) {
+    int idx = 0x7FFFFFFF;
+#pragma unroll
+    for (int k = DPD - 1; k >= 0; --k)
+        if (L[k] == m) idx = l * DPD + k;
+    return idx;
+}
+template <int CTRL>
+__device__ __forceinline__ void min_stage(int& a, int& b) {
+    a = min(a, dppi<CTRL>(0, a));
+    b = min(b, dppi<CTRL>(0, b));
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void row_min_both(int& a, int& b) {
+    min_stage<0x128>(a, b);
+    min_stage<0x124>(a, b);
+    min_stage<0x122>(a, b);
+    min_stage<0x121>(a, b);
+}
+
+// What a pixel's gradient G of one direction hands to the pixel before it
+// (w, ks: the pixel's winner codes and the previous pixel's argmin), and the
+// lane's shares of its penalty gradients.
+// The codes' two bits become masks, so a share is one three-input bit
+// operation; F is left without the argmin's term, whose amount is less the
+// sum of F (a code 3 hands nothing on).
+template <int DPD>
+__device__ __forceinline__ float bwd_flow(const float (&G)[DPD], uint32_t w, float (&F)[DPD], float* s12, float* s3) {
+    float A1[DPD], A2[DPD], a12 = 0.f, a3 = 0.f, rest = 0.f;
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) {
+        const uint32_t g = __builtin_bit_cast(uint32_t, G[k]);
+        // written out: the compiler turns shifted masks into compares and selects
+        uint32_t b0, b1;
+        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(b0) : "v"(w), "i"(2 * k));
+        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(b1) : "v"(w), "i"(2 * k + 1));
+        F[k] = __builtin_bit_cast(float, g & ~(b0 | b1));
+        A1[k] = __builtin_bit_cast(float, g & b0 & ~b1);   // to d - 1
+        A2[k] = __builtin_bit_cast(float, g & b1 & ~b0);   // to d + 1
+        a3 += __builtin_bit_cast(float, g & b0 & b1);
+        a12 += A1[k] + A2[k];
+    }
+    const float a1_next = dppf<kShl1>(0.f, A1[0]);
+    const float a2_prev = dppf<kShr1>(0.f, A2[DPD - 1]);
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) {
+        F[k] += (k == DPD - 1) ? a1_next : A1[k + 1 < DPD ? k + 1 : k];
+        F[k] += (k == 0) ? a2_prev : A2[k > 0 ? k - 1 : 0];
+        rest += F[k];
+    }
+    *s12 = a12;
+    *s3 = a3;
+    return rest;
+}
+// the argmin's term, to disparity ks
+template <int DPD>
+__device__ __forceinline__ void bwd_jump(float (&F)[DPD], int ks, float rest, int l) {
+    const int kl = ks - l * DPD;
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) F[k] -= (kl == k) ? rest : 0.f;
 }
 
 }  // namespace dsgm

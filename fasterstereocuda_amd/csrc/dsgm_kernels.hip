@@ -14,11 +14,13 @@
 // L'(d+1)+P1, m'+P2] wins; m' = L'(k*) with k* the smallest argmin.
 //
 // Memory: S is built in place and no per-direction volume is kept.  The
-// forward's first launch runs, per group of 4 rows, left->right (S = L_1)
-// and then right->left (S += L_3) in one wave, so the second pass adds onto
-// the first with no other writer; beside them the top->bottom groups write
-// L_0 into the one workspace volume.  The second launch runs bottom->top,
-// forms S = (S + L_0) + L_2 and the soft-argmin, and keeps the minimum of S
+// forward's first launch runs, per pair of rows, left->right and right->left
+// at the same time in one wave: each pixel is reached by one direction in the
+// first half of the walk, which stores its L, and by the other in the second
+// half, which adds onto it (two-term sums commute, so S = L_1 + L_3 whichever
+// came first).  Beside them the top->bottom groups write L_0 into the one
+// workspace volume.  The second launch runs bottom->top, forms
+// S = (S + L_0) + L_2 and the soft-argmin, and keeps the minimum of S
 // and the softmax normaliser per pixel.  Every direction also saves, per
 // step, the winner code of each disparity (2 bits) and k* of the previous
 // step's L (one byte per pixel): 1 byte per cell over the four directions,
@@ -26,15 +28,26 @@
 // forward.  The backward walks each scanline from its last step to its
 // first, once:
 //   G(s-1, d) = gS(s-1, d) + G(s, d)[w(s,d)=0] + G(s, d+1)[w(s,d+1)=1]
-//             + G(s, d-1)[w(s,d-1)=2] + [d = k*(s-1)] (sum_e G(s,e)[w(s,e)=3] - sum_e G(s,e))
+//             + G(s, d-1)[w(s,d-1)=2] - [d = k*(s-1)] sum_e G(s,e)[w(s,e)!=3]
 // with gS = dLoss/dS formed from S, the kept minimum and normaliser, and
 // emits dC_r(s, d) = G(s, d), dP1_r(s) = sum_d G(s,d)[w in {1,2}],
 // dP2_r(s) = sum_d G(s,d)[w = 3].  Its launches mirror the forward's: dC,
 // dP1 and dP2 are built in place by the horizontal pairs, the top->bottom
 // terms go to the workspace, and bottom->top adds both in the same order as S.
 //
-// Layout per wave as in the integer aggregation: four 16-lane DPP rows, one
-// scanline per row, D/16 disparities per lane.
+// Layout per wave: four 16-lane DPP rows, one scanline per row (two rows in
+// both directions, or four columns), D/16 disparities per lane.  Lanes past
+// the image repeat its last line: same values, same addresses.
+//
+// What bounds these passes: for one image or a few, the chain of a scanline's
+// steps, max(H, W) + H forward and again backward, each 130-300 instructions
+// of a wave that has its SIMD to itself; for many, the copy rate (93 bytes per
+// cell).  Walking a row's directions one after the other made the chain
+// 2 W + H: 2 images 321x119 D = 64 0.57 -> 0.28 ms forward + backward, one
+// image 1242x375 D = 128 3.24 -> 1.58, D = 256 6.04 -> 3.28 ms, 4 images
+// D = 64 3.13 -> 2.37 ms.
+#include <type_traits>
+
 #include "dsgm_device.h"
 #include "sgm_device.h"
 
@@ -44,411 +57,434 @@ namespace fsgm {
 using namespace dsgm;
 namespace {
 
-// Geometry of one scanline of one direction.
-struct LineGeo {
-    int n;            // steps
-    int line;         // row (horizontal) or column (vertical)
-    bool active;
-    int64_t pix0;     // pixel index of step 0 within the image
-    int64_t pstep;    // pixel index increment per step
-};
+// Steps of loads in flight: a wave that is alone on its SIMD would otherwise
+// wait the memory latency at every step.  The inputs of step s + kAhead are
+// issued right after step s has used its slot; steps past the end load the
+// last pixel again and are not used.
+// (Fewer at D = 256, where four would pass the 256 vector registers.)
+template <int D, bool LAST> constexpr int kAhead = D < 256 ? 4 : LAST ? 2 : 3;
 
-__device__ __forceinline__ LineGeo line_geo(const DsgmArgs& A, int path, int group, int sub) {
-    LineGeo g;
-    const bool horiz = (path == 1 || path == 3);
-    const bool fwd = (path == 0 || path == 1);
-    const int H = A.H, W = A.W;
-    const int nlines = horiz ? H : W;
-    int line = group * 4 + sub;
-    g.active = line < nlines;
-    if (!g.active) line = nlines - 1;
-    g.line = line;
-    g.n = horiz ? W : H;
-    if (horiz) {
-        g.pix0 = (int64_t)line * W + (fwd ? 0 : W - 1);
-        g.pstep = fwd ? 1 : -1;
-    } else {
-        g.pix0 = (int64_t)(fwd ? 0 : H - 1) * W + line;
-        g.pstep = fwd ? W : -W;
-    }
-    return g;
+// Offsets of a scanline's cells from a wave-uniform base: 32 bits unless the
+// image is so wide that two of its rows pass 2^31 bytes.
+template <bool WIDE> using Off = std::conditional_t<WIDE, int64_t, uint32_t>;
+
+template <int D, class T, class O>
+__device__ __forceinline__ T* cell_at(T* base, O pix, int l) {
+    return base + ((O)(pix * D) + (O)(l * (D / 16)));
 }
+// Winner codes are loaded as the dword that holds the lane's: the masking of a
+// 1- or 2-byte load would wait at the top of the loop for the whole ring.
+// (The codes of a pixel are D / 4 bytes, and the buffer starts on 8.)
+template <int D>
+__device__ __forceinline__ uint32_t load_codes(const uint8_t* pixel, int l) {
+    return *(const __attribute__((address_space(1))) uint32_t*)(pixel + ((l * (D / 64)) & ~3));
+}
+template <int D>
+__device__ __forceinline__ uint32_t shift_codes(uint32_t w, int l) { return w >> (8 * ((l * (D / 64)) & 3)); }
+template <int D>
+__device__ __forceinline__ void store_codes(uint8_t* pixel, int l, uint32_t w) {
+    *(__attribute__((address_space(1))) WinWord<D>*)(pixel + l * (D / 64)) = (WinWord<D>)w;
+}
+__device__ __forceinline__ void storeb(uint8_t* p, int v) { *(__attribute__((address_space(1))) uint8_t*)p = (uint8_t)v; }
+__device__ __forceinline__ int loadb(const uint8_t* p) { return *(const __attribute__((address_space(1))) uint8_t*)p; }
+__device__ __forceinline__ void store1(float* p, float v) { *(g_f*)p = v; }
+
+// Two rows of an image, walked from both ends at once: lanes 0-31 left->right
+// and lanes 32-63 right->left (in the backward, each reversed: lanes 0-31 from
+// the right).  At step t every lane is t pixels into its direction's walk.
+template <bool WIDE>
+struct RowPair {
+    int W, n1, n2;             // steps that reach a pixel first; first step that reaches one second
+    bool second;               // this lane walks right->left
+    Off<WIDE> pix0, step;      // pixel of step 0 from the pair's first, its move (all ones: -1)
+    int64_t q0;                // the pair's first pixel in the batch
+    __device__ RowPair(const DsgmArgs& A, int b, int g, int lane, bool reversed) {
+        W = A.W;
+        n1 = W / 2;
+        n2 = (W + 1) / 2;
+        const int sub = lane >> 4;
+        second = sub >= 2;
+        const bool from_right = second != reversed;
+        const int row = min(2 * g + (sub & 1), A.H - 1) - 2 * g;
+        pix0 = (Off<WIDE>)row * (Off<WIDE>)W + (Off<WIDE>)(from_right ? W - 1 : 0);
+        step = from_right ? (Off<WIDE>)-1 : (Off<WIDE>)1;
+        q0 = ((int64_t)b * A.H + 2 * g) * W;
+    }
+    __device__ Off<WIDE> pix(int t) const { return pix0 + step * (Off<WIDE>)t; }
+    // a walk's next pixel, staying on the last one (t: the step moved to)
+    __device__ Off<WIDE> move(Off<WIDE> p, int t) const { return t < W ? p + step : p; }
+};
+// the other direction's value of the same row
+__device__ __forceinline__ float other_half(float v, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, v)));
+}
+
+// Runs n steps with NA of them loaded ahead: whole blocks, then the remainder.
+// (An exit from the middle of a block would join the loop's head, whose wait
+// counts would then cover the shortest path: every block would wait for loads
+// just issued.)
+template <int NA, class Issue, class Step>
+__device__ __forceinline__ void run_steps(int n, Issue issue, Step step) {
+#pragma unroll
+    for (int u = 0; u < NA; ++u) issue(u);
+    int blocks = n / NA;
+    const int rest = n - blocks * NA;
+    if (blocks > 0) {
+        do {
+#pragma unroll
+            for (int u = 0; u < NA; ++u) {
+                step(u);
+                issue(u);
+            }
+        } while (--blocks > 0);
+    }
+#pragma unroll
+    for (int u = 0; u < NA - 1; ++u)
+        if (u < rest) step(u);
+}
+
+// Three phases of a pair of walks: pixels reached first (STORE), a middle
+// pixel reached by both at once when W is odd (both halves hold the sum), and
+// pixels reached second (ADD).
+enum PairPhase { kPairStore = 0, kPairMiddle = 1, kPairAdd = 2 };
 
 // ------------------------------------------------------------- forward ---
-// What a forward pass does with each step's L.
-enum FwdMode {
-    kFwdStoreS = 0,   // S = L          (left->right, first of the horizontal pair)
-    kFwdAddS = 1,     // S = S + L      (right->left, second of the pair)
-    kFwdStoreY = 2,   // Y = L          (top->bottom, into the workspace volume)
-    kFwdLast = 3,     // S = (S + Y) + L, then the soft-argmin (bottom->top)
-};
+template <int D, bool WIDE>
+__device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int lane) {
+    constexpr int DPD = D / 16, NA = kAhead<D, false>;
+    const float inf = __builtin_inff();
+    const int l = lane & 15;
+    const RowPair<WIDE> rp(A, b, g, lane, false);
+    const int64_t npix = (int64_t)A.B * A.H * A.W;
+    const float* cost = A.cost + rp.q0 * D;
+    float* S = A.S + rp.q0 * D;
+    const float *p1 = A.p1 + rp.q0, *p2 = A.p2 + rp.q0;
+    const int64_t line0 = (rp.second ? 3 : 1) * npix + rp.q0;
+    uint8_t* wout = A.wins + line0 * (D / 4);
+    uint8_t* kout = A.kstar + line0;
 
-// Loads run ahead of the arithmetic: a scanline step needs its inputs from
-// HBM, and a lone wave (the long horizontal pairs run about one per SIMD)
-// would otherwise wait the full memory latency at every step.  The inputs of
-// step s + kAheadF are issued right after step s has used its slot, into
-// register slots indexed by s % kAheadF (compile-time within the unrolled
-// block).  Steps past the end load the last pixel again and are never used.
-constexpr int kAheadF = 4;
-
-// One direction over a scanline group (forward), saving each step's winner
-// codes and the previous step's argmin for the backward.
-template <int D, int MODE>
-__device__ __forceinline__ void fwd_lines(const DsgmArgs& A, int b, int path, int group, int lane) {
-    constexpr int DPD = D / 16;
-    constexpr bool kPriorS = MODE == kFwdAddS || MODE == kFwdLast;
-    constexpr bool kPriorY = MODE == kFwdLast;
-    const int sub = lane >> 4, l = lane & 15;
-    const LineGeo g = line_geo(A, path, group, sub);
-    const int64_t img = (int64_t)A.H * A.W;
-    const float* cost = A.cost + (int64_t)b * img * D + l * DPD;
-    const float* p1 = A.p1 + (int64_t)b * img;
-    const float* p2 = A.p2 + (int64_t)b * img;
-    float* S = A.S + (int64_t)b * img * D + l * DPD;
-    float* Y = A.vol + (int64_t)b * img * D + l * DPD;
-    float* disp = A.disp + (int64_t)b * img;
-    float* stats = A.stats + (int64_t)b * img * 2;
-    const int64_t npix = (int64_t)A.B * img;
-    // saved for the backward: each step's winner codes (this lane's DPD
-    // disparities) and k* of the previous step's L
-    WinWord<D>* wout = reinterpret_cast<WinWord<D>*>(A.wins) + ((int64_t)path * npix + (int64_t)b * img) * 16 + l;
-    uint8_t* kout = A.kstar + (int64_t)path * npix + (int64_t)b * img;
-    const float invT = A.inv_temperature;
-    const int n = g.n;
-
-    // inputs of the steps in flight: cost, penalties, and what the pixel's
-    // earlier passes left (S, and Y for the last pass)
-    float qc[kAheadF][DPD], qp1[kAheadF], qp2[kAheadF];
-    float qs[kAheadF][DPD], qy[kAheadF][DPD];
-    auto issue = [&](int slot, int s) __attribute__((always_inline)) {
-        const int64_t q = g.pix0 + (int64_t)min(s, n - 1) * g.pstep;
-        loadf<DPD>(cost + q * D, qc[slot]);
-        qp1[slot] = loads(p1 + q);
-        qp2[slot] = loads(p2 + q);
-        if constexpr (kPriorS) loadf<DPD>(S + q * D, qs[slot]);
-        if constexpr (kPriorY) loadf<DPD>(Y + q * D, qy[slot]);
-    };
-    auto emit = [&](int64_t q, const float (&L)[DPD], int slot) __attribute__((always_inline)) {
-        if constexpr (MODE == kFwdLast) {
-            float sv[DPD];
-#pragma unroll
-            for (int k = 0; k < DPD; ++k) sv[k] = (qs[slot][k] + qy[slot][k]) + L[k];
-            float mn, z;
-            const float d = soft_argmin<DPD>(sv, l, invT, &mn, &z);
-            if (g.active) {
-                storef<DPD>(S + q * D, sv);
-                if (l == 0) {
-                    disp[q] = d;
-                    stats[2 * q] = mn;
-                    stats[2 * q + 1] = z;
-                }
-            }
-        } else if constexpr (MODE == kFwdAddS) {
-            float sv[DPD];
-#pragma unroll
-            for (int k = 0; k < DPD; ++k) sv[k] = qs[slot][k] + L[k];
-            if (g.active) storef<DPD>(S + q * D, sv);
-        } else {
-            if (g.active) storef<DPD>((MODE == kFwdStoreS ? S : Y) + q * D, L);
-        }
-    };
-
-#pragma unroll
-    for (int u = 0; u < kAheadF; ++u) issue(u, u);
+    float qc[NA][DPD], qp1[NA], qp2[NA], qs[NA][DPD];
     float L[DPD];
-    float m = 0.f;
-    for (int s0 = 0; s0 < n; s0 += kAheadF) {
 #pragma unroll
-        for (int u = 0; u < kAheadF; ++u) {
-            const int s = s0 + u;
-            if (s < n) {
-                const int64_t pix = g.pix0 + (int64_t)s * g.pstep;
-                if (s == 0) {
+    for (int k = 0; k < DPD; ++k) L[k] = 0.f;   // with infinite penalties: L = C at the first step
+
+    auto walk = [&](auto phase, int t0, int t1) __attribute__((always_inline)) {
+        constexpr int PHASE = decltype(phase)::value;
+        if (t0 >= t1) return;
+        Off<WIDE> pi = rp.pix(t0), ps = pi;      // pixels of the next issue and of the step
+        int ti = t0;
+        auto issue = [&](int u) __attribute__((always_inline)) {
+            loadf<DPD>(cell_at<D>(cost, pi, l), qc[u]);
+            if constexpr (PHASE == kPairAdd) loadf<DPD>(cell_at<D>(S, pi, l), qs[u]);
+            qp1[u] = loads(p1 + pi);
+            qp2[u] = loads(p2 + pi);
+            pi = rp.move(pi, ++ti);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int t = t0;
+        auto step = [&](int u) __attribute__((always_inline)) {
+            const float m = row_min(lane_min(L));
+            const int ks = row_mini(lane_argmin<DPD>(L, m, l));
+            const bool start = PHASE != kPairAdd && t == 0;
+            const uint32_t w = fwd_step<DPD>(L, qc[u], m, start ? inf : qp1[u], start ? inf : qp2[u]);
+            float sv[DPD];
 #pragma unroll
-                    for (int k = 0; k < DPD; ++k) L[k] = qc[u][k];
-                } else {
-                    const int ks = row_argmin<DPD>(L, m, l);
-                    const uint32_t w = fwd_step<DPD>(L, qc[u], m, qp1[u], qp2[u]);
-                    if (g.active) {
-                        wout[pix * 16] = (WinWord<D>)w;
-                        if (l == 0) kout[pix] = (uint8_t)ks;
-                    }
-                }
-                m = row_minf(lane_min(L));
-                emit(pix, L, u);
+            for (int k = 0; k < DPD; ++k) {
+                sv[k] = L[k];
+                if constexpr (PHASE == kPairAdd) sv[k] = qs[u][k] + L[k];
+                if constexpr (PHASE == kPairMiddle) sv[k] = L[k] + other_half(L[k], lane);
             }
-            issue(u, s + kAheadF);
+            storef<DPD>(cell_at<D>(S, ps, l), sv);
+            store_codes<D>(wout + (int64_t)ps * (D / 4), l, w);
+            storeb(kout + ps, ks);           // sixteen lanes, one value
+            ps += rp.step;
+            ++t;
+        };
+        if constexpr (PHASE == kPairMiddle) {    // one step at most
+            issue(0);
+            step(0);
+        } else {
+            run_steps<NA>(t1 - t0, issue, step);
         }
-    }
+    };
+    walk(std::integral_constant<int, kPairStore>{}, 0, rp.n1);
+    walk(std::integral_constant<int, kPairMiddle>{}, rp.n1, rp.n2);
+    // the other lanes' stores of the pixels that this phase loads
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.W);
 }
 
-// Items of the first launch (forward or backward): the horizontal pairs of
-// every image (4 rows each, left->right then right->left in one wave, so the
-// second accumulates onto the first without another writer), then the
-// top->bottom groups (4 columns each).  The long pairs are dispatched first.
-// The second launch is the bottom->top groups.  Column groups are spread so
-// that each XCD walks a contiguous run of them: the per-pixel maps (penalties,
-// statistics, disparity, gradients) of 32 neighbouring columns share a
-// 128-byte line, which is then fetched into one L2 instead of eight.
-__device__ __forceinline__ void first_item(const DsgmArgs& A, int item, int* b, bool* pair, int* group) {
-    const int nh = (A.H + 3) / 4, nv = (A.W + 3) / 4;
-    const int hp = A.B * nh;
-    *pair = item < hp;
-    const int local = *pair ? item : dev::xcd_item(item - hp, A.B * nv);
-    const int per = *pair ? nh : nv;
-    *b = local / per;
-    *group = local - *b * per;
-}
+// Four columns, top->bottom into the workspace volume or (LAST) bottom->top
+// with the sum and the soft-argmin.
+template <int D, bool LAST, bool WIDE>
+__device__ __forceinline__ void fwd_cols(const DsgmArgs& A, int b, int group, int lane) {
+    constexpr int DPD = D / 16, NA = kAhead<D, LAST>;
+    const float inf = __builtin_inff();
+    const int l = lane & 15, W = A.W, H = A.H;
+    const Off<WIDE> col = (Off<WIDE>)min(group * 4 + (lane >> 4), W - 1);
+    const int64_t npix = (int64_t)A.B * H * W, img = (int64_t)b * H * W, path = LAST ? 2 : 0;
 
-template <int D>
-__global__ __launch_bounds__(64) void dsgm_forward_first_kernel(DsgmArgs A) {
-    int b, group;
-    bool pair;
-    first_item(A, blockIdx.x, &b, &pair, &group);
-    if (pair) {
-        fwd_lines<D, kFwdStoreS>(A, b, 1, group, threadIdx.x);
-        fwd_lines<D, kFwdAddS>(A, b, 3, group, threadIdx.x);
-    } else {
-        fwd_lines<D, kFwdStoreY>(A, b, 0, group, threadIdx.x);
-    }
-}
-
-template <int D>
-__global__ __launch_bounds__(64) void dsgm_forward_last_kernel(DsgmArgs A) {
-    const int nv = (A.W + 3) / 4;
-    const int item = dev::xcd_item(blockIdx.x, gridDim.x);
-    const int b = item / nv, group = item - b * nv;
-    fwd_lines<D, kFwdLast>(A, b, 2, group, threadIdx.x);
+    float qc[NA][DPD], qs[NA][DPD], qy[NA][DPD], qp1[NA], qp2[NA];
+    int si = 0;
+    auto issue = [&](int u) __attribute__((always_inline)) {
+        const int s = min(si++, H - 1);
+        const int64_t r0 = img + (int64_t)(LAST ? H - 1 - s : s) * W;
+        loadf<DPD>(cell_at<D>(A.cost + r0 * D, col, l), qc[u]);
+        qp1[u] = loads(A.p1 + r0 + col);
+        qp2[u] = loads(A.p2 + r0 + col);
+        if constexpr (LAST) {
+            loadf<DPD>(cell_at<D>(A.S + r0 * D, col, l), qs[u]);
+            loadf<DPD>(cell_at<D>(A.vol + r0 * D, col, l), qy[u]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float L[DPD];
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) L[k] = 0.f;
+    int s = 0;
+    auto step = [&](int u) __attribute__((always_inline)) {
+        const int64_t r0 = img + (int64_t)(LAST ? H - 1 - s : s) * W;
+        const float m = row_min(lane_min(L));
+        const int ks = row_mini(lane_argmin<DPD>(L, m, l));
+        const uint32_t w = fwd_step<DPD>(L, qc[u], m, s == 0 ? inf : qp1[u], s == 0 ? inf : qp2[u]);
+        store_codes<D>(A.wins + (path * npix + r0) * (D / 4) + (Off<WIDE>)(col * (D / 4)), l, w);
+        storeb(A.kstar + path * npix + r0 + col, ks);
+        if constexpr (LAST) {
+            float sv[DPD], mn, z;
+#pragma unroll
+            for (int k = 0; k < DPD; ++k) sv[k] = (qs[u][k] + qy[u][k]) + L[k];
+            storef<DPD>(cell_at<D>(A.S + r0 * D, col, l), sv);
+            const float d = soft_argmin<DPD>(sv, l, A.inv_temperature, &mn, &z);
+            store1(A.disp + r0 + col, d);
+            store1(A.stats + 2 * r0 + 2 * col, mn);
+            store1(A.stats + 2 * r0 + 2 * col + 1, z);
+        } else {
+            storef<DPD>(cell_at<D>(A.vol + r0 * D, col, l), L);
+        }
+        ++s;
+    };
+    run_steps<NA>(H, issue, step);
 }
 
 // ------------------------------------------------------------ backward ---
-template <int DPD>
-__device__ __forceinline__ void grad_s_at(const DsgmArgs& A, const float* Sb, const float* stats,
-                                          const float* disp, const float* gdisp, int64_t q, int l,
-                                          float (&g)[DPD]) {
-    float s[DPD];
-    loadf<DPD>(Sb + q * A.D, s);
-    grad_s_from<DPD>(s, loads(stats + 2 * q), loads(stats + 2 * q + 1), loads(gdisp + q),
-                     loads(disp + q), A.inv_temperature, l, g);
-}
+template <int D, bool WIDE>
+__device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int lane) {
+    constexpr int DPD = D / 16, NA = kAhead<D, false>;
+    const int l = lane & 15;
+    const RowPair<WIDE> rp(A, b, g, lane, true);
+    const int64_t npix = (int64_t)A.B * A.H * A.W;
+    const float *S = A.S + rp.q0 * D, *stats = A.stats + 2 * rp.q0;
+    const float *disp = A.disp + rp.q0, *gdisp = A.grad_disp + rp.q0;
+    float *dc = A.grad_cost + rp.q0 * D, *dp1 = A.grad_p1 + rp.q0, *dp2 = A.grad_p2 + rp.q0;
+    const int64_t line0 = (rp.second ? 3 : 1) * npix + rp.q0;
+    const uint8_t* win = A.wins + line0 * (D / 4);
+    const uint8_t* kin = A.kstar + line0;
 
-// What a backward pass does with each pixel's gradients of its direction.
-enum BwdMode {
-    kBwdStore = 0,    // dC = G, dP1 = d1, dP2 = d2            (left->right)
-    kBwdAdd = 1,      // dC += G, dP1 += d1, dP2 += d2         (right->left)
-    kBwdStoreY = 2,   // workspace: gY = G, gY1 = d1, gY2 = d2 (top->bottom)
-    kBwdLast = 3,     // dC = (dC + gY) + G, likewise dP1, dP2 (bottom->top)
-};
+    float qs[NA][DPD], qmn[NA], qz[NA], qg[NA], qd[NA], qo[NA][DPD], qo1[NA], qo2[NA];
+    uint32_t qw[NA];
+    int qk[NA];
+    float F[DPD];                              // what the pixel after this one hands to it
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) F[k] = 0.f;
 
-// Loads ahead in the backward: what transition s needs (its winner codes
-// and k*, S and the soft-argmin statistics of the pixel before it, and, for
-// the passes that accumulate, the gradients the pixel already holds) is
-// issued kAheadV transitions earlier, into register slots indexed by the
-// position within an unrolled block.  Loads for transitions below 1 read
-// transition 1 again and are not used.
-constexpr int kAheadV = 4;
-
-// One direction's reverse recurrence over a scanline group.
-template <int D, int MODE>
-__device__ __forceinline__ void bwd_lines(const DsgmArgs& A, int b, int path, int group, int lane) {
-    constexpr int DPD = D / 16;
-    constexpr int V = kAheadV;
-    constexpr bool kPriorC = MODE == kBwdAdd || MODE == kBwdLast;
-    constexpr bool kPriorY = MODE == kBwdLast;
-    const int sub = lane >> 4, l = lane & 15;
-    const LineGeo g = line_geo(A, path, group, sub);
-    const int64_t img = (int64_t)A.H * A.W;
-    const int64_t npix = (int64_t)A.B * img;
-    const float* Sb = A.S + (int64_t)b * img * D + l * DPD;
-    const float* stats = A.stats + (int64_t)b * img * 2;
-    const float* dsp = A.disp + (int64_t)b * img;
-    const float* gdisp = A.grad_disp + (int64_t)b * img;
-    const WinWord<D>* win = reinterpret_cast<const WinWord<D>*>(A.wins) +
-                            ((int64_t)path * npix + (int64_t)b * img) * 16 + l;
-    const uint8_t* kin = A.kstar + (int64_t)path * npix + (int64_t)b * img;
-    float* out_c = A.grad_cost + (int64_t)b * img * D + l * DPD;
-    float* out_p1 = A.grad_p1 + (int64_t)b * img;
-    float* out_p2 = A.grad_p2 + (int64_t)b * img;
-    float* gy = A.vol + (int64_t)b * img * D + l * DPD;
-    float* gy1 = A.vol_p1 + (int64_t)b * img;
-    float* gy2 = A.vol_p2 + (int64_t)b * img;
-    const int n = g.n;
-    const float invT = A.inv_temperature;
-    auto pix_at = [&](int s) __attribute__((always_inline)) { return g.pix0 + (int64_t)s * g.pstep; };
-
-    // inputs of the transitions in flight
-    uint32_t vw[V], vk[V];
-    float vs[V][DPD], vmn[V], vz[V], vgd[V], vdq[V];
-    float vo[V][DPD], vo1[V], vo2[V];
-    float vy[V][DPD], vy1[V], vy2[V];
-    auto issue = [&](int slot, int s) __attribute__((always_inline)) {
-        if (n < 2) return;   // no transitions
-        const int64_t q = pix_at(max(s, 1)), qp = q - g.pstep;
-        vw[slot] = win[q * 16];
-        vk[slot] = kin[q];
-        loadf<DPD>(Sb + qp * D, vs[slot]);
-        vmn[slot] = loads(stats + 2 * qp);
-        vz[slot] = loads(stats + 2 * qp + 1);
-        vgd[slot] = loads(gdisp + qp);
-        vdq[slot] = loads(dsp + qp);
-        if constexpr (kPriorC) {
-            loadf<DPD>(out_c + q * D, vo[slot]);
-            vo1[slot] = loads(out_p1 + q);
-            vo2[slot] = loads(out_p2 + q);
-        }
-        if constexpr (kPriorY) {
-            loadf<DPD>(gy + q * D, vy[slot]);
-            vy1[slot] = loads(gy1 + q);
-            vy2[slot] = loads(gy2 + q);
-        }
-    };
-    // writes this direction's gradients of one pixel; o, o1, o2 (and y, y1,
-    // y2) are what the pixel held before, for the passes that accumulate
-    auto emit = [&](int64_t q, const float (&G)[DPD], float d1, float d2, const float (&o)[DPD],
-                    float o1, float o2, const float (&y)[DPD], float y1, float y2)
-        __attribute__((always_inline)) {
-        if (!g.active) return;
-        if constexpr (MODE == kBwdStore || MODE == kBwdStoreY) {
-            float* oc = MODE == kBwdStore ? out_c : gy;
-            storef<DPD>(oc + q * D, G);
-            if (l == 0) {
-                (MODE == kBwdStore ? out_p1 : gy1)[q] = d1;
-                (MODE == kBwdStore ? out_p2 : gy2)[q] = d2;
+    auto walk = [&](auto phase, int t0, int t1) __attribute__((always_inline)) {
+        constexpr int PHASE = decltype(phase)::value;
+        if (t0 >= t1) return;
+        Off<WIDE> pi = rp.pix(t0), ps = pi;
+        int ti = t0;
+        auto issue = [&](int u) __attribute__((always_inline)) {
+            loadf<DPD>(cell_at<D>(S, pi, l), qs[u]);
+            qmn[u] = loads(stats + 2 * pi);
+            qz[u] = loads(stats + 2 * pi + 1);
+            qg[u] = loads(gdisp + pi);
+            qd[u] = loads(disp + pi);
+            qw[u] = load_codes<D>(win + (int64_t)pi * (D / 4), l);
+            qk[u] = loadb(kin + pi);
+            if constexpr (PHASE == kPairAdd) {
+                loadf<DPD>(cell_at<D>(dc, pi, l), qo[u]);
+                qo1[u] = loads(dp1 + pi);
+                qo2[u] = loads(dp2 + pi);
             }
+            pi = rp.move(pi, ++ti);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int t = t0;
+        auto step = [&](int u) __attribute__((always_inline)) {
+            float G[DPD], v[DPD], s12, s3;
+            grad_s_from<DPD>(qs[u], qmn[u], qz[u], qg[u], qd[u], A.inv_temperature, l, G);
+#pragma unroll
+            for (int k = 0; k < DPD; ++k) G[k] += F[k];
+            // the direction's first pixel (the walk's last) hands on
+            // nothing and has no penalty gradient: code 0 everywhere
+            const uint32_t w = t == rp.W - 1 ? 0u : shift_codes<D>(qw[u], l);
+            float sums[3];
+            sums[0] = bwd_flow<DPD>(G, w, F, &s12, &s3);
+            sums[1] = s12;
+            sums[2] = s3;
+            row_sums(sums);
+            bwd_jump<DPD>(F, qk[u], sums[0], l);
+#pragma unroll
+            for (int k = 0; k < DPD; ++k) {
+                v[k] = G[k];
+                if constexpr (PHASE == kPairAdd) v[k] = qo[u][k] + G[k];
+                if constexpr (PHASE == kPairMiddle) v[k] = G[k] + other_half(G[k], lane);
+            }
+            if constexpr (PHASE == kPairAdd) {
+                sums[1] = qo1[u] + sums[1];
+                sums[2] = qo2[u] + sums[2];
+            }
+            if constexpr (PHASE == kPairMiddle) {
+                sums[1] += other_half(sums[1], lane);
+                sums[2] += other_half(sums[2], lane);
+            }
+            storef<DPD>(cell_at<D>(dc, ps, l), v);
+            store1(dp1 + ps, sums[1]);
+            store1(dp2 + ps, sums[2]);
+            ps += rp.step;
+            ++t;
+        };
+        if constexpr (PHASE == kPairMiddle) {    // one step at most
+            issue(0);
+            step(0);
         } else {
-            float v[DPD];
-#pragma unroll
-            for (int k = 0; k < DPD; ++k) v[k] = (MODE == kBwdLast) ? (o[k] + y[k]) + G[k] : o[k] + G[k];
-            storef<DPD>(out_c + q * D, v);
-            if (l == 0) {
-                out_p1[q] = (MODE == kBwdLast) ? (o1 + y1) + d1 : o1 + d1;
-                out_p2[q] = (MODE == kBwdLast) ? (o2 + y2) + d2 : o2 + d2;
-            }
+            run_steps<NA>(t1 - t0, issue, step);
         }
     };
+    walk(std::integral_constant<int, kPairStore>{}, 0, rp.n1);
+    walk(std::integral_constant<int, kPairMiddle>{}, rp.n1, rp.n2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.W);
+}
 
-    float G[DPD];
-    grad_s_at<DPD>(A, Sb, stats, dsp, gdisp, pix_at(n - 1), l, G);
-#pragma unroll
-    for (int u = 0; u < V; ++u) issue(u, n - 1 - u);
-    for (int s0 = n - 1; s0 >= 1; s0 -= V) {
-#pragma unroll
-        for (int u = 0; u < V; ++u) {
-            const int s = s0 - u;    // the transition s-1 -> s, in slot u
-            if (s >= 1) {
-                const int64_t pix = pix_at(s);
-                const uint32_t w = vw[u];
-                float all = 0.f, s3 = 0.f, s12 = 0.f;
-                float A1[DPD], A2[DPD];
-#pragma unroll
-                for (int k = 0; k < DPD; ++k) {
-                    const uint32_t wk = (w >> (2 * k)) & 3u;
-                    all += G[k];
-                    s3 += (wk == 3u) ? G[k] : 0.f;
-                    s12 += (wk == 1u || wk == 2u) ? G[k] : 0.f;
-                    A1[k] = (wk == 1u) ? G[k] : 0.f;   // flows to d-1
-                    A2[k] = (wk == 2u) ? G[k] : 0.f;   // flows to d+1
-                }
-                all = row_sumf(all);
-                s3 = row_sumf(s3);
-                s12 = row_sumf(s12);
-                emit(pix, G, s12, s3, vo[u], vo1[u], vo2[u], vy[u], vy1[u], vy2[u]);
-                const float a1_next = dppf<kShl1>(0.f, A1[0]);        // lane+1, d = lane end + 1
-                const float a2_prev = dppf<kShr1>(0.f, A2[DPD - 1]);  // lane-1, d = lane start - 1
-                const int ks = (int)vk[u];
-                float gprev[DPD];
-                grad_s_from<DPD>(vs[u], vmn[u], vz[u], vgd[u], vdq[u], invT, l, gprev);
-                const float jump = s3 - all;
-#pragma unroll
-                for (int k = 0; k < DPD; ++k) {
-                    const uint32_t wk = (w >> (2 * k)) & 3u;
-                    float x = gprev[k];
-                    x += (wk == 0u) ? G[k] : 0.f;
-                    x += (k == DPD - 1) ? a1_next : A1[k + 1];
-                    x += (k == 0) ? a2_prev : A2[k - 1];
-                    x += (l * DPD + k == ks) ? jump : 0.f;
-                    gprev[k] = x;
-                }
-#pragma unroll
-                for (int k = 0; k < DPD; ++k) G[k] = gprev[k];
-            }
-            issue(u, s - V);
+// Four columns: top->bottom reversed into the workspace, or (LAST)
+// bottom->top reversed, adding both onto the rows' gradients.
+template <int D, bool LAST, bool WIDE>
+__device__ __forceinline__ void bwd_cols(const DsgmArgs& A, int b, int group, int lane) {
+    constexpr int DPD = D / 16, NA = kAhead<D, LAST>;
+    const int l = lane & 15, W = A.W, H = A.H;
+    const Off<WIDE> col = (Off<WIDE>)min(group * 4 + (lane >> 4), W - 1);
+    const int64_t npix = (int64_t)A.B * H * W, img = (int64_t)b * H * W, path = LAST ? 2 : 0;
+
+    float qs[NA][DPD], qmn[NA], qz[NA], qg[NA], qd[NA], qo[NA][DPD], qo1[NA], qo2[NA], qy[NA][DPD], qy1[NA], qy2[NA];
+    uint32_t qw[NA];
+    int qk[NA];
+    int si = 0;
+    auto issue = [&](int u) __attribute__((always_inline)) {
+        const int s = min(si++, H - 1);
+        const int64_t r0 = img + (int64_t)(LAST ? s : H - 1 - s) * W;
+        loadf<DPD>(cell_at<D>(A.S + r0 * D, col, l), qs[u]);
+        qmn[u] = loads(A.stats + 2 * r0 + 2 * col);
+        qz[u] = loads(A.stats + 2 * r0 + 2 * col + 1);
+        qg[u] = loads(A.grad_disp + r0 + col);
+        qd[u] = loads(A.disp + r0 + col);
+        qw[u] = load_codes<D>(A.wins + (path * npix + r0) * (D / 4) + (Off<WIDE>)(col * (D / 4)), l);
+        qk[u] = loadb(A.kstar + path * npix + r0 + col);
+        if constexpr (LAST) {
+            loadf<DPD>(cell_at<D>(A.grad_cost + r0 * D, col, l), qo[u]);
+            loadf<DPD>(cell_at<D>(A.vol + r0 * D, col, l), qy[u]);
+            qo1[u] = loads(A.grad_p1 + r0 + col);
+            qo2[u] = loads(A.grad_p2 + r0 + col);
+            qy1[u] = loads(A.vol_p1 + r0 + col);
+            qy2[u] = loads(A.vol_p2 + r0 + col);
         }
-    }
-    // the first pixel (no penalty terms)
-    float o0[DPD], y0[DPD], o01 = 0.f, o02 = 0.f, y01 = 0.f, y02 = 0.f;
-    const int64_t q0 = g.pix0;
-    if constexpr (kPriorC) {
-        loadf<DPD>(out_c + q0 * D, o0);
-        o01 = loads(out_p1 + q0);
-        o02 = loads(out_p2 + q0);
-    }
-    if constexpr (kPriorY) {
-        loadf<DPD>(gy + q0 * D, y0);
-        y01 = loads(gy1 + q0);
-        y02 = loads(gy2 + q0);
-    }
-    emit(q0, G, 0.f, 0.f, o0, o01, o02, y0, y01, y02);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float F[DPD];
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) F[k] = 0.f;
+    int s = 0;
+    auto step = [&](int u) __attribute__((always_inline)) {
+        const int64_t r0 = img + (int64_t)(LAST ? s : H - 1 - s) * W;
+        float G[DPD], s12, s3, sums[3];
+        grad_s_from<DPD>(qs[u], qmn[u], qz[u], qg[u], qd[u], A.inv_temperature, l, G);
+#pragma unroll
+        for (int k = 0; k < DPD; ++k) G[k] += F[k];
+        sums[0] = bwd_flow<DPD>(G, s == H - 1 ? 0u : shift_codes<D>(qw[u], l), F, &s12, &s3);
+        sums[1] = s12;
+        sums[2] = s3;
+        row_sums(sums);
+        bwd_jump<DPD>(F, qk[u], sums[0], l);
+        if constexpr (LAST) {
+#pragma unroll
+            for (int k = 0; k < DPD; ++k) G[k] = (qo[u][k] + qy[u][k]) + G[k];
+            storef<DPD>(cell_at<D>(A.grad_cost + r0 * D, col, l), G);
+            store1(A.grad_p1 + r0 + col, (qo1[u] + qy1[u]) + sums[1]);
+            store1(A.grad_p2 + r0 + col, (qo2[u] + qy2[u]) + sums[2]);
+        } else {
+            storef<DPD>(cell_at<D>(A.vol + r0 * D, col, l), G);
+            store1(A.vol_p1 + r0 + col, sums[1]);
+            store1(A.vol_p2 + r0 + col, sums[2]);
+        }
+        ++s;
+    };
+    run_steps<NA>(H, issue, step);
 }
 
-template <int D>
-__global__ __launch_bounds__(64) void dsgm_backward_first_kernel(DsgmArgs A) {
-    int b, group;
-    bool pair;
-    first_item(A, blockIdx.x, &b, &pair, &group);
-    if (pair) {
-        bwd_lines<D, kBwdStore>(A, b, 1, group, threadIdx.x);
-        bwd_lines<D, kBwdAdd>(A, b, 3, group, threadIdx.x);
+// The first launch: the row pairs of every image, then the top->bottom column
+// groups; the second: the bottom->top groups.  Column groups are spread so
+// that each XCD walks a contiguous run of them: the per-pixel maps (penalties,
+// statistics, disparity, gradients) of 32 neighbouring columns share a
+// 128-byte line, which is then fetched into one L2 instead of eight.  A
+// workgroup is one wave: of few groups, four to a workgroup leave most CUs
+// idle, and the walks wait for the memory path of the rest (1242x375, forward
+// + backward, four / one: D = 128 2.56 / 1.58 ms, D = 256 6.23 / 3.28 ms;
+// 4 images D = 128 5.33 / 4.76 ms).
+
+template <int D, bool BWD, bool WIDE>
+__global__ __launch_bounds__(64) void dsgm_first_kernel(DsgmArgs A, int row_blocks) {
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x < row_blocks) {
+        const int nh = (A.H + 1) / 2, item = blockIdx.x;
+        const int b = item / nh;
+        if constexpr (BWD) bwd_rows<D, WIDE>(A, b, item - b * nh, lane);
+        else fwd_rows<D, WIDE>(A, b, item - b * nh, lane);
     } else {
-        bwd_lines<D, kBwdStoreY>(A, b, 0, group, threadIdx.x);
+        const int nv = (A.W + 3) / 4;
+        const int item = dev::xcd_item((int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks);
+        const int b = item / nv;
+        if constexpr (BWD) bwd_cols<D, false, WIDE>(A, b, item - b * nv, lane);
+        else fwd_cols<D, false, WIDE>(A, b, item - b * nv, lane);
     }
 }
 
-template <int D>
-__global__ __launch_bounds__(64) void dsgm_backward_last_kernel(DsgmArgs A) {
+template <int D, bool BWD, bool WIDE>
+__global__ __launch_bounds__(64) void dsgm_last_kernel(DsgmArgs A) {
     const int nv = (A.W + 3) / 4;
     const int item = dev::xcd_item(blockIdx.x, gridDim.x);
-    const int b = item / nv, group = item - b * nv;
-    bwd_lines<D, kBwdLast>(A, b, 2, group, threadIdx.x);
+    const int b = item / nv;
+    if constexpr (BWD) bwd_cols<D, true, WIDE>(A, b, item - b * nv, threadIdx.x);
+    else fwd_cols<D, true, WIDE>(A, b, item - b * nv, threadIdx.x);
+}
+
+template <int D, bool BWD, bool WIDE>
+hipError_t launch_passes(const DsgmArgs& A, hipStream_t s) {
+    const unsigned rows = (unsigned)A.B * ((A.H + 1) / 2);
+    const unsigned cols = (unsigned)A.B * ((A.W + 3) / 4);
+    hipLaunchKernelGGL((dsgm_first_kernel<D, BWD, WIDE>), dim3(rows + cols), dim3(64), 0, s, A, (int)rows);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((dsgm_last_kernel<D, BWD, WIDE>), dim3(cols), dim3(64), 0, s, A);
+    return hipGetLastError();
+}
+
+template <bool BWD>
+hipError_t launch_by_d(const DsgmArgs& A, hipStream_t s) {
+    const bool wide = (int64_t)2 * A.W * A.D * 4 > (int64_t)1 << 31;
+    switch (A.D) {
+        case 64: return wide ? launch_passes<64, BWD, true>(A, s) : launch_passes<64, BWD, false>(A, s);
+        case 128: return wide ? launch_passes<128, BWD, true>(A, s) : launch_passes<128, BWD, false>(A, s);
+        case 256: return wide ? launch_passes<256, BWD, true>(A, s) : launch_passes<256, BWD, false>(A, s);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace
 
-#define FSGM_DSGM_DISPATCH(KER, grid, block, A, s)                                       \
-    do {                                                                                \
-        switch ((A).D) {                                                                \
-            case 64: hipLaunchKernelGGL(KER<64>, grid, block, 0, s, A); break;          \
-            case 128: hipLaunchKernelGGL(KER<128>, grid, block, 0, s, A); break;        \
-            case 256: hipLaunchKernelGGL(KER<256>, grid, block, 0, s, A); break;        \
-            default: return hipErrorInvalidValue;                                       \
-        }                                                                               \
-    } while (0)
-
-// first launch: the horizontal pairs and the top->bottom groups of every
-// image; second launch: the bottom->top groups
-static unsigned dsgm_items_first(const DsgmArgs& A) {
-    return (unsigned)(A.B * ((A.H + 3) / 4 + (A.W + 3) / 4));
-}
-static unsigned dsgm_items_last(const DsgmArgs& A) { return (unsigned)(A.B * ((A.W + 3) / 4)); }
-
 hipError_t dsgm_launch_forward(const DsgmArgs& A, hipStream_t s) {
-    if (dsgm_sweep_ok(A)) return dsgm_sweep_forward(A, s);
-    const dim3 b1(64);
-    FSGM_DSGM_DISPATCH(dsgm_forward_first_kernel, dim3(dsgm_items_first(A)), b1, A, s);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    FSGM_DSGM_DISPATCH(dsgm_forward_last_kernel, dim3(dsgm_items_last(A)), b1, A, s);
-    return hipGetLastError();
+    return dsgm_sweep_ok(A) ? dsgm_sweep_forward(A, s) : launch_by_d<false>(A, s);
 }
-
 hipError_t dsgm_launch_backward(const DsgmArgs& A, hipStream_t s) {
-    if (dsgm_sweep_ok(A)) return dsgm_sweep_backward(A, s);
-    const dim3 b1(64);
-    FSGM_DSGM_DISPATCH(dsgm_backward_first_kernel, dim3(dsgm_items_first(A)), b1, A, s);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    FSGM_DSGM_DISPATCH(dsgm_backward_last_kernel, dim3(dsgm_items_last(A)), b1, A, s);
-    return hipGetLastError();
+    return dsgm_sweep_ok(A) ? dsgm_sweep_backward(A, s) : launch_by_d<true>(A, s);
 }
 
 }  // namespace fsgm

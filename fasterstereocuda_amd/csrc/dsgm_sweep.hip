@@ -86,7 +86,8 @@ struct CodeLane {
 template <int D>
 __device__ __forceinline__ void bstore_codes(Rsrc r, uint32_t off, uint32_t w) {
     if constexpr (D == 64) __builtin_amdgcn_raw_buffer_store_b8((uint8_t)w, r, (int)off, 0, 0);
-    else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)w, r, (int)off, 0, 0);
+    else if constexpr (D == 128) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)w, r, (int)off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(w, r, (int)off, 0, 0);
 }
 
 __device__ __forceinline__ int bands_of(int H) { return (H + 3) / 4; }
@@ -154,60 +155,6 @@ struct Handover {
     }
 };
 
-// Row reductions of several values stage by stage: a DPP read has to wait two
-// states after the write of its register, which the other values' moves fill.
-__device__ __forceinline__ void row_min_both(float& a, float& b) {
-    // written out: fminf of a moved value costs a separate move and a
-    // canonicalising v_max per stage
-    asm("s_nop 1\n\t"
-        "v_min_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-        "v_min_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 0\n\t"
-        "v_min_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
-        "v_min_f32_dpp %1, %1, %1 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 0\n\t"
-        "v_min_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
-        "v_min_f32_dpp %1, %1, %1 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 0\n\t"
-        "v_min_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf\n\t"
-        "v_min_f32_dpp %1, %1, %1 row_ror:1 row_mask:0xf bank_mask:0xf"
-        : "+v"(a), "+v"(b));
-}
-template <int CTRL, int N>
-__device__ __forceinline__ void add_stage(float (&v)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] += dppf<CTRL>(0.f, v[i]);
-    __builtin_amdgcn_sched_barrier(0);
-}
-template <int N>
-__device__ __forceinline__ void row_sums(float (&v)[N]) {
-    add_stage<0x128>(v);
-    add_stage<0x124>(v);
-    add_stage<0x122>(v);
-    add_stage<0x121>(v);
-}
-// smallest d with L(d) == m in a lane (none: a large value)
-template <int DPD>
-__device__ __forceinline__ int lane_argmin(const float (&L)[DPD], float m, int l) {
-    int idx = 0x7FFFFFFF;
-#pragma unroll
-    for (int k = DPD - 1; k >= 0; --k)
-        if (L[k] == m) idx = l * DPD + k;
-    return idx;
-}
-template <int CTRL>
-__device__ __forceinline__ void min_stage(int& a, int& b) {
-    a = min(a, dppi<CTRL>(0, a));
-    b = min(b, dppi<CTRL>(0, b));
-    __builtin_amdgcn_sched_barrier(0);
-}
-__device__ __forceinline__ void row_min_both(int& a, int& b) {
-    min_stage<0x128>(a, b);
-    min_stage<0x124>(a, b);
-    min_stage<0x122>(a, b);
-    min_stage<0x121>(a, b);
-}
-
 // Edge states of a vertical direction: [direction 0, 2][image][band 1 ..][walk column][D]
 __device__ __forceinline__ float* edge_at(const DsgmArgs& A, int second, int b, int band) {
     const int64_t nb1 = bands_of(A.H) - 1;
@@ -216,12 +163,13 @@ __device__ __forceinline__ float* edge_at(const DsgmArgs& A, int second, int b, 
 
 // Steps of loads in flight.  A band's walk runs about one wave per SIMD, so
 // the ring alone covers the memory latency: four steps of 2-5 KB per wave.
-constexpr int kAheadS = 4;
+// (Six steps: the same.  At D = 256 four would pass the vector registers.)
+template <int D> constexpr int kAheadS = D == 256 ? 2 : 4;
 
 // ------------------------------------------------------------- forward ---
 template <int D, bool LAST>
 __device__ __forceinline__ void fwd_sweep(const DsgmArgs& A, int b, int g, int lane, Handover<D>& ho) {
-    constexpr int DPD = D / 16, NA = kAheadS, PH = LAST ? 3 : 1, PV = LAST ? 2 : 0;
+    constexpr int DPD = D / 16, NA = kAheadS<D>, PH = LAST ? 3 : 1, PV = LAST ? 2 : 0;
     const float inf = __builtin_inff();
     const int sub = lane >> 4, l = lane & 15;
     const int W = A.W;
@@ -311,47 +259,6 @@ __device__ __forceinline__ void fwd_sweep(const DsgmArgs& A, int b, int g, int l
 }
 
 // ------------------------------------------------------------ backward ---
-// What a pixel's gradient G of one direction hands to the pixel before it
-// (w, ks: the pixel's winner codes and the previous pixel's argmin), and the
-// lane's shares of its penalty gradients.
-// The codes' two bits become masks, so a share is one three-input bit
-// operation; F is left without the argmin's term, whose amount is less the
-// sum of F (a code 3 hands nothing on).
-template <int DPD>
-__device__ __forceinline__ float bwd_flow(const float (&G)[DPD], uint32_t w, float (&F)[DPD], float* s12, float* s3) {
-    float A1[DPD], A2[DPD], a12 = 0.f, a3 = 0.f, rest = 0.f;
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) {
-        const uint32_t g = __builtin_bit_cast(uint32_t, G[k]);
-        // written out: the compiler turns shifted masks into compares and selects
-        uint32_t b0, b1;
-        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(b0) : "v"(w), "i"(2 * k));
-        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(b1) : "v"(w), "i"(2 * k + 1));
-        F[k] = __builtin_bit_cast(float, g & ~(b0 | b1));
-        A1[k] = __builtin_bit_cast(float, g & b0 & ~b1);   // to d - 1
-        A2[k] = __builtin_bit_cast(float, g & b1 & ~b0);   // to d + 1
-        a3 += __builtin_bit_cast(float, g & b0 & b1);
-        a12 += A1[k] + A2[k];
-    }
-    const float a1_next = dppf<kShl1>(0.f, A1[0]);
-    const float a2_prev = dppf<kShr1>(0.f, A2[DPD - 1]);
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) {
-        F[k] += (k == DPD - 1) ? a1_next : A1[k + 1 < DPD ? k + 1 : k];
-        F[k] += (k == 0) ? a2_prev : A2[k > 0 ? k - 1 : 0];
-        rest += F[k];
-    }
-    *s12 = a12;
-    *s3 = a3;
-    return rest;
-}
-// the argmin's term, to disparity ks
-template <int DPD>
-__device__ __forceinline__ void bwd_jump(float (&F)[DPD], int ks, float rest, int l) {
-    const int kl = ks - l * DPD;
-#pragma unroll
-    for (int k = 0; k < DPD; ++k) F[k] -= (kl == k) ? rest : 0.f;
-}
 // gS of a pixel from S, its minimum mn, coef = gdisp (-1/T) / z and disp
 template <int DPD>
 __device__ __forceinline__ void grad_s_coef(const float (&s)[DPD], float mn, float coef, float dq, float c, int l,
@@ -362,7 +269,7 @@ __device__ __forceinline__ void grad_s_coef(const float (&s)[DPD], float mn, flo
 
 template <int D, bool LAST>
 __device__ __forceinline__ void bwd_sweep(const DsgmArgs& A, int b, int g, int lane, Handover<D>& ho) {
-    constexpr int DPD = D / 16, NA = kAheadS, PH = LAST ? 3 : 1, PV = LAST ? 2 : 0;
+    constexpr int DPD = D / 16, NA = kAheadS<D>, PH = LAST ? 3 : 1, PV = LAST ? 2 : 0;
     const int sub = lane >> 4, l = lane & 15;
     const int W = A.W;
     Band<D, !LAST> bd(A, b, g, sub);
@@ -520,7 +427,7 @@ __device__ __forceinline__ void edge_lines(const DsgmArgs& A, int b, int second,
             if constexpr (!BWD) {
                 const bool start = u == 0 && band == 0;
                 const float inf = __builtin_inff();
-                const float m = row_minf(lane_min(v));
+                const float m = row_min(lane_min(v));
                 fwd_step<DPD>(v, q[u], m, start ? inf : q1[u], start ? inf : q2[u]);
             } else {
                 float gs[DPD], s12, s3;
@@ -537,33 +444,26 @@ __device__ __forceinline__ void edge_lines(const DsgmArgs& A, int b, int second,
     } while (++band < nb1);   // launched where nb1 >= 1
 }
 
-// Workgroups of several bands: the waves of one go to different SIMDs, and a
-// sweep of eight driving frames has less than one wave per SIMD.  What bounds a
-// sweep: about 300-420 VALU instructions per step and wave (4.5 cycles each,
-// alone on its SIMD), 0.9-1.2 ms over 1242 columns, beside its share of HBM
-// (8 images, D = 128: 3.5-4 TB/s; the edge passes run at 5).  Measured, 8 images
-// 1242x375 D = 128: edges 0.50 / 0.54, first sweeps with the other edges 1.66 /
-// 1.74, second sweeps 1.62 / 1.70 ms; the separate passes took 10.0 ms.
-constexpr int kSweepWaves = 4;
-
+// One wave per workgroup: the 752 bands of eight driving frames then spread
+// over all CUs (four waves to a workgroup 7.74 ms, one 7.03 ms).  What bounds a
+// sweep: 300-420 VALU instructions per step at about 4.5 cycles each (a wave
+// alone on its SIMD), 0.9-1.2 ms over 1242 columns, beside its share of HBM.
+//
 // The first sweep's launch also holds the edges of the second direction: the
 // sweep leaves memory bandwidth and wave slots that they fill.
 template <int D, bool BWD, bool LAST>
-__global__ __launch_bounds__(64 * kSweepWaves, 1) void dsgm_sweep_kernel(DsgmArgs A, int sweeps) {
-    __shared__ __align__(16) Handover<D> ho[kSweepWaves];
-    const int wave = dev::wave_in_group();
+__global__ __launch_bounds__(64) void dsgm_sweep_kernel(DsgmArgs A, int sweeps) {
+    __shared__ __align__(16) Handover<D> ho;
     if (LAST || (int)blockIdx.x < sweeps) {
-        const int nb = bands_of(A.H), item = (int)blockIdx.x * kSweepWaves + wave;
-        if (item >= A.B * nb) return;
+        const int nb = bands_of(A.H), item = blockIdx.x;
         const int b = item / nb, g = item - b * nb;
-        if constexpr (BWD) bwd_sweep<D, LAST>(A, b, g, threadIdx.x & 63, ho[wave]);
-        else fwd_sweep<D, LAST>(A, b, g, threadIdx.x & 63, ho[wave]);
+        if constexpr (BWD) bwd_sweep<D, LAST>(A, b, g, threadIdx.x, ho);
+        else fwd_sweep<D, LAST>(A, b, g, threadIdx.x, ho);
     } else {
         const int nv = (A.W + 3) / 4;
-        const int item = dev::xcd_item((int)blockIdx.x - sweeps, (int)gridDim.x - sweeps) * kSweepWaves + wave;
-        if (item >= A.B * nv) return;
+        const int item = dev::xcd_item((int)blockIdx.x - sweeps, (int)gridDim.x - sweeps);
         const int b = item / nv;
-        edge_lines<D, BWD>(A, b, 1, item - b * nv, threadIdx.x & 63);
+        edge_lines<D, BWD>(A, b, 1, item - b * nv, threadIdx.x);
     }
 }
 
@@ -584,9 +484,9 @@ __global__ __launch_bounds__(256) void dsgm_coef_kernel(DsgmArgs A, int64_t n) {
 template <int D, bool BWD>
 hipError_t launch_sweeps(const DsgmArgs& A, hipStream_t s) {
     const unsigned nb = (unsigned)((A.H + 3) / 4);
-    const unsigned sweeps = ((unsigned)A.B * nb + kSweepWaves - 1) / kSweepWaves;
+    const unsigned sweeps = (unsigned)A.B * nb;
     const unsigned columns = (unsigned)A.B * ((A.W + 3) / 4);
-    const unsigned edges = nb > 1 ? (columns + kSweepWaves - 1) / kSweepWaves : 0;
+    const unsigned edges = nb > 1 ? columns : 0;
     if constexpr (BWD) {
         const int64_t n = (int64_t)A.B * A.H * A.W;
         hipLaunchKernelGGL(dsgm_coef_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, A, n);
@@ -598,11 +498,11 @@ hipError_t launch_sweeps(const DsgmArgs& A, hipStream_t s) {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((dsgm_sweep_kernel<D, BWD, false>), dim3(sweeps + edges), dim3(64 * kSweepWaves), 0, s, A,
+    hipLaunchKernelGGL((dsgm_sweep_kernel<D, BWD, false>), dim3(sweeps + edges), dim3(64), 0, s, A,
                        (int)sweeps);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((dsgm_sweep_kernel<D, BWD, true>), dim3(sweeps), dim3(64 * kSweepWaves), 0, s, A, (int)sweeps);
+    hipLaunchKernelGGL((dsgm_sweep_kernel<D, BWD, true>), dim3(sweeps), dim3(64), 0, s, A, (int)sweeps);
     return hipGetLastError();
 }
 
@@ -611,24 +511,26 @@ hipError_t launch_by_d(const DsgmArgs& A, hipStream_t s) {
     switch (A.D) {
         case 64: return launch_sweeps<64, BWD>(A, s);
         case 128: return launch_sweeps<128, BWD>(A, s);
+        case 256: return launch_sweeps<256, BWD>(A, s);
         default: return hipErrorInvalidValue;
     }
 }
 
 }  // namespace
 
-// Taken from 560 bands on, about half a wave per SIMD: below that the walk of
+// Taken from 390 bands on (450 at D = 64), about 0.4 waves per SIMD: the walk of
 // a band's W + 3 steps of two directions lasts as long for few images as for
-// many, and the separate passes, with four times the waves, are sooner done.
-// Forward and backward, us, separate -> sweeps (D = 128, 375 rows of 1242):
-//   4 images (376 bands) 5337 -> 5850, 5 (470) 6281 -> 6416, 6 (564) 7834 ->
-//   6997, 8 (752) 10088 -> 7741; 8 images 800x300 (600) 5079 -> 4654, 160x375
-//   (752) 1473 -> 1266; D = 64, 8 images 1242x375 4934 -> 4286.
-// At D = 256 a lane's 16 disparities make a step twice as long (4 images:
-// 11892 against 12829), so it keeps the separate passes.  A band's cells stay
-// below 2^30 bytes, so that 32-bit offsets and kNoPixel hold.
+// many, and below that the separate passes are sooner done.  Forward +
+// backward, ms, separate -> sweeps, 375 rows of 1242 unless given:
+//   D = 128: 4 images (376 bands) 4.76 -> 4.96, 5 (470) 6.40 -> 5.22, 8 (752)
+//   9.97 -> 7.03; 8 images 1000x180 (360) 3.60 -> 3.97, 1242x200 (400) 5.75 -> 5.02
+//   D = 64: 4 images 2.37 -> 2.80, 5 3.11 -> 2.97, 8 5.07 -> 3.70; 8 images
+//   600x196 (392) 1.23 -> 1.35
+//   D = 256: 4 images 9.82 -> 9.75; 8 images 600x375 (752) 9.81 -> 7.21, 600x150
+//   (304) 4.04 -> 4.45
+// A band's cells stay below 2^30 bytes, so that 32-bit offsets and kNoPixel hold.
 bool dsgm_sweep_ok(const DsgmArgs& A) {
-    return A.D <= 128 && (int64_t)A.B * ((A.H + 3) / 4) >= 560 && (int64_t)A.W * A.D <= (int64_t)1 << 26;
+    return (int64_t)A.B * ((A.H + 3) / 4) >= (A.D == 64 ? 450 : 390) && (int64_t)A.W * A.D <= (int64_t)1 << 26;
 }
 hipError_t dsgm_sweep_forward(const DsgmArgs& A, hipStream_t s) { return launch_by_d<false>(A, s); }
 hipError_t dsgm_sweep_backward(const DsgmArgs& A, hipStream_t s) { return launch_by_d<true>(A, s); }

@@ -54,11 +54,20 @@ def test_forward_backward_match_fp64(cuda, B, H, W, D):
             assert np.abs(g - ref).max() <= 1e-4 * np.abs(ref).max(), f"{name} max err"
 
 
+# both directions of a row pair at once: widths 4 .. 9 around the load ring and
+# the middle pixel (odd widths), one row, an odd last row
+@pytest.mark.parametrize("B,H,W,D", [(1, 1, 1, 64), (1, 1, 4, 128), (2, 2, 5, 64), (1, 3, 6, 256), (1, 5, 7, 128),
+                                     (1, 2, 8, 64), (3, 3, 9, 128), (1, 6, 16, 256), (1, 4, 17, 64)])
+def test_row_pairs_match_fp64(cuda, B, H, W, D):
+    test_forward_backward_match_fp64(cuda, B, H, W, D)
+
+
 # many images of few rows, which take the form that walks bands of four rows
 # for two directions together: last bands of 1 to 4 rows, a single band (no
 # state handed between bands), lines shorter than the skew of a band's rows
 @pytest.mark.parametrize("B,H,W,D", [(141, 13, 70, 128), (188, 10, 33, 64), (560, 3, 9, 64),
-                                     (140, 16, 1, 128), (280, 7, 2, 64), (187, 12, 130, 128)])
+                                     (140, 16, 1, 128), (280, 7, 2, 64), (187, 12, 130, 128),
+                                     (98, 13, 20, 256)])
 def test_many_images_match_fp64(cuda, B, H, W, D):
     print(f"[dsgm] B{B} H{H} W{W} D{D}", flush=True)
     cost, p1, p2, gt = _inputs(B, H, W, D, seed=B + H + W + D)
