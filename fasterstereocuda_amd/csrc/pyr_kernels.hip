@@ -271,19 +271,31 @@ __global__ __launch_bounds__(64) void agg_init_kernel(PyrLevel a) {
     else agg_init_lines<LR, false>(a, dir, group, threadIdx.x, lds);
 }
 
-// The same aggregation with two disparities per lane as packed u16 pairs:
-// LR / 2 lanes per scanline, SPW = 128 / LR scanlines per wave, and every
-// VALU instruction of the step works on two cells.  The window shift goes
-// through LDS.  Each step writes the scanline's L + P1 into a row of
-// overlapping pairs, C[e] = (L'[e - PAD], L'[e - PAD + 1]) + P1, padded on
-// both sides with 127.  A lane then reads the four neighbour terms its two
-// disparities need, L'[2k + b - b' - 1 .. 2k + b - b' + 2] + P1, as the two
-// dwords C[e0] and C[e0 + 2]: dword-aligned whatever the parity of b - b'.
-// (Reading the four u16 of a plain row is a misaligned 8-byte LDS access,
-// and its stalls took most of the kernel's time.)  A pad is exactly the 127
-// of a neighbour outside the window, so no range test remains.  b - b' is
-// clamped to +-(LR + 1), past which every term is a pad, and, separately, to
-// [-254, 256] to index a table of max(P1, P2 / max(1, |b' - b + 1|)).
+// The same aggregation with NP packed u16 pairs per lane (2 NP disparities):
+// LPL = LR / (2 NP) lanes per scanline, SPW = 64 / LPL scanlines per wave, a
+// block of K = LR / 2 steps (NP pixels per lane), and every VALU instruction
+// of a step works on two cells.  A step needs the neighbour pairs that start
+// at f + q - 1, f + q + 1, .. (f: the lane's first disparity, q = b - b'); the
+// middle one of NP = 2 serves both of its pairs.
+//
+// Where no line of the wave shifts its window by more than one disparity, the
+// shifted pairs are this lane's and its neighbours' (DPP), picked by a byte
+// selector.  The selector, the P2 term, the validity and the base of the last
+// valid pixel before (a scan over the block's steps) are worked out per pixel
+// by the lane that loads it, not per step by every lane of the scanline, and
+// the steps where some line shifts by more are known to the wave, as bits of a
+// scalar, before the block is walked.  In such a step each line's L + P1 is
+// written as a row of overlapping pairs, C[e] = (L'[e - PAD], L'[e - PAD + 1])
+// + P1, padded on both sides with 127, and a lane reads the pairs it needs,
+// dword-aligned whatever the parity of q.  (Reading the u16 of a plain row is a
+// misaligned LDS access, and its stalls took most of the time.)  A pad is
+// exactly the 127 of a neighbour outside the window, so no range test remains.
+// q is clamped to +-(LR + 1), past which every term is a pad, and, separately,
+// to [-254, 256] to index a table of max(P1, P2 / max(1, |1 - q|)).
+//
+// A wave that is alone on its SIMD waits out every latency, so LDS is read a
+// block ahead: while block i is walked, block i + 1 is staged and read into
+// registers, and the results of block i - 1 are read back and stored.
 //
 // Exact when P1 <= 127 and P2 <= 254: the true (unbounded) values of the
 // recurrence then lie in [-382, 763] (l <= c + P2 <= 509, and l >= 127 - m
@@ -291,77 +303,95 @@ __global__ __launch_bounds__(64) void agg_init_kernel(PyrLevel a) {
 // representatives pick the same entries as those of their u32
 // representatives, and the stored low bytes agree.  Other penalties take
 // agg_init_kernel.
+//
+// What bounds it: the chain of a scanline's dependent steps at one or two waves
+// per SIMD (20 instructions per step, 16 more for its share of the staging; a
+// wide step waits for LDS).  Staging and streaming alone take 0.47 of 0.77 ms
+// for 4800x3409 in quads.  Rows of unpadded LDS put all of an access's lanes
+// on 8 banks (quads 0.87 -> 0.77 ms, window 32 0.77 -> 0.51 ms).  With that, the
+// reads a block ahead and the per-pixel preparation, against the form that
+// worked out every step's shift in the step: 4800x3409 window 16 0.79 -> 0.66
+// ms, 7000x5000 1.44 -> 1.20, 2900x2200 window 32 0.64 -> 0.49, 850x600 window
+// 32 0.27 -> 0.21, 1600x1200 window 16 0.20 -> 0.19, 800x600 0.094 -> 0.100.
 typedef unsigned short pk16 __attribute__((ext_vector_type(2)));
 typedef unsigned int pyr_u32x4 __attribute__((ext_vector_type(4)));
 
-// Block stores of the window aggregation: one LR-byte window per pixel, as
-// buffer stores from a base that moves by a fixed step per block, each pixel
-// of a block at an offset from it fixed for the whole walk.  A pixel past the
-// scanlines or the line's end gets an offset beyond the resource's range and
-// its store is dropped, so every block issues the same stores with no branch
-// around them: the compiler then counts the prefetch ring's outstanding loads
-// exactly instead of draining every load and store at each block.  Block blk
-// of scanline group l0 holds pixel (scanline l0 + ln, step blk K + j); the
-// base is the lowest such pixel, offsets stay below (64 + K) W LR bytes.
-template <int LR, int K>
-struct BlockStores {
+// A block's pixels as buffer accesses from a base that moves by a fixed step
+// per block, each pixel at an offset from it fixed for the whole walk.  A
+// pixel past the scanlines or the line's end gets an offset beyond the
+// resource's range: it loads 0 and its store is dropped, so every block issues
+// the same accesses with no branch around them, and the compiler counts the
+// prefetch ring's outstanding loads exactly instead of draining them.  Block
+// blk of scanline group l0 holds pixel (scanline l0 + ln, step blk K + j); the
+// base is the lowest such pixel, offsets stay below (64 + K) W LR bytes.  In
+// the reverse directions the base of a line's last, partial block (and of the
+// blocks past it) lies before the volume: only pixels inside the line are in
+// range, and their offsets land inside it.
+template <int K>
+struct BlockPixels {
     int64_t base0, step;   // base pixel at block 0, and its move per block
-    __device__ BlockStores(bool horiz, bool fwd, int W, int n, int l0) {
+    __device__ BlockPixels(bool horiz, bool fwd, int W, int n, int l0) {
         base0 = horiz ? (int64_t)l0 * W + (fwd ? 0 : n - K) : (fwd ? 0 : (int64_t)(n - K) * W) + l0;
         step = (horiz ? 1 : (int64_t)W) * (fwd ? K : -K);
     }
-    // byte offset of (ln, j) from the base
+    // pixels from the base to (ln, j)
     __device__ static uint32_t offset(bool horiz, bool fwd, int W, int ln, int j) {
         const int jj = fwd ? j : K - 1 - j;
-        return (uint32_t)((horiz ? ln * W + jj : jj * W + ln) * LR);
+        return (uint32_t)(horiz ? ln * W + jj : jj * W + ln);
     }
-    __device__ void store(uint8_t* out, int blk, uint32_t off, bool ok, const uint8_t* src) const {
-        // in the reverse directions the base of a line's last, partial block
-        // (and of the blocks past it) lies before the volume: only pixels
-        // inside the line are in range, and their offsets land inside it
-        const uintptr_t base = (uintptr_t)out + (uintptr_t)((base0 + blk * step) * LR);
-        const __amdgpu_buffer_rsrc_t rs =
-            __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, 0x7fffffff, 0x00020000);
-        const uint32_t o = ok ? off : 0x80000000u;
-#pragma unroll
-        for (int v = 0; v < LR / 16; ++v) {
-            const uint4 w = reinterpret_cast<const uint4*>(src)[v];
-            __builtin_amdgcn_raw_buffer_store_b128(pyr_u32x4{w.x, w.y, w.z, w.w}, rs, (int)(o + 16 * v), 0, 0);
-        }
+};
+// Successive blocks of a volume of `bytes` per pixel.
+struct BlockWalk {
+    uintptr_t base, step;
+    template <int K>
+    __device__ BlockWalk(const BlockPixels<K>& px, const void* volume, int bytes, int blk)
+        : base((uintptr_t)volume + (uintptr_t)((px.base0 + blk * px.step) * bytes)),
+          step((uintptr_t)(px.step * bytes)) {}
+    __device__ __amdgpu_buffer_rsrc_t next() {
+        const uintptr_t b = base;
+        base += step;
+        return __builtin_amdgcn_make_buffer_rsrc((void*)b, (short)0, 0x7fffffff, 0x00020000);
     }
 };
 
 constexpr int kPkDeltaLo = -254, kPkDeltaHi = 256;   // table range of b - b'
-// Blocks of cost loads in flight per wave.  A block is LR / 2 steps; its
-// loads are issued kPkAhead blocks before they are staged, so the HBM
-// latency (1-2 us under load) is spread over that many blocks of steps.
-constexpr int kPkAhead = 4;
+// Blocks of cost loads in flight per wave, so that the HBM latency (1-2 us
+// under load) is spread over that many blocks of steps.
+template <int LR> constexpr int kPkAheadOf = LR == 16 ? 4 : 2;   // 32 steps
 
-template <int LR>
+template <int LR, int NP>
 struct AggInitPkLds {
-    static constexpr int SPW = 128 / LR;
-    static constexpr int PAD = LR + 2;               // even: the lanes' pair stores stay 8-byte aligned
-    static constexpr int ROW = PAD + 2 * LR + 2;     // even; reads reach PAD + 2 LR
-    uint32_t cost[SPW][LR / 2][LR / 2];      // [line][pair k][step]: the pair's costs as u16
-    uint8_t out[64 * LR];                    // [line][step][t]
-    int16_t init[64];                        // [line][step]
+    static constexpr int LPL = LR / (2 * NP), SPW = 64 / LPL, K = LR / 2;
+    static constexpr int PAD = (LR + 2 + 3) / 4 * 4;         // a multiple of 4: aligned row stores
+    static constexpr int ROW = (PAD + 2 * LR + 1 + 3) / 4 * 4;   // reads reach PAD + 2 LR
+    // Strides that spread the lanes of an access over the 64 banks: staging
+    // writes K steps of 64 / K lines per pair (a line stride of K more than a
+    // multiple of 64 words), a step writes a word or half of one per lane.
+    static constexpr int PAIR = K + 4, LINE = LR / 2 * PAIR + K, OUT = LR * (K + 1);
+    uint32_t cost[SPW * LINE];               // [line][pair][step]: the pair's costs as u16
+    uint32_t sel[64 * NP], pen[64 * NP];     // [line][step]: selector and P2 term of a shift of at most
+                                             // one, or the shift itself
+    uint8_t out[SPW * OUT];                  // [line][step][t]
+    alignas(16) int16_t valid[64 * NP];      // [line][step]: 0 or all ones
     uint32_t pen2[kPkDeltaHi - kPkDeltaLo + 1];   // by b - b', both halves
-    uint32_t win[SPW][ROW];                  // overlapping pairs, see above
+    alignas(16) uint32_t win[SPW][ROW];      // overlapping pairs, see above
 };
 
 __device__ __forceinline__ uint32_t pk_bits(pk16 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ pk16 pk_of(uint32_t v) { return __builtin_bit_cast(pk16, v); }
+__device__ __forceinline__ pk16 pk_min2(pk16 a, pk16 b) { return __builtin_elementwise_min(a, b); }
 
 // v_perm selector of bytes 2 (q + 1) .. 2 (q + 1) + 3 of {hi, lo} for a
 // window shift q in {-1, 0, 1}: the dword starting one disparity below, at,
-// or one above the middle of the pair boundary.  Other q (lanes whose step
+// or one above the middle of the pair boundary.  Other q (pixels whose step
 // is skipped) are clamped into that range; their result is not used.
 // Three full-rate instructions: q clamped by v_med3, then 24-bit multiply-adds
 // (written out: the compiler merges the steps into one quarter-rate 32-bit
 // multiply).  The constants come in registers (no literals in VOP3).
 __device__ __forceinline__ uint32_t shift_sel(int q, uint32_t k0202, uint32_t k10001, uint32_t kbase) {
     uint32_t t, u, sel;
-    asm("v_med3_i32 %0, %3, -1, 1\n\t"
+    asm volatile(   // not moved into a branch
+        "v_med3_i32 %0, %3, -1, 1\n\t"
         "v_mad_i32_i24 %1, %0, %4, %4\n\t"     // (q + 1) * 0x0202
         "v_mad_u32_u24 %2, %1, %5, %6"           // u * 0x10001 + 0x03020100
         : "=&v"(t), "=&v"(u), "=v"(sel)
@@ -369,76 +399,62 @@ __device__ __forceinline__ uint32_t shift_sel(int q, uint32_t k0202, uint32_t k1
     return sel;
 }
 
-// minimum over the LR / 2 lanes of a scanline (STRIDE = 32 / LR apart in a
-// DPP row) of both halves; the result holds it in both halves
-template <int LR>
-__device__ __forceinline__ pk16 pk_group_min(pk16 v) {
-    constexpr int STRIDE = 32 / LR;
-    v = __builtin_elementwise_min(v, v.yx);
-    uint32_t m = pk_bits(v);                 // equal halves: u32 order = u16 order
-    m = min(m, dppu<0x120 + STRIDE>(m));     // row_ror by STRIDE, 2 STRIDE, ...
-    m = min(m, dppu<0x120 + 2 * STRIDE>(m));
-    m = min(m, dppu<0x120 + 4 * STRIDE>(m));
-    if constexpr (8 * STRIDE < 16) m = min(m, dppu<0x120 + 8 * STRIDE>(m));
-    return pk_of(m);
-}
-
-template <int LR>
+template <int LR, int NP>
 __device__ __forceinline__ void agg_init_pk_lines(const PyrLevel& a, int dir, int group, int lane,
-                                                  AggInitPkLds<LR>& S) {
-    constexpr int LPL = LR / 2, SPW = 128 / LR, K = LPL;
-    constexpr int PAD = AggInitPkLds<LR>::PAD, ROW = AggInitPkLds<LR>::ROW;
-    constexpr int NV = LR / 16;
+                                                  AggInitPkLds<LR, NP>& S) {
+    using Lds = AggInitPkLds<LR, NP>;
+    constexpr int LPL = Lds::LPL, SPW = Lds::SPW, K = Lds::K, PAD = Lds::PAD;
+    constexpr int NV = LR / 16, kPkAhead = kPkAheadOf<LR>;
     constexpr uint32_t kPadPair = 127u * 0x10001u;
-    // the lanes of a scanline sit STRIDE = 16 / LPL apart in one DPP row (see
-    // agg_init_pk2_lines): the edge pads stay in unwritten lanes
+    static_assert(SPW * K == 64 * NP, "a block is NP pixels per lane");
+    // The lanes of a scanline sit STRIDE = 16 / LPL apart in one DPP row, so a
+    // neighbouring lane's pair is a row shift by STRIDE.  The line's first and
+    // last lanes then read from outside the row, which leaves a move's old
+    // value in place: the 127 pads stay in those lanes of two persistent
+    // registers, with no select per step.
     constexpr int STRIDE = 16 / LPL;
     const int sub = (lane / 16) * STRIDE + lane % STRIDE;   // recurrence: line
-    const int k = (lane % 16) / STRIDE;                     // disparity pair
-    const int lsub = lane / K, lstep = lane % K;     // loads / stores: line, step
+    const int k = (lane % 16) / STRIDE;                     // lane of the line
     const bool horiz = (dir == 1 || dir == 3);
     const bool fwd = (dir == 0 || dir == 1);
     const int W = a.w, H = a.h;
     const int nlines = horiz ? H : W;
     const int n = horiz ? W : H;
-    auto pix_of = [&](int line, int step) -> int64_t {
-        line = min(line, nlines - 1);
-        step = min(step, n - 1);
-        const int pos = fwd ? step : n - 1 - step;
-        return horiz ? (int64_t)line * W + pos : (int64_t)pos * W + line;
-    };
-    const int line = min(group * SPW + sub, nlines - 1);
-    const int lline = group * SPW + lsub;
     uint8_t* out = (dir == 0) ? a.path[0] : (dir == 1) ? a.path[1] : (dir == 2) ? a.path[2] : a.path[3];
 
-    // a ring of kPkAhead blocks of loads in flight (slot = block mod kPkAhead)
-    uint4 ncs[kPkAhead][NV];
-    int nbs[kPkAhead];
-    auto fetch = [&](int slot, int blk) __attribute__((always_inline)) {
-        const int64_t p = pix_of(lline, blk * K + lstep);
-        const uint4* src = reinterpret_cast<const uint4*>(a.cost + p * LR);
+    // loads and stores: lane j handles the block's pixels j, j + 64 in
+    // [line][step] order
+    const BlockPixels<K> px(horiz, fwd, W, n, group * SPW);
+    const int lstep = lane % K;              // 64 is a multiple of K
+    uint32_t off[NP];
+    bool on_line[NP];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) ncs[slot][v] = src[v];
-        nbs[slot] = a.init[p];
+    for (int h = 0; h < NP; ++h) {
+        const int ln = (lane + 64 * h) / K;
+        off[h] = BlockPixels<K>::offset(horiz, fwd, W, ln, lstep);
+        on_line[h] = group * SPW + ln < nlines;
+    }
+    auto inside = [&](int h, int blk) __attribute__((always_inline)) {
+        return on_line[h] && lstep < n - blk * K;
     };
-    // the block in LDS, transposed so that a lane later reads the cost pairs
-    // of all K steps of its own (line, pair) with wide loads: pair j of
-    // this lane's pixel goes to cost[line][j][step], zero-extended to u16
-    auto stage = [&](int slot) __attribute__((always_inline)) {
-        uint32_t wv[LR / 4];
+    // a ring of kPkAhead blocks of loads in flight (slot = block mod kPkAhead)
+    pyr_u32x4 nc[kPkAhead][NP][NV];
+    uint16_t nb[kPkAhead][NP];
+    BlockWalk costs(px, a.cost, LR, 0), bases(px, a.init, 2, 0), outs(px, out, LR, -1);
+    auto fetch = [&](int slot, int blk) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rc = costs.next(), rb = bases.next();
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            wv[4 * v] = ncs[slot][v].x; wv[4 * v + 1] = ncs[slot][v].y;
-            wv[4 * v + 2] = ncs[slot][v].z; wv[4 * v + 3] = ncs[slot][v].w;
+        for (int h = 0; h < NP; ++h) {
+            const bool in = inside(h, blk);
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                nc[slot][h][v] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rc, (int)(in ? off[h] * LR + 16 * v : 0x80000000u), 0, 0);
+            nb[slot][h] = __builtin_amdgcn_raw_buffer_load_b16(rb, (int)(in ? off[h] * 2 : 0x80000000u), 0, 0);
         }
-#pragma unroll
-        for (int j = 0; j < LR / 2; ++j)
-            S.cost[lsub][j][lstep] = __builtin_amdgcn_perm(0u, wv[j / 2], (j & 1) ? 0x0c030c02u : 0x0c010c00u);
-        S.init[lane] = (int16_t)nbs[slot];
     };
 
-    // pads, and the P2 table by offset q = b - b' (divisor |1 - q|)
-    for (int e = lane; e < SPW * ROW; e += 64) (&S.win[0][0])[e] = kPadPair;
+    for (int e = lane; e < SPW * Lds::ROW; e += 64) (&S.win[0][0])[e] = kPadPair;
     for (int e = lane; e <= kPkDeltaHi - kPkDeltaLo; e += 64) {
         const int q = e + kPkDeltaLo;
         const uint32_t v = (uint32_t)max(a.p1, a.p2 / max(1, abs(1 - q)));
@@ -447,226 +463,36 @@ __device__ __forceinline__ void agg_init_pk_lines(const PyrLevel& a, int dir, in
     __builtin_amdgcn_wave_barrier();
 
     uint32_t* wrow = &S.win[sub][0];
-    const uint32_t* wlane = wrow + (PAD - 1 + 2 * k);     // + q: the pair before this lane's first term
+    const uint32_t* wlane = wrow + (PAD - 1 + 2 * NP * k);     // + q: the first neighbour pair
     const bool last_k = k == LPL - 1;
-    uint8_t* obase = S.out + sub * K * LR + 2 * k;
+    uint8_t* obase = S.out + sub * Lds::OUT + 2 * NP * k;
     const pk16 p1v = pk_of((uint32_t)a.p1 * 0x10001u);
     const pk16 m127 = pk_of(kPadPair);
     const uint32_t k10001 = 0x10001u;
-    // clamp bounds kept in registers (one v_med3 each per step) instead of
-    // rematerialised each step
-    int qlo = kPkDeltaLo, qhi = kPkDeltaHi, wlo = -(LR + 1);
-    asm volatile("" : "+v"(qlo), "+v"(qhi), "+v"(wlo));
-    // P2 terms of the offsets -1, 0 and 1 (divisors 2, 1 and 1)
-    const pk16 pen2_m1 = pk_of(S.pen2[-1 - kPkDeltaLo]);
-    const pk16 pen2_01 = pk_of(S.pen2[0 - kPkDeltaLo]);
-    // this lane's pairs of L + P1 into the window row: C[PAD + 2k] (its own
-    // pair), C[PAD + 2k + 1] (its high half and the next lane's low half or a
-    // pad) and, from lane 0, C[PAD - 1] (a pad and its low half)
-    auto put = [&](uint32_t own) __attribute__((always_inline)) {
-        uint32_t nxt = dppu<0x100 + STRIDE>(own);         // row_shl: lane k + 1
-        nxt = last_k ? kPadPair : nxt;
-        const uint32_t mid = __builtin_amdgcn_alignbit(nxt, own, 16);
-        *reinterpret_cast<uint2*>(wrow + PAD + 2 * k) = make_uint2(own, mid);
-        if (k == 0) wrow[PAD - 1] = (own << 16) | 127u;
+    // P2 terms of the shifts -1, 0 and 1 (divisors 2, 1 and 1)
+    const uint32_t pen2_m1 = S.pen2[-1 - kPkDeltaLo], pen2_01 = S.pen2[0 - kPkDeltaLo];
+    auto small_pen = [=](int q) __attribute__((always_inline)) {
+        const uint32_t neg = 0u - (uint32_t)(q < 0);
+        return (pen2_m1 & neg) | (pen2_01 & ~neg);
     };
 
-    pk16 L = pk_of(0u), m = pk_of(0u);
-    uint32_t nxt_r = kPadPair, prv_r = kPadPair;   // pads kept in the last / first lane of a line
-    int last_b = 0;
     // A11: vertical directions seed b' from row 0 whichever end they start at
-    const int seed_b = horiz ? 0 : a.init[line];
-    const int nblk = (n + K - 1) / K;
-    const BlockStores<LR, K> stores(horiz, fwd, W, n, group * SPW);
-    const uint32_t woff = BlockStores<LR, K>::offset(horiz, fwd, W, lsub, lstep);
-    const bool wline = lline < nlines;
-    auto process = [&](int blk) __attribute__((always_inline)) {
-        __builtin_amdgcn_wave_barrier();
-        // the bases of the block's K steps of this lane's line and this
-        // lane's cost pairs of those steps, in registers: no LDS read on the
-        // step's chain
-        uint32_t bw[K / 2], cwv[K];
+    int seed[NP], pb[NP];                    // pb: last valid bases of the block before
 #pragma unroll
-        for (int i = 0; i < K / 8; ++i) {
-            const uint4 v = reinterpret_cast<const uint4*>(&S.init[sub * K])[i];
-            bw[4 * i] = v.x; bw[4 * i + 1] = v.y; bw[4 * i + 2] = v.z; bw[4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int i = 0; i < K / 4; ++i) {
-            const uint4 v = reinterpret_cast<const uint4*>(&S.cost[sub][k][0])[i];
-            cwv[4 * i] = v.x; cwv[4 * i + 1] = v.y; cwv[4 * i + 2] = v.z; cwv[4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int s = 0; s < K; ++s) {
-            const int b = (int)(int16_t)(bw[s / 2] >> (16 * (s & 1)));
-            const pk16 c = pk_of(cwv[s]);
-            pk16 o;
-            if (s == 0 && blk == 0) {
-                L = c;
-                m = pk_group_min<LR>(L);
-                last_b = horiz ? b : seed_b;
-                o = L;
-            } else {
-                const bool valid = b != kInvalidShort;
-                const int q = b - last_b;
-                const uint32_t own = pk_bits(L + p1v);
-                pk16 bm, bp, pen2;                        // neighbour terms, + P1 already
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(valid && (q < -1 || q > 1)) == 0, 1)) {
-                    // every line shifts by at most one disparity: the terms are
-                    // this lane's pair and its neighbours' (DPP), no LDS
-                    // lane k + 1 and lane k - 1 (row_shl / row_shr by STRIDE,
-                    // out-of-row sources not written: the pads stay)
-                    nxt_r = (uint32_t)__builtin_amdgcn_update_dpp((int)nxt_r, (int)own, 0x100 + STRIDE, 0xF, 0xF,
-                                                                  false);
-                    prv_r = (uint32_t)__builtin_amdgcn_update_dpp((int)prv_r, (int)own, 0x110 + STRIDE, 0xF, 0xF,
-                                                                  false);
-                    const uint32_t nxt = nxt_r, prv = prv_r;
-                    // the pair starting at disparity 2k + q - 1 (2k + q + 1) is
-                    // bytes 2 (q + 1) .. 2 (q + 1) + 3 of {own, prv} ({nxt, own})
-                    const uint32_t sel = shift_sel(q, 0x0202u, k10001, 0x03020100u);
-                    bm = pk_of(__builtin_amdgcn_perm(own, prv, sel));
-                    bp = pk_of(__builtin_amdgcn_perm(nxt, own, sel));
-                    const uint32_t mneg = 0u - (uint32_t)(q < 0);
-                    pen2 = pk_of((pk_bits(pen2_m1) & mneg) | (pk_bits(pen2_01) & ~mneg));
-                } else {
-                    put(own);      // the window row holds L only when a step needs it
-                    const int qt = min(max(q, qlo), qhi);
-                    const int qw = min(max(q, wlo), LR + 1);
-                    uint32_t xm = wlane[qw], xp = wlane[qw + 2], pb = S.pen2[qt - kPkDeltaLo];
-                    // complete these reads inside the branch, so that no LDS read
-                    // is pending where the two paths meet (the fast path would
-                    // otherwise wait for every LDS operation, the output stores
-                    // included)
-                    asm volatile("" : "+v"(xm), "+v"(xp), "+v"(pb));
-                    bm = pk_of(xm);
-                    bp = pk_of(xp);
-                    pen2 = pk_of(pb);
-                }
-                const pk16 v = __builtin_elementwise_min(__builtin_elementwise_min(L, bm),
-                                                         __builtin_elementwise_min(bp, m + pen2));
-                const pk16 l = c + (v - m);
-                const pk16 mn = pk_group_min<LR>(l);
-                // selects as bit operations (v_bfi), so the step stays one block
-                const uint32_t vm = 0u - (uint32_t)valid;
-                o = pk_of(pk_bits(l) & vm);
-                L = pk_of((pk_bits(l) & vm) | (pk_bits(L) & ~vm));
-                m = pk_of((pk_bits(mn) & vm) | (pk_bits(m127) & ~vm));
-                last_b = (int)(((uint32_t)b & vm) | ((uint32_t)last_b & ~vm));
-            }
-            // low bytes of both halves
-            *reinterpret_cast<uint16_t*>(obase + s * LR) =
-                (uint16_t)__builtin_amdgcn_perm(0u, pk_bits(o), 0x0c0c0200u);
-        }
-        __builtin_amdgcn_wave_barrier();
-        // this block's results, one window per lane
-        stores.store(out, blk, woff, wline && lstep < n - blk * K, S.out + lane * LR);
-    };
-    // the prologue issues the ring's slots in the loop's order: the wait
-    // counts at the loop head merge both paths
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < kPkAhead; ++u) {
-        fetch(u, u);
-        __builtin_amdgcn_sched_barrier(0);
+    for (int h = 0; h < NP; ++h) {
+        seed[h] = horiz ? 0 : a.init[min(group * SPW + (lane + 64 * h) / K, nlines - 1)];
+        pb[h] = 0;
     }
-    for (int blk0 = 0; blk0 < nblk; blk0 += kPkAhead) {
+    // A block into LDS: the costs transposed, so that a lane later reads the
+    // cost pairs of all K steps of its line with wide loads (zero-extended to
+    // u16), and what each pixel's step needs.  Returns the steps at which some
+    // line shifts by more than one, as bits, and kInvalid if a pixel is invalid.
+    constexpr uint32_t kInvalid = 1u << 16;
+    auto stage = [&](int slot, int blk) __attribute__((always_inline)) -> uint32_t {
+        int b[NP], q[NP];
+        uint32_t kind = 0u;
 #pragma unroll
-        for (int u = 0; u < kPkAhead; ++u) {
-            // blocks past the last one (at most kPkAhead - 1) walk the
-            // line's last pixel again; their stores are dropped
-            const int blk = blk0 + u;
-            __builtin_amdgcn_wave_barrier();
-            stage(u);
-            fetch(u, blk + kPkAhead);
-            process(blk);
-        }
-    }
-}
-
-template <int LR>
-__global__ __launch_bounds__(64) void agg_init_pk_kernel(PyrLevel a) {
-    __shared__ __align__(16) AggInitPkLds<LR> lds;
-    constexpr int SPW = 128 / LR;
-    const int nh = (a.h + SPW - 1) / SPW, nv = (a.w + SPW - 1) / SPW;
-    const int item = blockIdx.x;
-    int dir, group;
-    if (item < nh) { dir = 1; group = item; }
-    else if (item < 2 * nh) { dir = 3; group = item - nh; }
-    else if (item < 2 * nh + nv) { dir = 0; group = item - 2 * nh; }
-    else { dir = 2; group = item - 2 * nh - nv; }
-    agg_init_pk_lines<LR>(a, dir, group, threadIdx.x, lds);
-}
-
-// The packed aggregation with four disparities per lane (two u16 pairs, A =
-// 4k, 4k+1 and B = 4k+2, 4k+3): LR / 4 lanes per scanline, 256 / LR
-// scanlines per wave.  Per step a lane needs the neighbour pairs starting
-// at 4k + q - 1, 4k + q + 1 and 4k + q + 3 (q = b - b'), the middle one
-// serving both of its pairs, so a step costs about as many instructions as
-// the two-disparity form for twice the cells.  It has half as many waves,
-// which suits the largest level; the launch picks the form.  Same window
-// row (overlapping pairs, 127 pads), table and exactness range.
-template <int LR>
-struct AggInitPk2Lds {
-    static constexpr int LPL = LR / 4, SPW = 64 / LPL, K = LR / 2;
-    static constexpr int PAD = (LR + 2 + 3) / 4 * 4;         // a multiple of 4: 16-byte row stores
-    static constexpr int ROW = (PAD + 2 * LR + 1 + 3) / 4 * 4;
-    uint32_t cost[SPW][LR / 2][K];           // [line][pair][step]: the pair's costs as u16
-    uint8_t out[2 * 64 * LR];                // [line][step][t]
-    int16_t init[2 * 64];                    // [line][step]
-    uint32_t pen2[kPkDeltaHi - kPkDeltaLo + 1];
-    uint32_t win[SPW][ROW];
-};
-
-template <int LR>
-__device__ __forceinline__ void agg_init_pk2_lines(const PyrLevel& a, int dir, int group, int lane,
-                                                   AggInitPk2Lds<LR>& S) {
-    using Lds = AggInitPk2Lds<LR>;
-    constexpr int LPL = Lds::LPL, SPW = Lds::SPW, K = Lds::K, PAD = Lds::PAD, ROW = Lds::ROW;
-    constexpr int NV = LR / 16;
-    constexpr uint32_t kPadPair = 127u * 0x10001u;
-    static_assert(SPW * K == 128, "a block is two pixels per lane");
-    // The lanes of a scanline sit STRIDE = 16 / LPL apart in one DPP row, so a
-    // neighbouring quad is a row shift by STRIDE.  The line's first and last
-    // lanes then read from outside the row, which leaves a move's old value in
-    // place: the 127 pads stay in those lanes of two persistent registers,
-    // with no select per step.
-    constexpr int STRIDE = 16 / LPL;
-    const int sub = (lane / 16) * STRIDE + lane % STRIDE;   // recurrence: line
-    const int k = (lane % 16) / STRIDE;                     // disparity quad
-    const bool horiz = (dir == 1 || dir == 3);
-    const bool fwd = (dir == 0 || dir == 1);
-    const int W = a.w, H = a.h;
-    const int nlines = horiz ? H : W;
-    const int n = horiz ? W : H;
-    auto pix_of = [&](int line, int step) -> int64_t {
-        line = min(line, nlines - 1);
-        step = min(step, n - 1);
-        const int pos = fwd ? step : n - 1 - step;
-        return horiz ? (int64_t)line * W + pos : (int64_t)pos * W + line;
-    };
-    const int line = min(group * SPW + sub, nlines - 1);
-    uint8_t* out = (dir == 0) ? a.path[0] : (dir == 1) ? a.path[1] : (dir == 2) ? a.path[2] : a.path[3];
-
-    // loads and stores: lane j handles the block's pixels j and j + 64 in
-    // [line][step] order
-    // a ring of kPkAhead blocks of loads in flight (slot = block mod kPkAhead)
-    uint4 nc[kPkAhead][2][NV];
-    int nb[kPkAhead][2];
-    auto fetch = [&](int slot, int blk) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int idx = lane + 64 * h;
-            const int64_t p = pix_of(group * SPW + idx / K, blk * K + idx % K);
-            const uint4* src = reinterpret_cast<const uint4*>(a.cost + p * LR);
-#pragma unroll
-            for (int v = 0; v < NV; ++v) nc[slot][h][v] = src[v];
-            nb[slot][h] = a.init[p];
-        }
-    };
-    auto stage = [&](int slot) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int idx = lane + 64 * h;
+        for (int h = 0; h < NP; ++h) {
             uint32_t wv[LR / 4];
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
@@ -675,155 +501,214 @@ __device__ __forceinline__ void agg_init_pk2_lines(const PyrLevel& a, int dir, i
             }
 #pragma unroll
             for (int j = 0; j < LR / 2; ++j)
-                S.cost[idx / K][j][idx % K] =
+                S.cost[(lane + 64 * h) / K * Lds::LINE + j * Lds::PAIR + lstep] =
                     __builtin_amdgcn_perm(0u, wv[j / 2], (j & 1) ? 0x0c030c02u : 0x0c010c00u);
-            S.init[idx] = (int16_t)nb[slot][h];
+            b[h] = (int)(int16_t)nb[slot][h];
+            // v: the base of the last valid pixel up to this one (none: the
+            // marker, whose distance is past every window, as it should be)
+            const int before = __builtin_amdgcn_mov_dpp(pb[h], 0x100 + K - 1, 0xF, 0xF, true);   // row_shl:K-1
+            int v = b[h];
+            if (lstep == 0) {
+                if (blk == 0) v = horiz ? v : seed[h];
+                else v = v == kInvalidShort ? before : v;
+            }
+            if (__builtin_amdgcn_ballot_w64(b[h] == kInvalidShort) != 0) {
+                kind |= kInvalid;
+                auto pull = [&](int d, int from) __attribute__((always_inline)) {
+                    v = v == kInvalidShort && lstep >= d ? from : v;
+                };
+                pull(1, __builtin_amdgcn_mov_dpp(v, 0x111, 0xF, 0xF, true));   // row_shr:1, 2, 4, 8
+                pull(2, __builtin_amdgcn_mov_dpp(v, 0x112, 0xF, 0xF, true));
+                pull(4, __builtin_amdgcn_mov_dpp(v, 0x114, 0xF, 0xF, true));
+                if constexpr (K == 16) pull(8, __builtin_amdgcn_mov_dpp(v, 0x118, 0xF, 0xF, true));
+            }
+            const int last = __builtin_amdgcn_mov_dpp(v, 0x111, 0xF, 0xF, true);
+            q[h] = b[h] - (lstep == 0 ? before : last);
+            pb[h] = v;
+            const bool far = (uint32_t)(q[h] + 1) > 2u && b[h] != kInvalidShort && inside(h, blk) &&
+                             (blk > 0 || lstep > 0);
+            uint64_t f = __builtin_amdgcn_ballot_w64(far);
+            f |= f >> 32;
+            f |= f >> 16;
+            if constexpr (K == 8) f |= f >> 8;
+            kind |= (uint32_t)f & ((1u << K) - 1u);
+        }
+#pragma unroll
+        for (int h = 0; h < NP; ++h) {
+            const int idx = lane + 64 * h;
+            S.valid[idx] = (int16_t)(b[h] == kInvalidShort ? 0 : -1);
+            const uint32_t sel = shift_sel(q[h], 0x0202u, k10001, 0x03020100u);
+            S.sel[idx] = (kind >> lstep) & 1u ? (uint32_t)q[h] : sel;
+            S.pen[idx] = small_pen(q[h]);
+        }
+        return kind;
+    };
+    // a staged block as this lane walks it
+    struct Block {
+        uint32_t valid[K / 2], cost[NP][K], sel[K], pen[K];
+    };
+    auto wide = [](const void* src, int words, uint32_t* dst) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < words / 4; ++i) {
+            const uint4 v = reinterpret_cast<const uint4*>(src)[i];
+            dst[4 * i] = v.x; dst[4 * i + 1] = v.y; dst[4 * i + 2] = v.z; dst[4 * i + 3] = v.w;
         }
     };
+    auto take = [&](Block& B) __attribute__((always_inline)) {
+        wide(&S.valid[sub * K], K / 2, B.valid);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) wide(&S.cost[sub * Lds::LINE + (NP * k + i) * Lds::PAIR], K, B.cost[i]);
+        wide(&S.sel[sub * K], K, B.sel);
+        wide(&S.pen[sub * K], K, B.pen);
+    };
 
-    for (int e = lane; e < SPW * ROW; e += 64) (&S.win[0][0])[e] = kPadPair;
-    for (int e = lane; e <= kPkDeltaHi - kPkDeltaLo; e += 64) {
-        const int q = e + kPkDeltaLo;
-        const uint32_t v = (uint32_t)max(a.p1, a.p2 / max(1, abs(1 - q)));
-        S.pen2[e] = v | (v << 16);
-    }
-    __builtin_amdgcn_wave_barrier();
-
-    uint32_t* wrow = &S.win[sub][0];
-    const uint32_t* wlane = wrow + (PAD - 1 + 4 * k);     // + q: the first neighbour pair
-    const bool last_k = k == LPL - 1;
-    uint8_t* obase = S.out + sub * K * LR + 4 * k;
-    const pk16 p1v = pk_of((uint32_t)a.p1 * 0x10001u);
-    const pk16 m127 = pk_of(kPadPair);
-    const uint32_t k10001 = 0x10001u;
-    const pk16 pen2_m1 = pk_of(S.pen2[-1 - kPkDeltaLo]);
-    const pk16 pen2_01 = pk_of(S.pen2[0 - kPkDeltaLo]);
-    int qlo = kPkDeltaLo, qhi = kPkDeltaHi, wlo = -(LR + 1);
-    asm volatile("" : "+v"(qlo), "+v"(qhi), "+v"(wlo));
-    // the window row from this lane's pairs of L + P1 (A, B): C[PAD + 4k ..
-    // PAD + 4k + 3] in one 16-byte store, and C[PAD - 1] from lane 0
-    auto put = [&](uint32_t oa, uint32_t ob) __attribute__((always_inline)) {
-        uint32_t nxt = dppu<0x100 + STRIDE>(oa);          // row_shl: lane k + 1's A
+    // the window row from this lane's pairs of L + P1: the lane's pairs and
+    // the ones between them, and C[PAD - 1] from the first lane
+    auto put = [&](const uint32_t (&o)[NP]) __attribute__((always_inline)) {
+        uint32_t nxt = dppu<0x100 + STRIDE>(o[0]);        // row_shl: the next lane's first pair
         nxt = last_k ? kPadPair : nxt;
-        const uint4 v = make_uint4(oa, __builtin_amdgcn_alignbit(ob, oa, 16), ob,
-                                   __builtin_amdgcn_alignbit(nxt, ob, 16));
-        *reinterpret_cast<uint4*>(wrow + PAD + 4 * k) = v;
-        if (k == 0) wrow[PAD - 1] = (oa << 16) | 127u;
+        uint32_t* dst = wrow + PAD + 2 * NP * k;
+        if constexpr (NP == 2)
+            *reinterpret_cast<uint4*>(dst) =
+                make_uint4(o[0], __builtin_amdgcn_alignbit(o[1], o[0], 16), o[1],
+                           __builtin_amdgcn_alignbit(nxt, o[1], 16));
+        else
+            *reinterpret_cast<uint2*>(dst) = make_uint2(o[0], __builtin_amdgcn_alignbit(nxt, o[0], 16));
+        if (k == 0) wrow[PAD - 1] = (o[0] << 16) | 127u;
     };
-    auto group_min4 = [&](pk16 v) __attribute__((always_inline)) {
-        v = __builtin_elementwise_min(v, v.yx);
-        uint32_t m = pk_bits(v);
-        m = min(m, dppu<0x120 + STRIDE>(m));              // row_ror by STRIDE, 2 STRIDE, ...
-        if constexpr (2 * STRIDE < 16) m = min(m, dppu<0x120 + 2 * STRIDE>(m));
-        if constexpr (4 * STRIDE < 16) m = min(m, dppu<0x120 + 4 * STRIDE>(m));
-        return pk_of(m);
+    // minimum over the scanline's lanes of both halves, in both halves
+    auto line_min = [&](const pk16 (&v)[NP]) __attribute__((always_inline)) {
+        pk16 w = v[0];
+        if constexpr (NP == 2) w = pk_min2(w, v[1]);
+        w = pk_min2(w, w.yx);
+        uint32_t r = pk_bits(w);                          // equal halves: u32 order = u16 order
+        r = min(r, dppu<0x120 + STRIDE>(r));              // row_ror by STRIDE, 2 STRIDE, ...
+        if constexpr (2 * STRIDE < 16) r = min(r, dppu<0x120 + 2 * STRIDE>(r));
+        if constexpr (4 * STRIDE < 16) r = min(r, dppu<0x120 + 4 * STRIDE>(r));
+        if constexpr (8 * STRIDE < 16) r = min(r, dppu<0x120 + 8 * STRIDE>(r));
+        return pk_of(r);
+    };
+    uint32_t nxt_r = kPadPair, prv_r = kPadPair;   // pads kept in the last / first lane of a line
+    // neighbour pairs for a shift in {-1, 0, 1}: bytes 2 (q + 1) .. 2 (q + 1) + 3
+    // of {first, the lane before's last}, ..., {the next lane's first, last}
+    auto dpp_pairs = [&](const uint32_t (&o)[NP], uint32_t sel, uint32_t (&x)[NP + 1]) __attribute__((always_inline)) {
+        nxt_r = (uint32_t)__builtin_amdgcn_update_dpp((int)nxt_r, (int)o[0], 0x100 + STRIDE, 0xF, 0xF, false);
+        prv_r = (uint32_t)__builtin_amdgcn_update_dpp((int)prv_r, (int)o[NP - 1], 0x110 + STRIDE, 0xF, 0xF, false);
+        x[0] = __builtin_amdgcn_perm(o[0], prv_r, sel);
+        if constexpr (NP == 2) x[1] = __builtin_amdgcn_perm(o[1], o[0], sel);
+        x[NP] = __builtin_amdgcn_perm(nxt_r, o[NP - 1], sel);
+    };
+    pk16 L[NP], m = pk_of(0u);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) L[i] = pk_of(0u);
+    // this step's L from the previous L, m and the neighbour pairs
+    auto relax = [&](const Block& B, int s, const uint32_t (&x)[NP + 1], uint32_t pen, pk16 (&l)[NP])
+        __attribute__((always_inline)) {
+        const pk16 t = pk_min2(pk_of(x[1]), m + pk_of(pen));
+        l[0] = pk_min2(pk_min2(L[0], pk_of(x[0])), t);
+        if constexpr (NP == 2) l[1] = pk_min2(pk_min2(L[1], pk_of(x[2])), t);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) l[i] = pk_of(B.cost[i][s]) - m + l[i];
+    };
+    // the low bytes of a step's results
+    auto emit = [&](int s, const pk16 (&l)[NP], uint32_t mask) __attribute__((always_inline)) {
+        if constexpr (NP == 2)
+            *reinterpret_cast<uint32_t*>(obase + s * LR) =
+                __builtin_amdgcn_perm(pk_bits(l[1]), pk_bits(l[0]), 0x06040200u) & mask;
+        else
+            *reinterpret_cast<uint16_t*>(obase + s * LR) =
+                (uint16_t)(__builtin_amdgcn_perm(0u, pk_bits(l[0]), 0x0c0c0200u) & mask);
     };
 
-    pk16 LA = pk_of(0u), LB = pk_of(0u), m = pk_of(0u);
-    int last_b = 0;
-    // A11: vertical directions seed b' from row 0 whichever end they start at
-    const int seed_b = horiz ? 0 : a.init[line];
-    const int nblk = (n + K - 1) / K;
-    const BlockStores<LR, K> stores(horiz, fwd, W, n, group * SPW);
-    uint32_t woff[2];
-    bool wline[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int idx = lane + 64 * h;
-        woff[h] = BlockStores<LR, K>::offset(horiz, fwd, W, idx / K, idx % K);
-        wline[h] = group * SPW + idx / K < nlines;
-    }
-    uint32_t nxt_r = kPadPair, prv_r = kPadPair;   // pads kept in the last / first lane of a line
-    // neighbour pairs at 4k + q - 1, 4k + q + 1, 4k + q + 3 for a base step q
-    // in {-1, 0, 1}: bytes 2 (q + 1) .. 2 (q + 1) + 3 of {oa, prv}, {ob, oa},
-    // {nxt, ob}, with `sel` the selector of q
-    auto dpp_terms = [&](uint32_t oa, uint32_t ob, uint32_t sel, int q, uint32_t& x0, uint32_t& x1,
-                         uint32_t& x2, pk16& pen2) __attribute__((always_inline)) {
-        // lane k + 1's A and lane k - 1's B (row_shl / row_shr by STRIDE,
-        // out-of-row sources not written)
-        nxt_r = (uint32_t)__builtin_amdgcn_update_dpp((int)nxt_r, (int)oa, 0x100 + STRIDE, 0xF, 0xF, false);
-        prv_r = (uint32_t)__builtin_amdgcn_update_dpp((int)prv_r, (int)ob, 0x110 + STRIDE, 0xF, 0xF, false);
-        x0 = __builtin_amdgcn_perm(oa, prv_r, sel);
-        x1 = __builtin_amdgcn_perm(ob, oa, sel);
-        x2 = __builtin_amdgcn_perm(nxt_r, ob, sel);
-        const uint32_t mneg = 0u - (uint32_t)(q < 0);
-        pen2 = pk_of((pk_bits(pen2_m1) & mneg) | (pk_bits(pen2_01) & ~mneg));
-    };
-    // this step's L of the lane's two pairs from the previous L, m and the
-    // neighbour terms
-    auto relax = [&](pk16 cA, pk16 cB, uint32_t x0, uint32_t x1, uint32_t x2, pk16 pen2, pk16& lA,
-                     pk16& lB) __attribute__((always_inline)) {
-        const pk16 t = __builtin_elementwise_min(pk_of(x1), m + pen2);
-        const pk16 vA = __builtin_elementwise_min(__builtin_elementwise_min(LA, pk_of(x0)), t);
-        const pk16 vB = __builtin_elementwise_min(__builtin_elementwise_min(LB, pk_of(x2)), t);
-        lA = cA + (vA - m);
-        lB = cB + (vB - m);
-    };
-    auto process = [&](int blk) __attribute__((always_inline)) {
-        __builtin_amdgcn_wave_barrier();
-        uint32_t bw[K / 2], ca[K], cb[K];
-#pragma unroll
-        for (int i = 0; i < K / 8; ++i) {
-            const uint4 v = reinterpret_cast<const uint4*>(&S.init[sub * K])[i];
-            bw[4 * i] = v.x; bw[4 * i + 1] = v.y; bw[4 * i + 2] = v.z; bw[4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int i = 0; i < K / 4; ++i) {
-            const uint4 va = reinterpret_cast<const uint4*>(&S.cost[sub][2 * k][0])[i];
-            const uint4 vb = reinterpret_cast<const uint4*>(&S.cost[sub][2 * k + 1][0])[i];
-            ca[4 * i] = va.x; ca[4 * i + 1] = va.y; ca[4 * i + 2] = va.z; ca[4 * i + 3] = va.w;
-            cb[4 * i] = vb.x; cb[4 * i + 1] = vb.y; cb[4 * i + 2] = vb.z; cb[4 * i + 3] = vb.w;
-        }
+    // a block with no invalid pixel and no wide step
+    auto straight = [&](const Block& B) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < K; ++s) {
-            const int b = (int)(int16_t)(bw[s / 2] >> (16 * (s & 1)));
-            const pk16 cA = pk_of(ca[s]), cB = pk_of(cb[s]);
-            uint32_t ow;   // the low bytes of the four halves
-            if (s == 0 && blk == 0) {
-                LA = cA;
-                LB = cB;
-                m = group_min4(__builtin_elementwise_min(LA, LB));
-                last_b = horiz ? b : seed_b;
-                ow = __builtin_amdgcn_perm(pk_bits(LB), pk_bits(LA), 0x06040200u);
-            } else {
-                const bool valid = b != kInvalidShort;
-                const int q = b - last_b;
-                const uint32_t oa = pk_bits(LA + p1v), ob = pk_bits(LB + p1v);
-                uint32_t x0, x1, x2;                     // pairs at 4k + q - 1, + 1, + 3
-                pk16 pen2;
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(valid && (q < -1 || q > 1)) == 0, 1)) {
-                    dpp_terms(oa, ob, shift_sel(q, 0x0202u, k10001, 0x03020100u), q, x0, x1, x2, pen2);
-                } else {
-                    put(oa, ob);   // the window row holds L only when a step needs it
-                    const int qt = min(max(q, qlo), qhi);
-                    const int qw = min(max(q, wlo), LR + 1);
-                    x0 = wlane[qw];
-                    x1 = wlane[qw + 2];
-                    x2 = wlane[qw + 4];
-                    uint32_t pb = S.pen2[qt - kPkDeltaLo];
-                    // complete these reads inside the branch (see agg_init_pk_lines)
-                    asm volatile("" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(pb));
-                    pen2 = pk_of(pb);
-                }
-                pk16 lA, lB;
-                relax(cA, cB, x0, x1, x2, pen2, lA, lB);
-                const pk16 mn = group_min4(__builtin_elementwise_min(lA, lB));
-                const uint32_t vm = 0u - (uint32_t)valid;
-                ow = __builtin_amdgcn_perm(pk_bits(lB), pk_bits(lA), 0x06040200u) & vm;
-                LA = pk_of((pk_bits(lA) & vm) | (pk_bits(LA) & ~vm));
-                LB = pk_of((pk_bits(lB) & vm) | (pk_bits(LB) & ~vm));
-                m = pk_of((pk_bits(mn) & vm) | (pk_bits(m127) & ~vm));
-                last_b = (int)(((uint32_t)b & vm) | ((uint32_t)last_b & ~vm));
-            }
-            *reinterpret_cast<uint32_t*>(obase + s * LR) = ow;
-        }
-        __builtin_amdgcn_wave_barrier();
+            uint32_t o[NP], x[NP + 1];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {   // this block's results, one window per pixel
-            const int idx = lane + 64 * h;
-            stores.store(out, blk, woff[h], wline[h] && idx % K < n - blk * K, S.out + idx * LR);
+            for (int i = 0; i < NP; ++i) o[i] = pk_bits(L[i] + p1v);
+            dpp_pairs(o, B.sel[s], x);
+            pk16 l[NP];
+            relax(B, s, x, B.pen[s], l);
+            m = line_min(l);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) L[i] = l[i];
+            emit(s, l, ~0u);
         }
     };
+    auto mixed = [&](const Block& B, uint32_t wide_steps, bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < K; ++s) {
+            if (s == 0 && first) {
+#pragma unroll
+                for (int i = 0; i < NP; ++i) L[i] = pk_of(B.cost[i][0]);
+                m = line_min(L);
+                emit(0, L, ~0u);
+                continue;
+            }
+            uint32_t o[NP], x[NP + 1], pen;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) o[i] = pk_bits(L[i] + p1v);
+            if ((wide_steps >> s & 1u) == 0) {
+                dpp_pairs(o, B.sel[s], x);
+                pen = B.pen[s];
+            } else {
+                const int q = (int)B.sel[s];
+                const int qw = min(max(q, -(LR + 1)), LR + 1);
+                if constexpr (NP == 1) {
+                    // the three pairs from disparity 2k + q - 1 (rounded down
+                    // to even) on, straight from their lanes
+                    const int e = 2 * k + qw - 1, j = e >> 1;
+                    uint32_t p[3];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const uint32_t v = bperm(lane - k * STRIDE + (j + i) * STRIDE, o[0]);
+                        p[i] = (uint32_t)(j + i) < (uint32_t)LPL ? v : kPadPair;
+                    }
+                    const uint32_t sel = e & 1 ? 0x05040302u : 0x03020100u;
+                    x[0] = __builtin_amdgcn_perm(p[1], p[0], sel);
+                    x[1] = __builtin_amdgcn_perm(p[2], p[1], sel);
+                } else {
+                    put(o);    // the window row holds L only when a step needs it
+#pragma unroll
+                    for (int i = 0; i <= NP; ++i) x[i] = wlane[qw + 2 * i];
+                }
+                pen = S.pen2[min(max(q, kPkDeltaLo), kPkDeltaHi) - kPkDeltaLo];
+            }
+            pk16 l[NP];
+            relax(B, s, x, pen, l);
+            const pk16 mn = line_min(l);
+            // an invalid pixel keeps L, sets m to 127 and leaves 0; selects as
+            // bit operations (v_bfi), so the step stays one block
+            const uint32_t vm = (uint32_t)(int)(int16_t)(B.valid[s / 2] >> (16 * (s & 1)));
+            emit(s, l, NP == 2 ? vm : vm & 0xFFFFu);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) L[i] = pk_of((pk_bits(l[i]) & vm) | (pk_bits(L[i]) & ~vm));
+            m = pk_of((pk_bits(mn) & vm) | (pk_bits(m127) & ~vm));
+        }
+    };
+
+    const int nblk = (n + K - 1) / K;
+    // a block's results, one window per pixel: read back, then stored
+    auto results = [&](uint4 (&r)[NP][NV]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < NP; ++h)
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                r[h][v] = reinterpret_cast<const uint4*>(S.out + (lane + 64 * h) / K * Lds::OUT + lstep * LR)[v];
+    };
+    auto store = [&](const uint4 (&r)[NP][NV], int blk) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rs = outs.next();
+#pragma unroll
+        for (int h = 0; h < NP; ++h) {
+            const uint32_t o = inside(h, blk) && blk >= 0 ? off[h] * LR : 0x80000000u;
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                __builtin_amdgcn_raw_buffer_store_b128(pyr_u32x4{r[h][v].x, r[h][v].y, r[h][v].z, r[h][v].w}, rs,
+                                                       (int)(o + 16 * v), 0, 0);
+        }
+    };
+
     // the prologue issues the ring's slots in the loop's order: the wait
     // counts at the loop head merge both paths
     __builtin_amdgcn_sched_barrier(0);
@@ -832,24 +717,40 @@ __device__ __forceinline__ void agg_init_pk2_lines(const PyrLevel& a, int dir, i
         fetch(u, u);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (int blk0 = 0; blk0 < nblk; blk0 += kPkAhead) {
+    Block B[2];
+    uint32_t kind = stage(0, 0);
+    fetch(0, kPkAhead);
+    __builtin_amdgcn_wave_barrier();
+    take(B[0]);
+    kind |= kInvalid;                        // the first pixel has a rule of its own
+    int blk0 = 0;
+    do {
 #pragma unroll
         for (int u = 0; u < kPkAhead; ++u) {
-            // blocks past the last one (at most kPkAhead - 1) walk the
-            // line's last pixel again; their stores are dropped
+            // blocks past the last one (at most kPkAhead - 1) hold nothing;
+            // their stores are dropped
             const int blk = blk0 + u;
+            uint4 r[NP][NV];
             __builtin_amdgcn_wave_barrier();
-            stage(u);
-            fetch(u, blk + kPkAhead);
-            process(blk);
+            results(r);                                          // block blk - 1
+            const uint32_t next = stage((u + 1) % kPkAhead, blk + 1);
+            __builtin_amdgcn_wave_barrier();
+            take(B[(u + 1) % 2]);
+            store(r, blk - 1);
+            fetch((u + 1) % kPkAhead, blk + 1 + kPkAhead);
+            __builtin_amdgcn_wave_barrier();
+            if (__builtin_expect(kind == 0, 1)) straight(B[u % 2]);
+            else mixed(B[u % 2], kind, blk == 0);
+            kind = next;
         }
-    }
+        blk0 += kPkAhead;
+    } while (blk0 <= nblk);                  // one block further: the last one's results
 }
 
-template <int LR>
-__global__ __launch_bounds__(64) void agg_init_pk2_kernel(PyrLevel a) {
-    __shared__ __align__(16) AggInitPk2Lds<LR> lds;
-    constexpr int SPW = AggInitPk2Lds<LR>::SPW;
+template <int LR, int NP>
+__global__ __launch_bounds__(64) void agg_init_pk_kernel(PyrLevel a) {
+    __shared__ __align__(16) AggInitPkLds<LR, NP> lds;
+    constexpr int SPW = AggInitPkLds<LR, NP>::SPW;
     const int nh = (a.h + SPW - 1) / SPW, nv = (a.w + SPW - 1) / SPW;
     const int item = blockIdx.x;
     int dir, group;
@@ -857,7 +758,7 @@ __global__ __launch_bounds__(64) void agg_init_pk2_kernel(PyrLevel a) {
     else if (item < 2 * nh) { dir = 3; group = item - nh; }
     else if (item < 2 * nh + nv) { dir = 0; group = item - 2 * nh; }
     else { dir = 2; group = item - 2 * nh - nv; }
-    agg_init_pk2_lines<LR>(a, dir, group, threadIdx.x, lds);
+    agg_init_pk_lines<LR, NP>(a, dir, group, threadIdx.x, lds);
 }
 
 // WTA with initial disparity (cusgm_ca.cu:3425-3512), one lane per pixel
@@ -984,18 +885,23 @@ hipError_t pyr_launch_aggregate_init(const PyrLevel& a, hipStream_t s) {
     auto items = [&](int spw) { return 2 * ((a.h + spw - 1) / spw) + 2 * ((a.w + spw - 1) / spw); };
     int form = window_form();
     if (!agg_init_packed_ok(a)) form = SGM_WINDOW_U32;
+    // Quads issue fewer instructions per cell, pairs have twice the waves and
+    // the shorter step.  Pairs / quads, us: window 16, 4800x3409 (1.0 quad waves
+    // per SIMD) 661 / 785, 7000x5000 (1.5) 1195 / 1221, 9600x6800 (2.0) 2330 /
+    // 2250; window 32, 1700x1200 (0.7) 205 / 271, 2900x2200 (1.2) 538 / 493.
     if (form == SGM_WINDOW_AUTO)
-        form = items(256 / a.level_range) >= device_simds() ? SGM_WINDOW_QUADS : SGM_WINDOW_PAIRS;
+        form = items(256 / a.level_range) >= (a.level_range == 16 ? 2 : 1) * device_simds() ? SGM_WINDOW_QUADS
+                                                                                           : SGM_WINDOW_PAIRS;
     if (form == SGM_WINDOW_QUADS) {
         const int n = items(256 / a.level_range);
-        if (a.level_range == 16) hipLaunchKernelGGL(agg_init_pk2_kernel<16>, dim3(n), dim3(64), 0, s, a);
-        else hipLaunchKernelGGL(agg_init_pk2_kernel<32>, dim3(n), dim3(64), 0, s, a);
+        if (a.level_range == 16) hipLaunchKernelGGL((agg_init_pk_kernel<16, 2>), dim3(n), dim3(64), 0, s, a);
+        else hipLaunchKernelGGL((agg_init_pk_kernel<32, 2>), dim3(n), dim3(64), 0, s, a);
         return hipGetLastError();
     }
     if (form == SGM_WINDOW_PAIRS) {
         const int n = items(128 / a.level_range);
-        if (a.level_range == 16) hipLaunchKernelGGL(agg_init_pk_kernel<16>, dim3(n), dim3(64), 0, s, a);
-        else hipLaunchKernelGGL(agg_init_pk_kernel<32>, dim3(n), dim3(64), 0, s, a);
+        if (a.level_range == 16) hipLaunchKernelGGL((agg_init_pk_kernel<16, 1>), dim3(n), dim3(64), 0, s, a);
+        else hipLaunchKernelGGL((agg_init_pk_kernel<32, 1>), dim3(n), dim3(64), 0, s, a);
         return hipGetLastError();
     }
     if (a.level_range == 16) {
