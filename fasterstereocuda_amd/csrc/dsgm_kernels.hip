@@ -43,9 +43,10 @@
 // steps, max(H, W) + H forward and again backward, each 130-300 instructions
 // of a wave that has its SIMD to itself; for many, the copy rate (93 bytes per
 // cell).  Walking a row's directions one after the other made the chain
-// 2 W + H: 2 images 321x119 D = 64 0.57 -> 0.28 ms forward + backward, one
+// 2 W + H: 2 images 321x119 D = 64 0.57 -> 0.27 ms forward + backward, one
 // image 1242x375 D = 128 3.24 -> 1.58, D = 256 6.04 -> 3.28 ms, 4 images
 // D = 64 3.13 -> 2.37 ms.
+#include <algorithm>
 #include <type_traits>
 
 #include "dsgm_device.h"
@@ -64,26 +65,28 @@ namespace {
 // (Fewer at D = 256, where four would pass the 256 vector registers.)
 template <int D, bool LAST> constexpr int kAhead = D < 256 ? 4 : LAST ? 2 : 3;
 
-// Offsets of a scanline's cells from a wave-uniform base: 32 bits unless the
-// image is so wide that two of its rows pass 2^31 bytes.
+// Byte offsets from a wave-uniform base: 32 bits, which an access takes beside
+// a scalar base, unless two rows of the image or two directions' codes pass
+// 2^31 bytes (64-bit address arithmetic took a sixth of a D = 64 step).
 template <bool WIDE> using Off = std::conditional_t<WIDE, int64_t, uint32_t>;
 
-template <int D, class T, class O>
-__device__ __forceinline__ T* cell_at(T* base, O pix, int l) {
-    return base + ((O)(pix * D) + (O)(l * (D / 16)));
+template <class T, class O>
+__device__ __forceinline__ T* at(T* base, O bytes) {
+    return (T*)((std::conditional_t<std::is_const_v<T>, const char, char>*)base + bytes);
 }
 // Winner codes are loaded as the dword that holds the lane's: the masking of a
 // 1- or 2-byte load would wait at the top of the loop for the whole ring.
 // (The codes of a pixel are D / 4 bytes, and the buffer starts on 8.)
-template <int D>
-__device__ __forceinline__ uint32_t load_codes(const uint8_t* pixel, int l) {
-    return *(const __attribute__((address_space(1))) uint32_t*)(pixel + ((l * (D / 64)) & ~3));
+template <int D> constexpr int kCodeBytes = D / 4;
+template <int D> __device__ __forceinline__ uint32_t code_byte(int l) { return (uint32_t)l * (D / 64); }
+__device__ __forceinline__ uint32_t load_codes(const uint8_t* p) {
+    return *(const __attribute__((address_space(1))) uint32_t*)p;
 }
 template <int D>
-__device__ __forceinline__ uint32_t shift_codes(uint32_t w, int l) { return w >> (8 * ((l * (D / 64)) & 3)); }
+__device__ __forceinline__ uint32_t shift_codes(uint32_t w, int l) { return w >> (8 * (code_byte<D>(l) & 3)); }
 template <int D>
-__device__ __forceinline__ void store_codes(uint8_t* pixel, int l, uint32_t w) {
-    *(__attribute__((address_space(1))) WinWord<D>*)(pixel + l * (D / 64)) = (WinWord<D>)w;
+__device__ __forceinline__ void store_codes(uint8_t* p, uint32_t w) {
+    *(__attribute__((address_space(1))) WinWord<D>*)p = (WinWord<D>)w;
 }
 __device__ __forceinline__ void storeb(uint8_t* p, int v) { *(__attribute__((address_space(1))) uint8_t*)p = (uint8_t)v; }
 __device__ __forceinline__ int loadb(const uint8_t* p) { return *(const __attribute__((address_space(1))) uint8_t*)p; }
@@ -159,9 +162,10 @@ __device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int la
     const float* cost = A.cost + rp.q0 * D;
     float* S = A.S + rp.q0 * D;
     const float *p1 = A.p1 + rp.q0, *p2 = A.p2 + rp.q0;
-    const int64_t line0 = (rp.second ? 3 : 1) * npix + rp.q0;
-    uint8_t* wout = A.wins + line0 * (D / 4);
-    uint8_t* kout = A.kstar + line0;
+    uint8_t* wout = A.wins + (npix + rp.q0) * kCodeBytes<D>;   // of direction 1; 3 is two planes on
+    uint8_t* kout = A.kstar + npix + rp.q0;
+    const Off<WIDE> plane = rp.second ? (Off<WIDE>)(2 * npix) : 0;
+    const Off<WIDE> lane_c = (Off<WIDE>)(l * DPD * 4), lane_w = plane * kCodeBytes<D> + code_byte<D>(l);
 
     float qc[NA][DPD], qp1[NA], qp2[NA], qs[NA][DPD];
     float L[DPD];
@@ -174,10 +178,10 @@ __device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int la
         Off<WIDE> pi = rp.pix(t0), ps = pi;      // pixels of the next issue and of the step
         int ti = t0;
         auto issue = [&](int u) __attribute__((always_inline)) {
-            loadf<DPD>(cell_at<D>(cost, pi, l), qc[u]);
-            if constexpr (PHASE == kPairAdd) loadf<DPD>(cell_at<D>(S, pi, l), qs[u]);
-            qp1[u] = loads(p1 + pi);
-            qp2[u] = loads(p2 + pi);
+            loadf<DPD>(at(cost, pi * (D * 4) + lane_c), qc[u]);
+            if constexpr (PHASE == kPairAdd) loadf<DPD>(at(S, pi * (D * 4) + lane_c), qs[u]);
+            qp1[u] = loads(at(p1, pi * 4));
+            qp2[u] = loads(at(p2, pi * 4));
             pi = rp.move(pi, ++ti);
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -194,9 +198,9 @@ __device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int la
                 if constexpr (PHASE == kPairAdd) sv[k] = qs[u][k] + L[k];
                 if constexpr (PHASE == kPairMiddle) sv[k] = L[k] + other_half(L[k], lane);
             }
-            storef<DPD>(cell_at<D>(S, ps, l), sv);
-            store_codes<D>(wout + (int64_t)ps * (D / 4), l, w);
-            storeb(kout + ps, ks);           // sixteen lanes, one value
+            storef<DPD>(at(S, ps * (D * 4) + lane_c), sv);
+            store_codes<D>(at(wout, ps * kCodeBytes<D> + lane_w), w);
+            storeb(at(kout, ps + plane), ks);           // sixteen lanes, one value
             ps += rp.step;
             ++t;
         };
@@ -223,18 +227,19 @@ __device__ __forceinline__ void fwd_cols(const DsgmArgs& A, int b, int group, in
     const int l = lane & 15, W = A.W, H = A.H;
     const Off<WIDE> col = (Off<WIDE>)min(group * 4 + (lane >> 4), W - 1);
     const int64_t npix = (int64_t)A.B * H * W, img = (int64_t)b * H * W, path = LAST ? 2 : 0;
+    const Off<WIDE> col_c = col * (D * 4) + (Off<WIDE>)(l * DPD * 4), col_w = col * kCodeBytes<D> + code_byte<D>(l);
 
     float qc[NA][DPD], qs[NA][DPD], qy[NA][DPD], qp1[NA], qp2[NA];
     int si = 0;
     auto issue = [&](int u) __attribute__((always_inline)) {
         const int s = min(si++, H - 1);
         const int64_t r0 = img + (int64_t)(LAST ? H - 1 - s : s) * W;
-        loadf<DPD>(cell_at<D>(A.cost + r0 * D, col, l), qc[u]);
-        qp1[u] = loads(A.p1 + r0 + col);
-        qp2[u] = loads(A.p2 + r0 + col);
+        loadf<DPD>(at(A.cost + r0 * D, col_c), qc[u]);
+        qp1[u] = loads(at(A.p1 + r0, col * 4));
+        qp2[u] = loads(at(A.p2 + r0, col * 4));
         if constexpr (LAST) {
-            loadf<DPD>(cell_at<D>(A.S + r0 * D, col, l), qs[u]);
-            loadf<DPD>(cell_at<D>(A.vol + r0 * D, col, l), qy[u]);
+            loadf<DPD>(at(A.S + r0 * D, col_c), qs[u]);
+            loadf<DPD>(at(A.vol + r0 * D, col_c), qy[u]);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -247,19 +252,19 @@ __device__ __forceinline__ void fwd_cols(const DsgmArgs& A, int b, int group, in
         const float m = row_min(lane_min(L));
         const int ks = row_mini(lane_argmin<DPD>(L, m, l));
         const uint32_t w = fwd_step<DPD>(L, qc[u], m, s == 0 ? inf : qp1[u], s == 0 ? inf : qp2[u]);
-        store_codes<D>(A.wins + (path * npix + r0) * (D / 4) + (Off<WIDE>)(col * (D / 4)), l, w);
-        storeb(A.kstar + path * npix + r0 + col, ks);
+        store_codes<D>(at(A.wins + (path * npix + r0) * kCodeBytes<D>, col_w), w);
+        storeb(at(A.kstar + path * npix + r0, col), ks);
         if constexpr (LAST) {
             float sv[DPD], mn, z;
 #pragma unroll
             for (int k = 0; k < DPD; ++k) sv[k] = (qs[u][k] + qy[u][k]) + L[k];
-            storef<DPD>(cell_at<D>(A.S + r0 * D, col, l), sv);
+            storef<DPD>(at(A.S + r0 * D, col_c), sv);
             const float d = soft_argmin<DPD>(sv, l, A.inv_temperature, &mn, &z);
-            store1(A.disp + r0 + col, d);
-            store1(A.stats + 2 * r0 + 2 * col, mn);
-            store1(A.stats + 2 * r0 + 2 * col + 1, z);
+            store1(at(A.disp + r0, col * 4), d);
+            store1(at(A.stats + 2 * r0, col * 8), mn);
+            store1(at(A.stats + 2 * r0, col * 8 + 4), z);
         } else {
-            storef<DPD>(cell_at<D>(A.vol + r0 * D, col, l), L);
+            storef<DPD>(at(A.vol + r0 * D, col_c), L);
         }
         ++s;
     };
@@ -276,9 +281,10 @@ __device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int la
     const float *S = A.S + rp.q0 * D, *stats = A.stats + 2 * rp.q0;
     const float *disp = A.disp + rp.q0, *gdisp = A.grad_disp + rp.q0;
     float *dc = A.grad_cost + rp.q0 * D, *dp1 = A.grad_p1 + rp.q0, *dp2 = A.grad_p2 + rp.q0;
-    const int64_t line0 = (rp.second ? 3 : 1) * npix + rp.q0;
-    const uint8_t* win = A.wins + line0 * (D / 4);
-    const uint8_t* kin = A.kstar + line0;
+    const uint8_t* win = A.wins + (npix + rp.q0) * kCodeBytes<D>;   // of direction 1; 3 is two planes on
+    const uint8_t* kin = A.kstar + npix + rp.q0;
+    const Off<WIDE> plane = rp.second ? (Off<WIDE>)(2 * npix) : 0;
+    const Off<WIDE> lane_c = (Off<WIDE>)(l * DPD * 4), lane_w = plane * kCodeBytes<D> + (code_byte<D>(l) & ~3u);
 
     float qs[NA][DPD], qmn[NA], qz[NA], qg[NA], qd[NA], qo[NA][DPD], qo1[NA], qo2[NA];
     uint32_t qw[NA];
@@ -293,17 +299,17 @@ __device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int la
         Off<WIDE> pi = rp.pix(t0), ps = pi;
         int ti = t0;
         auto issue = [&](int u) __attribute__((always_inline)) {
-            loadf<DPD>(cell_at<D>(S, pi, l), qs[u]);
-            qmn[u] = loads(stats + 2 * pi);
-            qz[u] = loads(stats + 2 * pi + 1);
-            qg[u] = loads(gdisp + pi);
-            qd[u] = loads(disp + pi);
-            qw[u] = load_codes<D>(win + (int64_t)pi * (D / 4), l);
-            qk[u] = loadb(kin + pi);
+            loadf<DPD>(at(S, pi * (D * 4) + lane_c), qs[u]);
+            qmn[u] = loads(at(stats, pi * 8));
+            qz[u] = loads(at(stats, pi * 8 + 4));
+            qg[u] = loads(at(gdisp, pi * 4));
+            qd[u] = loads(at(disp, pi * 4));
+            qw[u] = load_codes(at(win, pi * kCodeBytes<D> + lane_w));
+            qk[u] = loadb(at(kin, pi + plane));
             if constexpr (PHASE == kPairAdd) {
-                loadf<DPD>(cell_at<D>(dc, pi, l), qo[u]);
-                qo1[u] = loads(dp1 + pi);
-                qo2[u] = loads(dp2 + pi);
+                loadf<DPD>(at(dc, pi * (D * 4) + lane_c), qo[u]);
+                qo1[u] = loads(at(dp1, pi * 4));
+                qo2[u] = loads(at(dp2, pi * 4));
             }
             pi = rp.move(pi, ++ti);
             __builtin_amdgcn_sched_barrier(0);
@@ -337,9 +343,9 @@ __device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int la
                 sums[1] += other_half(sums[1], lane);
                 sums[2] += other_half(sums[2], lane);
             }
-            storef<DPD>(cell_at<D>(dc, ps, l), v);
-            store1(dp1 + ps, sums[1]);
-            store1(dp2 + ps, sums[2]);
+            storef<DPD>(at(dc, ps * (D * 4) + lane_c), v);
+            store1(at(dp1, ps * 4), sums[1]);
+            store1(at(dp2, ps * 4), sums[2]);
             ps += rp.step;
             ++t;
         };
@@ -364,6 +370,7 @@ __device__ __forceinline__ void bwd_cols(const DsgmArgs& A, int b, int group, in
     const int l = lane & 15, W = A.W, H = A.H;
     const Off<WIDE> col = (Off<WIDE>)min(group * 4 + (lane >> 4), W - 1);
     const int64_t npix = (int64_t)A.B * H * W, img = (int64_t)b * H * W, path = LAST ? 2 : 0;
+    const Off<WIDE> col_c = col * (D * 4) + (Off<WIDE>)(l * DPD * 4), col_w = col * kCodeBytes<D> + (code_byte<D>(l) & ~3u);
 
     float qs[NA][DPD], qmn[NA], qz[NA], qg[NA], qd[NA], qo[NA][DPD], qo1[NA], qo2[NA], qy[NA][DPD], qy1[NA], qy2[NA];
     uint32_t qw[NA];
@@ -372,20 +379,20 @@ __device__ __forceinline__ void bwd_cols(const DsgmArgs& A, int b, int group, in
     auto issue = [&](int u) __attribute__((always_inline)) {
         const int s = min(si++, H - 1);
         const int64_t r0 = img + (int64_t)(LAST ? s : H - 1 - s) * W;
-        loadf<DPD>(cell_at<D>(A.S + r0 * D, col, l), qs[u]);
-        qmn[u] = loads(A.stats + 2 * r0 + 2 * col);
-        qz[u] = loads(A.stats + 2 * r0 + 2 * col + 1);
-        qg[u] = loads(A.grad_disp + r0 + col);
-        qd[u] = loads(A.disp + r0 + col);
-        qw[u] = load_codes<D>(A.wins + (path * npix + r0) * (D / 4) + (Off<WIDE>)(col * (D / 4)), l);
-        qk[u] = loadb(A.kstar + path * npix + r0 + col);
+        loadf<DPD>(at(A.S + r0 * D, col_c), qs[u]);
+        qmn[u] = loads(at(A.stats + 2 * r0, col * 8));
+        qz[u] = loads(at(A.stats + 2 * r0, col * 8 + 4));
+        qg[u] = loads(at(A.grad_disp + r0, col * 4));
+        qd[u] = loads(at(A.disp + r0, col * 4));
+        qw[u] = load_codes(at(A.wins + (path * npix + r0) * kCodeBytes<D>, col_w));
+        qk[u] = loadb(at(A.kstar + path * npix + r0, col));
         if constexpr (LAST) {
-            loadf<DPD>(cell_at<D>(A.grad_cost + r0 * D, col, l), qo[u]);
-            loadf<DPD>(cell_at<D>(A.vol + r0 * D, col, l), qy[u]);
-            qo1[u] = loads(A.grad_p1 + r0 + col);
-            qo2[u] = loads(A.grad_p2 + r0 + col);
-            qy1[u] = loads(A.vol_p1 + r0 + col);
-            qy2[u] = loads(A.vol_p2 + r0 + col);
+            loadf<DPD>(at(A.grad_cost + r0 * D, col_c), qo[u]);
+            loadf<DPD>(at(A.vol + r0 * D, col_c), qy[u]);
+            qo1[u] = loads(at(A.grad_p1 + r0, col * 4));
+            qo2[u] = loads(at(A.grad_p2 + r0, col * 4));
+            qy1[u] = loads(at(A.vol_p1 + r0, col * 4));
+            qy2[u] = loads(at(A.vol_p2 + r0, col * 4));
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -407,13 +414,13 @@ __device__ __forceinline__ void bwd_cols(const DsgmArgs& A, int b, int group, in
         if constexpr (LAST) {
 #pragma unroll
             for (int k = 0; k < DPD; ++k) G[k] = (qo[u][k] + qy[u][k]) + G[k];
-            storef<DPD>(cell_at<D>(A.grad_cost + r0 * D, col, l), G);
-            store1(A.grad_p1 + r0 + col, (qo1[u] + qy1[u]) + sums[1]);
-            store1(A.grad_p2 + r0 + col, (qo2[u] + qy2[u]) + sums[2]);
+            storef<DPD>(at(A.grad_cost + r0 * D, col_c), G);
+            store1(at(A.grad_p1 + r0, col * 4), (qo1[u] + qy1[u]) + sums[1]);
+            store1(at(A.grad_p2 + r0, col * 4), (qo2[u] + qy2[u]) + sums[2]);
         } else {
-            storef<DPD>(cell_at<D>(A.vol + r0 * D, col, l), G);
-            store1(A.vol_p1 + r0 + col, sums[1]);
-            store1(A.vol_p2 + r0 + col, sums[2]);
+            storef<DPD>(at(A.vol + r0 * D, col_c), G);
+            store1(at(A.vol_p1 + r0, col * 4), sums[1]);
+            store1(at(A.vol_p2 + r0, col * 4), sums[2]);
         }
         ++s;
     };
@@ -469,7 +476,8 @@ hipError_t launch_passes(const DsgmArgs& A, hipStream_t s) {
 
 template <bool BWD>
 hipError_t launch_by_d(const DsgmArgs& A, hipStream_t s) {
-    const bool wide = (int64_t)2 * A.W * A.D * 4 > (int64_t)1 << 31;
+    const int64_t rows = (int64_t)2 * A.W * A.D * 4, codes = ((int64_t)2 * A.B * A.H + 2) * A.W * (A.D / 4);
+    const bool wide = std::max(rows, codes) > (int64_t)1 << 31;
     switch (A.D) {
         case 64: return wide ? launch_passes<64, BWD, true>(A, s) : launch_passes<64, BWD, false>(A, s);
         case 128: return wide ? launch_passes<128, BWD, true>(A, s) : launch_passes<128, BWD, false>(A, s);
