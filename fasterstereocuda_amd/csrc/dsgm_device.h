@@ -240,7 +240,7 @@ __device__ __forceinline__ float bwd_flow(const float (&G)[DPD], uint32_t w, flo
     }
     *s12 = a12;
     *s3 = a3;
-    return rest;
+    return rest + (a3 - a3);   // a gradient that is no number reaches the argmin too
 }
 // the argmin's term, to disparity ks
 template <int DPD>
