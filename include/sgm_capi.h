@@ -150,12 +150,12 @@ void sgm_roi_from_disparity(const float* disp, int32_t width, int32_t height, sg
 /* Where the aggregation takes its matching cost (no reference counterpart;
  * the reference always stores the cost volume, cusgm_cc.cu:118-172):
  *   SGM_COST_ON_THE_FLY  recompute it from the census words inside the
- *                        aggregation wherever the plan allows (D <= 256, not
- *                        the 5x5 right view): no cost volume is built or read
+ *                        aggregation wherever the plan allows (D <= 256): no
+ *                        cost volume is built or read
  *   SGM_COST_STORED      always build and read the u8 cost volume
  *   SGM_COST_AUTO        on the fly when the plan also has enough scanlines
- *                        to fill the device (batches), stored otherwise
- *                        (single pairs finish sooner that way)
+ *                        to fill the device (batches) or 250M cells and more,
+ *                        stored otherwise (small pairs finish sooner that way)
  * Process-wide; read when a handle, batch or pyramid is created.  All give
  * byte-identical results. */
 #define SGM_COST_AUTO 0
@@ -170,9 +170,9 @@ int32_t sgm_get_cost_mode(void);
  *   SGM_WINDOW_U32    one per lane in 32-bit arithmetic (any P1, P2)
  *   SGM_WINDOW_PAIRS  two per lane as packed u16 (P1 <= 127, P2 <= 254)
  *   SGM_WINDOW_QUADS  four per lane as two packed u16 pairs (same range)
- *   SGM_WINDOW_AUTO   the packed form with the fewest instructions that
- *                     still gives the device a wave per SIMD, the 32-bit
- *                     form outside the packed range
+ *   SGM_WINDOW_AUTO   quads once they give the device two waves per SIMD (one
+ *                     at window 32), pairs below, the 32-bit form outside the
+ *                     packed range
  * A packed form asked for outside its range runs the 32-bit form.
  * Process-wide, read at every launch.  All give byte-identical results. */
 #define SGM_WINDOW_AUTO 0
