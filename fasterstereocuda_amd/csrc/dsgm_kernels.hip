@@ -39,13 +39,17 @@
 // both directions, or four columns), D/16 disparities per lane.  Lanes past
 // the image repeat its last line: same values, same addresses.
 //
+// Little work (pairs_ok) runs as one launch of all four directions, columns too
+// as pairs walked from both ends into the workspace volume, and a pass that
+// joins the sums: S = (L_1 + L_3) + (L_0 + L_2), and the gradients likewise.
+//
 // What bounds these passes: for one image or a few, the chain of a scanline's
 // steps, max(H, W) + H forward and again backward, each 130-300 instructions
 // of a wave that has its SIMD to itself; for many, the copy rate (93 bytes per
 // cell).  Walking a row's directions one after the other made the chain
-// 2 W + H: 2 images 321x119 D = 64 0.57 -> 0.27 ms forward + backward, one
-// image 1242x375 D = 128 3.24 -> 1.58, D = 256 6.04 -> 3.28 ms, 4 images
-// D = 64 3.13 -> 2.37 ms.
+// 2 W + H: forward + backward of one image 1242x375 D = 128 3.24 -> 1.54 ms, D =
+// 256 6.04 -> 3.27 ms, 4 images D = 64 3.13 -> 2.37 ms, 2 images 321x119 D = 64
+// 0.57 -> 0.27 and, in one launch, 0.20 ms.
 #include <algorithm>
 #include <type_traits>
 
@@ -92,32 +96,34 @@ __device__ __forceinline__ void storeb(uint8_t* p, int v) { *(__attribute__((add
 __device__ __forceinline__ int loadb(const uint8_t* p) { return *(const __attribute__((address_space(1))) uint8_t*)p; }
 __device__ __forceinline__ void store1(float* p, float v) { *(g_f*)p = v; }
 
-// Two rows of an image, walked from both ends at once: lanes 0-31 left->right
-// and lanes 32-63 right->left (in the backward, each reversed: lanes 0-31 from
-// the right).  At step t every lane is t pixels into its direction's walk.
-template <bool WIDE>
-struct RowPair {
-    int W, n1, n2;             // steps that reach a pixel first; first step that reaches one second
-    bool second;               // this lane walks right->left
-    Off<WIDE> pix0, step;      // pixel of step 0 from the pair's first, its move (all ones: -1)
+// Two scanlines of an image, walked from both ends at once: lanes 0-31 in the
+// first direction (left->right, or top->bottom of columns), lanes 32-63 in the
+// second (in the backward, each reversed).  At step t every lane is t pixels
+// into its direction's walk.
+template <bool VERT, bool WIDE>
+struct LinePair {
+    int n, n1, n2;             // steps; those that reach a pixel first; first step that reaches one second
+    bool second;               // this lane walks the second direction
+    Off<WIDE> pix0, step;      // pixel of step 0 from q0, and its move
     int64_t q0;                // the pair's first pixel in the batch
-    __device__ RowPair(const DsgmArgs& A, int b, int g, int lane, bool reversed) {
-        W = A.W;
-        n1 = W / 2;
-        n2 = (W + 1) / 2;
-        const int sub = lane >> 4;
+    __device__ LinePair(const DsgmArgs& A, int b, int g, int lane, bool reversed) {
+        n = VERT ? A.H : A.W;
+        n1 = n / 2;
+        n2 = (n + 1) / 2;
+        const int sub = lane >> 4, lines = VERT ? A.W : A.H;
         second = sub >= 2;
-        const bool from_right = second != reversed;
-        const int row = min(2 * g + (sub & 1), A.H - 1) - 2 * g;
-        pix0 = (Off<WIDE>)row * (Off<WIDE>)W + (Off<WIDE>)(from_right ? W - 1 : 0);
-        step = from_right ? (Off<WIDE>)-1 : (Off<WIDE>)1;
-        q0 = ((int64_t)b * A.H + 2 * g) * W;
+        const bool from_end = second != reversed;
+        const int line = min(2 * g + (sub & 1), lines - 1) - 2 * g;
+        const Off<WIDE> along = VERT ? (Off<WIDE>)A.W : 1, across = VERT ? 1 : (Off<WIDE>)A.W;
+        pix0 = (Off<WIDE>)line * across + (Off<WIDE>)(from_end ? n - 1 : 0) * along;
+        step = from_end ? 0 - along : along;
+        q0 = (int64_t)b * A.H * A.W + (int64_t)2 * g * (VERT ? 1 : A.W);
     }
     __device__ Off<WIDE> pix(int t) const { return pix0 + step * (Off<WIDE>)t; }
     // a walk's next pixel, staying on the last one (t: the step moved to)
-    __device__ Off<WIDE> move(Off<WIDE> p, int t) const { return t < W ? p + step : p; }
+    __device__ Off<WIDE> move(Off<WIDE> p, int t) const { return t < n ? p + step : p; }
 };
-// the other direction's value of the same row
+// the other direction's value of the same line
 __device__ __forceinline__ float other_half(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, v)));
 }
@@ -152,18 +158,19 @@ __device__ __forceinline__ void run_steps(int n, Issue issue, Step step) {
 enum PairPhase { kPairStore = 0, kPairMiddle = 1, kPairAdd = 2 };
 
 // ------------------------------------------------------------- forward ---
-template <int D, bool WIDE>
-__device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int lane) {
+template <int D, bool VERT, bool WIDE>
+__device__ __forceinline__ void fwd_pair(const DsgmArgs& A, int b, int g, int lane) {
     constexpr int DPD = D / 16, NA = kAhead<D, false>;
     const float inf = __builtin_inff();
     const int l = lane & 15;
-    const RowPair<WIDE> rp(A, b, g, lane, false);
+    const LinePair<VERT, WIDE> rp(A, b, g, lane, false);
     const int64_t npix = (int64_t)A.B * A.H * A.W;
     const float* cost = A.cost + rp.q0 * D;
-    float* S = A.S + rp.q0 * D;
+    float* S = (VERT ? A.vol : A.S) + rp.q0 * D;   // where the pair's sum is built
     const float *p1 = A.p1 + rp.q0, *p2 = A.p2 + rp.q0;
-    uint8_t* wout = A.wins + (npix + rp.q0) * kCodeBytes<D>;   // of direction 1; 3 is two planes on
-    uint8_t* kout = A.kstar + npix + rp.q0;
+    constexpr int P = VERT ? 0 : 1;                // the first direction; the second is two planes on
+    uint8_t* wout = A.wins + (P * npix + rp.q0) * kCodeBytes<D>;
+    uint8_t* kout = A.kstar + P * npix + rp.q0;
     const Off<WIDE> plane = rp.second ? (Off<WIDE>)(2 * npix) : 0;
     const Off<WIDE> lane_c = (Off<WIDE>)(l * DPD * 4), lane_w = plane * kCodeBytes<D> + code_byte<D>(l);
 
@@ -215,7 +222,7 @@ __device__ __forceinline__ void fwd_rows(const DsgmArgs& A, int b, int g, int la
     walk(std::integral_constant<int, kPairMiddle>{}, rp.n1, rp.n2);
     // the other lanes' stores of the pixels that this phase loads
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.W);
+    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.n);
 }
 
 // Four columns, top->bottom into the workspace volume or (LAST) bottom->top
@@ -272,17 +279,19 @@ __device__ __forceinline__ void fwd_cols(const DsgmArgs& A, int b, int group, in
 }
 
 // ------------------------------------------------------------ backward ---
-template <int D, bool WIDE>
-__device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int lane) {
+template <int D, bool VERT, bool WIDE>
+__device__ __forceinline__ void bwd_pair(const DsgmArgs& A, int b, int g, int lane) {
     constexpr int DPD = D / 16, NA = kAhead<D, false>;
     const int l = lane & 15;
-    const RowPair<WIDE> rp(A, b, g, lane, true);
+    const LinePair<VERT, WIDE> rp(A, b, g, lane, true);
     const int64_t npix = (int64_t)A.B * A.H * A.W;
     const float *S = A.S + rp.q0 * D, *stats = A.stats + 2 * rp.q0;
     const float *disp = A.disp + rp.q0, *gdisp = A.grad_disp + rp.q0;
-    float *dc = A.grad_cost + rp.q0 * D, *dp1 = A.grad_p1 + rp.q0, *dp2 = A.grad_p2 + rp.q0;
-    const uint8_t* win = A.wins + (npix + rp.q0) * kCodeBytes<D>;   // of direction 1; 3 is two planes on
-    const uint8_t* kin = A.kstar + npix + rp.q0;
+    float* dc = (VERT ? A.vol : A.grad_cost) + rp.q0 * D;
+    float *dp1 = (VERT ? A.vol_p1 : A.grad_p1) + rp.q0, *dp2 = (VERT ? A.vol_p2 : A.grad_p2) + rp.q0;
+    constexpr int P = VERT ? 0 : 1;                // the first direction; the second is two planes on
+    const uint8_t* win = A.wins + (P * npix + rp.q0) * kCodeBytes<D>;
+    const uint8_t* kin = A.kstar + P * npix + rp.q0;
     const Off<WIDE> plane = rp.second ? (Off<WIDE>)(2 * npix) : 0;
     const Off<WIDE> lane_c = (Off<WIDE>)(l * DPD * 4), lane_w = plane * kCodeBytes<D> + (code_byte<D>(l) & ~3u);
 
@@ -322,7 +331,7 @@ __device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int la
             for (int k = 0; k < DPD; ++k) G[k] += F[k];
             // the direction's first pixel (the walk's last) hands on
             // nothing and has no penalty gradient: code 0 everywhere
-            const uint32_t w = t == rp.W - 1 ? 0u : shift_codes<D>(qw[u], l);
+            const uint32_t w = t == rp.n - 1 ? 0u : shift_codes<D>(qw[u], l);
             float sums[3];
             sums[0] = bwd_flow<DPD>(G, w, F, &s12, &s3);
             sums[1] = s12;
@@ -359,7 +368,7 @@ __device__ __forceinline__ void bwd_rows(const DsgmArgs& A, int b, int g, int la
     walk(std::integral_constant<int, kPairStore>{}, 0, rp.n1);
     walk(std::integral_constant<int, kPairMiddle>{}, rp.n1, rp.n2);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.W);
+    walk(std::integral_constant<int, kPairAdd>{}, rp.n2, rp.n);
 }
 
 // Four columns: top->bottom reversed into the workspace, or (LAST)
@@ -443,8 +452,8 @@ __global__ __launch_bounds__(64) void dsgm_first_kernel(DsgmArgs A, int row_bloc
     if ((int)blockIdx.x < row_blocks) {
         const int nh = (A.H + 1) / 2, item = blockIdx.x;
         const int b = item / nh;
-        if constexpr (BWD) bwd_rows<D, WIDE>(A, b, item - b * nh, lane);
-        else fwd_rows<D, WIDE>(A, b, item - b * nh, lane);
+        if constexpr (BWD) bwd_pair<D, false, WIDE>(A, b, item - b * nh, lane);
+        else fwd_pair<D, false, WIDE>(A, b, item - b * nh, lane);
     } else {
         const int nv = (A.W + 3) / 4;
         const int item = dev::xcd_item((int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks);
@@ -463,6 +472,63 @@ __global__ __launch_bounds__(64) void dsgm_last_kernel(DsgmArgs A) {
     else fwd_cols<D, true, WIDE>(A, b, item - b * nv, threadIdx.x);
 }
 
+// The form for little work: all four directions in one launch, rows and columns
+// both as pairs walked from both ends, then one pass that joins the two sums,
+// S = (L_1 + L_3) + (L_0 + L_2) (and dC, dP1, dP2 likewise).
+template <int D, bool BWD>
+__global__ __launch_bounds__(64) void dsgm_pairs_kernel(DsgmArgs A, int row_blocks) {
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x < row_blocks) {
+        const int nh = (A.H + 1) / 2, item = blockIdx.x, b = item / nh;
+        if constexpr (BWD) bwd_pair<D, false, false>(A, b, item - b * nh, lane);
+        else fwd_pair<D, false, false>(A, b, item - b * nh, lane);
+    } else {
+        const int nv = (A.W + 1) / 2;
+        const int item = dev::xcd_item((int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks), b = item / nv;
+        if constexpr (BWD) bwd_pair<D, true, false>(A, b, item - b * nv, lane);
+        else fwd_pair<D, true, false>(A, b, item - b * nv, lane);
+    }
+}
+template <int D, bool BWD>
+__global__ __launch_bounds__(256) void dsgm_join_kernel(DsgmArgs A, int64_t npix) {
+    constexpr int DPD = D / 16;
+    const int l = threadIdx.x & 15;
+    const int64_t q = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (q >= npix) return;                       // whole 16-lane rows
+    float* out = (BWD ? A.grad_cost : A.S) + q * D + l * DPD;
+    float x[DPD], y[DPD];
+    loadf<DPD>(out, x);
+    loadf<DPD>(A.vol + q * D + l * DPD, y);
+#pragma unroll
+    for (int k = 0; k < DPD; ++k) x[k] += y[k];
+    storef<DPD>(out, x);
+    if constexpr (BWD) {
+        if (l == 0) {
+            A.grad_p1[q] += A.vol_p1[q];
+            A.grad_p2[q] += A.vol_p2[q];
+        }
+    } else {
+        float mn, z;
+        const float d = soft_argmin<DPD>(x, l, A.inv_temperature, &mn, &z);
+        if (l == 0) {
+            A.disp[q] = d;
+            A.stats[2 * q] = mn;
+            A.stats[2 * q + 1] = z;
+        }
+    }
+}
+
+template <int D, bool BWD>
+hipError_t launch_pairs(const DsgmArgs& A, hipStream_t s) {
+    const unsigned rows = (unsigned)A.B * ((A.H + 1) / 2), cols = (unsigned)A.B * ((A.W + 1) / 2);
+    const int64_t npix = (int64_t)A.B * A.H * A.W;
+    hipLaunchKernelGGL((dsgm_pairs_kernel<D, BWD>), dim3(rows + cols), dim3(64), 0, s, A, (int)rows);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((dsgm_join_kernel<D, BWD>), dim3((unsigned)((npix + 15) / 16)), dim3(256), 0, s, A, npix);
+    return hipGetLastError();
+}
+
 template <int D, bool BWD, bool WIDE>
 hipError_t launch_passes(const DsgmArgs& A, hipStream_t s) {
     const unsigned rows = (unsigned)A.B * ((A.H + 1) / 2);
@@ -474,10 +540,36 @@ hipError_t launch_passes(const DsgmArgs& A, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Where all four directions in one launch are sooner done: the chain is
+// max(H, W) steps and a pass over the volumes instead of max(H, W) + H steps, but
+// it moves 12 more bytes per cell each way, and past about one wave per SIMD the
+// waves share the SIMDs anyway.  Forward + backward, us, separate -> pairs:
+//   D = 64: 2 images 321x119 (440 waves) 274 -> 198, 2 640x200 (840) 512 -> 412,
+//   4 321x119 (880) 280 -> 222, 1 1242x375 (808, 30M cells) 1010 -> 908, 8 321x119
+//   (1760) 320 -> 360
+//   D = 128: 1 100x300 (200) 626 -> 269, 3 280x134 (621) 406 -> 302, 4 300x100
+//   (800) 387 -> 337, 2 800x100 (900) 797 -> 777, 3 500x200 (1050) 827 -> 938, 1
+//   1242x375 (808, 60M cells) 1544 -> 1674
+//   D = 256: 1 300x200 (250) 845 -> 509, 2 280x134 (414) 693 -> 509, 3 280x134
+//   (621) 773 -> 819
+// Below the limit offsets fit 32 bits.
+bool pairs_ok(const DsgmArgs& A) {
+    const int64_t waves = (int64_t)A.B * ((A.H + 1) / 2 + (A.W + 1) / 2), cells = (int64_t)A.B * A.H * A.W * A.D;
+    return waves <= (A.D == 256 ? 500 : 950) && cells <= 30000000;
+}
+
 template <bool BWD>
 hipError_t launch_by_d(const DsgmArgs& A, hipStream_t s) {
     const int64_t rows = (int64_t)2 * A.W * A.D * 4, codes = ((int64_t)2 * A.B * A.H + 2) * A.W * (A.D / 4);
     const bool wide = std::max(rows, codes) > (int64_t)1 << 31;
+    if (pairs_ok(A)) {
+        switch (A.D) {
+            case 64: return launch_pairs<64, BWD>(A, s);
+            case 128: return launch_pairs<128, BWD>(A, s);
+            case 256: return launch_pairs<256, BWD>(A, s);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (A.D) {
         case 64: return wide ? launch_passes<64, BWD, true>(A, s) : launch_passes<64, BWD, false>(A, s);
         case 128: return wide ? launch_passes<128, BWD, true>(A, s) : launch_passes<128, BWD, false>(A, s);

@@ -67,7 +67,11 @@ def test_row_pairs_match_fp64(cuda, B, H, W, D):
 # state handed between bands), lines shorter than the skew of a band's rows
 @pytest.mark.parametrize("B,H,W,D", [(141, 13, 70, 128), (188, 10, 33, 64), (560, 3, 9, 64),
                                      (140, 16, 1, 128), (280, 7, 2, 64), (187, 12, 130, 128),
-                                     (98, 13, 20, 256)])
+                                     (98, 13, 20, 256)]
+                         # too many waves for one launch of all directions, too few
+                         # bands for the above: one pass per direction and set
+                         + [(12, 97, 71, 64), (12, 83, 90, 128), (200, 7, 5, 64),
+                            (180, 5, 9, 128), (90, 3, 7, 256), (240, 1, 8, 64), (120, 17, 1, 128)])
 def test_many_images_match_fp64(cuda, B, H, W, D):
     print(f"[dsgm] B{B} H{H} W{W} D{D}", flush=True)
     cost, p1, p2, gt = _inputs(B, H, W, D, seed=B + H + W + D)
