@@ -85,27 +85,34 @@ int waves_per_group(int n, int limit) {
     return 2 * n > simds && 4 * n <= limit * simds ? 4 : 1;
 }
 
+// 0: some matched image is over 2.5 times as wide as high, 1: over 1.5 times, 2:
+// not over 1.2 times as high as wide, 3: none of these (all tall).
+int plan_shape(const std::vector<SgmJob>& jobs, int n) {
+    int shape = n > 0 ? 3 : 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t w = jobs[i].W - jobs[i].roi_x, h = jobs[i].H;
+        shape = std::min(shape, 2 * w > 5 * h ? 0 : 2 * w > 3 * h ? 1 : 5 * h <= 6 * w ? 2 : 3);
+    }
+    return shape;
+}
+
 // Stored-cost plans: the four directions and then the WTA, or bottom->top
 // fused with the WTA after the other three.  The fused bottom->top walk is
 // latency-bound on a small plan, so it is better run beside the horizontal
 // ones (and the WTA left to its own memory-bound launch) while the four
 // directions have at most 2.5 waves per SIMD and the extra volume's traffic is
-// small: up to 200M cells, or 100M where the rows are much longer than the
-// columns and the fused walk is short (both views, separate / fused:
-// 1242x375 D = 64, 60M: 185 / 211 us; 640x480 D = 128, 79M: 240 / 268;
-// 1242x375 D = 128, 119M: 416 / 336; 1200x852, 131M: 405 / 429; 1280x720
-// D = 128, 236M: 643 / 626).
+// small: the more so, the longer the columns are beside the rows (both views,
+// separate / fused, us): wide 1242x375 D = 64, 60M 185 / 211, D = 128, 119M 416 /
+// 336; 640x480 D = 128, 79M 240 / 268, 1280x720 D = 128, 236M 643 / 626; square
+// 1200x852, 131M 405 / 429, 700x700 D = 256, 251M 700 / 762, 1200x1000 D = 128,
+// 307M 798 / 784; tall 500x1000 D = 256, 256M 722 / 917, 800x2500 D = 128, 512M
+// 1429 / 1573, 1200x1800 D = 128, 553M 1464 / 1441.
 bool separate_wta(const StagePlan& p) {
+    constexpr int64_t kCells[4] = {100000000, 200000000, 260000000, 540000000};
     const int f = g_wta_form.load();
     if (f == SGM_WTA_FUSED) return false;
     if (f == SGM_WTA_SEPARATE) return true;
-    return 4 * p.n_agg <= 5 * wide_min_groups() && p.cells <= (p.squarish ? 200000000 : 100000000);
-}
-
-bool squarish_jobs(const std::vector<SgmJob>& jobs, int n) {
-    for (int i = 0; i < n; ++i)
-        if (2 * (int64_t)(jobs[i].W - jobs[i].roi_x) > 5 * (int64_t)jobs[i].H) return false;
-    return n > 0;
+    return 4 * p.n_agg <= 5 * wide_min_groups() && p.cells <= kCells[p.shape];
 }
 
 bool choose_wide(bool eligible, int n_wh) {
@@ -115,16 +122,20 @@ bool choose_wide(bool eligible, int n_wh) {
 }
 
 // The 4-line on-the-fly form moves 6 bytes per cell where the stored cost
-// takes 11, but issues about 1.6 times the instructions per step: it wins once
-// memory, not the scanlines' serial steps, bounds the stored form (both views,
-// stored / on the fly: 1280x720 D = 128, 236M cells: 626 / 669 us; 1117x573
-// D = 256, 328M: 880 / 821; 1920x1080 D = 128, 531M: 1290 / 1100; 2400x1704
-// D = 256, 2.1G: 5.5 / 4.2 ms).
-constexpr int64_t kMidCells = 250000000;
-bool choose_mid(bool eligible, int n_wh, int64_t cells) {
+// takes 11, but issues about 1.6 times the instructions per step, and its
+// bottom->top walk always follows the others: it wins once memory, not the
+// scanlines' serial steps, bounds the stored form, the later the longer the
+// columns are (both views, stored / on the fly, us): wide 1280x720 D = 128, 236M
+// 626 / 669, 1000x500 D = 256, 256M 666 / 597, 1117x573 D = 256, 328M 880 / 821,
+// 1920x1080 D = 128, 531M 1290 / 1100; square 700x700 D = 256, 251M 700 / 854,
+// 1200x1000 D = 128, 307M 784 / 847, 1400x1100, 394M 996 / 988, 900x900 D = 256,
+// 415M 1154 / 1115, 1700x1700 D = 128, 740M 1758 / 1685; tall 500x1000 D = 256, 256M
+// 722 / 1081, 800x2500 D = 128, 512M 1429 / 1934, 1400x2200 D = 128, 788M 2002 / 2075.
+bool choose_mid(bool eligible, int n_wh, int64_t cells, int shape) {
+    constexpr int64_t kCells[4] = {250000000, 250000000, 400000000, 800000000};
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED || n_wh >= wide_min_groups()) return false;
-    return mode == SGM_COST_ON_THE_FLY || cells >= kMidCells;
+    return mode == SGM_COST_ON_THE_FLY || cells >= kCells[shape];
 }
 }  // namespace fsgm
 
@@ -255,12 +266,12 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmP
     plan->n_m3 = m3[nj];
     plan->n_mf = mf[nj];
     plan->wide = choose_wide(wide, w3[nj]);
-    plan->mid = choose_mid(mid, w3[nj], cells);
+    plan->shape = plan_shape(jobs, nj);
+    plan->mid = choose_mid(mid, w3[nj], cells, plan->shape);
     plan->cells = cells;
     plan->quirk = quirk;
     plan->big = big;
     plan->fast = !big;
-    plan->squarish = squarish_jobs(jobs, nj);
     plan->n_post = op[np];
     plan->dmax = dmax;
     plan->dmin = dmin;
@@ -295,9 +306,9 @@ void fsgm::restrict_matching(StagePlan* P, const std::vector<SgmJob>& jobs, int 
         P->n_dw += dw_items(jobs[i]);
     }
     P->wide = choose_wide(wide, P->n_wh);
-    P->mid = choose_mid(mid, P->n_wh, cells);
+    P->shape = plan_shape(jobs, n);
+    P->mid = choose_mid(mid, P->n_wh, cells, P->shape);
     P->cells = cells;
-    P->squarish = squarish_jobs(jobs, n);
 }
 
 // census, cost, three directions, bottom->top + WTA (or the four directions,

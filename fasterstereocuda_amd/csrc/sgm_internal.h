@@ -177,7 +177,7 @@ struct StagePlan {
     bool quirk = false;           // some matched job is a 5x5 right view
     bool big = false;             // some job's penalties need integer minima
     bool fast = false;            // not big, and every cost is a census distance (at most 64)
-    bool squarish = false;        // every matched job has W - roi_x <= 2.5 H
+    int shape = 0;                // how wide or tall the matched images are (plan_shape)
     IoBind io{};                  // host-side: bound caller buffers, if any
 };
 
@@ -237,9 +237,10 @@ hipError_t wide_occupancy(const StagePlan& p, int* per_cu);
 // (`eligible`) and that has n_wh horizontal scanline groups.
 int cost_mode();
 // choose_mid: whether an unscheduled run of it takes the 4-line form
-// (`eligible` by mid_ok; cells: matched pixels x D over the views).
+// (`eligible` by mid_ok; cells: matched pixels x D over the views; shape by
+// plan_shape).
 bool choose_wide(bool eligible, int n_wh);
-bool choose_mid(bool eligible, int n_wh, int64_t cells);
+bool choose_mid(bool eligible, int n_wh, int64_t cells, int shape);
 int wide_min_groups();
 hipError_t launch_wta(const StagePlan& p, hipStream_t s);
 hipError_t launch_post(const StagePlan& p, hipStream_t s);
