@@ -86,14 +86,19 @@ int waves_per_group(int n, int limit) {
 }
 
 // 0: some matched image is over 2.5 times as wide as high, 1: over 1.5 times, 2:
-// not over 1.2 times as high as wide, 3: none of these (all tall).
+// not over 1.2 times as high as wide, 3: none of these (all tall).  4: images of
+// several sizes, one pair of which has over half the cells; shape as for 0.
 int plan_shape(const std::vector<SgmJob>& jobs, int n) {
     int shape = n > 0 ? 3 : 0;
+    int64_t least = INT64_MAX, most = 0, total = 0;
     for (int i = 0; i < n; ++i) {
-        const int64_t w = jobs[i].W - jobs[i].roi_x, h = jobs[i].H;
+        const int64_t w = jobs[i].W - jobs[i].roi_x, h = jobs[i].H, cells = w * h * jobs[i].D;
+        least = std::min(least, cells);
+        most = std::max(most, cells);
+        total += cells;
         shape = std::min(shape, 2 * w > 5 * h ? 0 : 2 * w > 3 * h ? 1 : 5 * h <= 6 * w ? 2 : 3);
     }
-    return shape;
+    return n > 2 && least < most && 4 * most > total ? 4 : shape;   // two views a pair
 }
 
 // Stored-cost plans: the four directions and then the WTA, or bottom->top
@@ -108,7 +113,7 @@ int plan_shape(const std::vector<SgmJob>& jobs, int n) {
 // 307M 798 / 784; tall 500x1000 D = 256, 256M 722 / 917, 800x2500 D = 128, 512M
 // 1429 / 1573, 1200x1800 D = 128, 553M 1464 / 1441.
 bool separate_wta(const StagePlan& p) {
-    constexpr int64_t kCells[4] = {100000000, 200000000, 260000000, 540000000};
+    constexpr int64_t kCells[5] = {100000000, 200000000, 260000000, 540000000, 100000000};
     const int f = g_wta_form.load();
     if (f == SGM_WTA_FUSED) return false;
     if (f == SGM_WTA_SEPARATE) return true;
@@ -131,8 +136,12 @@ bool choose_wide(bool eligible, int n_wh) {
 // 1200x1000 D = 128, 307M 784 / 847, 1400x1100, 394M 996 / 988, 900x900 D = 256,
 // 415M 1154 / 1115, 1700x1700 D = 128, 740M 1758 / 1685; tall 500x1000 D = 256, 256M
 // 722 / 1081, 800x2500 D = 128, 512M 1429 / 1934, 1400x2200 D = 128, 788M 2002 / 2075.
+// A mixed plan whose largest pair has over half the cells stays with the stored
+// cost: that pair's steps outlast the rest, and the kernel for several D is
+// slower than the one for its own (6 pairs of 891M cells, 531M of them one
+// 1920x1080 D = 128: 2346 / 2694; 7 of 897M, 265M in one: 2375 / 2218).
 bool choose_mid(bool eligible, int n_wh, int64_t cells, int shape) {
-    constexpr int64_t kCells[4] = {250000000, 250000000, 400000000, 800000000};
+    constexpr int64_t kCells[5] = {250000000, 250000000, 400000000, 800000000, INT64_MAX};
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED || n_wh >= wide_min_groups()) return false;
     return mode == SGM_COST_ON_THE_FLY || cells >= kCells[shape];

@@ -154,8 +154,9 @@ void sgm_roi_from_disparity(const float* disp, int32_t width, int32_t height, sg
  *                        cost volume is built or read
  *   SGM_COST_STORED      always build and read the u8 cost volume
  *   SGM_COST_AUTO        on the fly when the plan also has enough scanlines
- *                        to fill the device (batches) or 250M cells and more,
- *                        stored otherwise (small pairs finish sooner that way)
+ *                        to fill the device (batches) or 250M cells and more
+ *                        (tall images more), stored otherwise (small pairs
+ *                        finish sooner that way)
  * Process-wide; read when a handle, batch or pyramid is created.  All give
  * byte-identical results. */
 #define SGM_COST_AUTO 0
