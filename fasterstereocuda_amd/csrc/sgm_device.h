@@ -18,10 +18,16 @@ __device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
     return as_u(__builtin_elementwise_min(as_v(a), as_v(b)));
 }
 
-// min of three packed pairs.  Costs and penalties below 2^15 - 2^10 are
-// positive finite f16 bit patterns, which order as the integers they are, so
-// one v_pk_minimum3_f16 stands for two v_pk_min_u16 (one 4-cycle issue
-// instead of two); BIG keeps the integer form (see big_penalties).
+// min of three packed pairs.  Values below kF16Inf are positive finite f16 bit
+// patterns, which order as the integers they are, so one v_pk_minimum3_f16
+// stands for two v_pk_min_u16 (one 4-cycle issue instead of two).  From there
+// on they are infinity and NaN, and a NaN wins over every value: BIG keeps the
+// integer form (see big_penalties and wta_key_max).
+constexpr uint32_t kF16Inf = 0x7C00u;
+// The largest argmin key S * DPL + j of a lane of DPL disparities: S is at most
+// 4 x 255.  16320 + 15 for DPL = 16, but 32671 for DPL = 32, past kF16Inf from
+// S = 992 on.
+__host__ __device__ constexpr uint32_t wta_key_max(int dpl) { return 4u * 255u * (uint32_t)dpl + (uint32_t)dpl - 1u; }
 template <bool BIG>
 __device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
     if constexpr (BIG) {

@@ -600,7 +600,9 @@ __device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int q, 
     for (int r = 0; r < 4; ++r) load_words<NW>(J.path[r] + off, w[r]);
     // pair 2k = (S(4k), S(4k + 2)), pair 2k + 1 = (S(4k + 1), S(4k + 3)): at
     // most 4 x 255 per half, so the sums are 32-bit and the keys S * DPL + j
-    // (j the disparity inside the lane) fit the halves, below 2^15
+    // (j the disparity inside the lane) fit the halves.  Their minimum is one of
+    // f16 patterns up to D = 256 and of integers at D = 512, whose keys pass them
+    // (450x375 D = 512, both views, with either minimum 653 us)
     constexpr int kLog = __builtin_ctz(DPL);
     uint32_t S[NP], keys[NP];
 #pragma unroll
@@ -610,7 +612,8 @@ __device__ __forceinline__ void wta_pixel(const SgmJob& J, int x, int y, int q, 
         S[k] = half(w[0][i]) + half(w[1][i]) + half(w[2][i]) + half(w[3][i]);
         keys[k] = (S[k] << kLog) | (uint32_t)((4 * i + o) | ((4 * i + o + 2) << 16));
     }
-    const uint32_t t = pk_min_all<false>(keys);
+    static_assert(wta_key_max(DPL) <= 0xFFFFu, "a key fits its half");
+    const uint32_t t = pk_min_all<(wta_key_max(DPL) >= kF16Inf)>(keys);
     const uint32_t key = min(t & 0xFFFFu, t >> 16);
     uint32_t best = ((key >> kLog) << 16) | (uint32_t)(DPL * q + (int)(key & (DPL - 1)));
     best = line_min<LPP>(best);

@@ -344,6 +344,7 @@ __device__ __forceinline__ void mid_vertical(const SgmJob& J, const MidColumns& 
     uint32_t wb[BLK], w1[BLK], w3[BLK];
     auto wta_step = [&](const uint32_t (&o3)[3][NW], int b) __attribute__((always_inline)) {
         constexpr int kLog = __builtin_ctz(DPL);
+        static_assert(wta_key_max(DPL) < kF16Inf, "argmin keys S * DPL + j are finite f16 patterns");
         uint32_t S[NP], keys[NP];
 #pragma unroll
         for (int k = 0; k < NP; ++k) {

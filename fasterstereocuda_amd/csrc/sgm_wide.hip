@@ -306,10 +306,10 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
             S[k] = a0 + a1 + a2 + (s.L[k] & 0x00FF00FFu);   // each half <= 1020
         }
         // argmin with the smallest d: inside the lane on u16 keys S * DPL + j
-        // (S <= 4 * 255 < 2^10 and j < DPL <= 16: the keys are below 2^14, so
-        // one 32-bit v_lshl_or_b32 per pair shifts both halves without a carry
-        // between them), then across the line's lanes on (S << 16) | d
-        static_assert(DPL <= 16 && (DPL & (DPL - 1)) == 0, "u16 argmin keys S * DPL + j");
+        // (one 32-bit v_lshl_or_b32 per pair shifts both halves without a carry
+        // between them, and the keys are finite f16 patterns), then across the
+        // line's lanes on (S << 16) | d
+        static_assert(wta_key_max(DPL) < kF16Inf && (DPL & (DPL - 1)) == 0, "argmin keys S * DPL + j");
         constexpr int kLog = __builtin_ctz(DPL);
         uint32_t keys[NP];
 #pragma unroll

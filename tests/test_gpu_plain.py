@@ -170,6 +170,55 @@ def test_stereocuda_match_matches_oracle(cuda, case, lr, median):
     st.Release()
 
 
+# Sums of the four directions up to their largest, 4 x 255: the WTA's argmin
+# keys carry the sum above the lane's disparity index and must order as integers
+@pytest.mark.parametrize("D", [64, 128, 256, 512])
+@pytest.mark.parametrize("low", [0, 240], ids=["any", "high"])
+def test_wta_sums_up_to_1020(cuda, D, low):
+    H, W = 17, 45
+    print(f"[wta sums] D{D} bytes {low}..255", flush=True)
+    rng = np.random.default_rng(D + low)
+    paths = [rng.integers(low, 256, (H, W, D), dtype=np.uint8) for _ in range(4)]
+    for p in paths:
+        p[::3] = 255          # whole rows of equal, largest sums, and one smaller sum
+        p[3::6, :, D // 3] = 251
+    got = stages.wta([torch.from_numpy(p).to(cuda) for p in paths], 0, UNIQ)
+    _eq_float(got.cpu().numpy(), oracle.wta(paths, 0, 0, UNIQ), "wta")
+    loose = stages.wta([torch.from_numpy(p).to(cuda) for p in paths], 0, 1.0)
+    _eq_float(loose.cpu().numpy(), oracle.wta(paths, 0, 0, 1.0), "wta without the uniqueness rule")
+
+
+# penalties that take the sums of real costs past 992, at every D
+HIGH_SUMS = [(600, 21, 512, 0, 1, 10, 190), (600, 21, 512, 0, 1, 10, 200), (530, 24, 512, 3, 0, 10, 220),
+             (300, 26, 256, 0, 1, 10, 190), (140, 30, 64, 0, 1, 10, 200), (190, 30, 128, 0, 1, 10, 200)]
+
+
+@pytest.mark.parametrize("case", HIGH_SUMS, ids=_ids)
+def test_stages_match_oracle_at_high_sums(cuda, case):
+    test_stages_match_oracle(cuda, case)
+
+
+@pytest.mark.parametrize("mode,form", [(0, stages.WTA_AUTO), (1, stages.WTA_FUSED), (1, stages.WTA_SEPARATE),
+                                       (2, stages.WTA_AUTO)])
+@pytest.mark.parametrize("case", HIGH_SUMS, ids=_ids)
+def test_match_at_high_sums(cuda, cost_mode, wta_form, mode, form, case):
+    W, H, D, min_d, cs, p1, p2 = case
+    print(f"[high sums] {case} mode={mode} form={form}", flush=True)
+    cost_mode(mode)
+    wta_form(form)
+    left, right = _pair(W, H, D, seed=7)
+    exp_l, exp_r = oracle.match(left, right, min_d, D, cs_type=cs, p1=p1, p2=p2, uniqueness=UNIQ,
+                                lr_threshold=LR_THR, do_median=False)
+    st = StereoCuda()
+    opt = CuSGMOption.benchmark(cs_type=cs, p1=p1, p2_init=p2, do_median_filter=False)
+    assert st.Init(W, H, min_d, D, opt), st.last_error
+    dl, dr = np.empty((H, W), np.float32), np.empty((H, W), np.float32)
+    assert st.Match(left, right, dl, dr), st.last_error
+    _eq_float(dl, exp_l, "left map")
+    _eq_float(dr, exp_r, "right map")
+    st.Release()
+
+
 @pytest.fixture
 def cost_mode():
     from fasterstereocuda_amd import stereo

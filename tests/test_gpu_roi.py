@@ -58,6 +58,22 @@ def test_match_with_regions_matches_oracle(cuda, case, lr, median):
     st.Release()
 
 
+# the region's WTA at sums of the four directions past 992
+@pytest.mark.parametrize("W,H,D,p2", [(600, 60, 512, 200), (600, 60, 512, 190), (300, 60, 256, 200)])
+def test_regions_at_high_sums(cuda, W, H, D, p2):
+    rl, rr = (30, 6, W - 60, H - 12), (10, 2, W - 30, H - 4)
+    print(f"[roi] high sums {W}x{H} D{D} p2={p2}", flush=True)
+    p = scenes.cone_like(W + H, H=H, W=W, D=128)
+    exp_l, exp_r = oracle.match_roi(p.left, p.right, 0, D, rl, rr, p2=p2, do_median=False)
+    st = StereoCuda()
+    assert st.Init(W, H, 0, D, CuSGMOption.benchmark(p2_init=p2, do_median_filter=False)), st.last_error
+    dl, dr = np.empty((H, W), np.float32), np.empty((H, W), np.float32)
+    assert st.Match(p.left, p.right, dl, dr, None, rl, rr), st.last_error
+    _eq(dl, exp_l, "left map")
+    _eq(dr, exp_r, "right map")
+    st.Release()
+
+
 def test_regions_with_peaks_and_depth(cuda):
     W, H, D = 400, 240, 64
     p = scenes.cone_like(7, H=H, W=W, D=D)
