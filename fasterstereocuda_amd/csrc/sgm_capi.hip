@@ -189,11 +189,12 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmP
     std::vector<int> o3(nj + 1, 0), od(nj + 1, 0), w3(nj + 1, 0), wd(nj + 1, 0), wf(nj + 1, 0);
     std::vector<int> m3(nj + 1, 0), mf(nj + 1, 0);
     int dmax = 64, dmin = kMaxD;
-    bool wide = true, big = false, mid = true, quirk = false;
+    bool wide = true, big = false, mid = true, quirk = false, far = false;
     int64_t cells = 0;
     for (int i = 0; i < nj; ++i) {
         wide = wide && wide_ok(jobs[i]);
         big = big || big_penalties(jobs[i]);
+        far = far || far_steps(jobs[i]);
         mid = mid && mid_ok(jobs[i]);
         quirk = quirk || mid_specials(jobs[i]) > 0;
         cells += (int64_t)(jobs[i].W - jobs[i].roi_x) * jobs[i].H * jobs[i].D;
@@ -280,6 +281,7 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmP
     plan->cells = cells;
     plan->quirk = quirk;
     plan->big = big;
+    plan->far = far;
     plan->fast = !big;
     plan->n_post = op[np];
     plan->dmax = dmax;

@@ -108,6 +108,11 @@ inline int wide_v_items(const SgmJob& j, int kind) {
 // Penalties whose sums leave the positive finite f16 patterns (below 0x7C00):
 // the aggregation then takes integer minima.
 inline bool big_penalties(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
+// Steps of the longest block of the stored-cost walk (agg_lines), and whether
+// that many rows pass 31 bits of bytes.  (Persistent schedules take sides up to
+// 65532, which never do.)
+__host__ __device__ constexpr int agg_block(int D) { return D <= 128 ? 16 : 2048 / D; }
+inline bool far_steps(const SgmJob& j) { return (int64_t)agg_block(j.D) * j.W * j.D > INT32_MAX; }
 inline bool wide_ok(const SgmJob& j) { return j.D <= 256 && !(j.is_right && j.cs_type == 0); }
 
 // Their 4-line form (sgm_mid.hip) for plans too small to fill the GPU that
@@ -176,6 +181,7 @@ struct StagePlan {
     bool mid = false;             // unless scheduled, it uses their 4-line form
     bool quirk = false;           // some matched job is a 5x5 right view
     bool big = false;             // some job's penalties need integer minima
+    bool far = false;             // some job has far_steps
     bool fast = false;            // not big, and every cost is a census distance (at most 64)
     int shape = 0;                // how wide or tall the matched images are (plan_shape)
     IoBind io{};                  // host-side: bound caller buffers, if any

@@ -259,7 +259,9 @@ __global__ __launch_bounds__(256) void cost_kernel(const SgmJob* __restrict__ jo
 //     whose out-of-row lanes no shift writes;
 //   * FAST (costs of at most 64, P1 + P2 <= 30000): no sum carries or borrows
 //     between u16 halves, so sums are 32-bit, and values are positive finite
-//     f16 patterns, so two minima are one v_pk_minimum3_f16.
+//     f16 patterns, so two minima are one v_pk_minimum3_f16;
+//   * FAR (rows so long that a block's steps pass 32 bits, see far_steps): each
+//     step has a 64-bit base of its own and no scalar offset.
 
 // Where a block of up to PF steps starts and how its steps lie from there:
 // byte offset `base` of its lowest address, the scalar offset of its first
@@ -280,7 +282,7 @@ __device__ __forceinline__ BlockWalk block_walk(int64_t first, int64_t step, int
     return w;
 }
 
-template <int D, bool FUSE, bool FAST>
+template <int D, bool FUSE, bool FAST, bool FAR = false>
 __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, int lane) {
     constexpr int DPD = D / 16;   // disparities per lane
     constexpr int NW = DPD / 4;   // u32 words of cost per lane
@@ -303,7 +305,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
     const int line0 = group * 4;
     const int64_t offL = horiz ? ((int64_t)line0 * W + xs) * D
                                : ((int64_t)ys * W + roi_x + line0) * D;
-    const uint32_t voff = (uint32_t)((line - line0) * (horiz ? W * D : D) + l * DPD);
+    const uint32_t voff = (uint32_t)(line - line0) * (horiz ? (uint32_t)W * D : (uint32_t)D) + l * DPD;
     uint8_t* const out_base = (path == 0) ? J.path[0] : (path == 1) ? J.path[1]
                             : (path == 2) ? J.path[2] : J.path[3];
     const uint32_t P1v = (uint32_t)J.p1 * 0x10001u;
@@ -317,8 +319,18 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
     // other directions).  Slot p holds step i0 + p of the current block.
     constexpr int NSRC = FUSE ? 4 : 1;
     constexpr int PF = FUSE ? (NW == 1 ? 8 : 16 / NW) : (NW >= 2 ? 32 / NW : 16);
+    static_assert(PF <= agg_block(D), "far_steps bounds a block's offsets");
     const uint8_t* srcs[4] = {J.cost, J.path[0], J.path[1], J.path[3]};
     uint32_t buf[PF][NSRC][NW];
+    // step j of a block walk, at scalar offset s
+    auto load_at = [&](const BlockWalk& w, int s, int j, int q, uint32_t (&d)[NW]) __attribute__((always_inline)) {
+        if constexpr (FAR) buf_load<NW>(buf_at(srcs[q] + block_walk(offL, step, j, 1, n).base, ~0u), voff, 0, d);
+        else buf_load<NW>(buf_at(srcs[q] + w.base), voff, s, d);
+    };
+    auto store_at = [&](const BlockWalk& w, int s, int j, const uint32_t (&o)[NW]) __attribute__((always_inline)) {
+        if constexpr (FAR) buf_store<NW>(buf_at(out_base + block_walk(offL, step, j, 1, n).base, ~0u), voff, 0, o);
+        else buf_store<NW>(buf_at(out_base + w.base), voff, s, o);
+    };
 
     uint32_t L[NP];
     uint32_t m;   // the line minimum in both u16 halves
@@ -329,7 +341,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
     {
         const BlockWalk w0 = block_walk(offL, step, 0, 1, n);
         uint32_t w[NW];
-        buf_load<NW>(buf_at(srcs[0] + w0.base), voff, w0.s, w);
+        load_at(w0, w0.s, 0, 0, w);
         // the ring's slots in the loop's own order (the scheduler may not
         // interleave them): the wait counts at the loop head are the merge of
         // both paths, and any other order collapses them to zero
@@ -339,13 +351,13 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
 #pragma unroll
-            for (int q = 0; q < NSRC; ++q) buf_load<NW>(buf_at(srcs[q] + b.base), voff, so, buf[p][q]);
+            for (int q = 0; q < NSRC; ++q) load_at(b, so, 1 + p, q, buf[p][q]);
             so = max(min(so + b.inc, b.last), 0);
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int k = 0; k < NW; ++k) { L[2 * k] = bytes01(w[k]); L[2 * k + 1] = bytes23(w[k]); }
-        if constexpr (!FUSE) buf_store<NW>(buf_at(out_base + w0.base), voff, w0.s, w);
+        if constexpr (!FUSE) store_at(w0, w0.s, 0, w);
         else if (active && l == 0) gst(J.disp + y0 * W + x0, kInvalidDisp);   // row H-1: border
         m = line_minimum();
     }
@@ -455,22 +467,19 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
         for (; i + PF <= n; i += PF) {
             const BlockWalk in = block_walk(offL, step, i + PF, PF, n);
             const BlockWalk out = block_walk(offL, step, i, PF, n);
-            const auto rin = buf_at(srcs[0] + in.base);
-            const auto rout = buf_at(out_base + out.base);
             int si = in.s, so = out.s;
 #pragma unroll
             for (int p = 0; p < PF; ++p) {
                 advance(buf[p][0]);
-                buf_load<NW>(rin, voff, si, buf[p][0]);
+                load_at(in, si, i + PF + p, 0, buf[p][0]);
                 uint32_t o[NW];
                 pack(o);
-                buf_store<NW>(rout, voff, so, o);
+                store_at(out, so, i + p, o);
                 si = max(min(si + in.inc, in.last), 0);
                 so += out.inc;
             }
         }
         const BlockWalk out = block_walk(offL, step, i, PF, n);
-        const auto rout = buf_at(out_base + out.base);
         int so = out.s;
 #pragma unroll
         for (int p = 0; p < PF - 1; ++p) {
@@ -478,7 +487,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
                 advance(buf[p][0]);
                 uint32_t o[NW];
                 pack(o);
-                buf_store<NW>(rout, voff, so, o);
+                store_at(out, so, i + p, o);
                 so += out.inc;
             }
         }
@@ -499,7 +508,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
             for (int p = 0; p < PF; ++p) {
                 consume(buf[p], at + p);
 #pragma unroll
-                for (int q = 0; q < NSRC; ++q) buf_load<NW>(buf_at(srcs[q] + in.base), voff, si, buf[p][q]);
+                for (int q = 0; q < NSRC; ++q) load_at(in, si, at + PF + p, q, buf[p][q]);
                 si = max(min(si + in.inc, in.last), 0);
             }
         };
@@ -523,7 +532,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
 // MODE 0: all four directions (stage entry point); MODE 1: left->right,
 // right->left, top->bottom; MODE 2: bottom->top fused with the WTA.
 // ONLY: every job has D = DMAX (other ranges' code would take its registers).
-template <int DMAX, int MODE, bool FAST, bool ONLY>
+template <int DMAX, int MODE, bool FAST, bool ONLY, bool FAR = false>
 __global__ __launch_bounds__(256) void aggregate_kernel(const SgmJob* __restrict__ jobs,
                                                         const int* __restrict__ offs, int njobs,
                                                         int n) {
@@ -543,10 +552,10 @@ __global__ __launch_bounds__(256) void aggregate_kernel(const SgmJob* __restrict
     const int lane = threadIdx.x & 63;
     constexpr bool F = (MODE == 2);
     switch (J.D) {
-        case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST>(J, path, group, lane); break;
-        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) agg_lines<128, F, FAST>(J, path, group, lane); break;
-        case 256: if constexpr (ONLY ? DMAX == 256 : DMAX >= 256) agg_lines<256, F, FAST>(J, path, group, lane); break;
-        case 512: if constexpr (ONLY ? DMAX == 512 : DMAX >= 512) agg_lines<512, F, FAST>(J, path, group, lane); break;
+        case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST, FAR>(J, path, group, lane); break;
+        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) agg_lines<128, F, FAST, FAR>(J, path, group, lane); break;
+        case 256: if constexpr (ONLY ? DMAX == 256 : DMAX >= 256) agg_lines<256, F, FAST, FAR>(J, path, group, lane); break;
+        case 512: if constexpr (ONLY ? DMAX == 512 : DMAX >= 512) agg_lines<512, F, FAST, FAR>(J, path, group, lane); break;
         default: break;
     }
 }
@@ -897,7 +906,8 @@ static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hi
     const int wg = p.cells <= 100000000 ? waves_per_group(n, 7) : 1;
     const dim3 g((n + wg - 1) / wg), b(64 * wg);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs, n); };
-    if (!p.fast) go(aggregate_kernel<512, MODE, false, false>);
+    if (p.far) go(aggregate_kernel<512, MODE, false, false, true>);
+    else if (!p.fast) go(aggregate_kernel<512, MODE, false, false>);
     else if (p.dmax <= 64) go(aggregate_kernel<64, MODE, true, true>);
     else if (p.dmin == p.dmax)
         p.dmax == 128 ? go(aggregate_kernel<128, MODE, true, true>)

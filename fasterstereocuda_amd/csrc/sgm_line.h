@@ -10,8 +10,8 @@ namespace dev {
 
 typedef unsigned int buf_u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int buf_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const uint8_t* p) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, 0x7fffffff, 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const uint8_t* p, uint32_t bytes = 0x7fffffffu) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)bytes, 0x00020000);
 }
 template <int NW>
 __device__ __forceinline__ void buf_load(__amdgpu_buffer_rsrc_t r, uint32_t v, int s, uint32_t (&w)[NW]) {

@@ -353,6 +353,49 @@ def test_wta_forms_match_oracle(cuda, cost_mode, wta_form, form, case, lr, media
     st.Release()
 
 
+# Rows so long that a block of the stored-cost walk's steps (16 rows, 8 at D = 256,
+# less one) passes 2^31 bytes of a volume: the steps then have 64-bit addresses.
+# Columns are independent in the vertical directions, so slices are checked there,
+# and the ends that the horizontal directions start from.
+@pytest.mark.parametrize("W,H,D", [(2240011, 19, 64), (1200007, 11, 256)])
+def test_very_long_rows(cuda, W, H, D):
+    print(f"[long rows] {W}x{H} D{D}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(W)
+    cost = torch.randint(0, 64, (H, W, D), dtype=torch.uint8, device=cuda, generator=g)
+    paths = stages.aggregate(cost, 0, 10, 150)
+    ends = {"first": slice(0, 70), "middle": slice(W // 2, W // 2 + 70), "last": slice(W - 70, W)}
+    for name, cols in ends.items():
+        c = cost[:, cols].cpu().numpy().copy()
+        for r in (0, 2) + ((1,) if name == "first" else (3,) if name == "last" else ()):
+            np.testing.assert_array_equal(paths[r][:, cols].cpu().numpy(), oracle.aggregate(c, 0, r, 10, 150),
+                                          err_msg=f"path {stages.DIRS[r]}, {name} columns")
+
+
+# the same rows through Match: bottom->top fused with the WTA against all four
+# directions and the WTA apart
+@pytest.mark.parametrize("W,H,D", [(1120003, 19, 128)])
+def test_very_long_rows_match(cuda, cost_mode, wta_form, W, H, D):
+    print(f"[long rows match] {W}x{H} D{D}", flush=True)
+    cost_mode(1)
+    rng = np.random.default_rng(W)
+    right = rng.integers(0, 256, (H, W), dtype=np.uint8)
+    left = np.roll(right, 17, axis=1)
+    opt = CuSGMOption.benchmark(do_median_filter=False)
+    maps = []
+    for form in (stages.WTA_FUSED, stages.WTA_SEPARATE):
+        wta_form(form)
+        st = StereoCuda()
+        assert st.Init(W, H, 0, D, opt), st.last_error
+        dl, dr = np.empty((H, W), np.float32), np.empty((H, W), np.float32)
+        assert st.Match(left, right, dl, dr), st.last_error
+        maps.append((dl, dr))
+        st.Release()
+    _eq_float(maps[0][0], maps[1][0], "left map")
+    _eq_float(maps[0][1], maps[1][1], "right map")
+    inside = maps[0][0][5:H - 5, 200:W - 5]
+    assert np.abs(inside[inside != oracle.INVALID] - 17).max() <= 1 and (inside != oracle.INVALID).mean() > 0.9
+
+
 def test_driving_full_size(cuda):
     pair = scenes.driving(0)
     print("[match] driving 1242x375", flush=True)
