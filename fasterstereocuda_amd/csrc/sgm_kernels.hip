@@ -18,6 +18,7 @@
 // Arithmetic matches the reference exactly (ethan-li-coding/FasterStereoCuda,
 // SgmStereoCuda/cusgm_cc.cu, cusgm_ca.cu, cusgm_df.cu); see each kernel.
 #include <algorithm>
+#include <cstdint>
 
 #include "sgm_device.h"
 #include "sgm_internal.h"
@@ -260,6 +261,11 @@ __global__ __launch_bounds__(256) void cost_kernel(const SgmJob* __restrict__ jo
 //   * FAST (costs of at most 64, P1 + P2 <= 30000): no sum carries or borrows
 //     between u16 halves, so sums are 32-bit, and values are positive finite
 //     f16 patterns, so two minima are one v_pk_minimum3_f16;
+//   * DEEP: the rings above are those of a kernel for one D.  One for several has
+//     the registers of its largest range in all its waves (fused, to D = 256: 201,
+//     so two waves per SIMD), and a mixed plan's waves then run in turns.  Without
+//     DEEP the fused form looks 4 (D = 64) or 2 steps ahead (121 registers) and the
+//     others 7 at D = 256 (62: eight waves); see launch_agg_mode;
 //   * FAR (rows so long that a block's steps pass 32 bits, see far_steps): each
 //     step has a 64-bit base of its own and no scalar offset.
 
@@ -282,7 +288,7 @@ __device__ __forceinline__ BlockWalk block_walk(int64_t first, int64_t step, int
     return w;
 }
 
-template <int D, bool FUSE, bool FAST, bool FAR = false>
+template <int D, bool FUSE, bool FAST, bool FAR = false, bool DEEP = true>
 __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, int lane) {
     constexpr int DPD = D / 16;   // disparities per lane
     constexpr int NW = DPD / 4;   // u32 words of cost per lane
@@ -318,7 +324,8 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
     // Register ring of prefetched words (the cost, and with FUSE the three
     // other directions).  Slot p holds step i0 + p of the current block.
     constexpr int NSRC = FUSE ? 4 : 1;
-    constexpr int PF = FUSE ? (NW == 1 ? 8 : 16 / NW) : (NW >= 2 ? 32 / NW : 16);
+    constexpr int PF = FUSE ? (DEEP ? (NW == 1 ? 8 : 16 / NW) : (NW == 1 ? 4 : 2))
+                            : (NW == 1 ? 16 : NW == 4 && !DEEP ? 7 : 32 / NW);
     static_assert(PF <= agg_block(D), "far_steps bounds a block's offsets");
     const uint8_t* srcs[4] = {J.cost, J.path[0], J.path[1], J.path[3]};
     uint32_t buf[PF][NSRC][NW];
@@ -532,7 +539,7 @@ __device__ __forceinline__ void agg_lines(const SgmJob& J, int path, int group, 
 // MODE 0: all four directions (stage entry point); MODE 1: left->right,
 // right->left, top->bottom; MODE 2: bottom->top fused with the WTA.
 // ONLY: every job has D = DMAX (other ranges' code would take its registers).
-template <int DMAX, int MODE, bool FAST, bool ONLY, bool FAR = false>
+template <int DMAX, int MODE, bool FAST, bool ONLY, bool FAR = false, bool DEEP = true>
 __global__ __launch_bounds__(256) void aggregate_kernel(const SgmJob* __restrict__ jobs,
                                                         const int* __restrict__ offs, int njobs,
                                                         int n) {
@@ -552,10 +559,10 @@ __global__ __launch_bounds__(256) void aggregate_kernel(const SgmJob* __restrict
     const int lane = threadIdx.x & 63;
     constexpr bool F = (MODE == 2);
     switch (J.D) {
-        case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST, FAR>(J, path, group, lane); break;
-        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) agg_lines<128, F, FAST, FAR>(J, path, group, lane); break;
-        case 256: if constexpr (ONLY ? DMAX == 256 : DMAX >= 256) agg_lines<256, F, FAST, FAR>(J, path, group, lane); break;
-        case 512: if constexpr (ONLY ? DMAX == 512 : DMAX >= 512) agg_lines<512, F, FAST, FAR>(J, path, group, lane); break;
+        case 64: if constexpr (!ONLY || DMAX == 64) agg_lines<64, F, FAST, FAR, DEEP>(J, path, group, lane); break;
+        case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) agg_lines<128, F, FAST, FAR, DEEP>(J, path, group, lane); break;
+        case 256: if constexpr (ONLY ? DMAX == 256 : DMAX >= 256) agg_lines<256, F, FAST, FAR, DEEP>(J, path, group, lane); break;
+        case 512: if constexpr (ONLY ? DMAX == 512 : DMAX >= 512) agg_lines<512, F, FAST, FAR, DEEP>(J, path, group, lane); break;
         default: break;
     }
 }
@@ -900,6 +907,12 @@ hipError_t launch_cost(const StagePlan& p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Plans of several D: without DEEP from D = 256 on, and to D = 128 where the fused
+// form's waves do not fit at two per SIMD (deep / not, us: three 640x480 D = 128
+// and four 450x375 D = 64, 1864 waves, whole match 820 / 855; two 1242x375 D = 128
+// and three 640x480 D = 64, 2204 waves, fused form 353 / 330; 1920x1080 D = 256 and
+// six 1242x375 D = 64, three directions + fused 1564 + 1379 / 1601 + 1218, the long
+// pair last 1862 + 1385 / 1605 + 1282).
 template <int MODE>
 static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
@@ -913,10 +926,12 @@ static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hi
         p.dmax == 128 ? go(aggregate_kernel<128, MODE, true, true>)
                       : p.dmax == 256 ? go(aggregate_kernel<256, MODE, true, true>)
                                       : go(aggregate_kernel<512, MODE, true, true>);
+    else if (p.dmax == 128)
+        MODE == 2 && n > wide_min_groups() ? go(aggregate_kernel<128, MODE, true, false, false, MODE != 2>)
+                                           : go(aggregate_kernel<128, MODE, true, false>);
     else
-        p.dmax == 128 ? go(aggregate_kernel<128, MODE, true, false>)
-                      : p.dmax == 256 ? go(aggregate_kernel<256, MODE, true, false>)
-                                      : go(aggregate_kernel<512, MODE, true, false>);
+        p.dmax == 256 ? go(aggregate_kernel<256, MODE, true, false, false, false>)
+                      : go(aggregate_kernel<512, MODE, true, false, false, false>);
     return hipGetLastError();
 }
 
@@ -979,7 +994,13 @@ hipError_t persistent_occupancy(const StagePlan& p, int* per_cu) {
     hipError_t e = occ_mode<1>(p.dmax, &a);
     if (e != hipSuccess) return e;
     if ((e = occ_mode<2>(p.dmax, &b)) != hipSuccess) return e;
-    *per_cu = std::max(1, std::min(a, b));
+    // From D = 256 on one wave per SIMD: its rings cover the memory latency, and
+    // more waves only share the path to memory (longest first, 4 / 8 / 12 waves per
+    // CU, us: four 1000x500 D = 256 2475 / 2599 / 2805, four 320x240 D = 256 470 /
+    // 516 / 544, 1920x1080 D = 256 and six 1242x375 D = 64 3574 / 3836 / 4040, two
+    // 640x480 D = 512 1987 / 2088 / 2160).
+    const int most = p.dmax >= 256 ? 4 : INT32_MAX;
+    *per_cu = std::max(1, std::min({a, b, most}));
     return hipSuccess;
 }
 

@@ -396,6 +396,32 @@ def test_very_long_rows_match(cuda, cost_mode, wta_form, W, H, D):
     assert np.abs(inside[inside != oracle.INVALID] - 17).max() <= 1 and (inside != oracle.INVALID).mean() > 0.9
 
 
+# several ranges in one stored-cost plan, whose kernels look fewer steps ahead:
+# heights and widths around whole rings of 2, 4, 7 and 16 steps
+@pytest.mark.parametrize("form", [stages.WTA_FUSED, stages.WTA_SEPARATE], ids=["fused", "separate"])
+@pytest.mark.parametrize("ranges", [(64, 128), (256, 64), (64, 128, 256), (512, 64, 256)])
+def test_stored_mixed_batch(cuda, cost_mode, wta_form, form, ranges):
+    from fasterstereocuda_amd.batch import SgmBatch
+    print(f"[stored mixed] {ranges} form={form}", flush=True)
+    cost_mode(1)
+    wta_form(form)
+    pairs, refs = [], []
+    for i, (W, H) in enumerate([(40, 13), (33, 14), (34, 16), (49, 15), (36, 22), (45, 23)]):
+        D, m = ranges[i % len(ranges)], (0, 3, -2)[i % 3]
+        left, right = _pair(W, H, D, seed=40 + i)
+        refs.append(oracle.match(left, right, m, D, uniqueness=UNIQ, lr_threshold=LR_THR, do_median=False))
+        pairs.append({"left": torch.from_numpy(left).to(cuda), "right": torch.from_numpy(right).to(cuda),
+                      "disp_left": torch.empty((H, W), device=cuda),
+                      "disp_right": torch.empty((H, W), device=cuda),
+                      "min_disparity": m, "disp_range": D})
+    b = SgmBatch(pairs, CuSGMOption.benchmark(do_median_filter=False))
+    b.run()
+    torch.cuda.synchronize()
+    for p, (exp_l, exp_r) in zip(pairs, refs):
+        _eq_float(p["disp_left"].cpu().numpy(), exp_l, "left map")
+        _eq_float(p["disp_right"].cpu().numpy(), exp_r, "right map")
+
+
 def test_driving_full_size(cuda):
     pair = scenes.driving(0)
     print("[match] driving 1242x375", flush=True)
