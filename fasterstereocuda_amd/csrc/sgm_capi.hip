@@ -85,66 +85,78 @@ int waves_per_group(int n, int limit) {
     return 2 * n > simds && 4 * n <= limit * simds ? 4 : 1;
 }
 
-// 0: some matched image is over 2.5 times as wide as high, 1: over 1.5 times, 2:
-// not over 1.2 times as high as wide, 3: none of these (all tall).  4: images of
-// several sizes, one pair of which has over half the cells; shape as for 0.
-int plan_shape(const std::vector<SgmJob>& jobs, int n) {
-    int shape = n > 0 ? 3 : 0;
-    int64_t least = INT64_MAX, most = 0, total = 0;
-    for (int i = 0; i < n; ++i) {
-        const int64_t w = jobs[i].W - jobs[i].roi_x, h = jobs[i].H, cells = w * h * jobs[i].D;
-        least = std::min(least, cells);
-        most = std::max(most, cells);
-        total += cells;
-        shape = std::min(shape, 2 * w > 5 * h ? 0 : 2 * w > 3 * h ? 1 : 5 * h <= 6 * w ? 2 : 3);
-    }
-    return n > 2 && least < most && 4 * most > total ? 4 : shape;   // two views a pair
-}
-
 // Stored-cost plans: the four directions and then the WTA, or bottom->top
-// fused with the WTA after the other three.  The fused bottom->top walk is
-// latency-bound on a small plan, so it is better run beside the horizontal
-// ones (and the WTA left to its own memory-bound launch) while the four
-// directions have at most 2.5 waves per SIMD and the extra volume's traffic is
-// small: the more so, the longer the columns are beside the rows (both views,
-// separate / fused, us): wide 1242x375 D = 64, 60M 185 / 211, D = 128, 119M 416 /
-// 336; 640x480 D = 128, 79M 240 / 268, 1280x720 D = 128, 236M 643 / 626; square
-// 1200x852, 131M 405 / 429, 700x700 D = 256, 251M 700 / 762, 1200x1000 D = 128,
-// 307M 798 / 784; tall 500x1000 D = 256, 256M 722 / 917, 800x2500 D = 128, 512M
-// 1429 / 1573, 1200x1800 D = 128, 553M 1464 / 1441.
+// fused with the WTA after the other three.
+//
+// The fused walk waits out `height` dependent steps of a few waves, while the
+// separate form runs it beside the other directions and pays 6 bytes per cell
+// (a volume more written and read, and the WTA's reads).  Cells over height are
+// the matched columns over all views, so those decide, whatever the shape; the
+// longer a D's step, the fewer columns (separate / fused, us, LR check on unless
+// given; columns):
+//   D = 64: 2500 1500x3000 off 903 / 1233, 2400 1200x852 405 / 429, 3000 1500x3000
+//   1598 / 1657, 3000 3000x3000 off 1683 / 1674, 3840 1920x1080 759 / 717
+//   D = 128: 1600 800x800 425 / 498, 1920 1920x1080 off 696 / 732, 2000 2000x2000
+//   off 1294 / 1379, 2400 1200x1000 798 / 784, 2484 1242x375 416 / 336, 2560
+//   1280x720 621 / 612
+//   D = 256: 1500 1500x1500 off 1470 / 1638, 1600 800x800 864 / 913, 1800 900x1500
+//   1965 / 1891, 1920 1920x1080 off 1383 / 1338
+//   D = 512: 1280 640x480 1083 / 1199, 1600 800x800 2115 / 2202, 1920 1920x1080
+//   off 3289 / 3227, 2000 2000x400 off 1482 / 1468
 bool separate_wta(const StagePlan& p) {
-    constexpr int64_t kCells[5] = {100000000, 200000000, 260000000, 540000000, 100000000};
     const int f = g_wta_form.load();
     if (f == SGM_WTA_FUSED) return false;
     if (f == SGM_WTA_SEPARATE) return true;
-    return 4 * p.n_agg <= 5 * wide_min_groups() && p.cells <= kCells[p.shape];
+    return p.work.walk < 12000;
 }
-
 bool choose_wide(bool eligible, int n_wh) {
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED) return false;
     return mode == SGM_COST_ON_THE_FLY || n_wh >= wide_min_groups();
 }
 
-// The 4-line on-the-fly form moves 6 bytes per cell where the stored cost
-// takes 11, but issues about 1.6 times the instructions per step, and its
-// bottom->top walk always follows the others: it wins once memory, not the
-// scanlines' serial steps, bounds the stored form, the later the longer the
-// columns are (both views, stored / on the fly, us): wide 1280x720 D = 128, 236M
-// 626 / 669, 1000x500 D = 256, 256M 666 / 597, 1117x573 D = 256, 328M 880 / 821,
-// 1920x1080 D = 128, 531M 1290 / 1100; square 700x700 D = 256, 251M 700 / 854,
-// 1200x1000 D = 128, 307M 784 / 847, 1400x1100, 394M 996 / 988, 900x900 D = 256,
-// 415M 1154 / 1115, 1700x1700 D = 128, 740M 1758 / 1685; tall 500x1000 D = 256, 256M
-// 722 / 1081, 800x2500 D = 128, 512M 1429 / 1934, 1400x2200 D = 128, 788M 2002 / 2075.
-// A mixed plan whose largest pair has over half the cells stays with the stored
-// cost: that pair's steps outlast the rest, and the kernel for several D is
-// slower than the one for its own (6 pairs of 891M cells, 531M of them one
-// 1920x1080 D = 128: 2346 / 2694; 7 of 897M, 265M in one: 2375 / 2218).
-bool choose_mid(bool eligible, int n_wh, int64_t cells, int shape) {
-    constexpr int64_t kCells[5] = {250000000, 250000000, 400000000, 800000000, INT64_MAX};
+// The 4-line on-the-fly form moves 6 bytes per cell where the stored cost takes
+// 11, but issues about 1.6 times the instructions per step, and its bottom->top
+// walk always follows the others: it wins once memory, not the lines' serial
+// steps, bounds the stored form.  A step of all columns moves columns x D bytes
+// of a volume, a step of all rows rows x D, over all views: the fewer, the more a
+// step's latency counts (columns x D, rows x D in K: the better stored form / on
+// the fly, us):
+//   1024, 1024: 2000x2000 D = 256 4592 / 3648; 983, 553: 3840x2160 D = 64 2599 /
+//   2629, D = 128, LR check off, 492, 276: 2376 / 2132; 572, 293: 1117x573 D = 256
+//   871 / 812; 512, 512: 2000x2000 D = 128 2298 / 2118; 512, 256: 1000x500 D = 256
+//   656 / 591; 492, 276: 1920x1080 D = 128 1290 / 1100, D = 256 off 1338 / 1222
+//   461, 768: 900x1500 D = 256 1891 / 1952; 410, 410: 800x800 D = 256 864 / 978;
+//   384, 640: 1500x2500 D = 128 2240 / 2337; 384, 384: 1500x1500 D = 256 off 1470 /
+//   1830, 3000x3000 D = 64 2712 / 2952; 256, 256: 2000x2000 D = 128 off 1294 / 1639
+//   768, 179: 3000x700 D = 128 1346 / 1413; 1280, 128: 5000x500 D = 128 1701 / 1947
+// Of several D the kernel has the registers of D = 256 in all its waves, which
+// only pays where most of them are D = 256 (share of the waves: 64%, 2000x800
+// D = 256 and 1242x375 D = 64 2144 / 1875; 50%, 1920x1080 D = 256 and two of those
+// 2884 / 3073; none, 1920x1080 D = 128 and 160x120 D = 64 1226 / 1261).  Of several
+// sizes the waves have to fit at once, or the longest lines end last (4 per SIMD:
+// 2840 waves, 1920x1080 and 640x480, D = 128, 1515 / 1367; 5694, 3000x1200 and three
+// 1242x375 2909 / 3000; 4680, 5000x500 and three 640x480 2173 / 2407).
+bool choose_mid(bool eligible, int n_wh, const PlanWork& w) {
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED || n_wh >= wide_min_groups()) return false;
-    return mode == SGM_COST_ON_THE_FLY || cells >= kCells[shape];
+    if (mode == SGM_COST_ON_THE_FLY) return true;
+    if (w.dmin != w.dmax && 5 * w.waves256 < 3 * w.waves) return false;
+    if (w.least != w.most && w.waves > 2 * wide_min_groups()) return false;
+    return w.col_bytes >= 470000 && w.row_bytes >= 230000;
+}
+void PlanWork::add(const SgmJob& j) {
+    const int64_t cols = j.W - j.roi_x, n = mid3_items(j), c = cols * j.H * j.D;
+    cells += c;
+    least = std::min(least, c);
+    most = std::max(most, c);
+    col_bytes += cols * j.D;
+    row_bytes += (int64_t)j.H * j.D;
+    walk += cols * (j.D <= 64 ? 4 : j.D <= 128 ? 5 : 7);   // 12000: 3000, 2400, 1714 columns
+    waves += n;
+    if (j.D == 256) waves256 += n;
+    dmin = std::min(dmin, j.D);
+    dmax = std::max(dmax, j.D);
 }
 }  // namespace fsgm
 
@@ -190,14 +202,14 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmP
     std::vector<int> m3(nj + 1, 0), mf(nj + 1, 0);
     int dmax = 64, dmin = kMaxD;
     bool wide = true, big = false, mid = true, quirk = false, far = false;
-    int64_t cells = 0;
+    PlanWork work;
     for (int i = 0; i < nj; ++i) {
         wide = wide && wide_ok(jobs[i]);
         big = big || big_penalties(jobs[i]);
         far = far || far_steps(jobs[i]);
         mid = mid && mid_ok(jobs[i]);
         quirk = quirk || mid_specials(jobs[i]) > 0;
-        cells += (int64_t)(jobs[i].W - jobs[i].roi_x) * jobs[i].H * jobs[i].D;
+        work.add(jobs[i]);
         m3[i + 1] = m3[i] + mid3_items(jobs[i]);
         mf[i + 1] = mf[i] + mid_v_items(jobs[i]);
         const bool w = jobs[i].D <= 256;
@@ -276,9 +288,8 @@ int fsgm::upload_plan(const std::vector<SgmJob>& jobs_in, const std::vector<SgmP
     plan->n_m3 = m3[nj];
     plan->n_mf = mf[nj];
     plan->wide = choose_wide(wide, w3[nj]);
-    plan->shape = plan_shape(jobs, nj);
-    plan->mid = choose_mid(mid, w3[nj], cells, plan->shape);
-    plan->cells = cells;
+    plan->work = work;
+    plan->mid = choose_mid(mid, w3[nj], work);
     plan->quirk = quirk;
     plan->big = big;
     plan->far = far;
@@ -296,13 +307,13 @@ void fsgm::restrict_matching(StagePlan* P, const std::vector<SgmJob>& jobs, int 
     P->n_cost = P->n_agg = P->n_wta = P->n_agg3 = P->n_dw = P->n_wh = P->n_wv = P->n_wf = 0;
     P->n_m3 = P->n_mf = 0;
     bool wide = true, mid = true;
-    int64_t cells = 0;
+    PlanWork work;
     P->quirk = false;
     for (int i = 0; i < n; ++i) {
         wide = wide && wide_ok(jobs[i]);
         mid = mid && mid_ok(jobs[i]);
         P->quirk = P->quirk || mid_specials(jobs[i]) > 0;
-        cells += (int64_t)(jobs[i].W - jobs[i].roi_x) * jobs[i].H * jobs[i].D;
+        work.add(jobs[i]);
         P->n_m3 += mid3_items(jobs[i]);
         P->n_mf += mid_v_items(jobs[i]);
         if (jobs[i].D <= 256) {
@@ -317,9 +328,8 @@ void fsgm::restrict_matching(StagePlan* P, const std::vector<SgmJob>& jobs, int 
         P->n_dw += dw_items(jobs[i]);
     }
     P->wide = choose_wide(wide, P->n_wh);
-    P->shape = plan_shape(jobs, n);
-    P->mid = choose_mid(mid, P->n_wh, cells, P->shape);
-    P->cells = cells;
+    P->work = work;
+    P->mid = choose_mid(mid, P->n_wh, work);
 }
 
 // census, cost, three directions, bottom->top + WTA (or the four directions,

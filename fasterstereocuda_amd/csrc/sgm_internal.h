@@ -155,6 +155,18 @@ struct IoBind {
     int32_t on;
 };
 
+// Sums over the matched views of a plan that decide its forms.
+struct PlanWork {
+    int64_t cells = 0;        // pixels x D
+    int64_t least = INT64_MAX, most = 0;   // of one view
+    int64_t col_bytes = 0;    // columns x D: a step of all vertical lines
+    int64_t row_bytes = 0;    // rows x D
+    int64_t walk = 0;         // columns by the length of their D's step (separate_wta)
+    int64_t waves = 0, waves256 = 0;   // of the 4-line form's first launch; those of D = 256
+    int dmin = INT32_MAX, dmax = 0;
+    void add(const SgmJob& j);
+};
+
 // Device-side launch plan: jobs, per-stage prefix sums and totals.
 struct StagePlan {
     SgmJob* jobs = nullptr;       // device
@@ -175,7 +187,7 @@ struct StagePlan {
     int njobs_ctw = 0;            // if > 0: jobs [0, njobs_ctw) run cost..wta
     int n_census = 0, n_cost = 0, n_agg = 0, n_wta = 0, n_post = 0, n_agg3 = 0, n_dw = 0;
     int n_wh = 0, n_wv = 0, n_wf = 0, n_m3 = 0, n_mf = 0;
-    int64_t cells = 0;            // matched pixels x D, over the views
+    PlanWork work;                // of the matched jobs
     int dmax = 64, dmin = 64;     // over all jobs; dmin over the matched ones
     bool wide = false;            // matching uses the on-the-fly cost kernels
     bool mid = false;             // unless scheduled, it uses their 4-line form
@@ -183,7 +195,6 @@ struct StagePlan {
     bool big = false;             // some job's penalties need integer minima
     bool far = false;             // some job has far_steps
     bool fast = false;            // not big, and every cost is a census distance (at most 64)
-    int shape = 0;                // how wide or tall the matched images are (plan_shape)
     IoBind io{};                  // host-side: bound caller buffers, if any
 };
 
@@ -222,8 +233,9 @@ unsigned spread_lds(int n, int used);
 // different SIMDs, while single-wave workgroups are placed unevenly: with few
 // waves some SIMDs get several and others none (1242x375 D = 64, four
 // directions and WTA: 211 us as 1620 single waves, 183 us by fours;
-// 1920x1080 D = 128, 2040 waves with on-the-fly cost: 1265 and 1097 us).  With
-// more waves, or where memory is the limit, the finer grain is the better one.
+// 1920x1080 D = 128, 2040 waves with on-the-fly cost: 1265 and 1097 us; with
+// 640x480 beside it, 2840 waves, 1515 and 1367 us).  With more waves, or where
+// memory is the limit, the finer grain is the better one.
 int waves_per_group(int n, int limit);
 // sgm_wide.hip: aggregation with the cost computed from the census words
 hipError_t launch_wide3(const StagePlan& p, hipStream_t s);
@@ -243,10 +255,9 @@ hipError_t wide_occupancy(const StagePlan& p, int* per_cu);
 // (`eligible`) and that has n_wh horizontal scanline groups.
 int cost_mode();
 // choose_mid: whether an unscheduled run of it takes the 4-line form
-// (`eligible` by mid_ok; cells: matched pixels x D over the views; shape by
-// plan_shape).
+// (`eligible` by mid_ok).
 bool choose_wide(bool eligible, int n_wh);
-bool choose_mid(bool eligible, int n_wh, int64_t cells, int shape);
+bool choose_mid(bool eligible, int n_wh, const PlanWork& w);
 int wide_min_groups();
 hipError_t launch_wta(const StagePlan& p, hipStream_t s);
 hipError_t launch_post(const StagePlan& p, hipStream_t s);

@@ -916,7 +916,7 @@ hipError_t launch_cost(const StagePlan& p, hipStream_t s) {
 template <int MODE>
 static hipError_t launch_agg_mode(const StagePlan& p, const int* offs, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    const int wg = p.cells <= 100000000 ? waves_per_group(n, 7) : 1;
+    const int wg = p.work.cells <= 100000000 ? waves_per_group(n, 7) : 1;
     const dim3 g((n + wg - 1) / wg), b(64 * wg);
     auto go = [&](auto ker) { hipLaunchKernelGGL(ker, g, b, 0, s, p.jobs, offs, p.njobs, n); };
     if (p.far) go(aggregate_kernel<512, MODE, false, false, true>);

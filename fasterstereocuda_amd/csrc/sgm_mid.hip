@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void census_pads_kernel(uint64_t* census, int 
 }  // namespace
 
 hipError_t launch_mid3(const StagePlan& p, hipStream_t s) {
-    const int n = p.n_m3, wg = waves_per_group(n, 8);
+    const int n = p.n_m3, wg = waves_per_group(n, 16);
     if (n <= 0) return hipSuccess;
     auto go = [&](auto ker, int lds) {
         hipLaunchKernelGGL(ker, dim3((n + wg - 1) / wg), dim3(64 * wg), wg * lds, s, p.jobs, p.offs_m3,

@@ -154,9 +154,10 @@ void sgm_roi_from_disparity(const float* disp, int32_t width, int32_t height, sg
  *                        cost volume is built or read
  *   SGM_COST_STORED      always build and read the u8 cost volume
  *   SGM_COST_AUTO        on the fly when the plan also has enough scanlines
- *                        to fill the device (batches) or 250M cells and more
- *                        (tall images more), stored otherwise (small pairs
- *                        finish sooner that way)
+ *                        to fill the device (batches) or enough columns and
+ *                        rows side by side (470K and 230K over D, both views;
+ *                        plans of several sizes or D within further limits),
+ *                        stored otherwise (small pairs finish sooner that way)
  * Process-wide; read when a handle, batch or pyramid is created.  All give
  * byte-identical results. */
 #define SGM_COST_AUTO 0
@@ -191,10 +192,9 @@ int32_t sgm_get_window_form(void);
  *   SGM_WTA_SEPARATE  the four directions in one launch, then the WTA: the
  *                     short bottom->top walk runs beside the long horizontal
  *                     ones instead of after them
- *   SGM_WTA_AUTO      SEPARATE when the four-direction launch has at most
- *                     2.5 waves per SIMD (single pairs, where the scanline
- *                     walks set the time) and no matched image is more than
- *                     2.5 times as wide as it is high; FUSED otherwise
+ *   SGM_WTA_AUTO      SEPARATE below 3000 matched columns over all views at
+ *                     D = 64, 2400 at D = 128 and 1714 beyond (few columns
+ *                     walk bottom->top too slowly alone); FUSED otherwise
  * The on-the-fly kernels and the persistent batch schedules always fuse.
  * Process-wide, read when the launches are enqueued (a batch's HIP graph keeps
  * the form it was captured with).  All give byte-identical results. */

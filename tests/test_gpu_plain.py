@@ -422,6 +422,58 @@ def test_stored_mixed_batch(cuda, cost_mode, wta_form, form, ranges):
         _eq_float(p["disp_right"].cpu().numpy(), exp_r, "right map")
 
 
+# Which form SGM_COST_AUTO and SGM_WTA_AUTO take, seen in the stage times: without
+# a cost volume the cost stage is empty, and the separate WTA is a short stage of
+# its own where the fused one walks the columns.  One view or two, one pair far
+# larger than the rest, one D or several.
+def _stage_times(sets, lr, mode, form, cost_mode, wta_form, cuda):
+    from fasterstereocuda_amd.batch import SgmBatch
+    cost_mode(mode)
+    wta_form(form)
+    pairs = [{"left": torch.zeros((H, W), dtype=torch.uint8, device=cuda),
+              "right": torch.zeros((H, W), dtype=torch.uint8, device=cuda),
+              "disp_left": torch.empty((H, W), device=cuda), "min_disparity": 0, "disp_range": D}
+             for W, H, D in sets]
+    b = SgmBatch(pairs, CuSGMOption.benchmark(do_lr_check=lr))
+    b.run()
+    torch.cuda.synchronize()
+    b.set_timing(True)
+    for _ in range(5):
+        b.run()
+    torch.cuda.synchronize()
+    return b.stage_times()[0]
+
+
+@pytest.mark.parametrize("sets,lr,on_the_fly", [
+    ([(1500, 1500, 256)], False, False), ([(2500, 2500, 64)], False, False),
+    ([(2000, 2000, 256)], True, True), ([(1117, 573, 256)], True, True),
+    ([(1117, 573, 256)] * 3 + [(450, 375, 64)], False, True),
+    ([(2400, 1704, 256), (160, 120, 64)], True, True),
+    ([(1920, 1080, 256)] + [(1242, 375, 64)] * 2, True, False),
+    ([(1920, 1080, 128), (160, 120, 64)], True, False),
+    ([(5000, 500, 128)] + [(640, 480, 128)] * 3, True, False),
+])
+def test_auto_cost_form(cuda, cost_mode, wta_form, sets, lr, on_the_fly):
+    print(f"[auto cost] {sets} lr={lr}", flush=True)
+    args = (cost_mode, wta_form, cuda)
+    auto = _stage_times(sets, lr, 0, stages.WTA_AUTO, *args)["cost"]
+    stored = _stage_times(sets, lr, 1, stages.WTA_AUTO, *args)["cost"]
+    assert (auto < 0.25 * stored) == on_the_fly, f"cost stage {auto:.3f} ms, with a cost volume {stored:.3f} ms"
+
+
+@pytest.mark.parametrize("sets,lr,separate", [
+    ([(700, 700, 256), (160, 120, 64)], True, True), ([(500, 1000, 256), (160, 120, 64)], True, True),
+    ([(2000, 2000, 128)], False, True), ([(800, 800, 512)], True, True), ([(1242, 375, 64)], True, True),
+    ([(900, 1500, 256)], True, False), ([(2560, 1440, 64)], True, False),
+])
+def test_auto_wta_form(cuda, cost_mode, wta_form, sets, lr, separate):
+    print(f"[auto wta] {sets} lr={lr}", flush=True)
+    t = [_stage_times(sets, lr, 1, form, cost_mode, wta_form, cuda)["aggregate_wta"]
+         for form in (stages.WTA_AUTO, stages.WTA_FUSED, stages.WTA_SEPARATE)]
+    assert t[2] < 0.8 * t[1], f"the two forms' last stages {t[1]:.3f} and {t[2]:.3f} ms"
+    assert (abs(t[0] - t[2]) < abs(t[0] - t[1])) == separate, t
+
+
 def test_driving_full_size(cuda):
     pair = scenes.driving(0)
     print("[match] driving 1242x375", flush=True)
