@@ -528,9 +528,24 @@ hipError_t launch_by_d(const DsgmArgs& A, hipStream_t s) {
 //   600x196 (392) 1.23 -> 1.35
 //   D = 256: 4 images 9.82 -> 9.75; 8 images 600x375 (752) 9.81 -> 7.21, 600x150
 //   (304) 4.04 -> 4.45
+// With that many bands there also have to be 24M cells (28M at D = 64), or the
+// launches and the walks' ends weigh more than the traffic, unless the images are
+// tall, whose column walks the sweeps run once fewer (us: D = 64, 32 images 120x64,
+// 16M, 217 -> 290, 250x64, 33M, 600 -> 573; D = 128, 32 images 64x64, 17M, 236 -> 293,
+// 120x64, 31M, 579 -> 493; D = 256, 100 images 30x20, 15M, 237 -> 270, 64x20, 33M,
+// 638 -> 535; 16 images 30x128, D = 64 194 -> 175, 128 302 -> 257; 60 images 8x40,
+// D = 64 72 -> 69, but 100 images 8x20, D = 128 64 -> 73), and a last band of
+// few rows wastes the rest of its wave (width 1000, of 1, 5, 6, 7, 9, 13 rows: D = 64
+// 821 -> 1936, 1624 -> 2176, 1903 -> 2234, 2370 -> 2294, 2098 -> 2254, 2418 -> 2543;
+// D = 128 1439 -> 3409, 3262 -> 3872, 3804 -> 3915, 4616 -> 4009, 4220 -> 3974, 4611 ->
+// 4665; D = 256 2854 -> 6406, 6730 -> 7446, 7998 -> 7676, 9714 -> 7907, 8801 -> 7775,
+// 9476 -> 9546).
 // A band's cells stay below 2^30 bytes, so that 32-bit offsets and kNoPixel hold.
 bool dsgm_sweep_ok(const DsgmArgs& A) {
-    return (int64_t)A.B * ((A.H + 3) / 4) >= (A.D == 64 ? 450 : 390) && (int64_t)A.W * A.D <= (int64_t)1 << 26;
+    const int64_t bands = (A.H + 3) / 4, cells = (int64_t)A.B * A.H * A.W * A.D;
+    const bool tall = A.H >= 40 && 2 * (int64_t)A.H >= 5 * (int64_t)A.W;
+    return A.B * bands >= (A.D == 64 ? 450 : 390) && (tall || cells >= (A.D == 64 ? 28000000 : 24000000)) &&
+           100 * (int64_t)A.H >= (A.D == 64 ? 85 : 70) * 4 * bands && (int64_t)A.W * A.D <= (int64_t)1 << 26;
 }
 hipError_t dsgm_sweep_forward(const DsgmArgs& A, hipStream_t s) { return launch_by_d<false>(A, s); }
 hipError_t dsgm_sweep_backward(const DsgmArgs& A, hipStream_t s) { return launch_by_d<true>(A, s); }

@@ -91,6 +91,15 @@ def test_many_images_match_fp64(cuda, B, H, W, D):
             assert np.abs(g - ref).max() <= 1e-4 * np.abs(ref).max(), f"{name} max err"
 
 
+# the bands' form where it is taken: narrow images (last bands of 1 to 4 rows),
+# and wide ones from the number of cells on that it needs
+@pytest.mark.parametrize("B,H,W,D", [(41, 41, 16, 64), (41, 42, 5, 64), (41, 43, 2, 64), (45, 40, 1, 64),
+                                     (36, 41, 1, 128), (36, 42, 13, 128), (36, 44, 3, 128), (36, 43, 4, 256),
+                                     (36, 41, 9, 256), (130, 13, 112, 128), (98, 14, 70, 256), (90, 18, 271, 64)])
+def test_bands_match_fp64(cuda, B, H, W, D):
+    test_many_images_match_fp64(cuda, B, H, W, D)
+
+
 def test_deterministic_and_repeatable(cuda):
     cost, p1, p2, gt = _inputs(2, 40, 50, 64, seed=1)
     outs = []
