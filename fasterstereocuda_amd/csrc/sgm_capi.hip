@@ -94,8 +94,9 @@ int waves_per_group(int n, int limit) {
 // the matched columns over all views, so those decide, whatever the shape; the
 // longer a D's step, the fewer columns (separate / fused, us, LR check on unless
 // given; columns):
-//   D = 64: 2500 1500x3000 off 903 / 1233, 2400 1200x852 405 / 429, 3000 1500x3000
-//   1598 / 1657, 3000 3000x3000 off 1683 / 1674, 3840 1920x1080 759 / 717
+//   D = 64: 1500 1500x3000 off 903 / 1233, 2400 1200x852 405 / 429, 3000 1500x3000
+//   1598 / 1657, 3000 3000x3000 off 1683 / 1674, 3000 1500x200 (a pyramid's
+//   coarsest level, whole pyramid) 584 / 600, 3840 1920x1080 759 / 717
 //   D = 128: 1600 800x800 425 / 498, 1920 1920x1080 off 696 / 732, 2000 2000x2000
 //   off 1294 / 1379, 2400 1200x1000 798 / 784, 2484 1242x375 416 / 336, 2560
 //   1280x720 621 / 612
@@ -107,8 +108,9 @@ bool separate_wta(const StagePlan& p) {
     const int f = g_wta_form.load();
     if (f == SGM_WTA_FUSED) return false;
     if (f == SGM_WTA_SEPARATE) return true;
-    return p.work.walk < 12000;
+    return p.work.walk <= 60000;
 }
+
 bool choose_wide(bool eligible, int n_wh) {
     const int mode = cost_mode();
     if (!eligible || mode == SGM_COST_STORED) return false;
@@ -152,7 +154,7 @@ void PlanWork::add(const SgmJob& j) {
     most = std::max(most, c);
     col_bytes += cols * j.D;
     row_bytes += (int64_t)j.H * j.D;
-    walk += cols * (j.D <= 64 ? 4 : j.D <= 128 ? 5 : 7);   // 12000: 3000, 2400, 1714 columns
+    walk += cols * (j.D <= 64 ? 20 : j.D <= 128 ? 26 : 35);   // 60000: 3000, 2307, 1714 columns
     waves += n;
     if (j.D == 256) waves256 += n;
     dmin = std::min(dmin, j.D);

@@ -192,8 +192,8 @@ int32_t sgm_get_window_form(void);
  *   SGM_WTA_SEPARATE  the four directions in one launch, then the WTA: the
  *                     short bottom->top walk runs beside the long horizontal
  *                     ones instead of after them
- *   SGM_WTA_AUTO      SEPARATE below 3000 matched columns over all views at
- *                     D = 64, 2400 at D = 128 and 1714 beyond (few columns
+ *   SGM_WTA_AUTO      SEPARATE up to 3000 matched columns over all views at
+ *                     D = 64, 2307 at D = 128 and 1714 beyond (few columns
  *                     walk bottom->top too slowly alone); FUSED otherwise
  * The on-the-fly kernels and the persistent batch schedules always fuse.
  * Process-wide, read when the launches are enqueued (a batch's HIP graph keeps
