@@ -20,8 +20,8 @@
 // end.  A map is mostly a few large segments, so one union per pixel edge and
 // one count per pixel all land on the same few roots (640x359 pixels: 390 us
 // of unions and 1070 us of counts, against 5-20 us a pass of the map); with
-// tiles, device memory sees one union per run of crossing edges (an 80th part
-// of the pixels at most) and one count per tile and component.
+// tiles, device memory sees one union per run of crossing edges (of edges, a
+// 13th part of the pixels) and one count per tile and component.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -72,14 +72,6 @@ int wide_min_groups() {
     return v;
 }
 
-unsigned spread_lds(int n, int used) {
-    constexpr int kLds = 160 * 1024, kUnit = 1280;   // per CU; allocation granule
-    const int cus = wide_min_groups() / 8;
-    const int want = std::max(4, (n + cus - 1) / cus);   // one per SIMD at least
-    const int bytes = kLds / want / kUnit * kUnit;
-    return bytes > used ? (unsigned)(bytes - used) : 0u;
-}
-
 int waves_per_group(int n, int limit) {
     const int simds = wide_min_groups() / 2;   // 4 per CU
     return 2 * n > simds && 4 * n <= limit * simds ? 4 : 1;

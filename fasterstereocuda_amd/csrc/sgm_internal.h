@@ -103,16 +103,17 @@ inline int wide_v_items(const SgmJob& j, int kind) {
     const int l = wide_lines(kind, j.D);
     return (j.W - j.roi_x + l - 1) / l;
 }
-// Whether a job's cost can come from the census on the fly: D <= 256, and not
-// the 5x5 right view, whose skipped-pixel rule needs the stored cost.
 // Penalties whose sums leave the positive finite f16 patterns (below 0x7C00):
 // the aggregation then takes integer minima.
 inline bool big_penalties(const SgmJob& j) { return (int64_t)j.p1 + j.p2 > 30000; }
 // Steps of the longest block of the stored-cost walk (agg_lines), and whether
-// that many rows pass 31 bits of bytes.  (Persistent schedules take sides up to
-// 65532, which never do.)
+// that many rows pass 31 bits of bytes: its steps then have 64-bit addresses.
+// (Persistent schedules take sides up to 65532, which never do.)  1120003x19
+// D = 128: 143 ms, with 64-bit addresses in all kernels 204 ms.
 __host__ __device__ constexpr int agg_block(int D) { return D <= 128 ? 16 : 2048 / D; }
 inline bool far_steps(const SgmJob& j) { return (int64_t)agg_block(j.D) * j.W * j.D > INT32_MAX; }
+// Whether a job's cost can come from the census on the fly: D <= 256, and not
+// the 5x5 right view, whose skipped-pixel rule needs the stored cost.
 inline bool wide_ok(const SgmJob& j) { return j.D <= 256 && !(j.is_right && j.cs_type == 0); }
 
 // Their 4-line form (sgm_mid.hip) for plans too small to fill the GPU that
@@ -188,7 +189,7 @@ struct StagePlan {
     int n_census = 0, n_cost = 0, n_agg = 0, n_wta = 0, n_post = 0, n_agg3 = 0, n_dw = 0;
     int n_wh = 0, n_wv = 0, n_wf = 0, n_m3 = 0, n_mf = 0;
     PlanWork work;                // of the matched jobs
-    int dmax = 64, dmin = 64;     // over all jobs; dmin over the matched ones
+    int dmax = 64, dmin = 64;     // over all jobs; equal: the kernels for one D do them all
     bool wide = false;            // matching uses the on-the-fly cost kernels
     bool mid = false;             // unless scheduled, it uses their 4-line form
     bool quirk = false;           // some matched job is a 5x5 right view
@@ -221,13 +222,6 @@ hipError_t launch_aggregate_wta_sched(const StagePlan& p, const AggSchedule& sc,
 // Resident 64-lane workgroups per compute unit of the persistent kernels.
 hipError_t persistent_occupancy(const StagePlan& p, int* per_cu);
 hipError_t launch_reset_counters(uint32_t* counters, int n, hipStream_t s);
-// Dynamic LDS (bytes) for a launch of n single-wave workgroups that spreads
-// them evenly: the dispatcher fills a compute unit up to its occupancy before
-// the waves are even (3072 waves that fit 16 to a CU ran on 192 CUs, a third
-// slower than 12 to each of 256), so a grid that fits at once is held to
-// ceil(n / CUs) workgroups per CU by the LDS each one claims.  `used` is the
-// kernel's static LDS.
-unsigned spread_lds(int n, int used);
 // Waves per workgroup of a launch of n scanline groups (one wave each): 4 from
 // half a wave per SIMD up to `limit` quarters of one, else 1.  A workgroup's waves go to
 // different SIMDs, while single-wave workgroups are placed unevenly: with few

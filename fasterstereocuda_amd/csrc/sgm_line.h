@@ -68,7 +68,6 @@ __device__ __forceinline__ uint32_t from_next(uint32_t v, uint32_t edge, bool la
     }
 }
 
-__device__ __forceinline__ uint32_t popc64(uint64_t a) { return (uint32_t)__popcll(a); }
 // popcount(a) + acc as two accumulating v_bcnt_u32_b32.  Written out, the
 // compiler regroups the sum and packs with a v_lshl_or_b32; this form packs
 // the upper count with a v_lshlrev_b32, which issues at twice the rate.

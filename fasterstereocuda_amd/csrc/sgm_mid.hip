@@ -8,7 +8,7 @@
 //   * census rows are padded with the word of column 0 (what a partner column
 //     outside the image reads; column 0 is a border pixel, so the word is a
 //     constant written once): no clamps.  A vertical step's partner words go
-//     through an LDS slot private to the single-wave workgroup, loaded PF steps
+//     through an LDS slot private to the wave, loaded PF steps
 //     ahead, and are read back a step ahead;
 //   * buffer accesses with a scalar offset per step; volumes are plain
 //     [H][W][D] (32-bit offsets, see mid_ok), only their words' byte order is
@@ -35,9 +35,6 @@ namespace fsgm {
 namespace {
 
 using namespace dev;
-
-constexpr uint32_t kMidSelFwd = 0x06020400u;   // bytes d, d + 2, d + 1, d + 3
-constexpr uint32_t kMidSelRev = 0x04000602u;   // the pairs' halves swapped (reversed lanes)
 
 // N consecutive census words (N a multiple of 4) in ascending address order
 template <int N>
@@ -76,7 +73,7 @@ __device__ __forceinline__ void mid_horizontal(const SgmJob& J, int path, int gr
     const int a = right ? (rev ? min_d + D - 1 : min_d) : (rev ? -min_d - (D - 1) : -min_d);
     const int st = (right != rev) ? 1 : -1;
     const uint32_t P1v = (uint32_t)J.p1 * 0x10001u, P2v = (uint32_t)J.p2 * 0x10001u;
-    const uint32_t sel = rev ? kMidSelRev : kMidSelFwd;
+    const uint32_t sel = rev ? kSelRev : kSelFwd;
     // census words: scalar row of the group's first line + the lane's rest
     const auto own_r = rows_of(J, J.census), oth_r = rows_of(J, J.census_other);
     const int rowb = J.cpitch * 8, srow = line0 * rowb;
@@ -329,7 +326,7 @@ __device__ __forceinline__ void mid_vertical(const SgmJob& J, const MidColumns& 
         line_init<BIG, 16>(s, c);
         if constexpr (!FUSE) {
             uint32_t o[NW];
-            pack_lane(s, kMidSelFwd, o);
+            pack_lane(s, kSelFwd, o);
             buf_store<NW>(ud_r, vvol, y0 * W * D, o);
         } else {
             // row H - 1 is a border row of the WTA
@@ -417,7 +414,7 @@ __device__ __forceinline__ void mid_vertical(const SgmJob& J, const MidColumns& 
             line_step<BIG, 16>(s, c, P1v, P2v, false, false);
             if constexpr (!FUSE) {
                 uint32_t o[NW];
-                pack_lane(s, kMidSelFwd, o);
+                pack_lane(s, kSelFwd, o);
                 if (full.value || i0 + b < H) buf_store<NW>(ud_r, vvol, st, o);
                 st += rowv;
             } else {

@@ -209,7 +209,6 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
     const int64_t ostep = dy * (int64_t)W * D;
     uint8_t* const out_base = FUSE ? J.path[kDU] : J.path[kUD];
 
-    // census words staged for step i: lane loads v = lane + 64 r
     // the other three directions' bytes of step i (FUSE): top->bottom by rows,
     // the horizontal pair in the row tiles of the horizontal kernel, one of
     // them (left->right of the right view, right->left of the left view) with
@@ -227,6 +226,7 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
         load_words<NW>(src_fwd + to + tv, w[1]);
         load_words<NW>(src_rev + to + tr, w[2]);
     };
+    // census words staged for step i: lane loads v = lane + 64 r
     auto load_step = [&](int i, uint64_t (&g)[NR]) __attribute__((always_inline)) {
         const int y = y0 + dy * min(i, H - 1);
         const uint64_t* cb = J.census + (int64_t)y * J.cpitch;
@@ -382,10 +382,8 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
             if (active && first) gst(J.disp + (int64_t)y0 * W + x, kInvalidDisp);
         }
     }
-    // row offsets of step i (stores) and of the refill step min(i + PF, H - 1)
-    // (loads), advanced by scalar adds: no 64-bit multiply per access
-    int64_t row_i = ubase + ostep, row_f = ubase + (int64_t)(1 + PF) * ostep;
-    const int64_t row_last = ubase + (int64_t)(H - 1) * ostep;
+    // row offset of step i's store, advanced by a scalar add
+    int64_t row_i = ubase + ostep;
     for (int i0 = 1; i0 < H; i0 += BLK) {
 #pragma unroll
         for (int b = 0; b < BLK; ++b) {
@@ -413,7 +411,6 @@ __device__ __forceinline__ void wide_vertical(const SgmJob& J, int group, int la
                 load_others(i + PF, pr[p]);
             }
             row_i += ostep;
-            row_f += ostep;
         }
         if constexpr (FUSE) wta_flush(i0);
     }
@@ -479,14 +476,13 @@ template <int DMAX, bool BIG>
 __global__ __launch_bounds__(64) void wide_h_persistent(const SgmJob* __restrict__ jobs,
                                                         const uint32_t* __restrict__ items, int n,
                                                         uint32_t* __restrict__ counter) {
-    constexpr bool ONLY = false;
     uint32_t it;
     while (next_item(items, n, counter, &it)) {
         const SgmJob& J = jobs[it >> 16];
         const int path = (int)((it >> 14) & 3u), group = (int)(it & 0x3FFFu);
         switch (J.D) {
-            case 64: if constexpr (!ONLY || DMAX == 64) wide_horizontal<64, BIG>(J, path, group, threadIdx.x); break;
-            case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_horizontal<128, BIG>(J, path, group, threadIdx.x); break;
+            case 64: wide_horizontal<64, BIG>(J, path, group, threadIdx.x); break;
+            case 128: if constexpr (DMAX >= 128) wide_horizontal<128, BIG>(J, path, group, threadIdx.x); break;
             case 256: if constexpr (DMAX >= 256) wide_horizontal<256, BIG>(J, path, group, threadIdx.x); break;
             default: break;
         }
@@ -497,7 +493,6 @@ template <int DMAX, bool FUSE, bool BIG>
 __global__ __launch_bounds__(64) void wide_v_persistent(const SgmJob* __restrict__ jobs,
                                                         const uint32_t* __restrict__ items, int n,
                                                         uint32_t* __restrict__ counter) {
-    constexpr bool ONLY = false;
     __shared__ uint64_t lds[2 * VertLds<DMAX, FUSE ? kWideF : kWideV>::NV];
     __shared__ __align__(16) uint16_t sums[FUSE ? kSumsLen<DMAX> : 1];
     uint32_t it;
@@ -505,8 +500,8 @@ __global__ __launch_bounds__(64) void wide_v_persistent(const SgmJob* __restrict
         const SgmJob& J = jobs[it >> 16];
         const int group = (int)(it & 0x3FFFu);
         switch (J.D) {
-            case 64: if constexpr (!ONLY || DMAX == 64) wide_vertical<64, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
-            case 128: if constexpr (ONLY ? DMAX == 128 : DMAX >= 128) wide_vertical<128, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+            case 64: wide_vertical<64, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
+            case 128: if constexpr (DMAX >= 128) wide_vertical<128, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
             case 256: if constexpr (DMAX >= 256) wide_vertical<256, FUSE, BIG>(J, group, threadIdx.x, lds, sums); break;
             default: break;
         }
