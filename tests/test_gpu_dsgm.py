@@ -100,6 +100,46 @@ def test_bands_match_fp64(cuda, B, H, W, D):
     test_many_images_match_fp64(cuda, B, H, W, D)
 
 
+# Rows whose pairs pass 2^32 bytes: the separate passes' 64-bit offsets.  A stretch
+# of columns is cut off by penalties P2 < 0 on both sides of its ends: the last term
+# then wins everywhere, L = C + P2, and nothing is handed across.  So the stretch
+# equals its own columns alone, up to a constant in S at its ends (and the penalty
+# gradients there).  Costs and penalties are multiples of 1/64, so L and S are exact
+# and the disparities equal; a gradient is a sum of the same four terms in another
+# order, within 4 roundings of terms not much above the largest.
+def test_very_long_rows(cuda):
+    H, W, D, n = 2, 3000001, 256, 64
+    print(f"[dsgm long rows] {W}x{H} D{D}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(5)
+
+    def ints(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, dtype=torch.uint8, device=cuda, generator=g).to(torch.float32).div_(64)
+
+    cost = ints(0, 64, 1, H, W, D).requires_grad_(True)
+    p1, p2, gd = ints(4, 16, 1, H, W), ints(32, 128, 1, H, W), ints(0, 64, 1, H, W) - 0.5
+    starts = [0, W // 4, W // 2, W - n - 1234567 // 2, W - n]
+    for a in starts:
+        for x in (a - 1, a, a + n - 1, a + n):
+            if 0 <= x < W:
+                p2[:, :, x] = -1 / 64
+    p1.requires_grad_(True)
+    p2.requires_grad_(True)
+    disp = diff_sgm(cost, p1, p2, T)
+    disp.backward(gd)
+    for a in starts:
+        cut = slice(a, a + n)
+        args = [x.detach()[:, :, cut].contiguous().requires_grad_(True) for x in (cost, p1, p2)]
+        part = diff_sgm(*args, T)
+        part.backward(gd[:, :, cut].contiguous())
+        np.testing.assert_array_equal(disp.detach()[:, :, cut].cpu().numpy(), part.detach().cpu().numpy(),
+                                      err_msg=f"disparity from column {a}")
+        for name, x, y in zip(("dC", "dP1", "dP2"), (cost, p1, p2), args):
+            got, ref = x.grad[:, :, cut].cpu().numpy(), y.grad.cpu().numpy()
+            if name != "dC":
+                got, ref = got[:, :, 1:-1], ref[:, :, 1:-1]
+            assert np.abs(ref).max() > 0 and np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max(), f"{name} from {a}"
+
+
 def test_deterministic_and_repeatable(cuda):
     cost, p1, p2, gt = _inputs(2, 40, 50, 64, seed=1)
     outs = []

@@ -320,6 +320,40 @@ def test_on_the_fly_mixed_batch(cuda, cost_mode, cs, p1, p2):
         _eq_float(p["disp_right"].cpu().numpy(), exp_r, "right map")
 
 
+# the 4-line form and the stored cost on a batch that fills the device: D = 256
+# beside larger pairs, whole images, several runs
+def test_on_the_fly_mixed_batch_under_load(cuda, cost_mode):
+    from fasterstereocuda_amd.batch import SgmBatch
+    sizes = [(1920, 1080, 128), (1242, 375, 64), (640, 360, 256)]
+    print(f"[otf mixed, load] {sizes}", flush=True)
+    rng = np.random.default_rng(9)
+    imgs = []
+    for W, H, _ in sizes:
+        right = rng.integers(0, 256, (H, W), dtype=np.uint8)
+        imgs.append([torch.from_numpy(np.ascontiguousarray(x)).to(cuda) for x in (np.roll(right, 23, axis=1), right)])
+
+    def run(mode, reps):
+        cost_mode(mode)
+        pairs = [{"left": l, "right": r, "disp_left": torch.empty((H, W), device=cuda),
+                  "disp_right": torch.empty((H, W), device=cuda), "min_disparity": 0, "disp_range": D}
+                 for (W, H, D), (l, r) in zip(sizes, imgs)]
+        b = SgmBatch(pairs, CuSGMOption.benchmark(do_median_filter=False))
+        out = []
+        for _ in range(reps):
+            b.run()
+            torch.cuda.synchronize()
+            out.append([p[k].cpu().numpy() for p in pairs for k in ("disp_left", "disp_right")])
+        return out
+
+    ref = run(1, 1)[0]
+    for (W, H, D), m in zip(sizes, ref[::2]):
+        inside = m[5:H - 5, D:W - 5]
+        assert (inside != oracle.INVALID).mean() > 0.9
+    for got in run(2, 4):
+        for k, (x, y) in enumerate(zip(got, ref)):
+            _eq_float(x, y, f"pair {k // 2}, {'right' if k % 2 else 'left'} map")
+
+
 @pytest.fixture
 def wta_form():
     before = stages.get_wta_form()
