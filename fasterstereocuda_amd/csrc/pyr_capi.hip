@@ -166,7 +166,14 @@ sgm_pyramid* build_pyramid(int32_t width, int32_t height, int32_t num_layers, in
     p->top_min = dmin; p->top_range = range;
     // memory
     const bool lr = opt->do_lr_check != 0;
-    const int pad = mid_pad(range, dmin);   // of the coarsest level's census rows
+    // pad words of the coarsest level's census rows
+    std::vector<SgmJob> views(lr ? 2 : 1);
+    for (size_t v = 0; v < views.size(); ++v) {
+        SgmJob& j = views[v];
+        j.W = p->lw[top]; j.H = p->lh[top]; j.D = range; j.roi_x = std::max(0, dmin);
+        j.is_right = (int)v; j.cs_type = opt->cs_type;
+    }
+    const int pad = wants_pads(views) ? mid_pad(range, dmin) : 0;
     size_t total = 0;
     for (int i = 0; i < layers; ++i) {
         const size_t npix = (size_t)p->lw[i] * p->lh[i];
@@ -212,12 +219,6 @@ sgm_pyramid* build_pyramid(int32_t width, int32_t height, int32_t num_layers, in
                                   v ? p->cl[top] : p->cr[top], w, h, opt->cs_type, v);
             j.D = range; j.min_d = dmin; j.roi_x = std::max(0, dmin);
             j.cpitch = w + 2 * pad; j.cpad = pad;
-            if (pad > 0 && (fill_census_pads(j, p->stream) != hipSuccess ||
-                            hipStreamSynchronize(p->stream) != hipSuccess)) {
-                set_global_error(SGM_E_HIP, "pyramid: census pads");
-                free_pyramid(p);
-                return nullptr;
-            }
             j.p1 = opt->p1; j.p2 = opt->p2_init;
             j.uniqueness = (top > 0) ? 1.0f : opt->unique_threshold;
             if (v == 0 || lr) {

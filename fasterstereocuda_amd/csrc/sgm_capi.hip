@@ -139,6 +139,17 @@ bool choose_mid(bool eligible, int n_wh, const PlanWork& w) {
     if (w.least != w.most && w.waves > 2 * wide_min_groups()) return false;
     return w.col_bytes >= 470000 && w.row_bytes >= 230000;
 }
+bool wants_pads(const std::vector<SgmJob>& views) {
+    PlanWork w;
+    bool ok = true;
+    int64_t groups = 0;
+    for (const SgmJob& j : views) {
+        ok = ok && j.D <= 256;
+        groups += j.D <= 256 ? wide_h_items(j) : 0;
+        w.add(j);
+    }
+    return choose_mid(ok, (int)std::min<int64_t>(groups, INT32_MAX), w);
+}
 void PlanWork::add(const SgmJob& j) {
     const int64_t cols = j.W - j.roi_x, n = mid3_items(j), c = cols * j.H * j.D;
     cells += c;
@@ -615,15 +626,20 @@ int sgm_init(sgm_handle* h, int32_t width, int32_t height, int32_t min_disparity
     h->opt = *opt;
     h->print_log = print_log != 0;
     HIP_TRY(&h->err, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-    h->cpad = h->window ? 0 : mid_pad(disp_range, min_disparity);
+    h->cpad = 0;
+    if (!h->window) {
+        // as for every column matched: a later offset may match more than this one
+        std::vector<SgmJob> views(opt->do_lr_check ? 2 : 1);
+        for (size_t v = 0; v < views.size(); ++v) {
+            SgmJob& j = views[v];
+            j.W = width; j.H = height; j.D = disp_range; j.is_right = (int)v; j.cs_type = opt->cs_type;
+        }
+        if (wants_pads(views)) h->cpad = mid_pad(disp_range, min_disparity);
+    }
     HIP_TRY(&h->err, hipMalloc(&h->arena, arena_bytes(width, height, disp_range, h->cpad)));
     if (opt->do_remove_peaks)
         HIP_TRY(&h->err, hipMalloc(&h->peaks, 2 * (size_t)width * height * sizeof(int)));
     carve(h);
-    if (h->cpad > 0) {
-        for (int v = 0; v < 2; ++v) HIP_TRY(&h->err, fill_census_pads(make_job(h, v), h->stream));
-        HIP_TRY(&h->err, hipStreamSynchronize(h->stream));
-    }
     if (int rc = build_handle_plan(h)) return rc;
     h->inited = true;
     if (h->print_log)
@@ -1039,14 +1055,17 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
         return nullptr;
     }
     const bool lr = opt->do_lr_check != 0;
-    // census rows are padded where the batch may take the 4-line form
-    int groups = 0;
-    for (int i = 0; i < n; ++i) {
-        SgmJob j{};
-        j.H = pairs[i].height; j.D = pairs[i].disp_range;
-        groups += j.D <= 256 ? (lr ? 2 : 1) * wide_h_items(j) : 0;
-    }
-    const bool padded = groups < wide_min_groups();
+    // census rows are padded where the batch takes the 4-line form
+    std::vector<SgmJob> views;
+    for (int i = 0; i < n; ++i)
+        for (int v = 0; v < (lr ? 2 : 1); ++v) {
+            SgmJob j{};
+            j.W = pairs[i].width; j.H = pairs[i].height; j.D = pairs[i].disp_range;
+            j.roi_x = std::max(0, pairs[i].min_disparity);
+            j.is_right = v; j.cs_type = opt->cs_type;
+            views.push_back(j);
+        }
+    const bool padded = wants_pads(views);
     auto pad_of = [&](const sgm_pair_desc& p) {
         return padded ? mid_pad(p.disp_range, p.min_disparity) : 0;
     };
@@ -1112,17 +1131,6 @@ sgm_batch* sgm_batch_create(const sgm_pair_desc* pairs, int32_t n, const sgm_opt
     }
     std::vector<SgmJob> jobs = left_jobs;
     jobs.insert(jobs.end(), right_jobs.begin(), right_jobs.end());
-    if (padded) {
-        hipError_t e = hipSuccess;
-        for (const SgmJob& j : jobs)
-            if (j.cpad > 0 && e == hipSuccess) e = fill_census_pads(j, nullptr);
-        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        if (e != hipSuccess) {
-            fail(nullptr, SGM_E_HIP, std::string("census pads: ") + hipGetErrorString(e));
-            free_batch(b);
-            return nullptr;
-        }
-    }
     if (upload_plan(jobs, posts, &b->plan, &b->plan_block, &b->err)) {
         g_last_error = b->err;
         free_batch(b);

@@ -239,10 +239,9 @@ hipError_t launch_wide_wta_sched(const StagePlan& p, const AggSchedule& sc, hipS
 // direction volumes as the launches above leave them (kUD, kLR, kRL) to plain ones
 hipError_t launch_wide_export(const SgmJob& j, const uint8_t* const (&src)[4],
                               uint8_t* const (&dst)[4], hipStream_t s);
-// sgm_mid.hip: the 4-line form; fill_census_pads writes a job's pad words
+// sgm_mid.hip: the 4-line form
 hipError_t launch_mid3(const StagePlan& p, hipStream_t s);
 hipError_t launch_mid_wta(const StagePlan& p, hipStream_t s);
-hipError_t fill_census_pads(const SgmJob& j, hipStream_t s);
 hipError_t wide_occupancy(const StagePlan& p, int* per_cu);
 // Process-wide SGM_COST_* mode, read when a plan is built; choose_wide
 // applies it to a plan whose views all allow the on-the-fly cost
@@ -252,6 +251,9 @@ int cost_mode();
 // (`eligible` by mid_ok).
 bool choose_wide(bool eligible, int n_wh);
 bool choose_mid(bool eligible, int n_wh, const PlanWork& w);
+// Whether a plan of these views (W, H, D, roi_x, is_right, cs_type set) would take it
+// if their census rows were padded.
+bool wants_pads(const std::vector<SgmJob>& views);
 int wide_min_groups();
 hipError_t launch_wta(const StagePlan& p, hipStream_t s);
 hipError_t launch_post(const StagePlan& p, hipStream_t s);

@@ -161,6 +161,18 @@ __global__ __launch_bounds__(128) void census_kernel(const SgmJob* __restrict__ 
             gst(J.census + (int64_t)y * J.cpitch + x, border ? invalid : v[rr][h]);
         }
     }
+    // the pad words of the tile's rows: column 0's word, a border pixel's, eight
+    // threads to a row (127 words a side of 1920x1080 23.7 -> 25.2 us, 255 of 1117x573
+    // 10.1 -> 12.3 us)
+    if (J.cpad > 0) {
+        const int y = y0 + (tid >> 3);
+        if (y < J.H)
+            for (int c = tid & 7; c < J.cpad; c += 8) {
+                uint64_t* const row = J.census + (int64_t)y * J.cpitch;
+                if (x0 == 0) gst(row - J.cpad + c, invalid);
+                if (x0 + 64 >= J.W) gst(row + J.W + c, invalid);
+            }
+    }
 }
 
 // ------------------------------------------------------------------ cost ---

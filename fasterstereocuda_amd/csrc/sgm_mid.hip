@@ -7,7 +7,7 @@
 // short: about one wave per SIMD, a step costs its instruction count.  Hence:
 //   * census rows are padded with the word of column 0 (what a partner column
 //     outside the image reads; column 0 is a border pixel, so the word is a
-//     constant written once): no clamps.  A vertical step's partner words go
+//     constant, which the census kernel writes): no clamps.  A vertical step's partner words go
 //     through an LDS slot private to the wave, loaded PF steps
 //     ahead, and are read back a step ahead;
 //   * buffer accesses with a scalar offset per step; volumes are plain
@@ -494,17 +494,6 @@ __global__ __launch_bounds__(256) void mid_wta_kernel(const SgmJob* __restrict__
     }
 }
 
-// The pad words of every census row: the border constant of column 0.
-__global__ __launch_bounds__(256) void census_pads_kernel(uint64_t* census, int W, int H, int pitch,
-                                                          int pad, uint64_t word) {
-    const int64_t n = (int64_t)2 * pad * H;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const int64_t y = i / (2 * pad);
-        const int k = (int)(i - y * 2 * pad);
-        census[y * pitch + (k < pad ? k - pad : W + k - pad)] = word;
-    }
-}
-
 }  // namespace
 
 hipError_t launch_mid3(const StagePlan& p, hipStream_t s) {
@@ -536,15 +525,6 @@ hipError_t launch_mid_wta(const StagePlan& p, hipStream_t s) {
     else if (p.dmax == 64) p.quirk ? go(mid_wta_kernel<64, false, true, true>, l64) : go(mid_wta_kernel<64, false, true, false>, l64);
     else if (p.dmax == 128) p.quirk ? go(mid_wta_kernel<128, false, true, true>, l128) : go(mid_wta_kernel<128, false, true, false>, l128);
     else p.quirk ? go(mid_wta_kernel<256, false, true, true>, l256) : go(mid_wta_kernel<256, false, true, false>, l256);
-    return hipGetLastError();
-}
-
-hipError_t fill_census_pads(const SgmJob& j, hipStream_t s) {
-    const int64_t n = (int64_t)2 * j.cpad * j.H;
-    if (n <= 0) return hipSuccess;
-    const unsigned blocks = (unsigned)std::min<int64_t>((n + 255) / 256, 65535);
-    hipLaunchKernelGGL(census_pads_kernel, dim3(blocks), dim3(256), 0, s, j.census, j.W, j.H,
-                       j.cpitch, j.cpad, j.is_right ? 0xFFFFFFFFull : 0ull);
     return hipGetLastError();
 }
 

@@ -289,3 +289,21 @@ def test_autotune_picks_and_remembers(cuda):
     b2.run()
     for g, r in zip(_outputs(pairs2), ref):
         np.testing.assert_array_equal(g, r)
+
+
+# census rows are padded (and written padded) only where the plan takes the 4-line
+# form; the arena shows it: two census maps of a pair, and per view cost, four
+# direction volumes and the raw map, each rounded up to 256 bytes
+@pytest.mark.parametrize("n,w,h,d,pad", [(8, 450, 375, 64, 0), (16, 160, 120, 64, 0), (1, 1242, 375, 64, 0),
+                                         (1, 1920, 1080, 128, 127), (1, 640, 480, 512, 0)])
+def test_census_pads_only_where_they_are_read(cuda, n, w, h, d, pad):
+    print(f"[pads] {n} x {w}x{h} D{d}", flush=True)
+    img = torch.zeros((h, w), dtype=torch.uint8, device=cuda)
+    pairs = [{"left": img, "right": img, "disp_left": torch.empty((h, w), device=cuda), "min_disparity": 0,
+              "disp_range": d} for _ in range(n)]
+    b = SgmBatch(pairs, CuSGMOption.benchmark())
+
+    def up(x):
+        return (x + 255) // 256 * 256
+    census = up(8 * ((w + 2 * pad) * h + (384 if pad else 0)))
+    assert b.device_bytes == n * (2 * census + 2 * (5 * up(w * h * d) + up(4 * w * h)))
