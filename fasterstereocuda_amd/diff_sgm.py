@@ -9,8 +9,11 @@ buffers with torch's caching allocator and passes the current stream.  The
 forward saves S (the 4-direction sum) and, per direction, the winning term of
 every cell (2 bits) and each pixel's argmin byte, about a quarter of one
 volume; no per-direction volume is kept.  Each call's transient workspace is
-one direction volume plus two per-pixel planes.  The torch-free C++ API never
-depends on this module.
+one direction volume plus two per-pixel planes.  The FP32 sum over the four
+directions is taken in one of three orders, chosen by the shape [B, H, W, D]
+(sgm_capi.h lists them): a call repeats bit for bit, but an image's last bits
+may depend on the batch it is in.  The torch-free C++ API never depends on this
+module.
 """
 from __future__ import annotations
 

@@ -154,8 +154,8 @@ WTA_AUTO, WTA_FUSED, WTA_SEPARATE = 0, 1, 2
 def set_wta_form(form: int) -> None:
     """How the stored-cost aggregation reaches the WTA: bottom->top fused
     with it after the other three directions, or the four directions in one
-    launch and then the WTA, or AUTO (separate for single pairs); process-wide,
-    read when the launches are enqueued.  Results are byte-identical."""
+    launch and then the WTA, or AUTO (separate for plans of few columns);
+    process-wide, read when the launches are enqueued.  Results are byte-identical."""
     check(lib().sgm_set_wta_form(int(form)))
 
 

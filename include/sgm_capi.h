@@ -259,7 +259,8 @@ void sgm_batch_destroy(sgm_batch* b);
  *                            groups from a device queue, pair by pair
  *   SGM_SCHED_LONGEST_FIRST  persistent, queue sorted by work (scanline length
  *                            x disparity range), longest first
- * waves = 0 picks occupancy x compute units.  Results are identical under
+ * waves = 0 picks occupancy x compute units (stored cost with D >= 256: at most
+ * one wave per SIMD).  Results are identical under
  * every schedule; only the order in which scanline groups run changes. */
 #define SGM_SCHED_GRID 0
 #define SGM_SCHED_JOB_MAJOR 1
@@ -290,7 +291,14 @@ int sgm_batch_use_graph(sgm_batch* b, int32_t on);
  * and the argmin of the previous step per pixel (1 byte), plus two floats
  * per pixel; about a quarter of one volume, and no per-direction volume.
  * The transient workspace (d_work, shared by forward and backward) is one
- * direction volume plus two per-pixel planes. */
+ * direction volume plus two per-pixel planes.
+ * B, H, W and D choose between three forms that sum the directions in FP32 in
+ * different orders (L1 left->right, L3 right->left, L0 top->bottom, L2
+ * bottom->top): ((L1 + L3) + L0) + L2 with one pass per direction,
+ * (L1 + L0) + (L3 + L2) in bands of rows, (L1 + L3) + (L0 + L2) where all
+ * directions share a launch; the gradients of the cost and the penalties
+ * likewise.  A call's forward and backward take the same form and repeat bit
+ * for bit, but an image's last bits may depend on the batch it is in. */
 size_t sgm_dsgm_checkpoint_floats(int32_t B, int32_t H, int32_t W, int32_t D);
 size_t sgm_dsgm_workspace_floats(int32_t B, int32_t H, int32_t W, int32_t D);
 int sgm_dsgm_forward(const float* d_cost, const float* d_p1, const float* d_p2, int32_t B,
@@ -379,7 +387,9 @@ int sgm_stage_aggregate(const uint8_t* d_cost, int32_t width, int32_t height,
  * d_paths[0] (top->bottom), d_paths[1] (left->right), d_paths[3]
  * (right->left) and the raw disparity map; d_paths[2] is not written (the
  * fused pass keeps bottom->top in registers) and may be NULL.  D <= 256,
- * not the 5x5 right view (SGM_E_UNSUPPORTED). */
+ * not the 5x5 right view (SGM_E_UNSUPPORTED).  For inspection: the kernels'
+ * own volumes keep another byte order, so the call allocates three for its
+ * length and copies them out in order. */
 int sgm_stage_aggregate_wta_otf(const uint64_t* d_census_base, const uint64_t* d_census_match,
                                 int32_t width, int32_t height, int32_t min_disparity,
                                 int32_t disp_range, int32_t is_right, int32_t cs_type, int32_t p1,
